@@ -27,6 +27,7 @@
 // (src/hip/kernel/moeKernel.h:37-107) and its TILE_M=1 GEMV tiles
 // (src/hip/kernel/tasks/internal/gemmImpl/basicGemmTileImpl.h:14-94).
 #include <type_traits>
+#include <utility>
 
 #define FMOE_PARAMS_IN_KERNARG 1
 #include "moe_device.h"
@@ -156,11 +157,6 @@ __device__ __forceinline__ void wg_broadcast_flag(ParamsRef p, int which) {
 // ------------------------------------------------- direct-to-LDS load helpers
 #define FMOE_G1 __attribute__((address_space(1)))
 #define FMOE_L3 __attribute__((address_space(3)))
-
-__device__ __forceinline__ f32x16 mma32(const uint4& a, const uint4& b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
 
 // wait until at most N of this wave's vector-memory operations are outstanding
 // (they complete in order); nothing else is waited for
@@ -468,12 +464,16 @@ __device__ void tiled_scatter_task(ParamsRef p, int blk) {
 // instructions, almost no vector-ALU work in the loop.
 //
 // One wave per SIMD, each with 64 weight rows x all token rows of the tile:
-// acc[2][JT] blocks of 32x32. The first 8 token blocks' accumulators fill the
+// acc[4][2*JT] blocks of 16x16. The first 16 token blocks' accumulators fill the
 // 256 accumulator registers a[0:255]; a tile of 257..320 rows (JT 9, 10) keeps
-// the last blocks' in v[...]. Per 16 k a wave reads 2 weight and JT token
-// fragments (16 bytes per lane each) for 2*JT matrix instructions. A tile's
-// time follows its rows down to about 160; below that the 32 load round trips
-// of its k-loop set it.
+// the last blocks' in v[...]. Per 32 k a wave reads 4 weight and 2*JT token
+// fragments (16 bytes per lane each) for 8*JT matrix instructions.
+//
+// Why 16x16x32 and not 32x32x16: at the board's power cap the smaller instruction
+// delivers more. Back to back on all CUs with normally distributed operands in
+// registers: 32x32x16 1717 TFLOP/s at 1.74 GHz, 16x16x32 1919 TFLOP/s at 1.99 GHz
+// (2478 and 2407 on 8 CUs, where the clock stays at 2.4 GHz). Per multiply-add it
+// reads twice the operand registers but moves half the accumulators.
 //
 // LDS stage layout: rows of 128 bytes, unpadded, weight rows 0..255 then token
 // rows. Row R keeps its eight 16-byte chunks permuted: chunk C sits at position
@@ -487,31 +487,43 @@ __device__ void tiled_scatter_task(ParamsRef p, int blk) {
 // chose the vector-register form of the instruction, which cannot reach a[...]).
 // The first instruction of every accumulator takes the constant 0 as its
 // addend, so nothing zeroes them.
+typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
+constexpr int JB_MAX = 2 * JT_MAX;  // 16-row token blocks of the tallest tile
+constexpr int JB_ACC = 16;          // of these, the ones whose accumulators are in a[...]
+
+// 16 bytes of LDS at a byte address. The k-loops address LDS by number: the dynamic block's
+// base is looked up in memory wherever its name is used inside a function that is not inlined,
+// and a scalar load in the loop makes every LDS read in flight be waited for.
+__device__ __forceinline__ v4u_t lds_read16(unsigned addr) {
+  return *(const FMOE_L3 v4u_t*)addr;
+}
+
 template <bool INIT, bool IN_V>
-__device__ __forceinline__ void mma32(const uint4& a, const uint4& b, f32x16& c) {
-  typedef unsigned v4u __attribute__((ext_vector_type(4)));
-  const v4u av = {a.x, a.y, a.z, a.w}, bv = {b.x, b.y, b.z, b.w};
+__device__ __forceinline__ void mma(const v4u_t& a, const v4u_t& b, f32x4& c) {
   if (IN_V) {
     if (INIT) {
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=v"(c) : "v"(av), "v"(bv));
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=v"(c) : "v"(a), "v"(b));
     } else {
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(av), "v"(bv));
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
     }
   } else {
     if (INIT) {
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(av), "v"(bv));
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
     } else {
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(av), "v"(bv));
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     }
   }
 }
 
-constexpr int ntl_of(int jt) { return jt > 8 ? 10 : 8; }            // 8-row token loads per wave and stage
-constexpr int stage_bytes_of(int jt) { return (TN + 4 * 8 * ntl_of(jt)) * ROWB; }
-constexpr int TILE_LDS_BYTES = 2 * stage_bytes_of(JT_MAX);          // 147456
-// behind the stages: the tile's destination rows and gate weights for the down epilogue
+constexpr int stage_bytes_of(int jt) { return (TN + 32 * jt) * ROWB; }
+// Stages of the LDS-staged pipeline: three where they fit. The tiles of a batch of some 40 to
+// 160 rows an expert are bound by how much of the weights is in flight, taller ones are not.
+constexpr int nst_of(int jt) { return jt <= 5 ? 3 : 2; }
+constexpr int TILE_LDS_BYTES = 3 * stage_bytes_of(5);               // 159744
+static_assert(TILE_LDS_BYTES >= 2 * stage_bytes_of(JT_MAX), "stages");
+// behind the stages: the tile's destination rows for the down epilogue
 constexpr int SIDE_OFF = TILE_LDS_BYTES;
-constexpr int SIDE_BYTES = TM_MAX * 8;
+constexpr int SIDE_BYTES = TM_MAX * 4;
 // and behind those one 16-byte line of words a GEMM task leaves for the worker loop: the ticket it
 // drew for the workgroup's next task. They live in
 // the dynamic block because a file-scope LDS variable written from a function that is not
@@ -541,90 +553,81 @@ __device__ __forceinline__ unsigned stage_chunk_bytes(int row) {
   return static_cast<unsigned>(((threadIdx.x & 7) ^ ((row >> 1) & 7)) << 4);
 }
 
-struct Frag {
-  uint4 a[2];
-  uint4 b[JT_MAX];
-};
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_(f, std::make_integer_sequence<int, N>{});
+}
 
-// acc[i][j] = W-block i (32 of this wave's 64 weight rows) x token-block j, j < JT, over
-// nstages * 64 k (nstages >= 2). Token rows from 32*JT on are neither loaded nor multiplied.
+// A stage is NSL = 4*JT slots, two sub-steps (32 k each) of 2*JT: slot n multiplies token
+// block n % (2*JT) of its sub-step with the wave's four weight blocks, four instructions of
+// 16 cycles. The token fragments pass through a ring of registers: a slot's fragment is
+// replaced, as soon as its instructions have been issued, by the one RING slots later, so
+// every LDS read has RING * 64 cycles to return. RING divides the slots of a stage.
+constexpr int ring_of(int jt) { return jt == 2 ? 4 : jt == 3 ? 6 : jt == 5 ? 5 : jt == 7 ? 7 : jt == 9 ? 6 : 8; }
+
+// acc[i][j] = weight block i (16 of this wave's 64 weight rows) x token block j (16 rows),
+// j < 2*JT, over nstages * 64 k (nstages >= 2). Token rows from 32*JT on are neither loaded
+// nor multiplied.
 //
-// A stage is 4 sub-steps of 16 k; a sub-step is NS = max(8, JT) slots; a slot is one pair of
-// matrix instructions and, behind it, the LDS reads and global loads the schedule puts there:
-//  * the fragments of sub-step u+1 are read under sub-step u, one token block per slot
-//  * hand-over in sub-step 3 after BAR pairs: this wave's reads of stage s have returned and
-//    its loads of stage s+1 have landed, then the workgroup barrier; from there on the next
-//    stage's first fragments are read and the loads of stage s+2 go out into the buffer just
-//    left, one per slot, the rest under the next stage's first sub-steps. (Measured on all
-//    256 CUs: all 16 loads behind the barrier at once, barrier in front of the sub-step: 51 us
-//    per 256x256x2048 tile; this schedule: 48 us.)
+// Hand-over between stages BAR slots after the last fragment of stage s has been asked for:
+// this wave's reads of stage s have returned and its loads of stage s+1 have landed, then
+// the workgroup barrier; from there on the next stage's first fragments are read and the
+// loads of stage s+NST go out into the buffer just left, LPS per slot, the rest under the next
+// stage's first slots. (With the 32x32 form of this loop, on all 256 CUs: all 16 loads behind
+// the barrier at once, barrier in front of the sub-step: 51 us per 256x256x2048 tile; spread
+// out: 48 us.)
 //
 // Bookkeeping rides along: at the first hand-over (every memory operation this wave issued
 // before it, the previous task's stores included, has completed there anyway) thread 0
 // signals the previous task's completion on `pend` (if any) and draws the workgroup's next
 // ticket from `queue` into `next`, so neither trip to memory is waited for between tasks.
 template <int JT, typename AfterFirstLoads>
-__device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f32x16 (&acc)[2][JT_MAX],
+__device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f32x4 (&acc)[4][JB_MAX],
                                           unsigned* pend, unsigned* queue, unsigned& next,
                                           AfterFirstLoads after_first_loads) {
   const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
-  const int r32 = lane & 31, kq = lane >> 5;
+  const int r16 = lane & 15, kg = lane >> 4;
   const unsigned lds_addr = uni(static_cast<unsigned>(
       reinterpret_cast<size_t>((FMOE_L3 unsigned char*)lds_raw)));
-  constexpr int TROWS = 32 * JT;
-  constexpr int NTL = ntl_of(JT);
-  constexpr int STG = stage_bytes_of(JT);
-  constexpr int NS = JT > 8 ? JT : 8;  // slots per sub-step
-  constexpr int NRD = 2 + JT;          // fragment reads per sub-step
-  constexpr int BAR = 2;               // pairs of sub-step 3 in front of the hand-over
-  constexpr int AFTER = NS - BAR;      // slots of sub-step 3 behind it
-  constexpr int RPS = (NRD + AFTER - 1) / AFTER;  // reads of the next stage's first fragments per slot there
+  constexpr int STG = stage_bytes_of(JT), NST = nst_of(JT);
+  constexpr int JB = 2 * JT, NSL = 2 * JB, RING = ring_of(JT);
+  constexpr int BAR = 2;                                     // slots between the last read of a stage and the hand-over
+  constexpr int HO = NSL - RING + BAR;                       // the slot the hand-over stands in front of
+  constexpr int AFTER = NSL - HO;                            // slots behind it
+  constexpr int NL = NLD + JT;                               // loads per wave and stage
+  constexpr int LPS = (NL + AFTER + JB - 1) / (AFTER + JB);  // loads per slot
+  constexpr int APS = (4 + AFTER - 1) / AFTER;               // weight fragments of the next stage read per slot behind the hand-over
+  static_assert(NSL % RING == 0 && RING > BAR && JB >= 4 && RING <= JB && HO >= JB, "slot schedule");
+  static_assert(NST * STG <= TILE_LDS_BYTES, "stages exceed the tile's LDS");
 
-  int fo[4];  // per-lane fragment offsets of the four 16-k sub-steps
+  unsigned fo[2];  // per-lane token fragment offsets of the two 32-k sub-steps
 #pragma unroll
-  for (int u = 0; u < 4; ++u) fo[u] = r32 * ROWB + (((2 * u + kq) ^ ((r32 >> 1) & 7)) << 4);
-
-  auto issue_one = [&](int s, int q) {  // q: 0..7 weights, 8..8+NTL-1 tokens
-    const unsigned st = uni(static_cast<int>(lds_addr + (s & 1) * STG));
-    if (q < NLD) {
-      load_to_lds(op.woff[q], op.wbase + static_cast<size_t>(s) * op.wstride, st + (wave * 64 + q * 8) * ROWB);
-    } else if (q < NLD + NTL) {
-      const int qq = q - NLD;
-      if ((NTL == 8 && JT == 8) || (wave * NTL + qq) * 8 < TROWS)
-        load_to_lds(op.toff[qq], op.tbase + static_cast<size_t>(s) * ROWB,
-                    st + TN * ROWB + ((wave * NTL + qq) * 8) * ROWB);
-    }
-  };
+  for (int u = 0; u < 2; ++u) fo[u] = lds_addr + r16 * ROWB + (((4 * u + kg) ^ ((r16 >> 1) & 7)) << 4);
   // weight fragments: from row-major stage rows as the token fragments, or, when the wave's
   // weight rows keep the packed order (eight runs [k-step 0..1][block 0..3] of [chunk][row]),
-  // row r32 of 32-row block i = row r32 % 16 of run block 2i + r32 / 16, chunk 2*(u % 2) + kq
-  // of k-step u / 2
-  int ao[4];
+  // 16 bytes per lane of the run of k-step u, block i
+  unsigned ao[2];
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
-    ao[u] = op.wpacked ? ((u >> 1) * 4 + (r32 >> 4)) * 1024 + (((2 * (u & 1) + kq) * 16 + (r32 & 15)) << 4)
-                       : fo[u];
-  const int ablock = uni(op.wpacked ? 2048 : 32 * ROWB);  // bytes from weight block 0 to block 1
-  auto read_n = [&](Frag& f, int s, int u, int r) {  // r-th of the NRD reads of a sub-step
-    const unsigned char* st = lds_raw + (s & 1) * STG + fo[u];
-    if (r < 2) {
-      f.a[r] = *reinterpret_cast<const uint4*>(lds_raw + (s & 1) * STG + wave * (64 * ROWB) + r * ablock + ao[u]);
-    } else if (r < NRD) {
-      f.b[r - 2] = *reinterpret_cast<const uint4*>(st + TN * ROWB + ((r - 2) * 32) * ROWB);
+  for (int u = 0; u < 2; ++u) ao[u] = wave * (64 * ROWB) + (op.wpacked ? lds_addr + u * 4096 + lane * 16 : fo[u]);
+  const int ablock = uni(op.wpacked ? 1024 : 16 * ROWB);  // bytes from one weight block to the next
+
+  auto issue_one = [&](int s, int buf, int q) {  // q: 0..7 weights, 8..8+JT-1 tokens; buf: the stage buffer's byte offset
+    const unsigned st = uni(static_cast<int>(lds_addr) + buf);
+    if (q < NLD) {
+      load_to_lds(op.woff[q], op.wbase + static_cast<size_t>(s) * op.wstride, st + (wave * 64 + q * 8) * ROWB);
+    } else if (q < NL) {
+      const int qq = q - NLD;
+      load_to_lds(op.toff[qq], op.tbase + static_cast<size_t>(s) * ROWB, st + TN * ROWB + ((wave * JT + qq) * 8) * ROWB);
     }
   };
-  auto pair = [&](auto init_tag, const Frag& cur, int j) {
-    constexpr bool INIT = decltype(init_tag)::value;
-    if (j < JT) {
-      if (j < 8) {
-        mma32<INIT, false>(cur.a[0], cur.b[j], acc[0][j]);
-        mma32<INIT, false>(cur.a[1], cur.b[j], acc[1][j]);
-      } else {
-        mma32<INIT, true>(cur.a[0], cur.b[j], acc[0][j]);
-        mma32<INIT, true>(cur.a[1], cur.b[j], acc[1][j]);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
+  auto read_a = [&](int buf, int u, int i) { return lds_read16(ao[u] + static_cast<unsigned>(buf + i * ablock)); };
+  auto read_b = [&](int buf, int n) {  // the fragment of slot n
+    return lds_read16(fo[n / JB] + static_cast<unsigned>(buf + TN * ROWB + (n % JB) * (16 * ROWB)));
   };
 
   auto bookkeeping = [&]() {
@@ -634,87 +637,104 @@ __device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f
     }
   };
 
-  Frag f0, f1;
+  v4u_t af[2][4], ring[RING];
 #pragma unroll
-  for (int q = 0; q < NLD + NTL; ++q) issue_one(0, q);
+  for (int st = 0; st < NST; ++st) {
+    if (st < 2 || nstages > st) {
 #pragma unroll
-  for (int q = 0; q < NLD + NTL; ++q) issue_one(1, q);
+      for (int q = 0; q < NL; ++q) issue_one(st, st * STG, q);
+    }
+  }
   // Loads to registers that the task still needs go out here, behind the loads to LDS: a
   // load to registers that is still on its way when a younger load to LDS is issued may not
   // deliver its data (seen with 16-byte loads; the register kept its old content). Every
-  // later load to LDS follows a wait for all outstanding loads.
+  // later load to LDS follows a wait for all outstanding loads to registers.
   after_first_loads();
   // stage 0 has landed, then everybody's. (The wait is for everything this wave has asked
-  // for, stage 1 and the loads to registers included: the two kinds of load are not counted
-  // in order with each other, so a count that leaves stage 1 in flight would not say that
-  // stage 0 is in.)
+  // for, the later stages and the loads to registers included: the two kinds of load are not
+  // counted in order with each other, so a count that leaves stage 1 in flight would not say
+  // that stage 0 is in.)
   wait_vm<0>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 #pragma unroll
-  for (int r = 0; r < NRD; ++r) read_n(f0, 0, 0, r);
+  for (int i = 0; i < 4; ++i) af[0][i] = read_a(0, 0, i);
+#pragma unroll
+  for (int n = 0; n < RING; ++n) ring[n] = read_b(0, n);
 
-  auto stage = [&](int s, auto first_tag, auto early_tag, auto late_tag, auto next_tag) {
-    constexpr bool EARLY = decltype(early_tag)::value;  // the tail of stage s+1's loads is still to go out
-    constexpr bool LATE = decltype(late_tag)::value;    // stage s+2 exists
-    constexpr bool NEXT = decltype(next_tag)::value;    // stage s+1 exists
-    using No = std::false_type;
+  // One stage. R: stages after it, NST meaning NST or more. cur, nxt, prv: byte offsets of the
+  // buffers of this stage, the next one and the last one (with two buffers the latter are one).
+  int cur = 0, nxt = STG, prv = (NST - 1) * STG;
+  auto stage = [&](int s, auto first_tag, auto rem_tag) {
+    constexpr bool FIRST = decltype(first_tag)::value;
+    constexpr int R = decltype(rem_tag)::value;
+    constexpr bool EARLY = !FIRST && R >= NST - 1;  // the tail of stage s+NST-1's loads is still to go out
+    constexpr bool LATE = R >= NST;                 // stage s+NST exists
+    constexpr bool NEXT = R >= 1;                   // stage s+1 exists
+    // loads of the stages behind the next one, which may still be in flight at the hand-over
+    constexpr int YOUNGER = NST == 3 && R >= 2 ? NL : 0;
 #pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      const Frag& cur = (u & 1) ? f1 : f0;
-      Frag& nxt = (u & 1) ? f0 : f1;
-#pragma unroll
-      for (int j = 0; j < NS; ++j) {
-        if (u == 0) {
-          pair(first_tag, cur, j);
-        } else {
-          pair(No{}, cur, j);
-        }
-        if (EARLY) issue_one(s + 1, AFTER + NS * u + j);
-        if (j == 0) {
-          read_n(nxt, s, u + 1, 0);
-          read_n(nxt, s, u + 1, 1);
-        }
-        read_n(nxt, s, u + 1, 2 + j);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NS; ++j) {
-      if (j == BAR) {
+    for (int n = 0; n < NSL; ++n) {
+      const int u = n / JB, j = n % JB;
+      if (n == HO && NEXT) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (NEXT) {
-          wait_vm<0>();
-          __builtin_amdgcn_s_barrier();
-          asm volatile("" ::: "memory");
-          if (decltype(first_tag)::value) bookkeeping();
-        }
+        wait_vm<YOUNGER>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (FIRST) bookkeeping();
       }
-      pair(No{}, f1, j);
-      if (j >= BAR) {
-        if (LATE) issue_one(s + 2, j - BAR);
-        if (NEXT) {
 #pragma unroll
-          for (int r = (j - BAR) * RPS; r < (j - BAR + 1) * RPS; ++r) read_n(f0, s + 1, 0, r);
+      for (int i = 0; i < 4; ++i) {
+        if (FIRST && u == 0) {
+          if (j < JB_ACC) mma<true, false>(af[u][i], ring[n % RING], acc[i][j]); else mma<true, true>(af[u][i], ring[n % RING], acc[i][j]);
+        } else {
+          if (j < JB_ACC) mma<false, false>(af[u][i], ring[n % RING], acc[i][j]); else mma<false, true>(af[u][i], ring[n % RING], acc[i][j]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
+      if (n + RING < NSL) ring[n % RING] = read_b(cur, n + RING);
+      if (n < 4) af[1][n] = read_a(cur, 1, n);
+      if (NEXT && n >= HO) {
+        if (n == HO) {
+#pragma unroll
+          for (int m = 0; m < BAR; ++m) ring[(NSL - RING + m) % RING] = read_b(nxt, m);
+        }
+        ring[n % RING] = read_b(nxt, n - (NSL - RING));
+#pragma unroll
+        for (int i = (n - HO) * APS; i < (n - HO + 1) * APS; ++i)
+          if (i < 4) af[0][i] = read_a(nxt, 0, i);
+      }
+#pragma unroll
+      for (int l = 0; l < LPS; ++l) {
+        if (EARLY && n < HO) issue_one(s + NST - 1, prv, (AFTER + n) * LPS + l);
+        if (LATE && n >= HO) issue_one(s + NST, cur, (n - HO) * LPS + l);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
+    prv = cur;
+    cur = nxt;
+    nxt = uni(nxt == (NST - 1) * STG ? 0 : nxt + STG);
   };
   using Yes = std::true_type;
   using No = std::false_type;
-  if (nstages > 2) {
-    stage(0, Yes{}, No{}, Yes{}, Yes{});
+  using Full = std::integral_constant<int, NST>;
+  if (nstages > NST) {
+    stage(0, Yes{}, Full{});
+  } else if (NST == 3 && nstages == 3) {
+    stage(0, Yes{}, std::integral_constant<int, 2>{});
   } else {
-    stage(0, Yes{}, No{}, No{}, Yes{});
+    stage(0, Yes{}, std::integral_constant<int, 1>{});
   }
   int s = 1;
-  for (; s + 2 < nstages; ++s) stage(s, No{}, Yes{}, Yes{}, Yes{});
-  if (s + 1 < nstages) {
-    stage(s, No{}, Yes{}, No{}, Yes{});
-    ++s;
-  }
-  stage(s, No{}, No{}, No{}, No{});
+  for (; s + NST < nstages; ++s) stage(s, No{}, Full{});
+  static_for<NST - 1>([&](auto i) {
+    constexpr int r = NST - 1 - decltype(i)::value;  // stages after the next one to run
+    if (s + r < nstages) {
+      stage(s, No{}, std::integral_constant<int, r>{});
+      ++s;
+    }
+  });
+  stage(s, No{}, std::integral_constant<int, 0>{});
   // the compiler does not see matrix instructions in the assembly above: keep the wait states
   // between the last of them and the first read of an accumulator
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -725,18 +745,17 @@ __device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f
 // keeps its depth in registers instead of LDS.
 //
 // A wave's 64 weight rows are its own: no other wave reads them. So they do not go through
-// LDS at all: every fragment (32 rows x 16 k, 16 bytes per lane) is one global load straight
-// into the registers the matrix instruction reads, four 256-byte segments of the packed runs
-// per instruction. Two register sets: the fragments of stage s+2 are requested into the
-// registers of stage s as soon as its sub-step is through, two stages (about 2 us) before
-// they are needed. The token rows, which all four waves read, still meet in LDS, but they
-// travel global -> registers -> LDS (ds_write_b128) instead of straight to LDS: a wave
-// requests its JT loads of 8 rows of stage s+3 during stage s, into the registers whose
-// previous content (stage s+1) it has just written to LDS. Two LDS buffers of 4 KiB per
-// 32-row block, written one stage before they are read. Half the LDS traffic of the version
-// above is gone (no weight rows written, no weight fragments read), the hand-over between
-// two stages waits for LDS only (this wave's writes of stage s+1 and reads of stage s, then
-// the workgroup barrier), and every global load has 1.75 to 2 stages to arrive.
+// LDS at all: every fragment (16 rows x 32 k, 16 bytes per lane) is one global load straight
+// into the registers the matrix instruction reads, one whole 1 KiB run of the packed layout
+// per instruction. D register sets: the fragments of stage s+D are requested into the
+// registers of stage s as soon as its sub-step is through. The token rows, which all four
+// waves read, still meet in LDS, but they travel global -> registers -> LDS (ds_write_b128)
+// instead of straight to LDS: a wave requests its JT loads of 8 rows of stage s+D+1 during
+// stage s, into the registers whose previous content (stage s+1) it has just written to LDS.
+// Three LDS buffers of 4 KiB per 32-row block, written one stage before they are read: the
+// buffer a wave writes during stage s was last read in stage s-2, and the workgroup barrier
+// of stage s-1 lies between, so a hand-over waits for nothing but this wave's writes of the
+// next stage (long done) and the slowest wave.
 //
 // Loads straight to LDS are not used here on purpose: a load to registers that was still
 // outstanding when a younger load-to-LDS was issued did not deliver its data (the register
@@ -746,18 +765,24 @@ __device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f
 // issues the same loads in the same order. direct_wait() counts them from the list of what
 // a stage issues (which also covers the last stages, where loads of stages that do not exist
 // are left out):
-//   sub-step 0: weights (s+1, sub-step 3); sub-step 1: weights (s+2, sub-step 0), then the
-//   token rows of stage s+3; sub-step 2, 3: weights (s+2, sub-step 1, 2).
-// The loads in front of the loop are issued in the same order, as if by stages -2 and -1.
-constexpr int DIRECT_GROUPS = 5;
+//   sub-step 0: weights (s+D-1, sub-step 1), then the token rows of stage s+D+1;
+//   sub-step 1: weights (s+D, sub-step 0).
+// The loads in front of the loop are issued in the same order, as if by stages -D ... -1.
+constexpr int DIRECT_GROUPS = 3;
 constexpr int DIRECT_JT_MAX = 8;     // taller tiles do not leave the registers for it
-constexpr int DIRECT_MIN_STAGES = 4;
+// Register sets. Short tiles have few accumulators and are bound by the weights' way from
+// memory: four sets. Two are enough for tall ones, whose stages last 2000 cycles.
+constexpr int direct_depth(int jt) { return jt <= 2 ? 4 : 2; }
+constexpr bool direct_takes(int jt, int nstages) {
+  return jt <= DIRECT_JT_MAX && nstages % direct_depth(jt) == 0 && nstages >= 2 * direct_depth(jt);
+}
 // Loads that group g (in issue order) of a stage with r stages after it puts out.
 constexpr int direct_group(int jt, int r, int g) {
+  const int d = direct_depth(jt);
   switch (g) {
-    case 0: return r >= 1 ? 2 : 0;
-    case 2: return r >= 3 ? jt : 0;
-    default: return r >= 2 ? 2 : 0;
+    case 0: return r >= d - 1 ? 4 : 0;
+    case 1: return r >= d + 1 ? jt : 0;
+    default: return r >= d ? 4 : 0;
   }
 }
 // Loads issued after group g0 of the stage `back` stages before the present one (which has
@@ -775,206 +800,179 @@ constexpr int direct_in_flight(int jt, int r, int back, int g0, int g1) {
 // wait in front of sub-step w of a stage with r stages after it: its weight fragments and,
 // for sub-step 0, the token rows of the next stage, which that sub-step writes to LDS
 constexpr int direct_wait(int jt, int r, int w) {
-  switch (w) {
-    case 0: return direct_in_flight(jt, r, 2, 2, 0);
-    case 1: return direct_in_flight(jt, r, 2, 3, 1);
-    case 2: return direct_in_flight(jt, r, 2, 4, 3);
-    default: return direct_in_flight(jt, r, 1, 0, 4);
-  }
+  const int d = direct_depth(jt);
+  return w == 0 ? direct_in_flight(jt, r, d, 2, 0) : direct_in_flight(jt, r, d - 1, 0, 1);
 }
+static_assert(direct_wait(2, 5, 0) < 64 && direct_wait(8, 3, 0) < 64, "vmcnt holds 6 bits");
 
-typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
-
-template <bool INIT>
-__device__ __forceinline__ void mma32v(const v4u_t& av, const uint4& b, f32x16& c) {
-  const v4u_t bv = {b.x, b.y, b.z, b.w};
-  if (INIT) {
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(av), "v"(bv));
-  } else {
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(av), "v"(bv));
-  }
-}
-
-// 16 bytes per lane from base + off into the registers of `dst`; completion is tracked by
-// hand (wait_vm), so the compiler must not believe it knows when the value is there: the
+// 16 bytes per lane from base + off + OFF into the registers of `dst`; completion is tracked
+// by hand (wait_vm), so the compiler must not believe it knows when the value is there: the
 // operand is read-write, which keeps the value in one place from the load to its last use.
+template <int OFF>
 __device__ __forceinline__ void load_fragment(v4u_t& dst, unsigned off, const unsigned char* base) {
-  asm volatile("global_load_dwordx4 %0, %1, %2" : "+v"(dst) : "v"(off), "s"(base) : "memory");
+  asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "+v"(dst) : "v"(off), "s"(base), "n"(OFF) : "memory");
 }
-// 16 bytes per lane from registers to LDS (byte address `lds_off`)
+// 16 bytes per lane from registers to LDS (byte address `lds_off` + OFF)
+template <int OFF>
 __device__ __forceinline__ void store_fragment(unsigned lds_off, const v4u_t& src) {
-  asm volatile("ds_write_b128 %0, %1" : : "v"(lds_off), "v"(src) : "memory");
+  asm volatile("ds_write_b128 %0, %1 offset:%2" : : "v"(lds_off), "v"(src), "n"(OFF) : "memory");
 }
-
+template <int N>
+__device__ __forceinline__ void wait_lds() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" : : "n"(N) : "memory");
+}
 template <int JT>
-__device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nstages, f32x16 (&acc)[2][JT_MAX],
+__device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nstages, f32x4 (&acc)[4][JB_MAX],
                                                  unsigned* pend, unsigned* queue, unsigned& next) {
   static_assert(JT <= DIRECT_JT_MAX, "tile too tall for the register-staged pipeline");
-  constexpr int NS = 8;                           // slots per sub-step
-  constexpr int BAR = 2;                          // pairs of sub-step 3 in front of the hand-over
-  constexpr int AFTER = NS - BAR;
+  constexpr int JB = 2 * JT, NSL = 2 * JB, RING = ring_of(JT);
+  constexpr int HO = NSL - RING;                  // the slot the hand-over stands in front of
   constexpr int STG = 32 * JT * ROWB;             // token rows of one stage
-  constexpr int RPS = (JT + AFTER - 1) / AFTER;   // reads of the next stage's first fragments per slot behind the hand-over
-  static_assert(2 * STG <= TILE_LDS_BYTES, "token stages exceed the tile's LDS");
+  // LDS operations a wave issues between its last write of the next stage (slot JT - 1) and the hand-over
+  constexpr int LDS_YOUNGER = HO - (JT - 1) < 15 ? HO - (JT - 1) : 15;
+  static_assert(3 * STG <= TILE_LDS_BYTES, "token stages exceed the tile's LDS");
+  static_assert(NSL % RING == 0 && HO >= JT && JB >= 4, "slot schedule");
   const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
-  const int r32 = lane & 31, kq = lane >> 5;
+  const int r16 = lane & 15, kg = lane >> 4;
   const unsigned lds_addr = uni(static_cast<unsigned>(
       reinterpret_cast<size_t>((FMOE_L3 unsigned char*)lds_raw)));
 
-  int fo[4];  // per-lane token fragment offsets of the four 16-k sub-steps
+  unsigned fo[2];  // per-lane token fragment offsets of the two 32-k sub-steps
 #pragma unroll
-  for (int u = 0; u < 4; ++u) fo[u] = r32 * ROWB + (((2 * u + kq) ^ ((r32 >> 1) & 7)) << 4);
-  // weight fragment (sub-step u, 32-row block i) of stage s in the wave's packed slice:
-  // 8192*s + 4096*(u/2) + 2048*i + 512*(u%2), plus this lane's part
-  const unsigned aoff = static_cast<unsigned>(((r32 >> 4) << 10) + (kq << 8) + ((r32 & 15) << 4));
+  for (int u = 0; u < 2; ++u) fo[u] = lds_addr + r16 * ROWB + (((4 * u + kg) ^ ((r16 >> 1) & 7)) << 4);
+  // weight fragment (sub-step u, block i) of stage s in the wave's packed slice: the run at
+  // 8192*s + 4096*u + 1024*i, 16 bytes per lane
+  const unsigned aoff = static_cast<unsigned>(lane) * 16u;
   // where this lane's 16 bytes of the wave's token load q belong in a stage buffer: the
   // eight rows of load q are one run of 1 KiB, lane l at 16*l
   const unsigned wr_off = lds_addr + static_cast<unsigned>((wave * JT) * 1024 + lane * 16);
 
-  v4u_t as[2][4][2];   // weight fragments: [stage parity][sub-step][block]
-  v4u_t bs[2][JT];     // token rows on their way to LDS: [stage parity][load]
+  constexpr int D = direct_depth(JT);
+  v4u_t as[D][2][4];   // weight fragments: [stage % D][sub-step][block]
+  v4u_t bs[D][JT];     // token rows on their way to LDS: [stage % D][load]
+  v4u_t ring[RING];
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
+  for (int p = 0; p < D; ++p) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) as[p][u][i] = v4u_t{0u, 0u, 0u, 0u};
+      for (int i = 0; i < 4; ++i) as[p][u][i] = v4u_t{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int q = 0; q < JT; ++q) bs[p][q] = v4u_t{0u, 0u, 0u, 0u};
   }
-  uint4 bf[2][JT_MAX];
+#pragma unroll
+  for (int n = 0; n < RING; ++n) ring[n] = v4u_t{0u, 0u, 0u, 0u};
 
-  auto issue_a = [&](int s, int u, int i, v4u_t& dst) {
-    load_fragment(dst, aoff, op.wbase + static_cast<size_t>(s) * 8192 + ((u >> 1) * 4096 + i * 2048 + (u & 1) * 512));
+  auto issue_a = [&](int s, int u, auto i_tag, v4u_t& dst) {
+    load_fragment<decltype(i_tag)::value * 1024>(dst, aoff, op.wbase + static_cast<size_t>(s) * 8192 + u * 4096);
   };
   auto issue_b = [&](int s, int q, v4u_t& dst) {  // q-th token load of this wave for stage s
-    load_fragment(dst, op.toff[q], op.tbase + static_cast<size_t>(s) * ROWB);
+    load_fragment<0>(dst, op.toff[q], op.tbase + static_cast<size_t>(s) * ROWB);
   };
-  auto write_b = [&](int buf, int q, const v4u_t& src) { store_fragment(wr_off + buf * STG + q * 1024, src); };
-  auto read_b = [&](int buf, int u, int j) {
-    return *reinterpret_cast<const uint4*>(
-        __builtin_assume_aligned(lds_raw + buf * STG + fo[u] + j * (32 * ROWB), 16));
-  };
-  auto pair = [&](auto init_tag, const v4u_t (&a)[2], const uint4 (&b)[JT_MAX], int j) {
-    constexpr bool INIT = decltype(init_tag)::value;
-    if (j < JT) {
-      mma32v<INIT>(a[0], b[j], acc[0][j]);
-      mma32v<INIT>(a[1], b[j], acc[1][j]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
+  // the fragment of token block j; `base`: this lane's address in the stage buffer and sub-step
+  auto read_b = [&](unsigned base, int j) { return lds_read16(base + static_cast<unsigned>(j * (16 * ROWB))); };
 
-  // ---- in front of the loop. First what stage 0 needs at once: its token rows, its weight
-  // fragments, and the token rows of stage 1 (which stage 0 writes to LDS).
+  // ---- in front of the loop. First what stage 0 needs at once: its token rows (through the
+  // ring's registers, idle until then), its weight fragments, and the token rows of stage 1
+  // (which stage 0 writes to LDS); then what the stages -D+1 ... -1 would have issued.
+  static_assert(JT <= RING, "stage 0's token rows pass through the ring's registers");
 #pragma unroll
-  for (int q = 0; q < JT; ++q) issue_b(0, q, bs[0][q]);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) issue_a(0, 0, i, as[0][0][i]);
+  for (int q = 0; q < JT; ++q) issue_b(0, q, ring[q]);
+  static_for<4>([&](auto i) { issue_a(0, 0, i, as[0][0][i]); });
 #pragma unroll
   for (int q = 0; q < JT; ++q) issue_b(1, q, bs[1][q]);
+  static_for<4>([&](auto i) { issue_a(0, 1, i, as[0][1][i]); });
 #pragma unroll
-  for (int u = 1; u < 4; ++u)
+  for (int b = 1; b < D; ++b) {
+    if (b > 1) static_for<4>([&](auto i) { issue_a(b - 1, 1, i, as[b - 1][1][i]); });
 #pragma unroll
-    for (int i = 0; i < 2; ++i) issue_a(0, u, i, as[0][u][i]);
-  // Everything requested so far has landed, and so have the stores of the previous task's
-  // epilogue (loads and stores do not complete in order with each other, so only a wait for
-  // all of them covers the stores): behind the workgroup barrier thread 0 may signal that
-  // task's completion, and draws the ticket of the task after this one.
-  wait_vm<0>();
-#pragma unroll
-  for (int q = 0; q < JT; ++q) write_b(0, q, bs[0][q]);
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    for (int q = 0; q < JT; ++q) issue_b(b + 1, q, bs[(b + 1) % D][q]);
+    static_for<4>([&](auto i) { issue_a(b, 0, i, as[b][0][i]); });
+  }
+  // What stage 0 needs has landed, and so have the stores of the previous task's epilogue,
+  // which were issued before (a wave's vector memory operations leave the counter in order):
+  // behind the workgroup barrier thread 0 may signal that task's completion, and draws the
+  // ticket of the task after this one.
+  wait_vm<(D - 1) * (JT + 4) + (D - 2) * 4>();
+  static_for<JT>([&](auto q) { store_fragment<q * 1024>(wr_off, ring[q]); });
+  wait_lds<0>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   if (threadIdx.x == 0) {
     if (pend != nullptr) (void)add_relaxed(pend, 1u);
     next = add_relaxed(queue, 1u);
   }
-  // then what stage -1 would have issued
 #pragma unroll
-  for (int i = 0; i < 2; ++i) issue_a(1, 0, i, as[1][0][i]);
-#pragma unroll
-  for (int q = 0; q < JT; ++q) issue_b(2, q, bs[0][q]);
-#pragma unroll
-  for (int u = 1; u < 3; ++u)
-#pragma unroll
-    for (int i = 0; i < 2; ++i) issue_a(1, u, i, as[1][u][i]);
-#pragma unroll
-  for (int j = 0; j < JT; ++j) bf[0][j] = read_b(0, 0, j);
+  for (int n = 0; n < RING; ++n) ring[n] = read_b(fo[0], n);
 
-  // One stage. P: its parity (which weight registers it multiplies, which LDS buffer it
-  // reads). R: stages after it, 3 meaning 3 or more.
+  // One stage. P: its register set, stage % D. R: stages after it, D+1 meaning D+1 or more. cur, nxt: byte offsets of its and the next stage's buffer;
+  // rd: where this lane reads sub-step 0 of the present stage.
+  static_assert(RING <= JB, "fragments of the next stage read in advance are sub-step 0's");
+  int cur = 0, nxt = STG;
+  unsigned rd = fo[0];
   auto stage = [&](auto par_tag, auto rem_tag, auto first_tag, int s) {
     constexpr int P = decltype(par_tag)::value;
     constexpr int R = decltype(rem_tag)::value;
-    constexpr bool A2 = R >= 2, A13 = R >= 1, B3 = R >= 3, NEXT = R >= 1;
-    using No = std::false_type;
-#pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      if (u == 0) wait_vm<direct_wait(JT, R, 0)>();
-      if (u == 1) wait_vm<direct_wait(JT, R, 1)>();
-      if (u == 2) wait_vm<direct_wait(JT, R, 2)>();
-      const uint4 (&cur)[JT_MAX] = bf[u & 1];
-      uint4 (&nxt)[JT_MAX] = bf[(u + 1) & 1];
-#pragma unroll
-      for (int j = 0; j < NS; ++j) {
-        if (u == 0) {
-          pair(first_tag, as[P][u], cur, j);
-        } else {
-          pair(No{}, as[P][u], cur, j);
-        }
-        if (u == 0) {
-          if (j < 2 && A13) issue_a(s + 1, 3, j, as[1 - P][3][j]);
-          if (j < JT && NEXT) write_b(1 - P, j, bs[1 - P][j]);   // token rows of stage s+1
-        } else if (u == 1) {
-          if (j == 0 && A2) {
-            issue_a(s + 2, 0, 0, as[P][0][0]);
-            issue_a(s + 2, 0, 1, as[P][0][1]);
-          }
-          if (j < JT && B3) issue_b(s + 3, j, bs[1 - P][j]);
-        } else if (j < 2 && A2) {
-          issue_a(s + 2, 1, j, as[P][1][j]);
-        }
-        if (j < JT) nxt[j] = read_b(P, u + 1, j);
-        __builtin_amdgcn_sched_barrier(0);
+    constexpr bool FIRST = decltype(first_tag)::value;
+    constexpr bool A0 = R >= D, A1 = R >= D - 1, NEXT = R >= 1, BN = R >= D + 1;
+    constexpr int P1 = (P + D - 1) % D;  // the set of the last stage, and of stage s+D-1
+    constexpr int PB = (P + 1) % D;      // the set of the next stage's token rows
+    // (pinned, so that the reads and writes below are these registers plus constants)
+    unsigned wr = wr_off + static_cast<unsigned>(nxt), rd1 = fo[1] + static_cast<unsigned>(cur),
+             rdn = fo[0] + static_cast<unsigned>(nxt);
+    asm volatile("" : "+v"(wr), "+v"(rd1), "+v"(rdn));
+    static_for<NSL>([&](auto n_tag) {
+      constexpr int n = decltype(n_tag)::value, u = n / JB, j = n % JB;
+      if (n == 0) wait_vm<direct_wait(JT, R, 0)>();
+      if (n == JB) wait_vm<direct_wait(JT, R, 1)>();
+      if (n == HO && NEXT) {
+        wait_lds<LDS_YOUNGER>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
       }
-    }
-    wait_vm<direct_wait(JT, R, 3)>();
 #pragma unroll
-    for (int j = 0; j < NS; ++j) {
-      if (j == BAR) {
-        // this wave no longer reads this stage's buffer and has written its part of the next
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (NEXT) {
-          __builtin_amdgcn_s_barrier();
-          asm volatile("" ::: "memory");
+      for (int i = 0; i < 4; ++i) mma<FIRST && u == 0, false>(as[P][u][i], ring[n % RING], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (u == 0) {
+        if constexpr (j < 2 && A1) {
+          issue_a(s + D - 1, 1, std::integral_constant<int, 2 * j>{}, as[P1][1][2 * j]);
+          issue_a(s + D - 1, 1, std::integral_constant<int, 2 * j + 1>{}, as[P1][1][2 * j + 1]);
         }
+        if constexpr (j < JT && NEXT) store_fragment<j * 1024>(wr, bs[PB][j]);  // token rows of stage s+1
+        if constexpr (j >= JT && BN) issue_b(s + D + 1, j - JT, bs[PB][j - JT]);
+      } else if constexpr (j < 2 && A0) {
+        issue_a(s + D, 0, std::integral_constant<int, 2 * j>{}, as[P][0][2 * j]);
+        issue_a(s + D, 0, std::integral_constant<int, 2 * j + 1>{}, as[P][0][2 * j + 1]);
       }
-      pair(No{}, as[P][3], bf[1], j);
-      if (j < 2 && A2) issue_a(s + 2, 2, j, as[P][2][j]);
-      if (j >= BAR && NEXT) {
-#pragma unroll
-        for (int r = (j - BAR) * RPS; r < (j - BAR + 1) * RPS; ++r)
-          if (r < JT) bf[0][r] = read_b(1 - P, 0, r);
+      if constexpr (n + RING < JB) {
+        ring[n % RING] = read_b(rd, n + RING);
+      } else if constexpr (n + RING < NSL) {
+        ring[n % RING] = read_b(rd1, n + RING - JB);
+      } else if constexpr (NEXT) {
+        ring[n % RING] = read_b(rdn, n + RING - NSL);
       }
       __builtin_amdgcn_sched_barrier(0);
-    }
+    });
+    rd = rdn;
+    cur = nxt;
+    nxt = uni(nxt == 2 * STG ? 0 : nxt + STG);
   };
   using Yes = std::true_type;
   using No = std::false_type;
-  using P0 = std::integral_constant<int, 0>;
-  using P1 = std::integral_constant<int, 1>;
-  using R3 = std::integral_constant<int, 3>;
-  // nstages is even and at least 4; stages with 3 or more after them: nstages - 3 (odd)
-  stage(P0{}, R3{}, Yes{}, 0);
+  // nstages is a multiple of D and at least 2*D; the last 2*D - 1 stages stand behind the loop.
+  // (One way through the code on purpose: where two ways meet or part the compiler may move
+  // registers about, and a value that is still on its way from memory must never be copied.)
+  stage(std::integral_constant<int, 0>{}, std::integral_constant<int, D + 1>{}, Yes{}, 0);
   int s = 1;
-  for (; s + 3 < nstages; s += 2) {
-    stage(P1{}, R3{}, No{}, s);
-    stage(P0{}, R3{}, No{}, s + 1);
-  }
-  stage(P1{}, std::integral_constant<int, 2>{}, No{}, s);
-  stage(P0{}, std::integral_constant<int, 1>{}, No{}, s + 1);
-  stage(P1{}, std::integral_constant<int, 0>{}, No{}, s + 2);
+  for (; s + 2 * D - 1 < nstages; s += D)
+    static_for<D>([&](auto i) {
+      stage(std::integral_constant<int, (1 + decltype(i)::value) % D>{}, std::integral_constant<int, D + 1>{}, No{},
+            s + decltype(i)::value);
+    });
+  static_for<2 * D - 1>([&](auto i) {
+    constexpr int k = decltype(i)::value, r = 2 * D - 2 - k;
+    stage(std::integral_constant<int, (1 + k) % D>{}, std::integral_constant<int, r < D + 1 ? r : D + 1>{}, No{}, s + k);
+  });
   // the compiler does not see matrix instructions in the assembly above: keep the wait states
   // between the last of them and the first read of an accumulator
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -1014,12 +1012,8 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
                                           unsigned* queue) {
   const int H = uni(p.H), I = uni(p.I), K = uni(p.K);
   const int wave = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  constexpr int NTL = ntl_of(JT);
-  // packed weights and at least four stages: the deeper pipeline (tile_gemm_direct), where a
-  // wave brings JT token loads per stage instead of NTL
-  const bool direct = JT <= DIRECT_JT_MAX &&
-                      uni(((down ? p.ffn2_packed : p.ffn1_packed) != nullptr && (down ? I : H) >= DIRECT_MIN_STAGES * KS) ? 1 : 0) != 0;
-  const int tl_per_wave = direct ? JT : NTL;
+  // packed weights and enough stages: the deeper pipeline
+  const bool direct = uni((down ? p.ffn2_packed : p.ffn1_packed) != nullptr && direct_takes(JT, (down ? I : H) / KS) ? 1 : 0) != 0;
   const int* perm = uni(p.perm) + row0;
   const int n0 = uni(nblk) * (down ? TN : G1_COLS);
   TileOperands op;
@@ -1046,8 +1040,8 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
                           : static_cast<unsigned>(row) * static_cast<unsigned>(I * 2) + stage_chunk_bytes(row);
     }
 #pragma unroll
-    for (int q = 0; q < NTL; ++q) {
-      const int row = stage_row(tl_per_wave, q);
+    for (int q = 0; q < JT; ++q) {
+      const int row = stage_row(JT, q);
       op.toff[q] = static_cast<unsigned>(min(row, rows - 1)) * static_cast<unsigned>(I * 2) + stage_chunk_bytes(row);
     }
   } else {
@@ -1074,13 +1068,13 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
                           : static_cast<unsigned>(wrow) * static_cast<unsigned>(H * 2) + stage_chunk_bytes(row);
     }
 #pragma unroll
-    for (int q = 0; q < NTL; ++q) {
-      const int row = stage_row(tl_per_wave, q);
+    for (int q = 0; q < JT; ++q) {
+      const int row = stage_row(JT, q);
       const int tok = ldc(&perm[min(row, rows - 1)]) / K;
       op.toff[q] = static_cast<unsigned>(tok) * static_cast<unsigned>(H * 2) + stage_chunk_bytes(row);
     }
   }
-  f32x16 acc[2][JT_MAX];
+  f32x4 acc[4][JB_MAX];
   unsigned next = 0u;
   // down: where the tile's rows go (token, slot), fetched while the k-loop runs
   auto load_side = [&]() {
@@ -1100,21 +1094,21 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
   }
   if (threadIdx.x == 0) task_notes()[0] = next;  // the epilogue's barriers publish it
 
-  const int r32 = lane & 31, kq = lane >> 5;
+  const int r16 = lane & 15, kg = lane >> 4;
   unsigned char* slab = lds_raw;
   if (!down) {
     constexpr int LD = G1_COLS * 2 + 16;  // slab row pitch in bytes
 #pragma unroll
-    for (int j = 0; j < JT; ++j)
+    for (int j = 0; j < 2 * JT; ++j)
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
+      for (int i = 0; i < 2; ++i) {  // gate blocks 0, 1 with their up blocks 2, 3
         float hv[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) hv[v] = silu_mul_fast(acc[0][j][g4 * 4 + v], acc[1][j][g4 * 4 + v]);
+        for (int v = 0; v < 4; ++v) hv[v] = silu_mul_fast(acc[i][j][v], acc[2 + i][j][v]);
         uint2 pk;
         pk.x = pack_bf16(hv[0], hv[1]);
         pk.y = pack_bf16(hv[2], hv[3]);
-        *reinterpret_cast<uint2*>(slab + (j * 32 + r32) * LD + (wave * 32 + g4 * 8 + kq * 4) * 2) = pk;
+        *reinterpret_cast<uint2*>(slab + (j * 16 + r16) * LD + (wave * 32 + i * 16 + kg * 4) * 2) = pk;
       }
     __syncthreads();
     // 16 lanes store one row's 256 bytes; a wave stores 4 rows per instruction
@@ -1150,19 +1144,16 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
 #pragma unroll
     for (int part = 0; part < (JT + 3) / 4; ++part) {
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int j = part * 4 + jj;
-        if (j < JT) {
+      for (int jj = 0; jj < 8; ++jj) {
+        const int j = part * 8 + jj;
+        if (j < 2 * JT) {
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-              uint2 pk;
-              pk.x = pack_bf16(acc[i][j][g4 * 4 + 0], acc[i][j][g4 * 4 + 1]);
-              pk.y = pack_bf16(acc[i][j][g4 * 4 + 2], acc[i][j][g4 * 4 + 3]);
-              *reinterpret_cast<uint2*>(slab + (jj * 32 + r32) * EPI_LD +
-                                        (wave * 64 + i * 32 + g4 * 8 + kq * 4) * 2) = pk;
-            }
+          for (int i = 0; i < 4; ++i) {
+            uint2 pk;
+            pk.x = pack_bf16(acc[i][j][0], acc[i][j][1]);
+            pk.y = pack_bf16(acc[i][j][2], acc[i][j][3]);
+            *reinterpret_cast<uint2*>(slab + (jj * 16 + r16) * EPI_LD + (wave * 64 + i * 16 + kg * 4) * 2) = pk;
+          }
         }
       }
       __syncthreads();
@@ -1205,17 +1196,21 @@ __device__ __noinline__ void tiled_gemm_task(ParamsRef pv, const TileDesc& tile_
     if (down) tile_task<8, true>(p, expert, row0, rows, nblk, pend, queue); else tile_task<8, false>(p, expert, row0, rows, nblk, pend, queue);
   } else if (jt > 6) {
     if (down) tile_task<7, true>(p, expert, row0, rows, nblk, pend, queue); else tile_task<7, false>(p, expert, row0, rows, nblk, pend, queue);
-  } else if (jt > 4) {
+  } else if (jt > 5) {
     if (down) tile_task<6, true>(p, expert, row0, rows, nblk, pend, queue); else tile_task<6, false>(p, expert, row0, rows, nblk, pend, queue);
-  } else if (jt > 2) {
+  } else if (jt > 4) {
+    if (down) tile_task<5, true>(p, expert, row0, rows, nblk, pend, queue); else tile_task<5, false>(p, expert, row0, rows, nblk, pend, queue);
+  } else if (jt > 3) {
     if (down) tile_task<4, true>(p, expert, row0, rows, nblk, pend, queue); else tile_task<4, false>(p, expert, row0, rows, nblk, pend, queue);
+  } else if (jt > 2) {
+    if (down) tile_task<3, true>(p, expert, row0, rows, nblk, pend, queue); else tile_task<3, false>(p, expert, row0, rows, nblk, pend, queue);
   } else {
     if (down) tile_task<2, true>(p, expert, row0, rows, nblk, pend, queue); else tile_task<2, false>(p, expert, row0, rows, nblk, pend, queue);
   }
 }
 
-constexpr int TILED_LDS_BYTES =
-    NOTE_OFF + NOTE_BYTES > ROUTER_LDS_BYTES ? NOTE_OFF + NOTE_BYTES : ROUTER_LDS_BYTES;
+constexpr int TILED_LDS_BYTES = NOTE_OFF + NOTE_BYTES;
+static_assert(TILED_LDS_BYTES >= ROUTER_LDS_BYTES && TILED_LDS_BYTES + 256 <= 160 * 1024, "LDS of a workgroup");
 
 // combine: out[t] = sum over slots, in slot order, of w[t,slot] * y[t*K+slot]
 // (refFullMoe.h:35,62-65): y holds each slot's down-projection row rounded to bf16; weight

@@ -208,6 +208,30 @@ def test_tiled_variant_forced(shape):
         case.close()
 
 
+@pytest.mark.parametrize("rows", [1, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 256, 257, 288,
+                                  289, 320, 321, 640, 641, 961])
+@pytest.mark.parametrize("I", [128, 192 * 2, 640])
+def test_tiled_tile_heights(rows, I):
+    """Every number of 32-row blocks a tile can have, at both edges, alone and as one of several tiles
+    of an expert (k == E: both experts hold every row), with 2,
+    6 and 10 stages of 64 k in the down projection and 4 in the gate/up one: on row-major weights
+    against the oracle, and the packed weights' pipeline must give the same bits."""
+    cfg = synth.MoeConfig("heights", rows, 256, 2, 2, I, "bf16")
+    print("tile heights", rows, I, flush=True)
+    case = GpuCase(cfg, seed=rows + I, sched=_lib.SCHED_TILED)
+    try:
+        out = case.run()
+        case.check_routing(case.inp["tokens"], case.launcher.routing(rows))
+        case.check_outputs(case.inp["tokens"], out, nthreads=4)
+        packed = GpuCase(cfg, seed=rows + I, sched=_lib.SCHED_TILED, inputs=case.inp, pack_weights=True)
+        try:
+            assert torch.equal(packed.run(), out)
+        finally:
+            packed.close()
+    finally:
+        case.close()
+
+
 @pytest.mark.parametrize("name,T", [("qwen3_30b_decode", 64), ("qwen3_30b_decode", 100),
                                     ("tiny_f32", 16)])
 def test_packed_weights_equal_unpacked(name, T):
