@@ -176,12 +176,36 @@ bool tiled_eligible(const FlashMoeLayerDesc& d, int tokens_num) {
          static_cast<long long>(tokens_num) * d.hidden * 2 < (1ll << 32);
 }
 
+// Whether the streaming variant may run this batch on its split-k kernel, and on how many 16-row
+// blocks a tile: 0 (no), 1 or 2. bf16; the shapes of the matrix-core router; k of at least a step a
+// wave in either projection; tables that fit the kernel's LDS; 4 KiB of router weights (where the
+// loads go that nobody needs); h rows that 31 bits address. One block up to 9 rows an expert on
+// average, two up to 24 (us, streaming kernel / one / two blocks, 30B shape: T=96 235 / 221 / 222,
+// T=144 260 / 230 / 229, T=160 252 / 228 / 225, T=200 266 / 253 / 234, T=256 275 / 301 / 241; 235B
+// shape: T=128 808 / 791 / 791, T=160 816 / 805 / 799, T=200 855 / 904 / 812, T=256 876 / 1124 / 836;
+// four hot experts, 30B: T=160 345 / 253 / 243, T=256 458 / 279 / 270).
+int split_row_blocks(const FlashMoeLayerDesc& d, int tokens_num) {
+  const long long slots = static_cast<long long>(tokens_num) * d.top_k;
+  if (d.dtype != FLASH_MOE_BF16 || d.hidden % fmoe::DOT16_KC != 0 || d.intermediate < 128 ||
+      slots > fmoe::SPLIT_MAX_SLOTS || slots > 24ll * d.experts ||
+      d.experts * ((tokens_num + 63) / 64) > fmoe::SCAN_LDS_WORDS ||
+      static_cast<long long>(d.experts) * d.hidden < 2048 || slots * d.intermediate * 2 >= (1ll << 31))
+    return 0;
+  return slots <= 9ll * d.experts ? 1 : 2;
+}
+
 int sched_for(const FlashMoeLayerDesc& d, int tokens_num) {
   if (d.sched == FLASH_MOE_SCHED_STREAM) return FLASH_MOE_SCHED_STREAM;
   if (!tiled_eligible(d, tokens_num)) return FLASH_MOE_SCHED_STREAM;
   if (d.sched == FLASH_MOE_SCHED_TILED) return FLASH_MOE_SCHED_TILED;
   const long long rows = static_cast<long long>(tokens_num) * d.top_k;
   const bool packed = (d.flags & (FLASH_MOE_FLAG_PACK_WEIGHTS | FLASH_MOE_FLAG_WEIGHTS_PREPACKED)) != 0;
+  // Row-major weights of moderate size: the split-k kernel is faster as far as it goes (us, tiled /
+  // split-k, 30B shape: T=224 309 / 277, T=256 313 / 292, with four hot experts 327 / 307; H=1024,
+  // I=512, 22 rows an expert 88 / 64; but 235B: T=224 975 / 1022, T=256 998 / 1067). The line lies
+  // between an expert's 1.6 M (30B) and 6.3 M (235B) weights a matrix.
+  if (!packed && static_cast<long long>(d.hidden) * d.intermediate <= 3ll << 20 && split_row_blocks(d, tokens_num) != 0)
+    return FLASH_MOE_SCHED_STREAM;
   return rows >= static_cast<long long>(packed ? kAutoTiledRowsPacked : kAutoTiledRowsRowMajor) * d.experts
              ? FLASH_MOE_SCHED_TILED
              : FLASH_MOE_SCHED_STREAM;
@@ -262,6 +286,14 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
              routing_groups <= p.n_groups / 2)
                 ? early_blocks
                 : 0;
+  // (a traced launch runs the streaming kernel, which writes the records)
+  p.split = p.dot16 && dot16_tasks <= p.n_groups / 2 && l->trace == nullptr ? split_row_blocks(d, T) : 0;
+  if (p.split) {
+    p.early = 1;
+    p.split_spec = reaches_experts ? 1 : 0;
+    // a down task in four parts, two of them to a workgroup, unless that leaves CUs without one
+    p.split_down = d.intermediate >= 256 && std::min<long long>(slots, d.experts) * (d.hidden / 128) < p.n_groups ? 8 : 4;
+  }
   p.max_mtiles = L.max_mtiles;
   p.spin_limit = l->spin_limit;
   p.tokens = (d.flags & FLASH_MOE_FLAG_RMSNORM) ? static_cast<const void*>(l->ws + L.xn) : tokens;

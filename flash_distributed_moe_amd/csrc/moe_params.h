@@ -26,6 +26,7 @@ constexpr int ROUTER_TOK = 8;    // streaming variant: tokens per router dot tas
 constexpr int ROUTER_EXP = 8;    // streaming variant: experts per router dot task
 constexpr int DOT16_KC = 256;    // streaming variant, matrix-core router: k per LDS stage
 constexpr int SCAN_LDS_WORDS = 1024;  // mask words (experts x 64-token words) the small-batch scan keeps in LDS
+constexpr int SPLIT_MAX_SLOTS = 2048;  // split-k kernel: (token, slot) entries its tables hold
 constexpr int EARLY_MAX_TOKENS = 384;  // batches up to this size may take their gate/up weights before the routing is known
 constexpr int MAX_EXPERTS = 256;  // experts are spread 64 per wave register slot
 constexpr int MAX_TOPK = 32;
@@ -120,6 +121,9 @@ struct Params {
   int fuse_scatter;                // 1: the scan task also writes the permutation
   int early;                       // 1, 2: row tile e belongs to expert e (empty or not), so gate/up tasks are
                                    //    handed out at launch and fetch their first weights under the routing
+  int split;                       // 1, 2: the split-k kernel runs, on tiles of so many 16-row blocks
+  int split_spec;                  //    1: its workgroups ask for gate/up weights before the routing is known
+  int split_down;                  //    waves that share a down task: 4 or 8
   int dot16;                       // 1 (streaming variant, bf16): the logit chains run on the matrix core, 16 tokens x
                                    //    16 experts per workgroup, on the first workgroups before they take tickets
   // What the last worker out needs when a launch has raised an error bit: it fills `out`
