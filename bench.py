@@ -85,6 +85,11 @@ def measured_traffic(workload, weights):
     return nbytes, entry.get("sources") != kernel_sources_digest()
 
 
+def kernel_of(tiled, dtype):
+    """The kernel a workload of this file runs (its bf16 decode batches have at most 24 rows an expert)."""
+    return "moe_tiled_kernel" if tiled else "moe_split_kernel" if dtype == "bf16" else "moe_stream_kernel"
+
+
 def record_traffic(workload, weights, fetch_kib, write_kib, kernel):
     try:
         with open(TRAFFIC_FILE) as f:
@@ -355,7 +360,7 @@ def measure(name, seed, steps, warmup, sched, weights, cold=False, balance=False
     routing = launcher.routing(cfg.T)
     active = int((routing["counts"] > 0).sum())
     tiled = launcher.sched_for(cfg.T) != 1
-    kernel = "moe_tiled_kernel" if tiled else "moe_stream_kernel"
+    kernel = kernel_of(tiled, cfg.dtype)
     extra = {}
     if cold:
         extra["cold_cache_us"] = cold_cache_us(launcher, x, out)
@@ -430,8 +435,9 @@ def main():
                  "multi-GPU path); run with --gpus 1")
     packed = args.weights
     if args.record_traffic:
-        kernel = "moe_tiled_kernel" if BOUND.get(args.config) == "mfma" or "4096" in args.config \
-            else "moe_stream_kernel"
+        from flash_distributed_moe_amd import synth
+
+        kernel = kernel_of(BOUND.get(args.config) == "mfma" or "4096" in args.config, synth.CONFIGS[args.config].dtype)
         record_traffic(args.config, packed, args.record_traffic[0], args.record_traffic[1], kernel)
         print(json.dumps({args.config: measured_traffic(args.config, packed)[0]}))
         return

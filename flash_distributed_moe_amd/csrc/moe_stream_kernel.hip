@@ -17,6 +17,10 @@
 // The down projection reads h rows that other workers wrote, so its B operand
 // uses coherent loads.
 //
+// bf16 batches of up to 24 rows an expert run a second kernel of this file instead, with
+// the same routing and combine: the split-k variant (moe_split_kernel, below), whose
+// workgroups share a task's k.
+//
 // Replaces, for this regime, the reference's moeKernel
 // (src/hip/kernel/moeKernel.h:37-107), its task executors
 // (src/hip/kernel/tasks/*.h) and its queue (src/hip/taskSystem/*.h).
@@ -1490,10 +1494,11 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
 // T=64 759 -> 762, T=256 876 -> 836. Four hot experts: T=16 146 -> 120, T=128 317 -> 240 (a tile of more
 // rows than an early task carries starts over there; here it is several tiles).
 //
-// Workgroups without a routing task ask for the first window of (expert b / nt1, columns b % nt1)
+// Where the batch reaches most experts, the first workgroups (as many as whole experts fill; those
+// with a routing task behind it) ask for the first window of (expert b / nt1, columns b % nt1)
 // before the routing is known and keep it if the expert turns out to be in use.
 // k-steps of a wave's window, by 16-row blocks of the tile (eight and six do not fit the registers
-// beside the epilogue: with eight the window's last loads were spilled, T = 64 306 us)
+// beside the epilogue: with eight for one block the window's last loads were spilled, T = 64 306 us)
 constexpr int split_u(int rb) { return rb == 1 ? 6 : 4; }
 constexpr int SPLIT_MAX_TILES = MAX_EXPERTS + SPLIT_MAX_SLOTS / 16;
 // LDS: the tables, then two sets of partial sums ([wave][weight block][row block][lane][4]); the

@@ -15,12 +15,13 @@
 //            and up rows side by side so that SiLU(gate)*up happens in registers
 //   down     (row tile, 256 output columns): same tile, weighted bf16 rows to y
 //   combine  8 tokens: out = sum over slots of y
-// GEMM tile: up to 256 token rows x 256 weight rows, K stepped by 64 through two
-// LDS stages that are filled straight from global memory in whole 128-byte
-// lines; each wave owns 64 weight rows x all token rows of it as 2x8 MFMA
-// 32x32x16 blocks, 256 accumulator registers. Weight rows are the MFMA "A"
-// operand so that a lane ends up with runs of 4 consecutive output columns of
-// one token row. A tile with fewer rows multiplies fewer token blocks, so its
+// GEMM tile: up to 320 token rows x 256 weight rows, K stepped by 64; each wave
+// owns 64 weight rows x all token rows of it as 4 x (2*JT) MFMA 16x16x32 blocks
+// (JT = 32-row blocks of the tile), up to 320 accumulator registers. Two
+// pipelines: both operands through LDS stages (row-major weights, tall tiles), or
+// packed weights straight to registers and token rows through LDS. Weight rows
+// are the MFMA "A" operand so that a lane ends up with runs of 4 consecutive
+// output columns of one token row. A tile with fewer rows multiplies fewer token blocks, so its
 // time follows its rows.
 //
 // Replaces, for this regime, the reference's moeKernel
@@ -460,7 +461,7 @@ __device__ void tiled_scatter_task(ParamsRef p, int blk) {
 // Operands go HBM/L2 -> LDS directly (global_load_lds_dwordx4: lane l's 16 bytes
 // land at LDS base + 16*l, from any global address), in stages of 64 k: one
 // 128-byte line of every operand row, so every request uses whole cache lines
-// whatever the row pitch. Two stages; no register staging, no LDS write
+// whatever the row pitch. Two or three stages; no register staging, no LDS write
 // instructions, almost no vector-ALU work in the loop.
 //
 // One wave per SIMD, each with 64 weight rows x all token rows of the tile:

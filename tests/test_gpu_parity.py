@@ -315,9 +315,12 @@ def test_prepacked_weights_equal_unpacked(name, T, sched):
     (67, 2304, 16, 2, 128, 2),      # ragged tiles; nine k-steps a wave, more than the window
     (72, 256, 256, 9, 128),         # every expert slot in use; two mask words
     (128, 256, 256, 9, 128, 3),     # 1152 routing entries, all workgroups busy with routing or early tasks
+    (40, 256, 4, 1, 128),           # ten rows an expert: tiles of two row blocks
+    (190, 768, 16, 2, 352, 2),      # 23.75 rows an expert; ragged tiles of up to 32 rows, two experts with several
+    (256, 512, 96, 8, 160, 4),      # 2048 routing entries: the tables are full
 ])
 def test_split_k_small_batches(shape):
-    """Small bf16 batches (at most nine rows an expert): the split-k kernel at the edges of its k
+    """Small bf16 batches (at most 24 rows an expert): the split-k kernel at the edges of its k
     parts, tiles and tables, on row-major weights against the oracle; the packed copy gives the same
     bits, and so does a second launch (every counter is back at zero)."""
     T, H, E, k, I = shape[:5]
