@@ -176,25 +176,38 @@ bool tiled_eligible(const FlashMoeLayerDesc& d, int tokens_num) {
          static_cast<long long>(tokens_num) * d.hidden * 2 < (1ll << 32);
 }
 
-// Whether the streaming variant may run this batch on its split-k kernel, and on how many 16-row
-// blocks a tile: 0 (no), 1 or 2. bf16; the shapes of the matrix-core router; k of at least a step a
-// wave in either projection; tables that fit the kernel's LDS; 4 KiB of router weights (where the
-// loads go that nobody needs); h rows that 31 bits address. One block up to 9 rows an expert on
+// What the choice of a kernel depends on beside the layer and the batch.
+struct Machine {
+  int n_groups;  // workgroups of a launch: one per CU
+  bool traced;   // task records are being written (the split-k kernel writes none)
+};
+
+// The matrix-core logit chains take 16 tokens x 16 experts per workgroup.
+int dot16_tasks_of(const FlashMoeLayerDesc& d, int tokens_num) {
+  return ((tokens_num + 15) / 16) * ((d.experts + 15) / 16);
+}
+
+// Whether the streaming variant runs this batch on its split-k kernel, and on how many 16-row
+// blocks a tile: 0 (no), 1 or 2. bf16; the shapes of the matrix-core router, with at most half of the
+// workgroups on it (the others have asked for weights by then); k of at least a step a wave in
+// either projection; tables that fit the kernel's LDS; 4 KiB of router weights (where the
+// loads go that nobody needs); h rows that 31 bits address; no trace. One block up to 9 rows an expert on
 // average, two up to 24 (us, streaming kernel / one / two blocks, 30B shape: T=96 235 / 221 / 222,
 // T=144 260 / 230 / 229, T=160 252 / 228 / 225, T=200 266 / 253 / 234, T=256 275 / 301 / 241; 235B
 // shape: T=128 808 / 791 / 791, T=160 816 / 805 / 799, T=200 855 / 904 / 812, T=256 876 / 1124 / 836;
 // four hot experts, 30B: T=160 345 / 253 / 243, T=256 458 / 279 / 270).
-int split_row_blocks(const FlashMoeLayerDesc& d, int tokens_num) {
+int split_row_blocks(const FlashMoeLayerDesc& d, int tokens_num, const Machine& m) {
   const long long slots = static_cast<long long>(tokens_num) * d.top_k;
   if (d.dtype != FLASH_MOE_BF16 || d.hidden % fmoe::DOT16_KC != 0 || d.intermediate < 128 ||
       slots > fmoe::SPLIT_MAX_SLOTS || slots > 24ll * d.experts ||
       d.experts * ((tokens_num + 63) / 64) > fmoe::SCAN_LDS_WORDS ||
-      static_cast<long long>(d.experts) * d.hidden < 2048 || slots * d.intermediate * 2 >= (1ll << 31))
+      static_cast<long long>(d.experts) * d.hidden < 2048 || slots * d.intermediate * 2 >= (1ll << 31) ||
+      dot16_tasks_of(d, tokens_num) > m.n_groups / 2 || m.traced)
     return 0;
   return slots <= 9ll * d.experts ? 1 : 2;
 }
 
-int sched_for(const FlashMoeLayerDesc& d, int tokens_num) {
+int sched_for(const FlashMoeLayerDesc& d, int tokens_num, const Machine& m) {
   if (d.sched == FLASH_MOE_SCHED_STREAM) return FLASH_MOE_SCHED_STREAM;
   if (!tiled_eligible(d, tokens_num)) return FLASH_MOE_SCHED_STREAM;
   if (d.sched == FLASH_MOE_SCHED_TILED) return FLASH_MOE_SCHED_TILED;
@@ -203,8 +216,12 @@ int sched_for(const FlashMoeLayerDesc& d, int tokens_num) {
   // Row-major weights of moderate size: the split-k kernel is faster as far as it goes (us, tiled /
   // split-k, 30B shape: T=224 309 / 277, T=256 313 / 292, with four hot experts 327 / 307; H=1024,
   // I=512, 22 rows an expert 88 / 64; but 235B: T=224 975 / 1022, T=256 998 / 1067). The line lies
-  // between an expert's 1.6 M (30B) and 6.3 M (235B) weights a matrix.
-  if (!packed && static_cast<long long>(d.hidden) * d.intermediate <= 3ll << 20 && split_row_blocks(d, tokens_num) != 0)
+  // between an expert's 1.6 M (30B) and 6.3 M (235B) weights a matrix. Where the split-k kernel
+  // does not start, the streaming kernel would run instead, and the tiled one is ahead of that (us,
+  // tiled / streaming, H=2048, I=768, even routing and four hot experts: E=128, k=4, T=480 307 / 334
+  // and 305 / 347; E=128, k=6, T=320 308 / 330 and 329 / 354; E=64, k=2, T=700 202 / 219 and
+  // 133 / 153; E=96, k=4, T=400 275 / 273 and 273 / 293).
+  if (!packed && static_cast<long long>(d.hidden) * d.intermediate <= 3ll << 20 && split_row_blocks(d, tokens_num, m) != 0)
     return FLASH_MOE_SCHED_STREAM;
   return rows >= static_cast<long long>(packed ? kAutoTiledRowsPacked : kAutoTiledRowsRowMajor) * d.experts
              ? FLASH_MOE_SCHED_TILED
@@ -238,6 +255,8 @@ struct FlashMoeLauncher {
 
 namespace {
 
+Machine machine(const FlashMoeLauncher& l) { return Machine{std::min(l.num_cus, kMaxGroups), l.trace != nullptr}; }
+
 fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* output, int T) {
   const FlashMoeLayerDesc& d = l->desc;
   const Layout& L = l->layout;
@@ -248,7 +267,8 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   p.K = d.top_k;
   p.I = d.intermediate;
   p.W = L.W;
-  p.n_groups = l->num_cus < kMaxGroups ? l->num_cus : kMaxGroups;
+  const Machine m = machine(*l);
+  p.n_groups = m.n_groups;
   p.n_workers = p.n_groups * 8;
   p.fuse_scatter = (static_cast<long long>(T) * d.top_k <= 2048) ? 1 : 0;
   // Early gate/up tasks wait inside the kernel for the routing, so every routing
@@ -259,7 +279,7 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
                         ((d.experts + fmoe::ROUTER_EXP - 1) / fmoe::ROUTER_EXP);
   // bf16 layers run the logit chains on the matrix core, 16 tokens x 16 experts
   // per workgroup, while every such task finds a workgroup of its own
-  const int dot16_tasks = ((T + 15) / 16) * ((d.experts + 15) / 16);
+  const int dot16_tasks = dot16_tasks_of(d, T);
   p.dot16 = (d.dtype == FLASH_MOE_BF16 && d.hidden % fmoe::DOT16_KC == 0 &&
              dot16_tasks <= p.n_groups)
                 ? 1
@@ -286,8 +306,7 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
              routing_groups <= p.n_groups / 2)
                 ? early_blocks
                 : 0;
-  // (a traced launch runs the streaming kernel, which writes the records)
-  p.split = p.dot16 && dot16_tasks <= p.n_groups / 2 && l->trace == nullptr ? split_row_blocks(d, T) : 0;
+  p.split = split_row_blocks(d, T, m);
   if (p.split) {
     p.early = 1;
     p.split_spec = reaches_experts ? 1 : 0;
@@ -499,7 +518,7 @@ int flashMoeCreate(FlashMoeLauncher** out, const FlashMoeLayerDesc* desc, void* 
 
 int flashMoeSchedFor(FlashMoeLauncher* l, int tokens_num) {
   if (l == nullptr) return -1;
-  return sched_for(l->desc, tokens_num);
+  return sched_for(l->desc, tokens_num, machine(*l));
 }
 
 int flashMoeLaunch(FlashMoeLauncher* l, const void* tokens, void* output, int tokens_num,
@@ -630,7 +649,10 @@ int flashMoeLaunchNoAlloc(const FlashMoeLayerDesc* desc, const void* tokens, voi
   FlashMoeLauncher l;
   l.desc = *desc;
   l.desc.max_tokens = tokens_num;
-  int sched = sched_for(l.desc, tokens_num);
+  // (what does not fit is refused before any device is asked for; where the number of CUs
+  // decides between the variants, below 26 rows an expert, both workspaces are of one size)
+  l.num_cus = kMaxGroups;
+  int sched = sched_for(l.desc, tokens_num, machine(l));
   l.layout = make_layout(l.desc, sched == FLASH_MOE_SCHED_TILED);
   if (sched == FLASH_MOE_SCHED_TILED && desc->sched == FLASH_MOE_SCHED_AUTO &&
       l.layout.total > static_cast<size_t>(FLASH_MOE_NOALLOC_SCRATCH_BYTES)) {
@@ -655,6 +677,7 @@ int flashMoeLaunchNoAlloc(const FlashMoeLayerDesc* desc, const void* tokens, voi
   l.num_cus = sd->num_cus;
   l.ticks_per_ms = sd->ticks_per_ms;
   l.spin_limit = 2000 * sd->ticks_per_ms;
+  sched = sched_for(l.desc, tokens_num, machine(l));
   // where a failing launch's last worker leaves its error bits: device memory here, no
   // pinned host word (that would be an allocation)
   l.host_error_dev = reinterpret_cast<unsigned*>(sd->ptr + kScratchErrorOffset);
@@ -752,7 +775,7 @@ int flashMoeReadDownRows(FlashMoeLauncher* l, int tokens_num, void* y, int* elem
   if (tokens_num < 0 || tokens_num > l->desc.max_tokens)
     FMOE_FAIL(hipErrorInvalidValue, "tokens_num = %i", tokens_num);
   FMOE_HIP_CHECK(hipStreamSynchronize(stream));
-  const bool tiled = sched_for(l->desc, tokens_num) == FLASH_MOE_SCHED_TILED;
+  const bool tiled = flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED;
   const size_t rows = static_cast<size_t>(tokens_num) * l->desc.top_k;
   const size_t bytes = rows * l->desc.hidden * (tiled ? 2 : 4);
   const size_t kept = (l->layout.xn - l->layout.y);  // the region's size up to the next one

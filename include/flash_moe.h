@@ -233,7 +233,8 @@ int flashMoeSetWaitLimitMs(FlashMoeLauncher* l, double ms);
  * `capacity` 48-byte records (0 frees them and turns tracing off); a traced
  * launch writes one record per task, indexed by ticket:
  *   { u32 ticket, kind, worker, aux; i64 t_fetch, t_ready, t_end, pad }
- * (a batch that would run the split-k kernel runs the streaming one while tracing is on);
+ * (a batch that would run the split-k kernel runs the streaming or the tiled one while tracing is
+ * on, see flashMoeSchedFor: read a launch's stage outputs before tracing is switched);
  * kind: 0 router dot, 1 scan, 2 scatter, 3 gate/up, 4 down, 5 combine, 6 router
  * select; times in
  * ticks of the 100 MHz device wall clock. Read waits for `stream`, copies up to

@@ -232,6 +232,33 @@ def test_tiled_tile_heights(rows, I):
         case.close()
 
 
+@pytest.mark.parametrize("E,k,last", [(128, 4, 256), (96, 4, 336), (64, 2, 512)])
+def test_auto_row_major_leaves_the_streaming_variant_with_the_split_k_kernel(E, k, last):
+    """AUTO sends row-major bf16 batches of 14 to 24 rows an expert to the streaming variant for its
+    split-k kernel only. That kernel starts with at most half of the 256 CUs on the logit chains
+    (16 tokens x 16 experts each): `last` tokens. From 14 rows an expert on, a batch it does not
+    start for is the tiled variant's, and so is every one of them while a trace is written."""
+    cfg = synth.MoeConfig("auto", 24 * E // k, 256, E, k, 128, "bf16")
+    line = -(-14 * E // k)   # tokens from which an expert has 14 rows on average
+    case = GpuCase(cfg, seed=E)
+    try:
+        sched = case.launcher.sched_for
+        above = max(last + 1, line)
+        print("row-major AUTO", E, k, "split-k up to", last, "tiled from", above, flush=True)
+        assert sched(last) == _lib.SCHED_STREAM
+        assert [sched(t) for t in (above, above + 16, cfg.T)] == [_lib.SCHED_TILED] * 3
+        x = case.inp["tokens"]
+        out = case.run()
+        case.check_routing(x, case.launcher.routing(cfg.T))
+        case.check_outputs(x, out, nthreads=4)
+        case.launcher.trace_enable(1 << 16)
+        assert sched(line) == _lib.SCHED_TILED
+        case.launcher.trace_enable(0)
+        assert sched(line) == (_lib.SCHED_STREAM if line <= last else _lib.SCHED_TILED)
+    finally:
+        case.close()
+
+
 @pytest.mark.parametrize("name,T", [("qwen3_30b_decode", 64), ("qwen3_30b_decode", 100),
                                     ("tiny_f32", 16)])
 def test_packed_weights_equal_unpacked(name, T):

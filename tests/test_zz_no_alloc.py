@@ -40,10 +40,10 @@ def no_alloc(cfg, inp, x, sched, inplace=False):
     return out
 
 
-def with_launcher(cfg, inp, x, sched):
+def with_launcher(cfg, inp, x, sched, **create):
     l = MoeKernelLauncher()
     l.create(inp["gate"], inp["ffn1"], inp["ffn2"], x.shape[0], l.getDistributedUniqueId(True), 0, 1,
-             top_k=cfg.k, router_bias=inp["bias"], sched=sched)
+             top_k=cfg.k, router_bias=inp["bias"], sched=sched, **create)
     try:
         out = torch.full_like(x, float("nan"))
         l.launch(x, out)
@@ -94,6 +94,19 @@ def test_no_alloc_equals_launcher_two_calls_in_a_row():
     # in place, as the reference's callers run it
     g = no_alloc(big, inp_big, inp_big["tokens"], _lib.SCHED_STREAM, inplace=True)
     assert torch.equal(g, no_alloc(big, inp_big, inp_big["tokens"], _lib.SCHED_STREAM))
+
+
+def test_no_alloc_takes_the_kernel_of_the_launcher():
+    """A row-major AUTO batch between the split-k kernel's last size and the packed weights'
+    switch-over: the number of CUs decides, and both entry points decide alike (the variants
+    round differently, so equal bits are the same variant's)."""
+    dev = torch.device("cuda:0")
+    cfg = synth.MoeConfig("between", 480, 256, 128, 4, 128, "bf16")
+    inp = synth.make_inputs_torch(cfg, 7907, dev)
+    for T in (256, 480):
+        x = inp["tokens"][:T].contiguous()
+        want = with_launcher(cfg, inp, x, _lib.SCHED_AUTO, pack_weights=False)
+        assert torch.equal(no_alloc(cfg, inp, x, _lib.SCHED_AUTO), want)
 
 
 def test_no_alloc_with_norm_and_residual():
