@@ -883,6 +883,13 @@ __device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nst
 #pragma unroll
   for (int q = 0; q < JT; ++q) issue_b(1, q, bs[1][q]);
   static_for<4>([&](auto i) { issue_a(0, 1, i, as[0][1][i]); });
+  // All of this has landed, and so have the stores of the previous task's epilogue (loads and
+  // stores are not taken to complete in order with each other, so only a wait for all of them
+  // covers the stores): behind the workgroup barrier below thread 0 may signal that task's
+  // completion. The later stages' loads go out behind the wait; in front of it, with a wait that
+  // left them in flight, they gained nothing (us, full wait / partial: T=600 305 / 305, T=8192
+  // 760 / 759, 235B shape T=1024 1018 / 1019).
+  wait_vm<0>();
 #pragma unroll
   for (int b = 1; b < D; ++b) {
     if (b > 1) static_for<4>([&](auto i) { issue_a(b - 1, 1, i, as[b - 1][1][i]); });
@@ -890,11 +897,6 @@ __device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nst
     for (int q = 0; q < JT; ++q) issue_b(b + 1, q, bs[(b + 1) % D][q]);
     static_for<4>([&](auto i) { issue_a(b, 0, i, as[b][0][i]); });
   }
-  // What stage 0 needs has landed, and so have the stores of the previous task's epilogue,
-  // which were issued before (a wave's vector memory operations leave the counter in order):
-  // behind the workgroup barrier thread 0 may signal that task's completion, and draws the
-  // ticket of the task after this one.
-  wait_vm<(D - 1) * (JT + 4) + (D - 2) * 4>();
   static_for<JT>([&](auto q) { store_fragment<q * 1024>(wr_off, ring[q]); });
   wait_lds<0>();
   __builtin_amdgcn_s_barrier();
