@@ -771,15 +771,20 @@ __device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f
 // The loads in front of the loop are issued in the same order, as if by stages -D ... -1.
 constexpr int DIRECT_GROUPS = 3;
 constexpr int DIRECT_JT_MAX = 8;     // taller tiles do not leave the registers for it
-// Register sets. Short tiles have few accumulators and are bound by the weights' way from
-// memory: four sets. Two are enough for tall ones, whose stages last 2000 cycles.
-constexpr int direct_depth(int jt) { return jt <= 2 ? 4 : 2; }
-constexpr bool direct_takes(int jt, int nstages) {
-  return jt <= DIRECT_JT_MAX && nstages % direct_depth(jt) == 0 && nstages >= 2 * direct_depth(jt);
+// Register sets for a product of nstages stages, 0: not this pipeline. Short tiles have few
+// accumulators and are bound by the weights' way from memory: four sets, where the stages are
+// enough to pay for filling and draining them (us, four / two sets: 30B shape T=512, 32 stages,
+// 302 / 303; 235B shape T=600, 64 stages, 983 / 985; but H=I=512 T=900, 8 stages, 71.4 / 70.4;
+// H=I=1024, 16 stages, 141.5 / 139.1; H=I=1536, 24 stages, 242.7 / 240.7). Two are enough for tall
+// ones, whose stages last 2000 cycles, and serve every other number of stages; against the LDS
+// pipeline (us, two sets / LDS): H=2048, I=256, 4 stages, T=448 162 / 166 and T=768 166 / 170; I=640,
+// 10 stages, T=768 276 / 275; I=1408, 22 stages, T=768 499 / 499.
+constexpr int direct_depth(int jt, int nstages) {
+  if (jt <= 2 && nstages % 4 == 0 && nstages >= 32) return 4;
+  return jt <= DIRECT_JT_MAX && nstages % 2 == 0 && nstages >= 4 ? 2 : 0;
 }
-// Loads that group g (in issue order) of a stage with r stages after it puts out.
-constexpr int direct_group(int jt, int r, int g) {
-  const int d = direct_depth(jt);
+// Loads that group g (in issue order) of a stage with r stages after it puts out, with d sets.
+constexpr int direct_group(int jt, int d, int r, int g) {
   switch (g) {
     case 0: return r >= d - 1 ? 4 : 0;
     case 1: return r >= d + 1 ? jt : 0;
@@ -789,22 +794,21 @@ constexpr int direct_group(int jt, int r, int g) {
 // Loads issued after group g0 of the stage `back` stages before the present one (which has
 // r stages after it) and before group g1 of the present stage: those may still be in flight
 // when everything up to and including that group has to have landed.
-constexpr int direct_in_flight(int jt, int r, int back, int g0, int g1) {
+constexpr int direct_in_flight(int jt, int d, int r, int back, int g0, int g1) {
   int n = 0;
   for (int b = back; b >= 0; --b) {
     const int lo = b == back ? g0 + 1 : 0;
     const int hi = b == 0 ? g1 : DIRECT_GROUPS;
-    for (int g = lo; g < hi; ++g) n += direct_group(jt, r + b, g);
+    for (int g = lo; g < hi; ++g) n += direct_group(jt, d, r + b, g);
   }
   return n;
 }
 // wait in front of sub-step w of a stage with r stages after it: its weight fragments and,
 // for sub-step 0, the token rows of the next stage, which that sub-step writes to LDS
-constexpr int direct_wait(int jt, int r, int w) {
-  const int d = direct_depth(jt);
-  return w == 0 ? direct_in_flight(jt, r, d, 2, 0) : direct_in_flight(jt, r, d - 1, 0, 1);
+constexpr int direct_wait(int jt, int d, int r, int w) {
+  return w == 0 ? direct_in_flight(jt, d, r, d, 2, 0) : direct_in_flight(jt, d, r, d - 1, 0, 1);
 }
-static_assert(direct_wait(2, 5, 0) < 64 && direct_wait(8, 3, 0) < 64, "vmcnt holds 6 bits");
+static_assert(direct_wait(2, 4, 5, 0) < 64 && direct_wait(8, 2, 3, 0) < 64, "vmcnt holds 6 bits");
 
 // 16 bytes per lane from base + off + OFF into the registers of `dst`; completion is tracked
 // by hand (wait_vm), so the compiler must not believe it knows when the value is there: the
@@ -822,7 +826,7 @@ template <int N>
 __device__ __forceinline__ void wait_lds() {
   asm volatile("s_waitcnt lgkmcnt(%0)" : : "n"(N) : "memory");
 }
-template <int JT>
+template <int JT, int D>
 __device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nstages, f32x4 (&acc)[4][JB_MAX],
                                                  unsigned* pend, unsigned* queue, unsigned& next) {
   static_assert(JT <= DIRECT_JT_MAX, "tile too tall for the register-staged pipeline");
@@ -848,7 +852,6 @@ __device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nst
   // eight rows of load q are one run of 1 KiB, lane l at 16*l
   const unsigned wr_off = lds_addr + static_cast<unsigned>((wave * JT) * 1024 + lane * 16);
 
-  constexpr int D = direct_depth(JT);
   v4u_t as[D][2][4];   // weight fragments: [stage % D][sub-step][block]
   v4u_t bs[D][JT];     // token rows on their way to LDS: [stage % D][load]
   v4u_t ring[RING];
@@ -926,8 +929,8 @@ __device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nst
     asm volatile("" : "+v"(wr), "+v"(rd1), "+v"(rdn));
     static_for<NSL>([&](auto n_tag) {
       constexpr int n = decltype(n_tag)::value, u = n / JB, j = n % JB;
-      if (n == 0) wait_vm<direct_wait(JT, R, 0)>();
-      if (n == JB) wait_vm<direct_wait(JT, R, 1)>();
+      if (n == 0) wait_vm<direct_wait(JT, D, R, 0)>();
+      if (n == JB) wait_vm<direct_wait(JT, D, R, 1)>();
       if (n == HO && NEXT) {
         wait_lds<LDS_YOUNGER>();
         __builtin_amdgcn_s_barrier();
@@ -1016,7 +1019,7 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
   const int H = uni(p.H), I = uni(p.I), K = uni(p.K);
   const int wave = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
   // packed weights and enough stages: the deeper pipeline
-  const bool direct = uni((down ? p.ffn2_packed : p.ffn1_packed) != nullptr && direct_takes(JT, (down ? I : H) / KS) ? 1 : 0) != 0;
+  const int depth = uni((down ? p.ffn2_packed : p.ffn1_packed) != nullptr ? direct_depth(JT, (down ? I : H) / KS) : 0);
   const int* perm = uni(p.perm) + row0;
   const int n0 = uni(nblk) * (down ? TN : G1_COLS);
   TileOperands op;
@@ -1089,9 +1092,14 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
       }
     }
   };
-  if (direct) {
+  if (depth != 0) {
     load_side();
-    if constexpr (JT <= DIRECT_JT_MAX) tile_gemm_direct<JT>(op, nstages, acc, pend, queue, next);
+    if constexpr (JT <= 2) {
+      if (depth == 4) tile_gemm_direct<JT, 4>(op, nstages, acc, pend, queue, next);
+      else tile_gemm_direct<JT, 2>(op, nstages, acc, pend, queue, next);
+    } else if constexpr (JT <= DIRECT_JT_MAX) {
+      tile_gemm_direct<JT, 2>(op, nstages, acc, pend, queue, next);
+    }
   } else {
     tile_gemm<JT>(op, nstages, acc, pend, queue, next, load_side);
   }

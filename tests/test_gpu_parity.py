@@ -215,9 +215,22 @@ def test_tiled_tile_heights(rows, I):
     """Every number of 32-row blocks a tile can have, at both edges, alone and as one of several tiles
     of an expert (k == E: both experts hold every row), with 2,
     6 and 10 stages of 64 k in the down projection and 4 in the gate/up one: on row-major weights
-    against the oracle, and the packed weights' pipeline must give the same bits."""
-    cfg = synth.MoeConfig("heights", rows, 256, 2, 2, I, "bf16")
-    print("tile heights", rows, I, flush=True)
+    against the oracle, and the packed weights must give the same bits (through the register-staged
+    pipeline with two sets of registers, but for the 2 stages and tiles of more than 256 rows)."""
+    check_tile_heights(rows, 256, I)
+
+
+@pytest.mark.parametrize("rows", [1, 33, 64])
+@pytest.mark.parametrize("H,I", [(512, 512), (2304, 2048), (2048, 2304)])
+def test_tiled_short_tiles_of_many_stages(rows, H, I):
+    """Tiles of up to 64 rows with 32 and 36 stages of 64 k, where the register-staged pipeline takes
+    four sets of registers, and with 8, where it still takes two."""
+    check_tile_heights(rows, H, I)
+
+
+def check_tile_heights(rows, H, I):
+    cfg = synth.MoeConfig("heights", rows, H, 2, 2, I, "bf16")
+    print("tile heights", rows, H, I, flush=True)
     case = GpuCase(cfg, seed=rows + I, sched=_lib.SCHED_TILED)
     try:
         out = case.run()
