@@ -24,6 +24,9 @@
 namespace fmoe {
 hipError_t launch_stream_kernel(const Params& p, int dtype, int grid, hipStream_t stream);
 hipError_t prepare_stream_kernel();
+hipError_t launch_split_kernel(const Params& p, int grid, hipStream_t stream);
+hipError_t prepare_split_kernel();
+hipError_t split_kernel_occupancy(int* per_cu);
 hipError_t pack_weights(const void* src, void* dst, int dtype, int E, int H, int I, int which,
                         hipStream_t stream);
 hipError_t launch_tiled_kernel(const Params& p, int grid, hipStream_t stream);
@@ -478,11 +481,14 @@ int flashMoeCreate(FlashMoeLauncher** out, const FlashMoeLayerDesc* desc, void* 
     l->ticks_per_ms = khz;
   l->spin_limit = 2000 * l->ticks_per_ms;
   if ((e = fmoe::prepare_stream_kernel()) != hipSuccess) return fail(e);
+  if ((e = fmoe::prepare_split_kernel()) != hipSuccess) return fail(e);
   if ((e = fmoe::prepare_tiled_kernel()) != hipSuccess) return fail(e);
   // Waits happen inside the kernels, so every workgroup of a launch must be resident at
-  // once: one per CU, which both kernels' resources allow only if nothing else is asked of them.
+  // once: one per CU, which the kernels' resources allow only if nothing else is asked of them.
   int per_cu = 0;
   if ((e = fmoe::stream_kernel_occupancy(desc->dtype, &per_cu)) != hipSuccess) return fail(e);
+  if (per_cu < 1) return fail(hipErrorLaunchOutOfResources);
+  if ((e = fmoe::split_kernel_occupancy(&per_cu)) != hipSuccess) return fail(e);
   if (per_cu < 1) return fail(hipErrorLaunchOutOfResources);
   if ((e = fmoe::tiled_kernel_occupancy(&per_cu)) != hipSuccess) return fail(e);
   if (per_cu < 1) return fail(hipErrorLaunchOutOfResources);
@@ -552,6 +558,8 @@ int flashMoeLaunch(FlashMoeLauncher* l, const void* tokens, void* output, int to
                                         tokens_num, l->desc.hidden, l->desc.norm_eps, stream));
   if (flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED) {
     FMOE_HIP_CHECK(fmoe::launch_tiled_kernel(p, p.n_groups, stream));
+  } else if (p.split) {
+    FMOE_HIP_CHECK(fmoe::launch_split_kernel(p, p.n_groups, stream));
   } else {
     FMOE_HIP_CHECK(fmoe::launch_stream_kernel(p, l->desc.dtype, p.n_groups, stream));
   }
@@ -601,6 +609,7 @@ hipError_t static_device(int device, const StaticDevice** out) {
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
       sd.ticks_per_ms = khz;
     FMOE_HIP_CHECK(fmoe::prepare_stream_kernel());
+    FMOE_HIP_CHECK(fmoe::prepare_split_kernel());
     FMOE_HIP_CHECK(fmoe::prepare_tiled_kernel());
     // as in flashMoeCreate: every workgroup of a launch must be resident at once
     int per_cu = 0;
@@ -608,6 +617,8 @@ hipError_t static_device(int device, const StaticDevice** out) {
     if (per_cu < 1) FMOE_FAIL(hipErrorLaunchOutOfResources, "the streaming kernel does not fit a CU");
     FMOE_HIP_CHECK(fmoe::stream_kernel_occupancy(FLASH_MOE_F32, &per_cu));
     if (per_cu < 1) FMOE_FAIL(hipErrorLaunchOutOfResources, "the streaming kernel does not fit a CU");
+    FMOE_HIP_CHECK(fmoe::split_kernel_occupancy(&per_cu));
+    if (per_cu < 1) FMOE_FAIL(hipErrorLaunchOutOfResources, "the split-k kernel does not fit a CU");
     FMOE_HIP_CHECK(fmoe::tiled_kernel_occupancy(&per_cu));
     if (per_cu < 1) FMOE_FAIL(hipErrorLaunchOutOfResources, "the tiled kernel does not fit a CU");
     // the error word starts at zero (the array is zero-initialised with the code object,
@@ -695,6 +706,8 @@ int flashMoeLaunchNoAlloc(const FlashMoeLayerDesc* desc, const void* tokens, voi
                                         desc->hidden, desc->norm_eps, stream));
   if (sched == FLASH_MOE_SCHED_TILED) {
     FMOE_HIP_CHECK(fmoe::launch_tiled_kernel(p, p.n_groups, stream));
+  } else if (p.split) {
+    FMOE_HIP_CHECK(fmoe::launch_split_kernel(p, p.n_groups, stream));
   } else {
     FMOE_HIP_CHECK(fmoe::launch_stream_kernel(p, desc->dtype, p.n_groups, stream));
   }

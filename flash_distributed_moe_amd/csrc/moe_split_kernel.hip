@@ -1,0 +1,638 @@
+// Persistent MoE kernel, split-k variant for gfx950: batches of up to 24 rows an expert (bf16,
+// tiles of one or two 16-row blocks). A wave of the streaming
+// variant carries a task of 64 weight rows over the whole of k alone: with few experts in use
+// most waves have no task at all and the others need 256 KiB each through one wave's window of
+// loads (one token on the 30B shape: 192 tasks on 2048 waves), and with many the launch ends in
+// a tail of whole tasks. Here the eight waves of a workgroup share a task's k (gate/up: eight
+// parts; down: two tasks side by side in four parts, or one in eight where that leaves a CU idle),
+// so tasks are an eighth as long, and meet in LDS: every wave leaves its partial sums there, one
+// barrier, and one or two waves add the parts in k order and store. The window of loads does not
+// drain between tasks: a slot is asked for again, for the step SPLIT_U later of the wave's sequence
+// of tasks, as soon as its matrix instructions have read it. Tasks are handed out statically
+// (equal shares of equal tasks), the routing tables are built by every workgroup for itself in
+// LDS from the top-k entries, and there is one grid-wide dependency between gate/up and down,
+// under which the first window of down weights is on its way.
+//
+// Bound by HBM from some 16 tokens on, below by the chain of waits (logit chains 14 us, selection,
+// gate/up, down, combine). Against the streaming kernel, us, 30B shape, weights packed in place:
+// T=1 59.5 -> 42, T=8 120 -> 103, T=16 164 -> 150, T=64 225 -> 217 (1.19 GB: 5.5 TB/s), T=128 243 -> 223,
+// T=200 266 -> 234, T=256 275 -> 241; row-major T=32 249 -> 226, T=128 290 -> 261; 235B T=1 102 -> 87,
+// T=64 759 -> 762, T=256 876 -> 836. Four hot experts: T=16 146 -> 120, T=128 317 -> 240 (a tile of more
+// rows than an early task carries starts over there; here it is several tiles).
+//
+// Where the batch reaches most experts, the first workgroups (as many as whole experts fill; those
+// with a routing task behind it) ask for the first window of (expert b / nt1, columns b % nt1)
+// before the routing is known and keep it if the expert turns out to be in use.
+//
+// Replaces, for this regime, the reference's moeKernel
+// (src/hip/kernel/moeKernel.h:37-107), its task executors
+// (src/hip/kernel/tasks/*.h) and its queue (src/hip/taskSystem/*.h).
+#include "moe_stream_device.h"
+
+namespace fmoe {
+
+// k-steps of a wave's window, by 16-row blocks of the tile (eight and six do not fit the registers
+// beside the epilogue: with eight for one block the window's last loads were spilled, T = 64 306 us)
+constexpr int split_u(int rb) { return rb == 1 ? 6 : 4; }
+constexpr int SPLIT_MAX_TILES = MAX_EXPERTS + SPLIT_MAX_SLOTS / 16;
+// LDS: the tables, then two sets of partial sums ([wave][weight block][row block][lane][4]); the
+// routing tasks use it from its first byte on before that
+constexpr int SPLIT_TILE_OFF = 0;
+constexpr int SPLIT_MASK_OFF = SPLIT_TILE_OFF + SPLIT_MAX_TILES * 8;
+constexpr int SPLIT_W_OFF = SPLIT_MASK_OFF + SCAN_LDS_WORDS * 8;
+constexpr int SPLIT_PERM_OFF = SPLIT_W_OFF + SPLIT_MAX_SLOTS * 4;
+constexpr int SPLIT_TOK_OFF = SPLIT_PERM_OFF + SPLIT_MAX_SLOTS * 2;
+constexpr int SPLIT_OFF_OFF = SPLIT_TOK_OFF + SPLIT_MAX_SLOTS * 2;
+constexpr int SPLIT_SPEC_OFF = SPLIT_OFF_OFF + MAX_EXPERTS * 4;
+constexpr int SPLIT_NOTE_OFF = SPLIT_SPEC_OFF + MAX_EXPERTS * 4;
+constexpr int SPLIT_PART_OFF = SPLIT_NOTE_OFF + 64;
+static_assert(SPLIT_PART_OFF % 16 == 0, "partial sums are read 16 bytes at a time");
+constexpr int split_part_bytes(int rb) { return 8 * 4 * rb * 64 * 16; }
+constexpr int split_lds_bytes(int rb) {
+  const int n = SPLIT_PART_OFF + 2 * split_part_bytes(rb);
+  return n > 8 * ROUTER_LDS_FLOATS * 4 ? n : 8 * ROUTER_LDS_FLOATS * 4;
+}
+static_assert(split_lds_bytes(2) + 64 <= 160 * 1024, "LDS of a workgroup");
+
+// LDS operations of this wave are done, then the workgroup barrier (loads from memory stay in flight)
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// A tile as the tables hold it: at most 16 * RB rows of one expert.
+struct SplitTile {
+  int expert, row0, rows;
+};
+__device__ __forceinline__ SplitTile split_tile(const uint2* tiles, int i) {
+  const uint2 v = tiles[i];
+  SplitTile t;
+  t.expert = __builtin_amdgcn_readfirstlane(static_cast<int>(v.x));
+  const int rr = __builtin_amdgcn_readfirstlane(static_cast<int>(v.y));
+  t.row0 = rr & 0xFFFF;
+  t.rows = rr >> 16;
+  return t;
+}
+
+// The window: U k-steps of four 16-row weight blocks and RB blocks of token rows. PACKED weights
+// are one run of 4 KiB a step; row-major ones four row-order loads (see fragment_from_row_order).
+template <bool PACKED, bool DOWN, int RB>
+struct SplitStream {
+  static constexpr int NP = PACKED ? 1 : 4;
+  static constexpr int U = split_u(RB);
+  uint4 a[U][4], b[U][RB];
+  const unsigned char* ap[NP];   // where the next step's weights are
+  const unsigned char* bp[RB];   // ... and its token rows (gate/up)
+  unsigned boff[RB];             // ... or h rows, as offsets (down)
+  int astep, bstep, left;        // bytes to the next step (0 behind the last task); steps left of the task
+  CoherentBuffer cb;
+
+  __device__ __forceinline__ void load_a(int u) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[u][i] = PACKED ? ld16_once(ap[0] + i * 1024) : ld16(ap[i]);
+#pragma unroll
+    for (int q = 0; q < NP; ++q) ap[q] += astep;
+  }
+  __device__ __forceinline__ void load_b(int u) {
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      if (DOWN) {
+        b[u][r] = ld16_agent(cb, boff[r]);
+        boff[r] += static_cast<unsigned>(bstep);
+      } else {
+        b[u][r] = ld16(bp[r]);
+        bp[r] += bstep;
+      }
+    }
+  }
+  // Behind the last task the loads go on (their number must not depend on a branch, or the
+  // compiler waits for all of them at every step), all lanes at one address that exists.
+  __device__ __forceinline__ void park(const void* somewhere) {
+#pragma unroll
+    for (int q = 0; q < NP; ++q) ap[q] = reinterpret_cast<const unsigned char*>(somewhere);
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      bp[r] = reinterpret_cast<const unsigned char*>(somewhere);
+      boff[r] = 0u;
+    }
+    astep = bstep = 0;
+    left = 0x7FFFFFFF;
+  }
+  __device__ __forceinline__ void mma(int u, int pull_from, f32x4 (&acc)[4][RB]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint4 w = PACKED ? a[u][i] : fragment_from_row_order(a[u][i], pull_from);
+#pragma unroll
+      for (int r = 0; r < RB; ++r) acc[i][r] = mma16<BF16>(w, b[u][r], acc[i][r]);
+    }
+  }
+  // this wave's partial sums of a task go to LDS, and the accumulators back to zero
+  __device__ __forceinline__ void leave(f32x4* part, int wave, f32x4 (&acc)[4][RB]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < RB; ++r) {
+        part[((wave * 4 + i) * RB + r) * 64 + lane_id()] = acc[i][r];
+        acc[i][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  }
+};
+
+template <bool PACKED, int RB>
+__global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_split_kernel(const Params params) {
+  ParamsRef p = kernel_params();
+  __shared__ unsigned lds_flag[4];
+  __shared__ unsigned lds_poller[4];
+  if (threadIdx.x < 4) {
+    lds_flag[threadIdx.x] = 0u;
+    lds_poller[threadIdx.x] = 0u;
+  }
+  __syncthreads();
+  const int tid = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int G = static_cast<int>(gridDim.x), b = static_cast<int>(blockIdx.x);
+  Control* ctl = p.ctl;
+  const int T = p.T, E = p.E, H = p.H, K = p.K, I = p.I, W = p.W;
+  unsigned char* lds = reinterpret_cast<unsigned char*>(lds_dyn);
+  constexpr int U = split_u(RB), TILE_ROWS = 16 * RB;
+  unsigned short* lperm = reinterpret_cast<unsigned short*>(lds + SPLIT_PERM_OFF);  // permuted row -> token*K + slot
+  unsigned short* ltok = reinterpret_cast<unsigned short*>(lds + SPLIT_TOK_OFF);    // permuted row -> token
+  float* lw = reinterpret_cast<float*>(lds + SPLIT_W_OFF);      // permuted row -> gate weight
+  unsigned long long* lmask = reinterpret_cast<unsigned long long*>(lds + SPLIT_MASK_OFF);
+  int* loff = reinterpret_cast<int*>(lds + SPLIT_OFF_OFF);      // expert -> first permuted row
+  uint2* tiles = reinterpret_cast<uint2*>(lds + SPLIT_TILE_OFF);
+  int* spec_tile = reinterpret_cast<int*>(lds + SPLIT_SPEC_OFF);  // expert -> its early tile, or -1
+  int* note = reinterpret_cast<int*>(lds + SPLIT_NOTE_OFF);
+
+  const int n_eg = (E + 15) >> 4;
+  const int n_dot = ((T + 15) >> 4) * n_eg;
+  const int nt1 = I / (16 * G1_NB), nt2 = H / (16 * G2_NB);
+  const int ks1 = H >> 5, ks2 = I >> 5;
+  const int pull_from = (((lane & 15) << 2) | (lane >> 4)) << 2;
+
+  // ---- routing: logit chains on the first workgroups, then one select a wave there
+  if (b < n_dot) {
+    router_dot16_task(p, b / n_eg, b % n_eg);
+    for (int t = b + n_dot * wave; t < T; t += 8 * n_dot) {
+      if (!wave_wait_ge(&p.tok_arrive[t], static_cast<unsigned>(n_eg), ctl, p.spin_limit)) break;
+      router_select_task(p, t);
+    }
+  }
+
+  // ---- gate/up weights before the routing is known
+  const int n_spec_experts = p.split_spec ? min(G / nt1, E) : 0;
+  const int n_spec = n_spec_experts * nt1;  // workgroups b < n_spec
+  const int k0 = ks1 * wave / 8, steps1 = ks1 * (wave + 1) / 8 - k0;
+  f32x4 acc[4][RB];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < RB; ++r) acc[i][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bool ok;
+  int ntiles = 0;
+  int cnt = 0;  // tasks this workgroup has finished: its parity names the set of partial sums
+  {
+    SplitStream<PACKED, false, RB> st;
+    st.cb = coherent_buffer(p.h, 0u);
+    auto weights = [&](int expert, int nblk) {
+      if constexpr (PACKED) {
+        const size_t task = static_cast<size_t>(expert) * nt1 + nblk;
+        st.ap[0] = reinterpret_cast<const unsigned char*>(p.ffn1_packed) + (task * ks1 + k0) * 4096 + lane * 16;
+        st.astep = 4096;
+      } else {
+        const unsigned char* w13 = reinterpret_cast<const unsigned char*>(p.ffn1) +
+                                   static_cast<size_t>(expert) * 2 * I * H * 2 + k0 * 64 + row_order_chunk() * 16;
+        const int n0 = nblk * (16 * G1_NB) + row_order_row();
+#pragma unroll
+        for (int q = 0; q < G1_NB; ++q) {
+          st.ap[q] = w13 + static_cast<size_t>(n0 + 16 * q) * H * 2;
+          st.ap[G1_NB + q] = w13 + static_cast<size_t>(I + n0 + 16 * q) * H * 2;
+        }
+        st.astep = 64;
+      }
+      st.left = steps1;
+    };
+    if (b < n_spec) {
+      weights(b / nt1, b % nt1);
+    } else {
+      st.park(p.gate);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      st.load_a(u);
+      // (a task shorter than the window: the slots behind it are filled again below)
+      if (u + 1 == steps1) st.park(p.gate);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+
+    // ---- tables, by every workgroup for itself
+    ok = wait_flag(p, FLAG_ROUTED, lds_flag, lds_poller);
+    const int wact = (T + 63) >> 6;
+    const int n = T * K;
+    lds_barrier();  // the routing tasks' use of the LDS is over
+    int ee[SPLIT_MAX_SLOTS / 512];
+    float ww[SPLIT_MAX_SLOTS / 512];
+    if (ok) {
+#pragma unroll
+      for (int q = 0; q < SPLIT_MAX_SLOTS / 512; ++q) {
+        const int i = tid + 512 * q;
+        ee[q] = i < n ? ldc(&p.topk_idx[i]) : -1;
+        ww[q] = i < n ? ldc(&p.topk_w[i]) : 0.0f;
+      }
+      for (int i = tid; i < E * wact; i += 512) lmask[i] = ldc(&p.masks[static_cast<size_t>(i / wact) * W + i % wact]);
+    }
+    lds_barrier();
+    if (ok && wave == 0) {
+      int base = 0, rest = 0, spec = 0;
+      const int epl = (E + 63) >> 6;
+      for (int pass = 0; pass < 2; ++pass) {  // the early tiles stand behind all others
+        if (pass == 1) base = 0;
+        for (int j = 0; j < epl; ++j) {
+          const int e = lane + 64 * j;
+          int c = 0;
+          if (e < E)
+            for (int w = 0; w < wact; ++w) c += __popcll(lmask[e * wact + w]);
+          const int off = base + wave_inclusive_scan(c) - c;
+          base = __shfl(off + c, 63, 64);
+          const int nt = (c + TILE_ROWS - 1) / TILE_ROWS;
+          const bool early = e < n_spec_experts && c > 0;
+          const int mine = pass == 0 ? nt - (early ? 1 : 0) : (early ? 1 : 0);
+          const int incl = wave_inclusive_scan(mine);
+          if (pass == 0) {
+            if (e < E) loff[e] = off;
+            for (int i = 0; i < mine; ++i) {
+              const int r = (i + (early ? 1 : 0)) * TILE_ROWS;
+              tiles[rest + incl - mine + i] =
+                  make_uint2(static_cast<unsigned>(e), static_cast<unsigned>((off + r) | (min(TILE_ROWS, c - r) << 16)));
+            }
+            rest += __shfl(incl, 63, 64);
+          } else {
+            if (e < E) spec_tile[e] = early ? rest + spec + incl - 1 : -1;
+            if (early)
+              tiles[rest + spec + incl - 1] =
+                  make_uint2(static_cast<unsigned>(e), static_cast<unsigned>(off | (min(TILE_ROWS, c) << 16)));
+            spec += __shfl(incl, 63, 64);
+          }
+        }
+      }
+      if (lane == 0) {
+        note[0] = rest;
+        note[1] = rest + spec;
+        note[2] = base;
+      }
+    }
+    lds_barrier();
+    int n_rest = 0;
+    if (ok) {
+      n_rest = __builtin_amdgcn_readfirstlane(note[0]);
+      ntiles = __builtin_amdgcn_readfirstlane(note[1]);
+#pragma unroll
+      for (int q = 0; q < SPLIT_MAX_SLOTS / 512; ++q) {
+        const int i = tid + 512 * q;
+        if (ee[q] >= 0) {
+          const int t = i / K, wd = t >> 6;
+          int pos = loff[ee[q]] + __popcll(lmask[ee[q] * wact + wd] & ((1ull << (t & 63)) - 1ull));
+          for (int w = 0; w < wd; ++w) pos += __popcll(lmask[ee[q] * wact + w]);
+          lperm[pos] = static_cast<unsigned short>(i);
+          ltok[pos] = static_cast<unsigned short>(t);
+          lw[pos] = ww[q];
+          if (b == G - 1) stc(&p.perm[pos], i);
+        }
+      }
+      if (b == G - 1) {  // the tables the host may read back
+        const int total = note[2];
+        for (int e = tid; e < E; e += 512) {
+          const int off = loff[e];
+          stc(&p.expert_offset[e], off);
+          stc(&p.expert_count[e], (e + 1 < E ? loff[e + 1] : total) - off);
+        }
+        if (tid == 0) stc(&p.expert_offset[E], total);
+      }
+    }
+    lds_barrier();
+
+    // ---- gate/up: the early task, then an equal share of the rest (workgroups without an early
+    // task first)
+    const int my_spec = ok && b < n_spec ? __builtin_amdgcn_readfirstlane(spec_tile[b / nt1]) : -1;
+    const int rank = b >= n_spec ? b - n_spec : b + G - n_spec;
+    const int n_tasks = n_rest * nt1;
+    int ntask = (my_spec >= 0 ? 1 : 0) + (rank < n_tasks ? (n_tasks - rank + G - 1) / G : 0);
+    int lq = rank;  // next task of the rest to load, and (cq) to finish
+    int cq = rank;
+    bool cspec = my_spec >= 0;
+    auto rows_of = [&](const SplitTile& t) {
+#pragma unroll
+      for (int r = 0; r < RB; ++r)
+        st.bp[r] = reinterpret_cast<const unsigned char*>(p.tokens) +
+                   (static_cast<size_t>(ltok[t.row0 + min(16 * r + r16, t.rows - 1)]) * H + k0 * 32 + g * 8) * 2;
+      st.bstep = 64;
+    };
+    auto next_task = [&]() {
+      if (lq < n_tasks) {
+        const SplitTile t = split_tile(tiles, lq / nt1);
+        weights(t.expert, lq % nt1);
+        rows_of(t);
+        lq += G;
+      } else {
+        st.park(p.gate);
+      }
+    };
+    auto finish = [&]() {  // the task's eight parts: add up, SiLU(gate) * up, store
+      const int q = cspec ? b : cq;
+      const SplitTile t = split_tile(tiles, cspec ? my_spec : q / nt1);
+      const int n0 = (q % nt1) * (16 * G1_NB);
+      if (!cspec) cq += G;
+      cspec = false;
+      f32x4* part = reinterpret_cast<f32x4*>(lds + SPLIT_PART_OFF + (cnt & 1) * split_part_bytes(RB));
+      st.leave(part, wave, acc);
+      lds_barrier();
+      const int turn = (wave - 2 * RB * cnt) & 7;  // the adding waves take turns
+      const int i = turn & 1, r = turn >> 1;
+      ++cnt;
+      if (r < RB) {
+        f32x4 s = part[(i * RB + r) * 64 + lane], v = part[((i + 2) * RB + r) * 64 + lane];
+#pragma unroll 1  // (more reads in flight cost the window its registers)
+        for (int w = 1; w < 8; ++w) {
+          s += part[((w * 4 + i) * RB + r) * 64 + lane];
+          v += part[((w * 4 + i + 2) * RB + r) * 64 + lane];
+        }
+        const int row = 16 * r + r16;
+        if (row < t.rows) {
+          unsigned hv[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {  // (one after the other, for the same reason)
+            hv[k] = f2bf(silu_mul(s[k], v[k]));
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          const unsigned lo = hv[0] | (hv[1] << 16), hi = hv[2] | (hv[3] << 16);
+          stc(reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned short*>(p.h) +
+                                                    static_cast<size_t>(t.row0 + row) * I + n0 + 16 * i + 4 * g),
+              static_cast<unsigned long long>(lo) | (static_cast<unsigned long long>(hi) << 32));
+        }
+      }
+    };
+    if (ntask > 0) {
+      if (my_spec >= 0 && steps1 >= U) {
+        // the window is this task's: its token rows join it
+        rows_of(split_tile(tiles, my_spec));
+        if (steps1 == U) {
+          st.left = 0;
+        } else {
+          st.left = steps1 - U;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) st.load_b(u);
+        if (st.left == 0) next_task();
+      } else {
+        if (my_spec >= 0) {
+          weights(b / nt1, b % nt1);
+          rows_of(split_tile(tiles, my_spec));
+        } else {
+          next_task();
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          st.load_a(u);
+          st.load_b(u);
+          if (--st.left == 0) next_task();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      int cleft = steps1;
+      auto round = [&]() {  // true: the last task is finished
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          st.mma(u, pull_from, acc);
+          __builtin_amdgcn_sched_barrier(0);
+          st.load_a(u);
+          st.load_b(u);
+          __builtin_amdgcn_sched_barrier(0);
+          if (--st.left == 0) next_task();
+          if (--cleft == 0) {
+            finish();
+            if (--ntask == 0) return true;
+            cleft = steps1;
+          }
+        }
+        return false;
+      };
+      if (!round()) {
+        asm volatile("; end of the first round" ::: "memory");  // as in stream_mma
+        while (!round()) {
+        }
+      }
+    }
+  }
+
+  // ---- every h row is final once all workgroups have been here
+  const int parts = p.split_down;            // waves that share a down task: 4 or 8
+  const int sub = wave & (parts - 1), grp = parts == 8 ? 0 : wave >> 2;
+  const int per_tile = parts == 8 ? nt2 : nt2 >> 1;  // workgroup tasks of one tile
+  if (ok) {
+    fence_release();
+    lds_barrier();
+    if (wave == 0) {
+      unsigned old = 0;
+      if (lane == 0) old = add_relaxed(&ctl->perm_done.v, 1u);
+      old = __builtin_amdgcn_readfirstlane(old);
+      if (old == static_cast<unsigned>(G) - 1u) broadcast_flag(p, FLAG_PERM);
+    }
+    const int d0 = ks2 * sub / parts, steps2 = ks2 * (sub + 1) / parts - d0;
+    const int n_tasks = ntiles * per_tile;
+    int ntask = b < n_tasks ? (n_tasks - b + G - 1) / G : 0;
+    if (ntask > 0) {
+      SplitStream<PACKED, true, RB> st;
+      st.cb = coherent_buffer(p.h, static_cast<unsigned>(T * K * I * 2));
+      int lq = b, cq = b;
+      auto next_task = [&]() {
+        if (lq < n_tasks) {
+          const SplitTile t = split_tile(tiles, lq / per_tile);
+          const int nblk = parts == 8 ? lq % per_tile : (lq % per_tile) * 2 + grp;
+          if constexpr (PACKED) {
+            const size_t task = static_cast<size_t>(t.expert) * nt2 + nblk;
+            st.ap[0] = reinterpret_cast<const unsigned char*>(p.ffn2_packed) + (task * ks2 + d0) * 4096 + lane * 16;
+            st.astep = 4096;
+          } else {
+            const unsigned char* w2 = reinterpret_cast<const unsigned char*>(p.ffn2) +
+                                      static_cast<size_t>(t.expert) * H * I * 2 + d0 * 64 + row_order_chunk() * 16;
+            const int n0 = nblk * (16 * G2_NB) + row_order_row();
+#pragma unroll
+            for (int q = 0; q < st.NP; ++q) st.ap[q] = w2 + static_cast<size_t>(n0 + 16 * q) * I * 2;
+            st.astep = 64;
+          }
+#pragma unroll
+          for (int r = 0; r < RB; ++r)
+            st.boff[r] = static_cast<unsigned>(((t.row0 + min(16 * r + r16, t.rows - 1)) * I + d0 * 32 + g * 8) * 2);
+          st.bstep = 64;
+          st.left = steps2;
+          lq += G;
+        } else {
+          st.park(p.gate);
+        }
+      };
+      // The weights of the first window go out before the wait, the h rows behind it: both walk
+      // through the same steps.
+      next_task();
+      const int lq0 = lq;
+      unsigned boff0[RB];
+#pragma unroll
+      for (int r = 0; r < RB; ++r) boff0[r] = st.boff[r];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        st.load_a(u);
+        if (--st.left == 0) next_task();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      ok = wait_flag(p, FLAG_PERM, lds_flag, lds_poller);
+      if (ok) {
+        const unsigned char* keep[st.NP];
+#pragma unroll
+        for (int q = 0; q < st.NP; ++q) keep[q] = st.ap[q];
+        lq = lq0;
+#pragma unroll
+        for (int r = 0; r < RB; ++r) st.boff[r] = boff0[r];
+        st.bstep = 64;
+        st.left = steps2;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          st.load_b(u);
+          if (--st.left == 0) next_task();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 0; q < st.NP; ++q) st.ap[q] = keep[q];
+        auto finish = [&]() {
+          const SplitTile t = split_tile(tiles, cq / per_tile);
+          const int n0 = (parts == 8 ? cq % per_tile : (cq % per_tile) * 2 + grp) * (16 * G2_NB);
+          cq += G;
+          f32x4* part = reinterpret_cast<f32x4*>(lds + SPLIT_PART_OFF + (cnt & 1) * split_part_bytes(RB));
+          st.leave(part, wave, acc);
+          lds_barrier();
+          // (four blocks for eight waves: one half of them, then the other)
+          const int first = parts > 4 * RB ? (sub + 4 * (cnt & 1)) & 7 : sub;
+          ++cnt;
+          for (int blk = first; blk < 4 * RB; blk += parts) {
+            const int i = blk & 3, r = blk >> 2;
+            f32x4 s = part[((grp * 16 + i) * RB + r) * 64 + lane];
+#pragma unroll 1
+            for (int w = 1; w < parts; ++w) s += part[(((grp * 4 + w) * 4 + i) * RB + r) * 64 + lane];
+            const int row = 16 * r + r16;
+            if (row < t.rows) {
+              const float wt = lw[t.row0 + row];
+              st16_through(p.y + static_cast<size_t>(lperm[t.row0 + row]) * H + n0 + 16 * i + 4 * g,
+                           make_uint4(__float_as_uint(s[0] * wt), __float_as_uint(s[1] * wt),
+                                      __float_as_uint(s[2] * wt), __float_as_uint(s[3] * wt)));
+            }
+          }
+        };
+        int cleft = steps2;
+        auto round = [&]() {
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            st.mma(u, pull_from, acc);
+            __builtin_amdgcn_sched_barrier(0);
+            st.load_a(u);
+            st.load_b(u);
+            __builtin_amdgcn_sched_barrier(0);
+            if (--st.left == 0) next_task();
+            if (--cleft == 0) {
+              finish();
+              if (--ntask == 0) return true;
+              cleft = steps2;
+            }
+          }
+          return false;
+        };
+        if (!round()) {
+          asm volatile("; end of the first round" ::: "memory");
+          while (!round()) {
+          }
+        }
+      }
+    }
+  }
+
+  // ---- combine, by the waves that have an item
+  if (ok) {
+    fence_release();
+    lds_barrier();
+    if (wave == 0) {
+      unsigned old = 0;
+      if (lane == 0) old = add_relaxed(&ctl->g2_done.v, 1u);
+      old = __builtin_amdgcn_readfirstlane(old);
+      if (old == static_cast<unsigned>(G) - 1u) broadcast_flag(p, FLAG_G2);
+    }
+    const unsigned ncomb = static_cast<unsigned>((H + COMBINE_COLS - 1) / COMBINE_COLS);
+    const unsigned nc = static_cast<unsigned>(T) * ncomb;
+    const unsigned slot = static_cast<unsigned>(wave * G + b);
+    if (slot < nc && wait_flag(p, FLAG_G2, lds_flag, lds_poller))
+      combine_items<BF16>(p, slot, nc, ncomb, static_cast<unsigned>(b * 8 + wave), 0u, 0);
+  }
+
+  // ---- the last workgroup out returns every counter to zero for the next launch
+  __syncthreads();
+  if (wave == 0) {
+    fence_release();  // flags this wave has raised for others have landed before anybody clears them
+    unsigned last = 0;
+    if (lane == 0) last = add_relaxed(&ctl->exit_count.v, 1u) == static_cast<unsigned>(G) - 1u ? 1u : 0u;
+    if (__builtin_amdgcn_readfirstlane(last) != 0u) {
+      const unsigned err = ldc(&ctl->error.v);
+      if (err != 0u) recover_after_error(p, err, lane, 64);
+      for (int q = lane; q < p.n_groups; q += 64) {
+        stc(&p.wgflags[q].f[FLAG_PERM], 0u);
+        stc(&p.wgflags[q].f[FLAG_G2], 0u);
+        stc(&p.wgflags[q].f[FLAG_ROUTED], 0u);
+      }
+      if (lane == 0) {
+        stc(&ctl->launches.v, ldc(&ctl->launches.v) + 1u);
+        stc(&ctl->router_done.v, 0u);
+        stc(&ctl->perm_done.v, 0u);
+        stc(&ctl->g2_done.v, 0u);
+        stc(&ctl->exit_count.v, 0u);
+      }
+    }
+  }
+}
+
+namespace {
+// The four kernels, and the dynamic LDS each is launched with.
+struct SplitUse {
+  const void* kernel;
+  int lds;
+};
+const SplitUse kSplitUses[] = {{reinterpret_cast<const void*>(moe_split_kernel<true, 1>), split_lds_bytes(1)},
+                               {reinterpret_cast<const void*>(moe_split_kernel<false, 1>), split_lds_bytes(1)},
+                               {reinterpret_cast<const void*>(moe_split_kernel<true, 2>), split_lds_bytes(2)},
+                               {reinterpret_cast<const void*>(moe_split_kernel<false, 2>), split_lds_bytes(2)}};
+}  // namespace
+
+hipError_t launch_split_kernel(const Params& p, int grid, hipStream_t stream) {
+  auto* kernel = p.split == 1 ? (p.ffn1_packed != nullptr ? moe_split_kernel<true, 1> : moe_split_kernel<false, 1>)
+                              : (p.ffn1_packed != nullptr ? moe_split_kernel<true, 2> : moe_split_kernel<false, 2>);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), split_lds_bytes(p.split), stream, p);
+  return hipGetLastError();
+}
+
+hipError_t prepare_split_kernel() {
+  for (const SplitUse& u : kSplitUses) {
+    const hipError_t e = hipFuncSetAttribute(u.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, u.lds);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+// the least of the kernels' numbers of workgroups a CU holds
+hipError_t split_kernel_occupancy(int* per_cu) {
+  *per_cu = 0x7FFFFFFF;
+  for (const SplitUse& u : kSplitUses) {
+    int n = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, u.kernel, 512, u.lds);
+    if (e != hipSuccess) return e;
+    if (n < *per_cu) *per_cu = n;
+  }
+  return hipSuccess;
+}
+
+}  // namespace fmoe

@@ -17,15 +17,14 @@
 // The down projection reads h rows that other workers wrote, so its B operand
 // uses coherent loads.
 //
-// bf16 batches of up to 24 rows an expert run a second kernel of this file instead, with
-// the same routing and combine: the split-k variant (moe_split_kernel, below), whose
-// workgroups share a task's k.
+// bf16 batches of up to 24 rows an expert run the split-k variant instead (moe_split_kernel.hip),
+// with the same routing and combine, whose workgroups share a task's k. It has a file of its own
+// because the float32 kernel's time depends on where its loops lie (see build.py).
 //
 // Replaces, for this regime, the reference's moeKernel
 // (src/hip/kernel/moeKernel.h:37-107), its task executors
 // (src/hip/kernel/tasks/*.h) and its queue (src/hip/taskSystem/*.h).
-#define FMOE_PARAMS_IN_KERNARG 1
-#include "moe_device.h"
+#include "moe_stream_device.h"
 
 namespace fmoe {
 
@@ -43,13 +42,7 @@ namespace fmoe {
 // wave's private LDS slice in k-chunks, and feed one sequential chain per lane
 // (k ascending). Each chain ends as a 64-bit candidate key in HBM. A "select"
 // task per token waits for all of the token's expert groups and picks the
-// winners.
-constexpr int ROUTER_KC = 256;   // k-chunk staged in LDS
-constexpr int ROUTER_LD = ROUTER_KC + 4;  // LDS row stride in floats (bank spread)
-constexpr int ROUTER_LDS_FLOATS = 2 * ROUTER_EXP * ROUTER_LD;  // per wave
-
-extern __shared__ __align__(16) float lds_dyn[];  // ROUTER_LDS_FLOATS per wave
-
+// winners. (bf16 layers of suitable shape run the chains on the matrix core: router_dot16_task.)
 template <typename DT>
 __device__ __noinline__ void router_dot_task(ParamsRef pv, int tg, int eg) {
   ParamsRef p = uniform_params(pv);
@@ -182,157 +175,6 @@ __device__ __noinline__ void router_dot_task(ParamsRef pv, int tg, int eg) {
   }
   fence_release();
   if (ei == 0 && t < T) add_relaxed(&p.tok_arrive[t], 1u);
-}
-
-// The same chains on the matrix core, for bf16 layers: V_MFMA_F32_16X16X4_F32 adds
-// its four products to the accumulator one after the other in k order, one
-// rounding each, so a chain of them is the same sequential sum (and a dependent
-// chain issues back to back, 32 cycles an instruction: 512 of them for H = 2048
-// against 2048 dependent FMAs on the vector unit). A whole workgroup takes 16
-// tokens x 16 experts: wave 0 only multiplies, waves 1..4 prepare its operands so
-// that it has nothing else to do: they load 32 bytes of a row (16 k), widen them
-// to float and leave them in LDS in the order the instruction wants them: the 16
-// k of a group as [k % 4][row][k / 4], so lane l of the multiplying wave (row
-// l % 16, k % 4 = l / 16) reads its operand of four consecutive instructions with
-// one 16-byte read at 16 * l. Two stages of DOT16_KC k; one workgroup barrier per
-// stage; the preparing waves hold the loads of eight stages in registers.
-// Called by all eight waves of the workgroup.
-constexpr int DOT16_GROUPS = DOT16_KC / 16;             // 16-k groups per stage
-constexpr int DOT16_OP_BYTES = DOT16_GROUPS * 1024;     // one operand of one stage
-constexpr int DOT16_STAGE_BYTES = 2 * DOT16_OP_BYTES;   // expert rows, then token rows
-constexpr int DOT16_AHEAD = 8;                          // stages whose loads are in flight together (even)
-
-__device__ __noinline__ void router_dot16_task(ParamsRef pv, int tg, int eg) {
-  ParamsRef p = uniform_params(pv);
-  const int H = p.H, E = p.E, T = p.T;
-  const int lane = lane_id();
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int nc = H / DOT16_KC;
-  unsigned char* lds = reinterpret_cast<unsigned char*>(lds_dyn);
-  auto barrier = [] {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-  if (wave == 0) {
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const unsigned char* mine = lds + lane * 16;
-    float4 wc, xc, wn, xn;
-    barrier();  // stage 0 is written
-    wc = *reinterpret_cast<const float4*>(mine);
-    xc = *reinterpret_cast<const float4*>(mine + DOT16_OP_BYTES);
-    for (int c = 0; c < nc; ++c) {
-      const unsigned char* st = mine + (c & 1) * DOT16_STAGE_BYTES;
-      const unsigned char* st_next = mine + ((c + 1) & 1) * DOT16_STAGE_BYTES;
-#pragma unroll
-      for (int g = 0; g < DOT16_GROUPS; ++g) {
-        if (g + 1 < DOT16_GROUPS) {
-          wn = *reinterpret_cast<const float4*>(st + (g + 1) * 1024);
-          xn = *reinterpret_cast<const float4*>(st + DOT16_OP_BYTES + (g + 1) * 1024);
-        } else {
-          // every read of this stage has returned: the stage may be refilled, and
-          // the next one is complete once the others have arrived too
-          barrier();
-          if (c + 1 < nc) {
-            wn = *reinterpret_cast<const float4*>(st_next);
-            xn = *reinterpret_cast<const float4*>(st_next + DOT16_OP_BYTES);
-          }
-        }
-        // the reads of the next group go out before this group's instructions, not after
-        __builtin_amdgcn_sched_barrier(0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wc.x, xc.x, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wc.y, xc.y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wc.z, xc.z, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wc.w, xc.w, acc, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        wc = wn;
-        xc = xn;
-      }
-    }
-    // acc[v] of lane l: expert 16*eg + 4*(l/16) + v, token 16*tg + l%16
-    const int t = tg * 16 + (lane & 15);
-    const int e0 = eg * 16 + 4 * (lane >> 4);
-    if (t < T) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int e = e0 + v;
-        if (e < E) {
-          float x = acc[v];
-          if (p.bias != nullptr) x = __fadd_rn(x, as_global(p.bias)[e]);
-          stc(&p.cand[static_cast<size_t>(t) * E + e], make_key(x, e, true));
-        }
-      }
-    }
-    fence_release();
-    if (lane < 16 && t < T) add_relaxed(&p.tok_arrive[t], 1u);
-  } else if (wave <= 4) {
-    // lane -> (row, group): four lanes cover 128 contiguous bytes of a row
-    const int hl = (wave - 1) * 64 + lane;
-    const int row = (hl & 63) >> 2;
-    const int g = (hl >> 6) * 4 + (hl & 3);
-    const unsigned short* wsrc = reinterpret_cast<const unsigned short*>(p.gate) +
-                                 static_cast<size_t>(min(eg * 16 + row, E - 1)) * H + g * 16;
-    const unsigned short* xsrc = reinterpret_cast<const unsigned short*>(p.tokens) +
-                                 static_cast<size_t>(min(tg * 16 + row, T - 1)) * H + g * 16;
-    unsigned char* dst = lds + g * 1024 + row * 16;
-    struct Regs {
-      uint4 w0, w1, x0, x1;
-    };
-    auto load = [&](Regs& r, int c) {
-      const int k = min(c, nc - 1) * DOT16_KC;  // past the end: the last stage again, never written
-      r.w0 = ld16(wsrc + k);
-      r.w1 = ld16(wsrc + k + 8);
-      r.x0 = ld16(xsrc + k);
-      r.x1 = ld16(xsrc + k + 8);
-    };
-    auto widen = [](unsigned char* d, const uint4& a, const uint4& b) {
-      // k % 4 = 0 and 1: low and high halves of the even words; 2 and 3: of the odd words
-      *reinterpret_cast<uint4*>(d) = make_uint4(a.x << 16, a.z << 16, b.x << 16, b.z << 16);
-      *reinterpret_cast<uint4*>(d + 256) =
-          make_uint4(a.x & 0xFFFF0000u, a.z & 0xFFFF0000u, b.x & 0xFFFF0000u, b.z & 0xFFFF0000u);
-      *reinterpret_cast<uint4*>(d + 512) = make_uint4(a.y << 16, a.w << 16, b.y << 16, b.w << 16);
-      *reinterpret_cast<uint4*>(d + 768) =
-          make_uint4(a.y & 0xFFFF0000u, a.w & 0xFFFF0000u, b.y & 0xFFFF0000u, b.w & 0xFFFF0000u);
-    };
-    // The loads of DOT16_AHEAD stages go out together (straight-line code, so each
-    // stage waits for exactly its own four): a load takes 2 to 3 us to come back
-    // here, three times what the multiplying wave spends on a stage.
-    for (int c0 = 0; c0 < nc; c0 += DOT16_AHEAD) {
-      Regs r[DOT16_AHEAD];
-#pragma unroll
-      for (int i = 0; i < DOT16_AHEAD; ++i) load(r[i], c0 + i);
-#pragma unroll
-      for (int i = 0; i < DOT16_AHEAD; ++i) {
-        if (c0 + i < nc) {
-          unsigned char* d = dst + (i & 1) * DOT16_STAGE_BYTES;
-          widen(d, r[i].w0, r[i].w1);
-          widen(d + DOT16_OP_BYTES, r[i].x0, r[i].x1);
-          barrier();  // the stage is written; the multiplying wave is done with the one before
-        }
-      }
-    }
-    barrier();  // the multiplying wave has read everything: the LDS is free again
-  } else {
-    for (int c = 0; c <= nc; ++c) barrier();
-  }
-}
-
-// All expert groups of token t have left their keys: pick the winners.
-__device__ __noinline__ void router_select_task(ParamsRef pv, int t) {
-  ParamsRef p = uniform_params(pv);
-  constexpr int MAXEPL = MAX_EXPERTS / 64;
-  const int lane = lane_id();
-  unsigned val[MAXEPL];  // the ordered logit bits are the upper half of a candidate key
-#pragma unroll
-  for (int j = 0; j < MAXEPL; ++j) {
-    const int e = lane + 64 * j;
-    val[j] = e < p.E ? static_cast<unsigned>(ldc(&p.cand[static_cast<size_t>(t) * p.E + e]) >> 32) : 0u;
-  }
-  if (lane == 0) stc(&p.tok_arrive[t], 0u);
-  router_select_max(p, t, val,
-                    reinterpret_cast<double*>(lds_dyn + (threadIdx.x >> 6) * ROUTER_LDS_FLOATS));
-  const unsigned old = wave_arrive(&p.ctl->router_done.v);
-  if (p.early && old == static_cast<unsigned>(p.T) - 1u) broadcast_flag(p, FLAG_ROUTED);
 }
 
 // ------------------------------------------------------------- scan / scatter
@@ -548,78 +390,14 @@ __device__ void scatter_task(ParamsRef p, int t) {
   if (old == static_cast<unsigned>(r.T) - 1u) broadcast_flag(p, FLAG_PERM);
 }
 
-// Wave-uniform bounded wait for this workgroup's copy of a phase flag. Only one
-// wave of the workgroup polls HBM; the others watch a word in LDS that the
-// polling wave sets (1 = flag seen, 2 = failed).
-__device__ __forceinline__ bool wait_flag(ParamsRef p, int which, unsigned* lds_flag,
-                                          unsigned* lds_poller) {
-  int ok = 1;
-  if (lane_id() == 0) {
-    while (true) {
-      const unsigned f = __hip_atomic_load(&lds_flag[which], __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-      if (f != 0u) {
-        ok = f == 1u;
-        break;
-      }
-      if (__hip_atomic_exchange(&lds_poller[which], 1u, __ATOMIC_RELAXED,
-                                __HIP_MEMORY_SCOPE_WORKGROUP) == 0u) {
-        // this wave polls for the workgroup
-        const unsigned* g = &p.wgflags[blockIdx.x].f[which];
-        const long long t0 = wall_clock64();
-        unsigned spins = 0;
-        unsigned res = 1u;
-        while (ld_relaxed(g) == 0u) {
-          if ((++spins & 31u) == 0u && ld_relaxed(&p.ctl->error.v) != 0u) {
-            res = 2u;
-            break;
-          }
-          if (wall_clock64() - t0 > p.spin_limit) {
-            or_relaxed(&p.ctl->error.v, ERR_TIMEOUT);
-            res = 2u;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(16);
-        }
-        __hip_atomic_store(&lds_flag[which], res, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        ok = res == 1u;
-        break;
-      }
-      __builtin_amdgcn_s_sleep(8);
-    }
-  }
-  ok = __builtin_amdgcn_readfirstlane(ok);
-  fence_acquire();
-  return ok != 0;
-}
-
 // ------------------------------------------------- streaming 16x16 MFMA sweep
 // acc[i][r] += A_i (16 weight rows) . B_r (16 token rows)^T over `ksteps` steps
 // of 4*EPV elements. ap[i] / bp[r] already point at this lane's row and
 // k-offset. Each round issues U steps' worth of 16-byte loads and then feeds
 // the MFMAs; the other waves of the CU keep HBM busy meanwhile. `pre` runs once
 // after the first round's weight loads are in flight and before any B row is
-// touched (the down projection waits for its h rows there).
-//
-// transpose_a (the caller's row-major weights): a fragment wants lane l to hold row l % 16,
-// 16-byte chunk l / 16 of a 64-byte row segment, which read that way makes every lane of a
-// load touch a line of its own.
-// So lane l loads chunk l % 4 of row l / 4 instead, four neighbouring lanes one contiguous
-// 64-byte segment, and the fragment is put right in registers afterwards: lane l takes the
-// four dwords of lane 4 * (l % 16) + l / 16 (ds_bpermute_b32: the LDS crossbar, no LDS memory).
-__device__ __forceinline__ uint4 fragment_from_row_order(const uint4& v, int pull_from) {
-  uint4 r;
-  r.x = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(pull_from, static_cast<int>(v.x)));
-  r.y = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(pull_from, static_cast<int>(v.y)));
-  r.z = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(pull_from, static_cast<int>(v.z)));
-  r.w = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(pull_from, static_cast<int>(v.w)));
-  return r;
-}
-// row and 16-byte chunk (of the 64-byte segment of one k-step) that this lane loads of a
-// 16-row weight block in the caller's row-major layout
-__device__ __forceinline__ int row_order_row() { return lane_id() >> 2; }
-__device__ __forceinline__ int row_order_chunk() { return lane_id() & 3; }
-
+// touched (the down projection waits for its h rows there). transpose_a: row-major weights,
+// loaded in row order (see fragment_from_row_order).
 template <typename DT, int NA, int RB, int U, bool COH_B, bool transpose_a, bool once_a, typename Pre>
 __device__ __forceinline__ bool stream_mma(const typename DT::elem* const (&ap)[NA],
                                            const typename DT::elem* const (&bp)[RB], int ksteps,
@@ -1066,95 +844,6 @@ __device__ __noinline__ bool down_task(ParamsRef pv, int expert, int row0, int r
   return true;
 }
 
-// -------------------------------------------------------------------- combine
-// out[t, c0..c0+256) = sum over slots, in slot order, of the weighted rows
-// (refFullMoe.h:35,62-65; src/hip/kernel/tasks/internal/reduceBlock.h:35-53).
-template <typename DT>
-__device__ void combine_task(ParamsRef p, int t, int chunk) {
-  const int lane = lane_id();
-  const int c = chunk * COMBINE_COLS + lane * 4;
-  if (c < p.H) {
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    // eight slots at a time: their validity and their rows are loaded together
-    // (one memory latency per group instead of two per slot), then added in slot order
-    for (int k0 = 0; k0 < p.K; k0 += 8) {
-      int idx[8];
-      uint4 v[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int kk = min(k0 + k, p.K - 1);
-        idx[k] = ldc(&p.topk_idx[static_cast<size_t>(t) * p.K + kk]);
-        v[k] = ld16_once(p.y + (static_cast<size_t>(t) * p.K + kk) * p.H + c);
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if (k0 + k < p.K && idx[k] >= 0) {
-          s.x += __uint_as_float(v[k].x);
-          s.y += __uint_as_float(v[k].y);
-          s.z += __uint_as_float(v[k].z);
-          s.w += __uint_as_float(v[k].w);
-        }
-      }
-    }
-    const size_t off = static_cast<size_t>(t) * p.H + c;
-    if (p.residual != nullptr) {  // output = input row + layer, the row added last
-      if constexpr (DT::EPV == 8) {
-        const unsigned long long xx = *as_global(
-            reinterpret_cast<const unsigned long long*>(reinterpret_cast<const unsigned short*>(p.residual) + off));
-        const uint2 x = make_uint2(static_cast<unsigned>(xx), static_cast<unsigned>(xx >> 32));
-        s.x += bf16_lo(x.x);
-        s.y += bf16_hi(x.x);
-        s.z += bf16_lo(x.y);
-        s.w += bf16_hi(x.y);
-      } else {
-        const uint4 x = ld16(reinterpret_cast<const float*>(p.residual) + off);
-        s.x += __uint_as_float(x.x);
-        s.y += __uint_as_float(x.y);
-        s.z += __uint_as_float(x.z);
-        s.w += __uint_as_float(x.w);
-      }
-    }
-    if constexpr (DT::EPV == 8) {
-      uint2 pk;
-      pk.x = f2bf(s.x) | (f2bf(s.y) << 16);
-      pk.y = f2bf(s.z) | (f2bf(s.w) << 16);
-      *reinterpret_cast<uint2*>(reinterpret_cast<unsigned short*>(p.out) + off) = pk;
-    } else {
-      *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.out) + off) = s;
-    }
-  }
-  // the selection masks are dead once the permutation is written: clear this
-  // token block's words for the next launch
-  if (chunk == 0 && (t & 63) == 0) {
-    for (int e = lane; e < p.E; e += 64) stc(&p.masks[static_cast<size_t>(e) * p.W + (t >> 6)], 0ull);
-  }
-}
-
-// The combine items slot, slot + n_workers, ... of one worker (a function of its
-// own so that the worker loop's registers are not shared with it).
-template <typename DT>
-__device__ __noinline__ void combine_items(ParamsRef pv, unsigned slot, unsigned nc,
-                                           unsigned ncomb, unsigned worker, unsigned id0,
-                                           long long t_fetch) {
-  ParamsRef p = uniform_params(pv);
-  const int lane = lane_id();
-  for (unsigned q = slot; q < nc; q += static_cast<unsigned>(p.n_workers)) {
-    const long long t_item = p.trace ? wall_clock64() : 0;
-    combine_task<DT>(p, static_cast<int>(q / ncomb), static_cast<int>(q % ncomb));
-    const unsigned id = id0 + q;
-    if (p.trace && lane == 0 && id < p.trace_cap) {
-      const long long t_end = wall_clock64();
-      TraceRec* r = p.trace + id;
-      st16(r, u32x4{id, 5u, worker, q / ncomb});
-      st16(reinterpret_cast<char*>(r) + 16,
-           u32x4{static_cast<unsigned>(t_fetch), static_cast<unsigned>(t_fetch >> 32),
-                 static_cast<unsigned>(t_item), static_cast<unsigned>(t_item >> 32)});
-      st16(reinterpret_cast<char*>(r) + 32,
-           u32x4{static_cast<unsigned>(t_end), static_cast<unsigned>(t_end >> 32), 0u, 0u});
-    }
-  }
-}
-
 // ---------------------------------------------------------------- worker loop
 // Nothing the tasks are called with lives in the wave's private memory: the
 // launch parameters are read in place (ParamsRef), a row tile travels as three
@@ -1472,596 +1161,6 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   }
 }
 
-// ------------------------------------------------- small batches: split-k variant
-// A batch of up to 24 rows an expert (bf16, tiles of one or two 16-row blocks). A wave of the streaming
-// variant carries a task of 64 weight rows over the whole of k alone: with few experts in use
-// most waves have no task at all and the others need 256 KiB each through one wave's window of
-// loads (one token on the 30B shape: 192 tasks on 2048 waves), and with many the launch ends in
-// a tail of whole tasks. Here the eight waves of a workgroup share a task's k (gate/up: eight
-// parts; down: two tasks side by side in four parts, or one in eight where that leaves a CU idle),
-// so tasks are an eighth as long, and meet in LDS: every wave leaves its partial sums there, one
-// barrier, and one or two waves add the parts in k order and store. The window of loads does not
-// drain between tasks: a slot is asked for again, for the step SPLIT_U later of the wave's sequence
-// of tasks, as soon as its matrix instructions have read it. Tasks are handed out statically
-// (equal shares of equal tasks), the routing tables are built by every workgroup for itself in
-// LDS from the top-k entries, and there is one grid-wide dependency between gate/up and down,
-// under which the first window of down weights is on its way.
-//
-// Bound by HBM from some 16 tokens on, below by the chain of waits (logit chains 14 us, selection,
-// gate/up, down, combine). Against the streaming kernel, us, 30B shape, weights packed in place:
-// T=1 59.5 -> 42, T=8 120 -> 103, T=16 164 -> 150, T=64 225 -> 217 (1.19 GB: 5.5 TB/s), T=128 243 -> 223,
-// T=200 266 -> 234, T=256 275 -> 241; row-major T=32 249 -> 226, T=128 290 -> 261; 235B T=1 102 -> 87,
-// T=64 759 -> 762, T=256 876 -> 836. Four hot experts: T=16 146 -> 120, T=128 317 -> 240 (a tile of more
-// rows than an early task carries starts over there; here it is several tiles).
-//
-// Where the batch reaches most experts, the first workgroups (as many as whole experts fill; those
-// with a routing task behind it) ask for the first window of (expert b / nt1, columns b % nt1)
-// before the routing is known and keep it if the expert turns out to be in use.
-// k-steps of a wave's window, by 16-row blocks of the tile (eight and six do not fit the registers
-// beside the epilogue: with eight for one block the window's last loads were spilled, T = 64 306 us)
-constexpr int split_u(int rb) { return rb == 1 ? 6 : 4; }
-constexpr int SPLIT_MAX_TILES = MAX_EXPERTS + SPLIT_MAX_SLOTS / 16;
-// LDS: the tables, then two sets of partial sums ([wave][weight block][row block][lane][4]); the
-// routing tasks use it from its first byte on before that
-constexpr int SPLIT_TILE_OFF = 0;
-constexpr int SPLIT_MASK_OFF = SPLIT_TILE_OFF + SPLIT_MAX_TILES * 8;
-constexpr int SPLIT_W_OFF = SPLIT_MASK_OFF + SCAN_LDS_WORDS * 8;
-constexpr int SPLIT_PERM_OFF = SPLIT_W_OFF + SPLIT_MAX_SLOTS * 4;
-constexpr int SPLIT_TOK_OFF = SPLIT_PERM_OFF + SPLIT_MAX_SLOTS * 2;
-constexpr int SPLIT_OFF_OFF = SPLIT_TOK_OFF + SPLIT_MAX_SLOTS * 2;
-constexpr int SPLIT_SPEC_OFF = SPLIT_OFF_OFF + MAX_EXPERTS * 4;
-constexpr int SPLIT_NOTE_OFF = SPLIT_SPEC_OFF + MAX_EXPERTS * 4;
-constexpr int SPLIT_PART_OFF = SPLIT_NOTE_OFF + 64;
-static_assert(SPLIT_PART_OFF % 16 == 0, "partial sums are read 16 bytes at a time");
-constexpr int split_part_bytes(int rb) { return 8 * 4 * rb * 64 * 16; }
-constexpr int split_lds_bytes(int rb) {
-  const int n = SPLIT_PART_OFF + 2 * split_part_bytes(rb);
-  return n > 8 * ROUTER_LDS_FLOATS * 4 ? n : 8 * ROUTER_LDS_FLOATS * 4;
-}
-static_assert(split_lds_bytes(2) + 64 <= 160 * 1024, "LDS of a workgroup");
-
-// LDS operations of this wave are done, then the workgroup barrier (loads from memory stay in flight)
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// A tile as the tables hold it: at most 16 * RB rows of one expert.
-struct SplitTile {
-  int expert, row0, rows;
-};
-__device__ __forceinline__ SplitTile split_tile(const uint2* tiles, int i) {
-  const uint2 v = tiles[i];
-  SplitTile t;
-  t.expert = __builtin_amdgcn_readfirstlane(static_cast<int>(v.x));
-  const int rr = __builtin_amdgcn_readfirstlane(static_cast<int>(v.y));
-  t.row0 = rr & 0xFFFF;
-  t.rows = rr >> 16;
-  return t;
-}
-
-// The window: U k-steps of four 16-row weight blocks and RB blocks of token rows. PACKED weights
-// are one run of 4 KiB a step; row-major ones four row-order loads (see fragment_from_row_order).
-template <bool PACKED, bool DOWN, int RB>
-struct SplitStream {
-  static constexpr int NP = PACKED ? 1 : 4;
-  static constexpr int U = split_u(RB);
-  uint4 a[U][4], b[U][RB];
-  const unsigned char* ap[NP];   // where the next step's weights are
-  const unsigned char* bp[RB];   // ... and its token rows (gate/up)
-  unsigned boff[RB];             // ... or h rows, as offsets (down)
-  int astep, bstep, left;        // bytes to the next step (0 behind the last task); steps left of the task
-  CoherentBuffer cb;
-
-  __device__ __forceinline__ void load_a(int u) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) a[u][i] = PACKED ? ld16_once(ap[0] + i * 1024) : ld16(ap[i]);
-#pragma unroll
-    for (int q = 0; q < NP; ++q) ap[q] += astep;
-  }
-  __device__ __forceinline__ void load_b(int u) {
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      if (DOWN) {
-        b[u][r] = ld16_agent(cb, boff[r]);
-        boff[r] += static_cast<unsigned>(bstep);
-      } else {
-        b[u][r] = ld16(bp[r]);
-        bp[r] += bstep;
-      }
-    }
-  }
-  // Behind the last task the loads go on (their number must not depend on a branch, or the
-  // compiler waits for all of them at every step), all lanes at one address that exists.
-  __device__ __forceinline__ void park(const void* somewhere) {
-#pragma unroll
-    for (int q = 0; q < NP; ++q) ap[q] = reinterpret_cast<const unsigned char*>(somewhere);
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      bp[r] = reinterpret_cast<const unsigned char*>(somewhere);
-      boff[r] = 0u;
-    }
-    astep = bstep = 0;
-    left = 0x7FFFFFFF;
-  }
-  __device__ __forceinline__ void mma(int u, int pull_from, f32x4 (&acc)[4][RB]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint4 w = PACKED ? a[u][i] : fragment_from_row_order(a[u][i], pull_from);
-#pragma unroll
-      for (int r = 0; r < RB; ++r) acc[i][r] = mma16<BF16>(w, b[u][r], acc[i][r]);
-    }
-  }
-  // this wave's partial sums of a task go to LDS, and the accumulators back to zero
-  __device__ __forceinline__ void leave(f32x4* part, int wave, f32x4 (&acc)[4][RB]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < RB; ++r) {
-        part[((wave * 4 + i) * RB + r) * 64 + lane_id()] = acc[i][r];
-        acc[i][r] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-  }
-};
-
-template <bool PACKED, int RB>
-__global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_split_kernel(const Params params) {
-  ParamsRef p = kernel_params();
-  __shared__ unsigned lds_flag[4];
-  __shared__ unsigned lds_poller[4];
-  if (threadIdx.x < 4) {
-    lds_flag[threadIdx.x] = 0u;
-    lds_poller[threadIdx.x] = 0u;
-  }
-  __syncthreads();
-  const int tid = threadIdx.x, lane = lane_id();
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r16 = lane & 15, g = lane >> 4;
-  const int G = static_cast<int>(gridDim.x), b = static_cast<int>(blockIdx.x);
-  Control* ctl = p.ctl;
-  const int T = p.T, E = p.E, H = p.H, K = p.K, I = p.I, W = p.W;
-  unsigned char* lds = reinterpret_cast<unsigned char*>(lds_dyn);
-  constexpr int U = split_u(RB), TILE_ROWS = 16 * RB;
-  unsigned short* lperm = reinterpret_cast<unsigned short*>(lds + SPLIT_PERM_OFF);  // permuted row -> token*K + slot
-  unsigned short* ltok = reinterpret_cast<unsigned short*>(lds + SPLIT_TOK_OFF);    // permuted row -> token
-  float* lw = reinterpret_cast<float*>(lds + SPLIT_W_OFF);      // permuted row -> gate weight
-  unsigned long long* lmask = reinterpret_cast<unsigned long long*>(lds + SPLIT_MASK_OFF);
-  int* loff = reinterpret_cast<int*>(lds + SPLIT_OFF_OFF);      // expert -> first permuted row
-  uint2* tiles = reinterpret_cast<uint2*>(lds + SPLIT_TILE_OFF);
-  int* spec_tile = reinterpret_cast<int*>(lds + SPLIT_SPEC_OFF);  // expert -> its early tile, or -1
-  int* note = reinterpret_cast<int*>(lds + SPLIT_NOTE_OFF);
-
-  const int n_eg = (E + 15) >> 4;
-  const int n_dot = ((T + 15) >> 4) * n_eg;
-  const int nt1 = I / (16 * G1_NB), nt2 = H / (16 * G2_NB);
-  const int ks1 = H >> 5, ks2 = I >> 5;
-  const int pull_from = (((lane & 15) << 2) | (lane >> 4)) << 2;
-
-  // ---- routing: logit chains on the first workgroups, then one select a wave there
-  if (b < n_dot) {
-    router_dot16_task(p, b / n_eg, b % n_eg);
-    for (int t = b + n_dot * wave; t < T; t += 8 * n_dot) {
-      if (!wave_wait_ge(&p.tok_arrive[t], static_cast<unsigned>(n_eg), ctl, p.spin_limit)) break;
-      router_select_task(p, t);
-    }
-  }
-
-  // ---- gate/up weights before the routing is known
-  const int n_spec_experts = p.split_spec ? min(G / nt1, E) : 0;
-  const int n_spec = n_spec_experts * nt1;  // workgroups b < n_spec
-  const int k0 = ks1 * wave / 8, steps1 = ks1 * (wave + 1) / 8 - k0;
-  f32x4 acc[4][RB];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int r = 0; r < RB; ++r) acc[i][r] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bool ok;
-  int ntiles = 0;
-  int cnt = 0;  // tasks this workgroup has finished: its parity names the set of partial sums
-  {
-    SplitStream<PACKED, false, RB> st;
-    st.cb = coherent_buffer(p.h, 0u);
-    auto weights = [&](int expert, int nblk) {
-      if constexpr (PACKED) {
-        const size_t task = static_cast<size_t>(expert) * nt1 + nblk;
-        st.ap[0] = reinterpret_cast<const unsigned char*>(p.ffn1_packed) + (task * ks1 + k0) * 4096 + lane * 16;
-        st.astep = 4096;
-      } else {
-        const unsigned char* w13 = reinterpret_cast<const unsigned char*>(p.ffn1) +
-                                   static_cast<size_t>(expert) * 2 * I * H * 2 + k0 * 64 + row_order_chunk() * 16;
-        const int n0 = nblk * (16 * G1_NB) + row_order_row();
-#pragma unroll
-        for (int q = 0; q < G1_NB; ++q) {
-          st.ap[q] = w13 + static_cast<size_t>(n0 + 16 * q) * H * 2;
-          st.ap[G1_NB + q] = w13 + static_cast<size_t>(I + n0 + 16 * q) * H * 2;
-        }
-        st.astep = 64;
-      }
-      st.left = steps1;
-    };
-    if (b < n_spec) {
-      weights(b / nt1, b % nt1);
-    } else {
-      st.park(p.gate);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      st.load_a(u);
-      // (a task shorter than the window: the slots behind it are filled again below)
-      if (u + 1 == steps1) st.park(p.gate);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-
-    // ---- tables, by every workgroup for itself
-    ok = wait_flag(p, FLAG_ROUTED, lds_flag, lds_poller);
-    const int wact = (T + 63) >> 6;
-    const int n = T * K;
-    lds_barrier();  // the routing tasks' use of the LDS is over
-    int ee[SPLIT_MAX_SLOTS / 512];
-    float ww[SPLIT_MAX_SLOTS / 512];
-    if (ok) {
-#pragma unroll
-      for (int q = 0; q < SPLIT_MAX_SLOTS / 512; ++q) {
-        const int i = tid + 512 * q;
-        ee[q] = i < n ? ldc(&p.topk_idx[i]) : -1;
-        ww[q] = i < n ? ldc(&p.topk_w[i]) : 0.0f;
-      }
-      for (int i = tid; i < E * wact; i += 512) lmask[i] = ldc(&p.masks[static_cast<size_t>(i / wact) * W + i % wact]);
-    }
-    lds_barrier();
-    if (ok && wave == 0) {
-      int base = 0, rest = 0, spec = 0;
-      const int epl = (E + 63) >> 6;
-      for (int pass = 0; pass < 2; ++pass) {  // the early tiles stand behind all others
-        if (pass == 1) base = 0;
-        for (int j = 0; j < epl; ++j) {
-          const int e = lane + 64 * j;
-          int c = 0;
-          if (e < E)
-            for (int w = 0; w < wact; ++w) c += __popcll(lmask[e * wact + w]);
-          const int off = base + wave_inclusive_scan(c) - c;
-          base = __shfl(off + c, 63, 64);
-          const int nt = (c + TILE_ROWS - 1) / TILE_ROWS;
-          const bool early = e < n_spec_experts && c > 0;
-          const int mine = pass == 0 ? nt - (early ? 1 : 0) : (early ? 1 : 0);
-          const int incl = wave_inclusive_scan(mine);
-          if (pass == 0) {
-            if (e < E) loff[e] = off;
-            for (int i = 0; i < mine; ++i) {
-              const int r = (i + (early ? 1 : 0)) * TILE_ROWS;
-              tiles[rest + incl - mine + i] =
-                  make_uint2(static_cast<unsigned>(e), static_cast<unsigned>((off + r) | (min(TILE_ROWS, c - r) << 16)));
-            }
-            rest += __shfl(incl, 63, 64);
-          } else {
-            if (e < E) spec_tile[e] = early ? rest + spec + incl - 1 : -1;
-            if (early)
-              tiles[rest + spec + incl - 1] =
-                  make_uint2(static_cast<unsigned>(e), static_cast<unsigned>(off | (min(TILE_ROWS, c) << 16)));
-            spec += __shfl(incl, 63, 64);
-          }
-        }
-      }
-      if (lane == 0) {
-        note[0] = rest;
-        note[1] = rest + spec;
-        note[2] = base;
-      }
-    }
-    lds_barrier();
-    int n_rest = 0;
-    if (ok) {
-      n_rest = __builtin_amdgcn_readfirstlane(note[0]);
-      ntiles = __builtin_amdgcn_readfirstlane(note[1]);
-#pragma unroll
-      for (int q = 0; q < SPLIT_MAX_SLOTS / 512; ++q) {
-        const int i = tid + 512 * q;
-        if (ee[q] >= 0) {
-          const int t = i / K, wd = t >> 6;
-          int pos = loff[ee[q]] + __popcll(lmask[ee[q] * wact + wd] & ((1ull << (t & 63)) - 1ull));
-          for (int w = 0; w < wd; ++w) pos += __popcll(lmask[ee[q] * wact + w]);
-          lperm[pos] = static_cast<unsigned short>(i);
-          ltok[pos] = static_cast<unsigned short>(t);
-          lw[pos] = ww[q];
-          if (b == G - 1) stc(&p.perm[pos], i);
-        }
-      }
-      if (b == G - 1) {  // the tables the host may read back
-        const int total = note[2];
-        for (int e = tid; e < E; e += 512) {
-          const int off = loff[e];
-          stc(&p.expert_offset[e], off);
-          stc(&p.expert_count[e], (e + 1 < E ? loff[e + 1] : total) - off);
-        }
-        if (tid == 0) stc(&p.expert_offset[E], total);
-      }
-    }
-    lds_barrier();
-
-    // ---- gate/up: the early task, then an equal share of the rest (workgroups without an early
-    // task first)
-    const int my_spec = ok && b < n_spec ? __builtin_amdgcn_readfirstlane(spec_tile[b / nt1]) : -1;
-    const int rank = b >= n_spec ? b - n_spec : b + G - n_spec;
-    const int n_tasks = n_rest * nt1;
-    int ntask = (my_spec >= 0 ? 1 : 0) + (rank < n_tasks ? (n_tasks - rank + G - 1) / G : 0);
-    int lq = rank;  // next task of the rest to load, and (cq) to finish
-    int cq = rank;
-    bool cspec = my_spec >= 0;
-    auto rows_of = [&](const SplitTile& t) {
-#pragma unroll
-      for (int r = 0; r < RB; ++r)
-        st.bp[r] = reinterpret_cast<const unsigned char*>(p.tokens) +
-                   (static_cast<size_t>(ltok[t.row0 + min(16 * r + r16, t.rows - 1)]) * H + k0 * 32 + g * 8) * 2;
-      st.bstep = 64;
-    };
-    auto next_task = [&]() {
-      if (lq < n_tasks) {
-        const SplitTile t = split_tile(tiles, lq / nt1);
-        weights(t.expert, lq % nt1);
-        rows_of(t);
-        lq += G;
-      } else {
-        st.park(p.gate);
-      }
-    };
-    auto finish = [&]() {  // the task's eight parts: add up, SiLU(gate) * up, store
-      const int q = cspec ? b : cq;
-      const SplitTile t = split_tile(tiles, cspec ? my_spec : q / nt1);
-      const int n0 = (q % nt1) * (16 * G1_NB);
-      if (!cspec) cq += G;
-      cspec = false;
-      f32x4* part = reinterpret_cast<f32x4*>(lds + SPLIT_PART_OFF + (cnt & 1) * split_part_bytes(RB));
-      st.leave(part, wave, acc);
-      lds_barrier();
-      const int turn = (wave - 2 * RB * cnt) & 7;  // the adding waves take turns
-      const int i = turn & 1, r = turn >> 1;
-      ++cnt;
-      if (r < RB) {
-        f32x4 s = part[(i * RB + r) * 64 + lane], v = part[((i + 2) * RB + r) * 64 + lane];
-#pragma unroll 1  // (more reads in flight cost the window its registers)
-        for (int w = 1; w < 8; ++w) {
-          s += part[((w * 4 + i) * RB + r) * 64 + lane];
-          v += part[((w * 4 + i + 2) * RB + r) * 64 + lane];
-        }
-        const int row = 16 * r + r16;
-        if (row < t.rows) {
-          unsigned hv[4];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {  // (one after the other, for the same reason)
-            hv[k] = f2bf(silu_mul(s[k], v[k]));
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          const unsigned lo = hv[0] | (hv[1] << 16), hi = hv[2] | (hv[3] << 16);
-          stc(reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned short*>(p.h) +
-                                                    static_cast<size_t>(t.row0 + row) * I + n0 + 16 * i + 4 * g),
-              static_cast<unsigned long long>(lo) | (static_cast<unsigned long long>(hi) << 32));
-        }
-      }
-    };
-    if (ntask > 0) {
-      if (my_spec >= 0 && steps1 >= U) {
-        // the window is this task's: its token rows join it
-        rows_of(split_tile(tiles, my_spec));
-        if (steps1 == U) {
-          st.left = 0;
-        } else {
-          st.left = steps1 - U;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) st.load_b(u);
-        if (st.left == 0) next_task();
-      } else {
-        if (my_spec >= 0) {
-          weights(b / nt1, b % nt1);
-          rows_of(split_tile(tiles, my_spec));
-        } else {
-          next_task();
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          st.load_a(u);
-          st.load_b(u);
-          if (--st.left == 0) next_task();
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      int cleft = steps1;
-      auto round = [&]() {  // true: the last task is finished
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          st.mma(u, pull_from, acc);
-          __builtin_amdgcn_sched_barrier(0);
-          st.load_a(u);
-          st.load_b(u);
-          __builtin_amdgcn_sched_barrier(0);
-          if (--st.left == 0) next_task();
-          if (--cleft == 0) {
-            finish();
-            if (--ntask == 0) return true;
-            cleft = steps1;
-          }
-        }
-        return false;
-      };
-      if (!round()) {
-        asm volatile("; end of the first round" ::: "memory");  // as in stream_mma
-        while (!round()) {
-        }
-      }
-    }
-  }
-
-  // ---- every h row is final once all workgroups have been here
-  const int parts = p.split_down;            // waves that share a down task: 4 or 8
-  const int sub = wave & (parts - 1), grp = parts == 8 ? 0 : wave >> 2;
-  const int per_tile = parts == 8 ? nt2 : nt2 >> 1;  // workgroup tasks of one tile
-  if (ok) {
-    fence_release();
-    lds_barrier();
-    if (wave == 0) {
-      unsigned old = 0;
-      if (lane == 0) old = add_relaxed(&ctl->perm_done.v, 1u);
-      old = __builtin_amdgcn_readfirstlane(old);
-      if (old == static_cast<unsigned>(G) - 1u) broadcast_flag(p, FLAG_PERM);
-    }
-    const int d0 = ks2 * sub / parts, steps2 = ks2 * (sub + 1) / parts - d0;
-    const int n_tasks = ntiles * per_tile;
-    int ntask = b < n_tasks ? (n_tasks - b + G - 1) / G : 0;
-    if (ntask > 0) {
-      SplitStream<PACKED, true, RB> st;
-      st.cb = coherent_buffer(p.h, static_cast<unsigned>(T * K * I * 2));
-      int lq = b, cq = b;
-      auto next_task = [&]() {
-        if (lq < n_tasks) {
-          const SplitTile t = split_tile(tiles, lq / per_tile);
-          const int nblk = parts == 8 ? lq % per_tile : (lq % per_tile) * 2 + grp;
-          if constexpr (PACKED) {
-            const size_t task = static_cast<size_t>(t.expert) * nt2 + nblk;
-            st.ap[0] = reinterpret_cast<const unsigned char*>(p.ffn2_packed) + (task * ks2 + d0) * 4096 + lane * 16;
-            st.astep = 4096;
-          } else {
-            const unsigned char* w2 = reinterpret_cast<const unsigned char*>(p.ffn2) +
-                                      static_cast<size_t>(t.expert) * H * I * 2 + d0 * 64 + row_order_chunk() * 16;
-            const int n0 = nblk * (16 * G2_NB) + row_order_row();
-#pragma unroll
-            for (int q = 0; q < st.NP; ++q) st.ap[q] = w2 + static_cast<size_t>(n0 + 16 * q) * I * 2;
-            st.astep = 64;
-          }
-#pragma unroll
-          for (int r = 0; r < RB; ++r)
-            st.boff[r] = static_cast<unsigned>(((t.row0 + min(16 * r + r16, t.rows - 1)) * I + d0 * 32 + g * 8) * 2);
-          st.bstep = 64;
-          st.left = steps2;
-          lq += G;
-        } else {
-          st.park(p.gate);
-        }
-      };
-      // The weights of the first window go out before the wait, the h rows behind it: both walk
-      // through the same steps.
-      next_task();
-      const int lq0 = lq;
-      unsigned boff0[RB];
-#pragma unroll
-      for (int r = 0; r < RB; ++r) boff0[r] = st.boff[r];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        st.load_a(u);
-        if (--st.left == 0) next_task();
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      ok = wait_flag(p, FLAG_PERM, lds_flag, lds_poller);
-      if (ok) {
-        const unsigned char* keep[st.NP];
-#pragma unroll
-        for (int q = 0; q < st.NP; ++q) keep[q] = st.ap[q];
-        lq = lq0;
-#pragma unroll
-        for (int r = 0; r < RB; ++r) st.boff[r] = boff0[r];
-        st.bstep = 64;
-        st.left = steps2;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          st.load_b(u);
-          if (--st.left == 0) next_task();
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int q = 0; q < st.NP; ++q) st.ap[q] = keep[q];
-        auto finish = [&]() {
-          const SplitTile t = split_tile(tiles, cq / per_tile);
-          const int n0 = (parts == 8 ? cq % per_tile : (cq % per_tile) * 2 + grp) * (16 * G2_NB);
-          cq += G;
-          f32x4* part = reinterpret_cast<f32x4*>(lds + SPLIT_PART_OFF + (cnt & 1) * split_part_bytes(RB));
-          st.leave(part, wave, acc);
-          lds_barrier();
-          // (four blocks for eight waves: one half of them, then the other)
-          const int first = parts > 4 * RB ? (sub + 4 * (cnt & 1)) & 7 : sub;
-          ++cnt;
-          for (int blk = first; blk < 4 * RB; blk += parts) {
-            const int i = blk & 3, r = blk >> 2;
-            f32x4 s = part[((grp * 16 + i) * RB + r) * 64 + lane];
-#pragma unroll 1
-            for (int w = 1; w < parts; ++w) s += part[(((grp * 4 + w) * 4 + i) * RB + r) * 64 + lane];
-            const int row = 16 * r + r16;
-            if (row < t.rows) {
-              const float wt = lw[t.row0 + row];
-              st16_through(p.y + static_cast<size_t>(lperm[t.row0 + row]) * H + n0 + 16 * i + 4 * g,
-                           make_uint4(__float_as_uint(s[0] * wt), __float_as_uint(s[1] * wt),
-                                      __float_as_uint(s[2] * wt), __float_as_uint(s[3] * wt)));
-            }
-          }
-        };
-        int cleft = steps2;
-        auto round = [&]() {
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            st.mma(u, pull_from, acc);
-            __builtin_amdgcn_sched_barrier(0);
-            st.load_a(u);
-            st.load_b(u);
-            __builtin_amdgcn_sched_barrier(0);
-            if (--st.left == 0) next_task();
-            if (--cleft == 0) {
-              finish();
-              if (--ntask == 0) return true;
-              cleft = steps2;
-            }
-          }
-          return false;
-        };
-        if (!round()) {
-          asm volatile("; end of the first round" ::: "memory");
-          while (!round()) {
-          }
-        }
-      }
-    }
-  }
-
-  // ---- combine, by the waves that have an item
-  if (ok) {
-    fence_release();
-    lds_barrier();
-    if (wave == 0) {
-      unsigned old = 0;
-      if (lane == 0) old = add_relaxed(&ctl->g2_done.v, 1u);
-      old = __builtin_amdgcn_readfirstlane(old);
-      if (old == static_cast<unsigned>(G) - 1u) broadcast_flag(p, FLAG_G2);
-    }
-    const unsigned ncomb = static_cast<unsigned>((H + COMBINE_COLS - 1) / COMBINE_COLS);
-    const unsigned nc = static_cast<unsigned>(T) * ncomb;
-    const unsigned slot = static_cast<unsigned>(wave * G + b);
-    if (slot < nc && wait_flag(p, FLAG_G2, lds_flag, lds_poller))
-      combine_items<BF16>(p, slot, nc, ncomb, static_cast<unsigned>(b * 8 + wave), 0u, 0);
-  }
-
-  // ---- the last workgroup out returns every counter to zero for the next launch
-  __syncthreads();
-  if (wave == 0) {
-    fence_release();  // flags this wave has raised for others have landed before anybody clears them
-    unsigned last = 0;
-    if (lane == 0) last = add_relaxed(&ctl->exit_count.v, 1u) == static_cast<unsigned>(G) - 1u ? 1u : 0u;
-    if (__builtin_amdgcn_readfirstlane(last) != 0u) {
-      const unsigned err = ldc(&ctl->error.v);
-      if (err != 0u) recover_after_error(p, err, lane, 64);
-      for (int q = lane; q < p.n_groups; q += 64) {
-        stc(&p.wgflags[q].f[FLAG_PERM], 0u);
-        stc(&p.wgflags[q].f[FLAG_G2], 0u);
-        stc(&p.wgflags[q].f[FLAG_ROUTED], 0u);
-      }
-      if (lane == 0) {
-        stc(&ctl->launches.v, ldc(&ctl->launches.v) + 1u);
-        stc(&ctl->router_done.v, 0u);
-        stc(&ctl->perm_done.v, 0u);
-        stc(&ctl->g2_done.v, 0u);
-        stc(&ctl->exit_count.v, 0u);
-      }
-    }
-  }
-}
-
 // ------------------------------------------------------------ weight packing
 // dst chunk c (16 bytes) of the packed gate/up or down weights <- its source.
 // which = 0: ffn1 [E,2I,H] -> tasks of 2*G1_NB blocks (gate blocks, then up
@@ -2113,68 +1212,32 @@ hipError_t pack_weights(const void* src, void* dst, int dtype, int E, int H, int
 
 template __global__ void moe_stream_kernel<F32>(const Params);
 template __global__ void moe_stream_kernel<BF16>(const Params);
-template __global__ void moe_split_kernel<true, 1>(const Params);
-template __global__ void moe_split_kernel<false, 1>(const Params);
-template __global__ void moe_split_kernel<true, 2>(const Params);
-template __global__ void moe_split_kernel<false, 2>(const Params);
+
+namespace {
+constexpr int STREAM_LDS_BYTES = 8 * ROUTER_LDS_FLOATS * static_cast<int>(sizeof(float));
+}
 
 hipError_t launch_stream_kernel(const Params& p, int dtype, int grid, hipStream_t stream) {
-  const size_t lds = static_cast<size_t>(8) * ROUTER_LDS_FLOATS * sizeof(float);
-  if (p.split) {
-    auto* kernel = p.split == 1 ? (p.ffn1_packed != nullptr ? moe_split_kernel<true, 1> : moe_split_kernel<false, 1>)
-                                : (p.ffn1_packed != nullptr ? moe_split_kernel<true, 2> : moe_split_kernel<false, 2>);
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), split_lds_bytes(p.split), stream, p);
-  } else if (dtype == DT_BF16) {
-    hipLaunchKernelGGL(moe_stream_kernel<BF16>, dim3(grid), dim3(512), lds, stream, p);
+  if (dtype == DT_BF16) {
+    hipLaunchKernelGGL(moe_stream_kernel<BF16>, dim3(grid), dim3(512), STREAM_LDS_BYTES, stream, p);
   } else {
-    hipLaunchKernelGGL(moe_stream_kernel<F32>, dim3(grid), dim3(512), lds, stream, p);
+    hipLaunchKernelGGL(moe_stream_kernel<F32>, dim3(grid), dim3(512), STREAM_LDS_BYTES, stream, p);
   }
   return hipGetLastError();
 }
 
-namespace {
-// Every kernel a layer of this type may run here, and the dynamic LDS it is launched with.
-struct KernelUse {
-  const void* kernel;
-  int lds;
-};
-template <typename F>
-hipError_t for_kernels(int dtype, F f) {
-  const int stream_lds = 8 * ROUTER_LDS_FLOATS * static_cast<int>(sizeof(float));
-  if (dtype != DT_BF16) return f(KernelUse{reinterpret_cast<const void*>(moe_stream_kernel<F32>), stream_lds});
-  const KernelUse uses[] = {
-      {reinterpret_cast<const void*>(moe_stream_kernel<BF16>), stream_lds},
-      {reinterpret_cast<const void*>(moe_split_kernel<true, 1>), split_lds_bytes(1)},
-      {reinterpret_cast<const void*>(moe_split_kernel<false, 1>), split_lds_bytes(1)},
-      {reinterpret_cast<const void*>(moe_split_kernel<true, 2>), split_lds_bytes(2)},
-      {reinterpret_cast<const void*>(moe_split_kernel<false, 2>), split_lds_bytes(2)}};
-  for (const KernelUse& u : uses) {
-    const hipError_t e = f(u);
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
-}
-}  // namespace
-
 hipError_t prepare_stream_kernel() {
-  auto prepare = [](const KernelUse& u) {
-    return hipFuncSetAttribute(u.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, u.lds);
-  };
-  const hipError_t e = for_kernels(DT_BF16, prepare);
-  return e != hipSuccess ? e : for_kernels(DT_F32, prepare);
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_stream_kernel<BF16>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS_BYTES);
+  if (e != hipSuccess) return e;
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(moe_stream_kernel<F32>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS_BYTES);
 }
 
-// the least of the kernels' numbers of workgroups a CU holds
 hipError_t stream_kernel_occupancy(int dtype, int* per_cu) {
-  int least = 0x7FFFFFFF;
-  const hipError_t e = for_kernels(dtype, [&](const KernelUse& u) {
-    int n = 0;
-    const hipError_t r = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, u.kernel, 512, u.lds);
-    if (n < least) least = n;
-    return r;
-  });
-  *per_cu = least;
-  return e;
+  return dtype == DT_BF16
+             ? hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, moe_stream_kernel<BF16>, 512, STREAM_LDS_BYTES)
+             : hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, moe_stream_kernel<F32>, 512, STREAM_LDS_BYTES);
 }
 
 }  // namespace fmoe
