@@ -527,6 +527,12 @@ int flashMoeSchedFor(FlashMoeLauncher* l, int tokens_num) {
   return sched_for(l->desc, tokens_num, machine(*l));
 }
 
+int flashMoeSplitBlocksFor(FlashMoeLauncher* l, int tokens_num) {
+  if (l == nullptr) return -1;
+  const Machine m = machine(*l);
+  return sched_for(l->desc, tokens_num, m) == FLASH_MOE_SCHED_TILED ? 0 : split_row_blocks(l->desc, tokens_num, m);
+}
+
 int flashMoeLaunch(FlashMoeLauncher* l, const void* tokens, void* output, int tokens_num,
                    void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);

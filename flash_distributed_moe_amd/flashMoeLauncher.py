@@ -244,3 +244,7 @@ class MoeKernelLauncher:
 
     def sched_for(self, tokens_num):
         return self._lib.flashMoeSchedFor(self._h, int(tokens_num))
+
+    def split_blocks_for(self, tokens_num):
+        """16-row blocks a tile of the split-k kernel for this batch: 1 or 2, 0 if it does not run."""
+        return self._lib.flashMoeSplitBlocksFor(self._h, int(tokens_num))

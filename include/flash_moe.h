@@ -245,6 +245,11 @@ int flashMoeTraceRead(FlashMoeLauncher* l, void* records, unsigned max_records, 
 /* Which scheduling variant a launch of tokens_num tokens would use. */
 int flashMoeSchedFor(FlashMoeLauncher* l, int tokens_num);
 
+/* Whether that launch runs the streaming variant's split-k kernel, and on how many 16-row
+ * blocks a tile: 1 or 2; 0 if it does not. (Added without a new interface revision: symbol
+ * version LIBFLASHMOE_MI355X_0.4.) */
+int flashMoeSplitBlocksFor(FlashMoeLauncher* l, int tokens_num);
+
 const char* flashMoeVersion(void);
 
 /* Binary interface revision, for bindings that were built against another header.

@@ -346,35 +346,42 @@ def test_prepacked_weights_equal_unpacked(name, T, sched):
         a.close()
 
 
-@pytest.mark.parametrize("shape", [
-    (1, 256, 8, 2, 128),            # one k-step a wave; most workgroups without a task
-    (1, 256, 8, 8, 256),            # one down task to a workgroup (eight parts)
-    (10, 512, 8, 1, 352),           # eleven down k-steps over four waves; early gate/up tasks of unused experts
-    (33, 768, 32, 4, 160),          # three k-steps a wave, five in the down projection; two mask words of experts
-    (64, 2048, 64, 8, 416, 4),      # four experts with 64 rows: tiles of one expert among the rest; a full window
-    (67, 2304, 16, 2, 128, 2),      # ragged tiles; nine k-steps a wave, more than the window
-    (72, 256, 256, 9, 128),         # every expert slot in use; two mask words
-    (128, 256, 256, 9, 128, 3),     # 1152 routing entries, all workgroups busy with routing or early tasks
-    (40, 256, 4, 1, 128),           # ten rows an expert: tiles of two row blocks
-    (190, 768, 16, 2, 352, 2),      # 23.75 rows an expert; ragged tiles of up to 32 rows, two experts with several
-    (256, 512, 96, 8, 160, 4),      # 2048 routing entries: the tables are full
+@pytest.mark.parametrize("blocks,shape", [
+    (1, (1, 256, 8, 2, 128)),            # one k-step a wave; most workgroups without a task
+    (1, (1, 256, 8, 8, 256)),            # one down task to a workgroup (eight parts)
+    (1, (10, 512, 8, 1, 352)),           # eleven down k-steps over four waves; early gate/up tasks of unused experts
+    (1, (33, 768, 32, 4, 160)),          # three k-steps a wave, five in the down projection; two mask words of experts
+    (1, (64, 2048, 64, 8, 416, 4)),      # four experts with 64 rows: tiles of one expert among the rest; a full window
+    (1, (67, 2304, 16, 2, 128, 2)),      # ragged tiles; nine k-steps a wave, more than the window
+    (1, (72, 256, 256, 9, 128)),         # every expert slot in use; two mask words
+    (1, (128, 256, 256, 9, 128, 3)),     # 1152 routing entries, all workgroups busy with routing or early tasks
+    (2, (80, 256, 8, 1, 128)),           # ten rows an expert: tiles of two row blocks, most with one block in use
+    (2, (128, 256, 8, 1, 128)),          # 16 rows an expert: the second block empty, full or anywhere between
+    (2, (190, 768, 16, 2, 352, 2)),      # 23.75 rows an expert; ragged tiles of up to 32 rows, two experts with several
+    (2, (256, 512, 96, 8, 160, 4)),      # 2048 routing entries: the tables are full
+    (0, (40, 256, 4, 1, 128)),           # too few router weights for the loads nobody needs
+    (0, (98, 256, 8, 2, 256)),           # 24.5 rows an expert
 ])
-def test_split_k_small_batches(shape):
+def test_split_k_small_batches(blocks, shape):
     """Small bf16 batches (at most 24 rows an expert): the split-k kernel at the edges of its k
     parts, tiles and tables, on row-major weights against the oracle; the packed copy gives the same
-    bits, and so does a second launch (every counter is back at zero)."""
+    bits, and so does a second launch (every counter is back at zero). `blocks`: the 16-row blocks
+    of its tiles, 0 just outside its range (another kernel runs, the packed copy's may differ)."""
     T, H, E, k, I = shape[:5]
     cfg = synth.MoeConfig("split", T, H, E, k, I, "bf16", hot=shape[5] if len(shape) > 5 else 0)
     print("split-k", shape, flush=True)
     case = GpuCase(cfg, seed=T + E)
     try:
+        assert case.launcher.split_blocks_for(T) == blocks
         out = case.run()
         case.check_routing(case.inp["tokens"], case.launcher.routing(T))
         case.check_outputs(case.inp["tokens"], out, nthreads=4)
         assert torch.equal(case.run(), out)
         packed = GpuCase(cfg, seed=T + E, inputs=case.inp, pack_weights=True)
         try:
-            assert torch.equal(packed.run(), out)
+            assert packed.launcher.split_blocks_for(T) == blocks
+            if blocks:
+                assert torch.equal(packed.run(), out)
         finally:
             packed.close()
     finally:
