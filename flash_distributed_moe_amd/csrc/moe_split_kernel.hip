@@ -11,11 +11,13 @@
 // of tasks, as soon as its matrix instructions have read it. Tasks are handed out statically
 // (equal shares of equal tasks), the routing tables are built by every workgroup for itself in
 // LDS from the top-k entries, and there is one grid-wide dependency between gate/up and down,
-// under which the first window of down weights is on its way.
+// under which the first window of down weights is on its way. T=64 on the 30B shape, us from the
+// launch's first workgroup: routed 21, tables 24, gate/up done 119 to 141, h everywhere 144, down
+// done 204, out 208.
 //
 // Bound by HBM from some 16 tokens on, below by the chain of waits (logit chains 14 us, selection,
 // gate/up, down, combine). Against the streaming kernel, us, 30B shape, weights packed in place:
-// T=1 59.5 -> 42, T=8 120 -> 103, T=16 164 -> 150, T=64 225 -> 217 (1.19 GB: 5.5 TB/s), T=128 243 -> 223,
+// T=1 59.5 -> 42 (routed 16, tables 19, gate/up 28, h everywhere 32, down 34), T=8 120 -> 103, T=16 164 -> 150, T=64 225 -> 217 (1.19 GB: 5.5 TB/s), T=128 243 -> 223,
 // T=200 266 -> 234, T=256 275 -> 241; row-major T=32 249 -> 226, T=128 290 -> 261; 235B T=1 102 -> 87,
 // T=64 759 -> 762, T=256 876 -> 836. Four hot experts: T=16 146 -> 120, T=128 317 -> 240 (a tile of more
 // rows than an early task carries starts over there; here it is several tiles).
@@ -88,6 +90,10 @@ struct SplitStream {
   int astep, bstep, left;        // bytes to the next step (0 behind the last task); steps left of the task
   CoherentBuffer cb;
 
+  // Packed weights pass through the caches without staying, also where an expert has several tiles
+  // that read them (unlike the streaming kernel's sweep): with ordinary loads they push the token
+  // rows, h and y out of the L2s. us, non-temporal / ordinary, 30B shape: T=64 217 / 237, T=256 240 / 261,
+  // with four hot experts T=64 207 / 220, T=256 269 / 272; 235B shape with four hot experts T=200 895 / 933.
   __device__ __forceinline__ void load_a(int u) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) a[u][i] = PACKED ? ld16_once(ap[0] + i * 1024) : ld16(ap[i]);

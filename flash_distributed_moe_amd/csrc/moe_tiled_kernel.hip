@@ -474,7 +474,10 @@ __device__ void tiled_scatter_task(ParamsRef p, int blk) {
 // delivers more. Back to back on all CUs with normally distributed operands in
 // registers: 32x32x16 1717 TFLOP/s at 1.74 GHz, 16x16x32 1919 TFLOP/s at 1.99 GHz
 // (2478 and 2407 on 8 CUs, where the clock stays at 2.4 GHz). Per multiply-add it
-// reads twice the operand registers but moves half the accumulators.
+// reads twice the operand registers but moves half the accumulators. What it gains is therefore
+// there in a row of launches that keep the board at its cap (T=8192 on the 30B shape 769 -> 746 us),
+// hardly in one launch behind a pause (792 -> 786), and it costs a little where a few tall tiles
+// have the chip to themselves (E=64, k=2, T=700, four hot experts, row-major 128 -> 133 us).
 //
 // LDS stage layout: rows of 128 bytes, unpadded, weight rows 0..255 then token
 // rows. Row R keeps its eight 16-byte chunks permuted: chunk C sits at position

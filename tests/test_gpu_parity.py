@@ -155,7 +155,7 @@ def test_relaunch_across_batch_sizes(sched):
 
 
 @pytest.mark.parametrize("shape", [
-    # T, H, E, k, I: the tiled (MFMA 32x32, LDS-staged) variant forced on small problems
+    # T, H, E, k, I: the tiled variant (MFMA 16x16x32, both of its pipelines) forced on small problems
     (300, 256, 8, 2, 128),      # ragged last row tile (75 rows per expert on average)
     (700, 512, 4, 2, 256),      # several 256-row tiles per expert, ragged tail
     (64, 256, 200, 6, 128),     # E > 128: two expert slabs in the router; tiny tiles
