@@ -949,9 +949,10 @@ __device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nst
         }
         if constexpr (j < JT && NEXT) store_fragment<j * 1024>(wr, bs[PB][j]);  // token rows of stage s+1
         if constexpr (j >= JT && BN) issue_b(s + D + 1, j - JT, bs[PB][j - JT]);
-      } else if constexpr (j < 2 && A0) {
-        issue_a(s + D, 0, std::integral_constant<int, 2 * j>{}, as[P][0][2 * j]);
-        issue_a(s + D, 0, std::integral_constant<int, 2 * j + 1>{}, as[P][0][2 * j + 1]);
+      } else if constexpr (j < 4 && A0) {
+        // (one a slot; before, two in each of the first two slots: us, T=600 304.1 -> 303.5, behind other
+        // launchers' memory 317.2 -> 316.3, T=900 307.8 -> 306.9, 235B shape T=1024 1017 -> 1016)
+        issue_a(s + D, 0, std::integral_constant<int, j>{}, as[P][0][j]);
       }
       if constexpr (n + RING < JB) {
         ring[n % RING] = read_b(rd, n + RING);
