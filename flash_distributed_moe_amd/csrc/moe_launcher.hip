@@ -111,9 +111,9 @@ Layout make_layout(const FlashMoeLayerDesc& d, bool need_tiled) {
   L.perm = take(sizeof(int) * rows);
   L.row_w = take(sizeof(float) * rows);
   L.mtiles = take(sizeof(fmoe::TileDesc) * L.max_mtiles);
-  (void)need_tiled;  // both variants keep h as [rows, I], rows in permuted order
-  const size_t h_rows = rows;
-  L.h = take(esz * h_rows * d.intermediate);
+  // Both variants keep h as [rows, I], rows in permuted order. The tiled one reads them through the
+  // caches, so its rows are whole 128-byte lines: no line then holds rows of two tiles.
+  L.h = take(esz * rows * (need_tiled ? fmoe::tiled_h_pitch(d.intermediate) : d.intermediate));
   // y: the streaming variant keeps every (token, slot) row in float, the tiled variant in
   // bf16. When every batch that asks for the tiled variant gets it (tiled_all) and AUTO hands
   // it the large batches, the streaming one only ever sees batches below the switch-over.
@@ -165,8 +165,12 @@ hipError_t validate(const FlashMoeLayerDesc* d) {
   return hipSuccess;
 }
 
-// The tiled variant needs bf16, tile-aligned shapes and token rows it can
-// address with 32-bit byte offsets. AUTO takes it once an expert sees about 26
+// The tiled variant needs bf16, two 64-k stages in either projection, and token rows and an expert's
+// weights that it can address with 32-bit byte offsets. H need be no multiple of its 256 columns nor I
+// one of 128: what stands out over the last column costs less than the streaming variant's tiles of 64
+// rows, each of which reads its expert's weights again (us, streaming / tiled: E=40, k=5, H=1344, I=736
+// T=200 107 / 107, T=400 150 / 105, T=8000 1112 / 391; E=16, k=2, H=320, I=160 T=300 58 / 48, T=4000
+// 201 / 74; E=100, k=6, H=3904, I=1952 T=600 1044 / 956, T=4000 3746 / 1386). AUTO takes it once an expert sees about 26
 // rows on average when the weights are packed (30B shape, us, streaming / tiled:
 // T=320 284 / 301, T=384 293 / 301, T=448 314 / 299, T=512 339 / 304; 235B shape:
 // T=320 905 / 960, T=384 934 / 969, T=512 1054 / 976), and from about 14 rows on
@@ -174,9 +178,10 @@ hipError_t validate(const FlashMoeLayerDesc* d) {
 // cache line at a time (30B: T=192 309 / 318, T=256 318 / 318, T=320 346 / 320;
 // 235B: T=192 1030 / 1001, T=256 1055 / 1007, T=384 1142 / 1015).
 bool tiled_eligible(const FlashMoeLayerDesc& d, int tokens_num) {
-  return d.dtype == FLASH_MOE_BF16 && d.hidden % 256 == 0 && d.intermediate % 128 == 0 &&
+  return d.dtype == FLASH_MOE_BF16 && d.hidden >= 128 && d.intermediate >= 128 &&
          tokens_num <= fmoe::tiled_max_tokens() &&
-         static_cast<long long>(tokens_num) * d.hidden * 2 < (1ll << 32);
+         static_cast<long long>(tokens_num) * d.hidden * 2 < (1ll << 32) &&
+         static_cast<long long>(d.intermediate) * d.hidden * 4 < (1ll << 32);
 }
 
 // What the choice of a kernel depends on beside the layer and the batch.
@@ -667,7 +672,8 @@ int flashMoeLaunchNoAlloc(const FlashMoeLayerDesc* desc, const void* tokens, voi
   l.desc = *desc;
   l.desc.max_tokens = tokens_num;
   // (what does not fit is refused before any device is asked for; where the number of CUs
-  // decides between the variants, below 26 rows an expert, both workspaces are of one size)
+  // decides between the variants, below 26 rows an expert, the workspaces differ by the padding of
+  // h's rows at most, and the streaming variant runs where only its own fits)
   l.num_cus = kMaxGroups;
   int sched = sched_for(l.desc, tokens_num, machine(l));
   l.layout = make_layout(l.desc, sched == FLASH_MOE_SCHED_TILED);
@@ -694,7 +700,16 @@ int flashMoeLaunchNoAlloc(const FlashMoeLayerDesc* desc, const void* tokens, voi
   l.num_cus = sd->num_cus;
   l.ticks_per_ms = sd->ticks_per_ms;
   l.spin_limit = 2000 * sd->ticks_per_ms;
+  const bool made_for_tiled = sched == FLASH_MOE_SCHED_TILED;
   sched = sched_for(l.desc, tokens_num, machine(l));
+  if (sched == FLASH_MOE_SCHED_TILED && !made_for_tiled) {
+    const Layout tiled = make_layout(l.desc, true);
+    if (tiled.total <= static_cast<size_t>(FLASH_MOE_NOALLOC_SCRATCH_BYTES)) {
+      l.layout = tiled;
+    } else {
+      sched = l.desc.sched = FLASH_MOE_SCHED_STREAM;
+    }
+  }
   // where a failing launch's last worker leaves its error bits: device memory here, no
   // pinned host word (that would be an allocation)
   l.host_error_dev = reinterpret_cast<unsigned*>(sd->ptr + kScratchErrorOffset);
@@ -781,8 +796,12 @@ int flashMoeReadIntermediate(FlashMoeLauncher* l, int tokens_num, void* h, void*
     FMOE_FAIL(hipErrorInvalidValue, "tokens_num = %i", tokens_num);
   FMOE_HIP_CHECK(hipStreamSynchronize(stream));
   const size_t esz = l->desc.dtype == FLASH_MOE_BF16 ? 2 : 4;
-  const size_t bytes = esz * static_cast<size_t>(tokens_num) * l->desc.top_k * l->desc.intermediate;
-  FMOE_HIP_CHECK(hipMemcpy(h, l->ws + l->layout.h, bytes, hipMemcpyDeviceToHost));
+  const size_t rows = static_cast<size_t>(tokens_num) * l->desc.top_k;
+  const size_t row_bytes = esz * l->desc.intermediate;
+  const bool tiled = flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED;
+  const size_t pitch = tiled ? esz * fmoe::tiled_h_pitch(l->desc.intermediate) : row_bytes;
+  if (rows != 0)
+    FMOE_HIP_CHECK(hipMemcpy2D(h, row_bytes, l->ws + l->layout.h, pitch, row_bytes, rows, hipMemcpyDeviceToHost));
   return hipSuccess;
 }
 

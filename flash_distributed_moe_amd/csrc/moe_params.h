@@ -28,6 +28,8 @@ constexpr int DOT16_KC = 256;    // streaming variant, matrix-core router: k per
 constexpr int SCAN_LDS_WORDS = 1024;  // mask words (experts x 64-token words) the small-batch scan keeps in LDS
 constexpr int SPLIT_MAX_SLOTS = 2048;  // split-k kernel: (token, slot) entries its tables hold
 constexpr int EARLY_MAX_TOKENS = 384;  // batches up to this size may take their gate/up weights before the routing is known
+// Elements from one row of h to the next in the bf16 tiled variant: whole 128-byte lines.
+constexpr __host__ __device__ int tiled_h_pitch(int intermediate) { return (intermediate + 63) & ~63; }
 constexpr int MAX_EXPERTS = 256;  // experts are spread 64 per wave register slot
 constexpr int MAX_TOPK = 32;
 
@@ -110,7 +112,7 @@ struct Params {
   int* perm;                  // [T*K] permuted row -> t*K+slot
   float* row_w;               // [T*K] gate weight of the permuted row
   TileDesc* mtiles;           // [max_mtiles]
-  void* h;                    // [T*K, I] SwiGLU output, layer dtype
+  void* h;                    // [T*K, I] SwiGLU output, layer dtype; bf16 tiled variant: rows of tiled_h_pitch(I) elements
   float* y;                   // [T*K, H] weighted down-projection rows, by t*K+slot
   Control* ctl;
   WgFlags* wgflags;                // [n_groups]

@@ -543,6 +543,7 @@ struct TileOperands {
   const unsigned char* tbase;  // uniform: tokens, or h
   unsigned wstride;            // uniform: bytes from one stage's weights to the next
   bool wpacked;                // uniform: the weights come from the packed layout (see packed_run_offset)
+  unsigned wlast, tlast;       // uniform: byte offsets of the last stage's weights and token rows
   unsigned woff[NLD];          // this lane's 16 bytes of weight load q at stage 0
   unsigned toff[10];           // the same for the token rows
 };
@@ -590,7 +591,13 @@ constexpr int ring_of(int jt) { return jt == 2 ? 4 : jt == 3 ? 6 : jt == 5 ? 5 :
 // before it, the previous task's stores included, has completed there anyway) thread 0
 // signals the previous task's completion on `pend` (if any) and draws the workgroup's next
 // ticket from `queue` into `next`, so neither trip to memory is waited for between tasks.
-template <int JT, typename AfterFirstLoads>
+//
+// HALF: k is an odd number of 32-k steps. The last stage then covers the last 64 k, the first 32
+// of which the stage before it has multiplied already, and only its second sub-step runs (`wlast`,
+// `tlast`: the byte offsets of the last stage's operands, which no stage's exceed). A template
+// parameter and not a branch: where two ways part or meet the compiler may copy accumulators, and
+// it does not know that a matrix instruction in assembly has yet to write them.
+template <int JT, bool HALF, typename AfterFirstLoads>
 __device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f32x4 (&acc)[4][JB_MAX],
                                           unsigned* pend, unsigned* queue, unsigned& next,
                                           AfterFirstLoads after_first_loads) {
@@ -623,10 +630,12 @@ __device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f
   auto issue_one = [&](int s, int buf, int q) {  // q: 0..7 weights, 8..8+JT-1 tokens; buf: the stage buffer's byte offset
     const unsigned st = uni(static_cast<int>(lds_addr) + buf);
     if (q < NLD) {
-      load_to_lds(op.woff[q], op.wbase + static_cast<size_t>(s) * op.wstride, st + (wave * 64 + q * 8) * ROWB);
+      const size_t at = HALF ? min(static_cast<unsigned>(s) * op.wstride, op.wlast) : static_cast<size_t>(s) * op.wstride;
+      load_to_lds(op.woff[q], op.wbase + at, st + (wave * 64 + q * 8) * ROWB);
     } else if (q < NL) {
       const int qq = q - NLD;
-      load_to_lds(op.toff[qq], op.tbase + static_cast<size_t>(s) * ROWB, st + TN * ROWB + ((wave * JT + qq) * 8) * ROWB);
+      const size_t at = HALF ? min(static_cast<unsigned>(s * ROWB), op.tlast) : static_cast<size_t>(s) * ROWB;
+      load_to_lds(op.toff[qq], op.tbase + at, st + TN * ROWB + ((wave * JT + qq) * 8) * ROWB);
     }
   };
   auto read_a = [&](int buf, int u, int i) { return lds_read16(ao[u] + static_cast<unsigned>(buf + i * ablock)); };
@@ -738,7 +747,20 @@ __device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f
       ++s;
     }
   });
-  stage(s, No{}, std::integral_constant<int, 0>{});
+  if constexpr (HALF) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) af[1][i] = read_a(cur, 1, i);
+#pragma unroll
+    for (int j = 0; j < JB; ++j) {
+      ring[j % RING] = read_b(cur, JB + j);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (j < JB_ACC) mma<false, false>(af[1][i], ring[j % RING], acc[i][j]); else mma<false, true>(af[1][i], ring[j % RING], acc[i][j]);
+      }
+    }
+  } else {
+    stage(s, No{}, std::integral_constant<int, 0>{});
+  }
   // the compiler does not see matrix instructions in the assembly above: keep the wait states
   // between the last of them and the first read of an accumulator
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -1017,48 +1039,57 @@ __device__ __forceinline__ unsigned packed_run_offset(int q) {
 // behind the stages, so the epilogue waits for no memory. The slot's gate weight is applied
 // by the combine task, which has instruction slots to spare; here every instruction of the
 // epilogue is one the matrix cores wait for.
-template <int JT, bool down>
+//
+// HALF (down): I is an odd number of 32-k steps (see tile_gemm).
+template <int JT, bool down, bool HALF = false>
 __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int rows, int nblk, unsigned* pend,
                                           unsigned* queue) {
   const int H = uni(p.H), I = uni(p.I), K = uni(p.K);
   const int wave = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
   // packed weights and enough stages: the deeper pipeline
-  const int depth = uni((down ? p.ffn2_packed : p.ffn1_packed) != nullptr ? direct_depth(JT, (down ? I : H) / KS) : 0);
+  const int hp = tiled_h_pitch(I);
+  const int depth = HALF ? 0 : uni((down ? p.ffn2_packed : p.ffn1_packed) != nullptr ? direct_depth(JT, (down ? I : H) / KS) : 0);
   const int* perm = uni(p.perm) + row0;
   const int n0 = uni(nblk) * (down ? TN : G1_COLS);
+  // The last task of a row tile may stand out over the last column: a wave whose columns do not exist
+  // repeats the last ones that do, and its results are not stored.
+  const int wblk = down ? min(n0 / 64 + wave, H / 64 - 1) : min(n0 / 32 + wave, I / 32 - 1);
   TileOperands op;
   int side_dst[2] = {-1, -1};
   int nstages;
   if (down) {
-    nstages = I / KS;
+    nstages = (I + KS - 1) / KS;
+    op.tlast = static_cast<unsigned>(I - KS) * 2u;
     const bool packed = uni(p.ffn2_packed != nullptr ? 1 : 0) != 0;
+    op.wlast = packed ? static_cast<unsigned>(I / 32 - 2) * 4096u : op.tlast;
     if (packed) {
-      const size_t task = static_cast<size_t>(expert) * (H / 64) + (n0 / 64 + wave);
+      const size_t task = static_cast<size_t>(expert) * (H / 64) + wblk;
       op.wbase = uni(reinterpret_cast<const unsigned char*>(p.ffn2_packed)) + task * (static_cast<size_t>(I / 32) * 4096);
       op.wstride = 8192u;
       op.wpacked = true;
     } else {
       op.wpacked = false;
-      op.wbase = uni(reinterpret_cast<const unsigned char*>(p.ffn2)) + (static_cast<size_t>(expert) * H + n0) * I * 2;
+      op.wbase = uni(reinterpret_cast<const unsigned char*>(p.ffn2)) + (static_cast<size_t>(expert) * H + 64 * wblk) * I * 2;
       op.wstride = static_cast<unsigned>(ROWB);
     }
-    op.tbase = uni(reinterpret_cast<const unsigned char*>(p.h)) + static_cast<size_t>(row0) * I * 2;
+    op.tbase = uni(reinterpret_cast<const unsigned char*>(p.h)) + static_cast<size_t>(row0) * hp * 2;
 #pragma unroll
     for (int q = 0; q < NLD; ++q) {
       const int row = stage_row(NLD, q);
       op.woff[q] = packed ? packed_run_offset(q)
-                          : static_cast<unsigned>(row) * static_cast<unsigned>(I * 2) + stage_chunk_bytes(row);
+                          : static_cast<unsigned>(row & 63) * static_cast<unsigned>(I * 2) + stage_chunk_bytes(row);
     }
 #pragma unroll
     for (int q = 0; q < JT; ++q) {
       const int row = stage_row(JT, q);
-      op.toff[q] = static_cast<unsigned>(min(row, rows - 1)) * static_cast<unsigned>(I * 2) + stage_chunk_bytes(row);
+      op.toff[q] = static_cast<unsigned>(min(row, rows - 1)) * static_cast<unsigned>(hp * 2) + stage_chunk_bytes(row);
     }
   } else {
     nstages = H / KS;
+    op.wlast = op.tlast = 0u;  // (not looked at)
     const bool packed = uni(p.ffn1_packed != nullptr ? 1 : 0) != 0;
     if (packed) {
-      const size_t task = static_cast<size_t>(expert) * (I / 32) + (n0 / 32 + wave);
+      const size_t task = static_cast<size_t>(expert) * (I / 32) + wblk;
       op.wbase = uni(reinterpret_cast<const unsigned char*>(p.ffn1_packed)) + task * (static_cast<size_t>(H / 32) * 4096);
       op.wstride = 8192u;
       op.wpacked = true;
@@ -1073,7 +1104,7 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
       const int row = stage_row(NLD, q);
       // weight stage rows 64w..64w+31: gate rows n0+32w.., 64w+32..64w+63: up rows I+n0+32w..
       const int wl = row & 63;
-      const int wrow = (wl < 32 ? n0 : I + n0 - 32) + 32 * wave + wl;
+      const int wrow = (wl < 32 ? 0 : I - 32) + 32 * wblk + wl;
       op.woff[q] = packed ? packed_run_offset(q)
                           : static_cast<unsigned>(wrow) * static_cast<unsigned>(H * 2) + stage_chunk_bytes(row);
     }
@@ -1105,7 +1136,7 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
       tile_gemm_direct<JT, 2>(op, nstages, acc, pend, queue, next);
     }
   } else {
-    tile_gemm<JT>(op, nstages, acc, pend, queue, next, load_side);
+    tile_gemm<JT, HALF>(op, nstages, acc, pend, queue, next, load_side);
   }
   if (threadIdx.x == 0) task_notes()[0] = next;  // the epilogue's barriers publish it
 
@@ -1127,7 +1158,8 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
       }
     __syncthreads();
     // 16 lanes store one row's 256 bytes; a wave stores 4 rows per instruction
-    unsigned char* h = uni(reinterpret_cast<unsigned char*>(p.h)) + (static_cast<size_t>(row0) * I + n0) * 2;
+    unsigned char* h = uni(reinterpret_cast<unsigned char*>(p.h)) + (static_cast<size_t>(row0) * hp + n0) * 2;
+    const bool live = n0 + (lane & 15) * 8 < I;  // the lane's columns exist
     // (the reads of a batch first, then its stores: a store's assembly orders memory
     // operations around it, and one LDS round trip per store would add up to microseconds)
     constexpr int NIT = 8 * JT / WAVES, BATCH = 8;
@@ -1142,8 +1174,8 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
         const int row = ((it0 + u) * WAVES + wave) * 4 + (lane >> 4);
-        if (it0 + u < NIT && row < rows)
-          st16_through(h + static_cast<size_t>(row) * I * 2 + (lane & 15) * 16, v[u]);
+        if (it0 + u < NIT && ((row < rows) & live))
+          st16_through(h + static_cast<size_t>(row) * hp * 2 + (lane & 15) * 16, v[u]);
       }
     }
     __syncthreads();  // the slab is stage memory again
@@ -1156,6 +1188,7 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
     }
     __syncthreads();
     unsigned char* y = uni(reinterpret_cast<unsigned char*>(p.y)) + n0 * 2;
+    const bool live = n0 + (lane & 31) * 8 < H;  // the lane's columns exist
 #pragma unroll
     for (int part = 0; part < (JT + 3) / 4; ++part) {
 #pragma unroll
@@ -1187,7 +1220,7 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
         }
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
-          if (dst[u] >= 0) st16_through(y + static_cast<size_t>(dst[u]) * H * 2 + (lane & 31) * 16, v[u]);
+          if ((dst[u] >= 0) & live) st16_through(y + static_cast<size_t>(dst[u]) * H * 2 + (lane & 31) * 16, v[u]);
       }
       __syncthreads();
     }
@@ -1221,6 +1254,27 @@ __device__ __noinline__ void tiled_gemm_task(ParamsRef pv, const TileDesc& tile_
     if (down) tile_task<3, true>(p, expert, row0, rows, nblk, pend, queue); else tile_task<3, false>(p, expert, row0, rows, nblk, pend, queue);
   } else {
     if (down) tile_task<2, true>(p, expert, row0, rows, nblk, pend, queue); else tile_task<2, false>(p, expert, row0, rows, nblk, pend, queue);
+  }
+}
+
+// the down tasks of layers whose I is an odd number of 32-k steps
+__device__ __noinline__ void tiled_odd_down_task(ParamsRef pv, const TileDesc& tile_in, int nblk, unsigned* pend_in,
+                                                 unsigned* queue_in) {
+  ParamsRef p = uniform_params(pv);
+  unsigned* pend = uni(pend_in);
+  unsigned* queue = uni(queue_in);
+  const int expert = uni(tile_in.expert), row0 = uni(tile_in.row0), rows = uni(tile_in.rows);
+  switch ((rows + 31) >> 5) {
+    case 1:
+    case 2: tile_task<2, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 3: tile_task<3, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 4: tile_task<4, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 5: tile_task<5, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 6: tile_task<6, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 7: tile_task<7, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 8: tile_task<8, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 9: tile_task<9, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
+    default: tile_task<10, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
   }
 }
 
@@ -1391,6 +1445,9 @@ __device__ __forceinline__ int xcc_id() {
 
 // The launch parameters are read in place and the task calls keep the local
 // calling convention, as in the streaming variant (see its worker loop).
+// ODD: I is an odd number of 32-k steps (a kernel of its own: as a branch of this one it cost every
+// task of the others half a microsecond).
+template <bool ODD>
 __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void moe_tiled_kernel(
     const Params params) {
   ParamsRef p = kernel_params();
@@ -1414,8 +1471,8 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
   const unsigned t_scan = n_rt + n_es;
   const unsigned t_scatter0 = t_scan + 1u;
   const unsigned t_dyn0 = t_scatter0 + n_sc;
-  const unsigned nt1 = static_cast<unsigned>(p.I / G1_COLS);
-  const unsigned nt2 = static_cast<unsigned>(p.H / TN);
+  const unsigned nt1 = static_cast<unsigned>((p.I + G1_COLS - 1) / G1_COLS);
+  const unsigned nt2 = static_cast<unsigned>((p.H + TN - 1) / TN);
   const unsigned ncmb = (T + CMB_TOK - 1u) / CMB_TOK;
   const unsigned n_groups = gridDim.x;
   const int home = xcc_id();
@@ -1537,7 +1594,11 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
         ok = wg_wait_ge(p, &p.g1_done[m].v, nt1, &sh);
         if (ok) {
           if (p.trace) t_ready = wall_clock64();
-          tiled_gemm_task(p, tile, static_cast<int>(jj % nt2), 1, pend, &ctl->xq[q].v);
+          if constexpr (ODD) {
+            tiled_odd_down_task(p, tile, static_cast<int>(jj % nt2), pend, &ctl->xq[q].v);
+          } else {
+            tiled_gemm_task(p, tile, static_cast<int>(jj % nt2), 1, pend, &ctl->xq[q].v);
+          }
           pend = &ctl->g2_done.v;
           trace(t_dyn0 + nm * nt1 + lo * nt2 + jj, 4, m, t_fetch, t_ready);
           j = task_notes()[0];
@@ -1599,17 +1660,30 @@ int tiled_max_tokens() { return 1 << 21; }
 size_t tiled_y_bytes(size_t rows, size_t hidden) { return rows * hidden * 2; }
 
 hipError_t launch_tiled_kernel(const Params& p, int grid, hipStream_t stream) {
-  hipLaunchKernelGGL(moe_tiled_kernel, dim3(grid), dim3(T_THREADS), TILED_LDS_BYTES, stream, p);
+  auto* kernel = p.I % KS == 0 ? moe_tiled_kernel<false> : moe_tiled_kernel<true>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(T_THREADS), TILED_LDS_BYTES, stream, p);
   return hipGetLastError();
 }
 
 hipError_t prepare_tiled_kernel() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(moe_tiled_kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, TILED_LDS_BYTES);
+  for (auto* kernel : {moe_tiled_kernel<false>, moe_tiled_kernel<true>}) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, TILED_LDS_BYTES);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
+// the lesser of the two kernels' numbers of workgroups a CU holds
 hipError_t tiled_kernel_occupancy(int* per_cu) {
-  return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, moe_tiled_kernel, T_THREADS, TILED_LDS_BYTES);
+  *per_cu = 0x7FFFFFFF;
+  for (auto* kernel : {moe_tiled_kernel<false>, moe_tiled_kernel<true>}) {
+    int n = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, T_THREADS, TILED_LDS_BYTES);
+    if (e != hipSuccess) return e;
+    if (n < *per_cu) *per_cu = n;
+  }
+  return hipSuccess;
 }
 
 }  // namespace fmoe

@@ -228,6 +228,16 @@ def test_tiled_short_tiles_of_many_stages(rows, H, I):
     check_tile_heights(rows, H, I)
 
 
+@pytest.mark.parametrize("rows", [1, 70, 161, 300, 330])
+@pytest.mark.parametrize("H,I", [(128, 128), (192, 160), (320, 224), (448, 352), (576, 672), (64 * 9, 32 * 9)])
+def test_tiled_ragged_columns(rows, H, I):
+    """Hidden sizes that are no multiple of a task's 256 columns and intermediate sizes that are none of
+    its 128 (a wave's columns exist or not as a whole), with k an even or an odd number of 32-k steps
+    (the last stage of the odd ones starts 32 k early and multiplies its second half only; h rows are
+    padded to whole lines), on every depth of the staged pipeline."""
+    check_tile_heights(rows, H, I)
+
+
 def check_tile_heights(rows, H, I):
     cfg = synth.MoeConfig("heights", rows, H, 2, 2, I, "bf16")
     print("tile heights", rows, H, I, flush=True)
