@@ -14,7 +14,7 @@
 //   gate/up  (row tile, 128 h columns): 256 token rows x 256 weight rows, gate
 //            and up rows side by side so that SiLU(gate)*up happens in registers
 //   down     (row tile, 256 output columns): same tile, weighted bf16 rows to y
-//   combine  8 tokens: out = sum over slots of y
+//   combine  1 to 8 tokens: out = sum over slots of y
 // GEMM tile: up to 320 token rows x 256 weight rows, K stepped by 64; each wave
 // owns 64 weight rows x all token rows of it as 4 x (2*JT) MFMA 16x16x32 blocks
 // (JT = 32-row blocks of the tile), up to 320 accumulator registers. Two
@@ -48,7 +48,7 @@ constexpr int WAVES = T_THREADS / 64;  // one per SIMD
 constexpr int NLD = 8;             // 8-row loads per wave, operand and stage
 constexpr int G1_COLS = TN / 2;    // h columns per gate/up task
 constexpr int RT_TOK = 32;         // tokens per scatter task
-constexpr int CMB_TOK = 8;         // tokens per combine task
+constexpr int CMB_TOK = 8;         // tokens per combine task at most
 
 extern __shared__ __align__(16) unsigned char lds_raw[];
 
@@ -1365,8 +1365,8 @@ __device__ __forceinline__ void combine_units(const unsigned short* y, const uns
       for (int i = 0; i < 8; ++i) s[i] = 0.0f;
     }
   };
-  // Units go in straight-line runs of CMB_RUN (no loop-carried registers: a value that is
-  // still on its way from memory must never be copied), the rest one by one.
+  // Units go in straight-line runs of CMB_RUN, 4, 2 and 1 (no loop-carried registers: a value that is
+  // still on its way from memory must never be copied).
   auto run = [&](auto n_tag, int u0) {
     constexpr int N = decltype(n_tag)::value;
 #pragma unroll
@@ -1390,10 +1390,18 @@ __device__ __forceinline__ void combine_units(const unsigned short* y, const uns
   };
   int u0 = 0;
   for (; u0 + CMB_RUN <= nunits; u0 += CMB_RUN) run(std::integral_constant<int, CMB_RUN>{}, u0);
-  for (; u0 < nunits; ++u0) run(std::integral_constant<int, 1>{}, u0);
+  if (u0 + 4 <= nunits) {
+    run(std::integral_constant<int, 4>{}, u0);
+    u0 += 4;
+  }
+  if (u0 + 2 <= nunits) {
+    run(std::integral_constant<int, 2>{}, u0);
+    u0 += 2;
+  }
+  if (u0 < nunits) run(std::integral_constant<int, 1>{}, u0);
 }
 
-__device__ __noinline__ void tiled_combine_task(ParamsRef pv, int blk) {
+__device__ __noinline__ void tiled_combine_task(ParamsRef pv, int blk, int tok_in) {
   ParamsRef p = uniform_params(pv);
   const int H = uni(p.H), K = uni(p.K), T = uni(p.T), E = uni(p.E), W = uni(p.W);
   unsigned short* out = uni(reinterpret_cast<unsigned short*>(p.out));
@@ -1403,8 +1411,9 @@ __device__ __noinline__ void tiled_combine_task(ParamsRef pv, int blk) {
   const float* topk_w = uni(p.topk_w);
   unsigned long long* masks = uni(p.masks);
   const int tid = threadIdx.x;
-  const int t0 = uni(blk) * CMB_TOK;
-  const int ntok = uni(min(CMB_TOK, T - t0));
+  const int tok = uni(tok_in);
+  const int t0 = uni(blk) * tok;
+  const int ntok = uni(min(tok, T - t0));
   // which (token, slot) pairs of this task hold an expert, and their gate weights: one load each
   float* wts = reinterpret_cast<float*>(lds_raw);                      // [CMB_TOK * MAX_TOPK]
   unsigned char* flag = lds_raw + CMB_TOK * MAX_TOPK * sizeof(float);  // [CMB_TOK * MAX_TOPK]
@@ -1473,7 +1482,12 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
   const unsigned t_dyn0 = t_scatter0 + n_sc;
   const unsigned nt1 = static_cast<unsigned>((p.I + G1_COLS - 1) / G1_COLS);
   const unsigned nt2 = static_cast<unsigned>((p.H + TN - 1) / TN);
-  const unsigned ncmb = (T + CMB_TOK - 1u) / CMB_TOK;
+  // as few tokens to a combine task as one round of tasks allows (8 tokens always, us, 30B shape: T=600
+  // 306.5 -> 302.3, where 75 workgroups had a task and the others none; 235B shape T=700 1027 -> 1021; two
+  // rounds of half as many tokens: T=600 303.9)
+  int cmb_tok = 1;
+  while (cmb_tok < CMB_TOK && T > gridDim.x * cmb_tok) cmb_tok *= 2;
+  const unsigned ncmb = (T + cmb_tok - 1u) / cmb_tok;
   const unsigned n_groups = gridDim.x;
   const int home = xcc_id();
   bool first = true, ok = true;
@@ -1618,7 +1632,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
     __syncthreads();
     if (c >= ncmb) break;
     const long long t_ready = p.trace ? wall_clock64() : 0;
-    tiled_combine_task(p, static_cast<int>(c));
+    tiled_combine_task(p, static_cast<int>(c), cmb_tok);
     trace(t_dyn0 + nm * (nt1 + nt2) + c, 5, c, t_fetch, t_ready);
   }
 
