@@ -45,8 +45,8 @@ BOUND = {
 FETCH_SCALE = 0.5
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 # device code only: the host launcher does not change what a kernel reads or writes
-KERNEL_SOURCES = ["moe_stream_kernel.hip", "moe_split_kernel.hip", "moe_tiled_kernel.hip", "moe_stream_device.h",
-                  "moe_device.h", "moe_params.h"]
+KERNEL_SOURCES = ["moe_stream_kernel.hip", "moe_split_kernel.hip", "moe_tiled_kernel.hip", "moe_tiled_f32_kernel.hip",
+                  "moe_stream_device.h", "moe_tiled_device.h", "moe_device.h", "moe_params.h"]
 
 
 def kernel_sources_digest():

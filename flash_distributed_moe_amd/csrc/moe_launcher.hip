@@ -30,6 +30,9 @@ hipError_t split_kernel_occupancy(int* per_cu);
 hipError_t pack_weights(const void* src, void* dst, int dtype, int E, int H, int I, int which,
                         hipStream_t stream);
 hipError_t launch_tiled_kernel(const Params& p, int grid, hipStream_t stream);
+hipError_t launch_tiled_f32_kernel(const Params& p, int grid, hipStream_t stream);
+hipError_t prepare_tiled_f32_kernel();
+hipError_t tiled_f32_kernel_occupancy(int* per_cu);
 hipError_t prepare_tiled_kernel();
 hipError_t stream_kernel_occupancy(int dtype, int* per_cu);
 hipError_t tiled_kernel_occupancy(int* per_cu);
@@ -77,14 +80,16 @@ struct Layout {
 constexpr int kMaxGroups = 1024;  // workgroups a launch may use (one per CU)
 
 // AUTO hands a batch to the tiled variant from this many rows an expert on (on average):
-// packed weights / the caller's row-major weights. Below it the streaming variant runs, which
-// is what its share of `y` is sized for.
+// packed weights / the caller's row-major weights / float32. Below it the streaming variant runs,
+// which is what its share of `y` is sized for (bf16).
 constexpr int kAutoTiledRowsPacked = 26;
 constexpr int kAutoTiledRowsRowMajor = 14;
+constexpr int kAutoTiledRowsF32 = 10;
 
 // need_tiled: the tiled variant may run on this workspace.
 Layout make_layout(const FlashMoeLayerDesc& d, bool need_tiled) {
   Layout L{};
+  need_tiled = need_tiled && d.dtype == FLASH_MOE_BF16;  // (float32 layers have one layout for both variants)
   const size_t rows = static_cast<size_t>(d.max_tokens) * d.top_k;
   const size_t esz = d.dtype == FLASH_MOE_BF16 ? 2 : 4;
   L.W = (d.max_tokens + 63) / 64;
@@ -165,7 +170,7 @@ hipError_t validate(const FlashMoeLayerDesc* d) {
   return hipSuccess;
 }
 
-// The tiled variant needs bf16, two 64-k stages in either projection, and token rows and an expert's
+// The tiled variant needs two 64-k stages in either projection, and token rows and an expert's
 // weights that it can address with 32-bit byte offsets. H need be no multiple of its 256 columns nor I
 // one of 128: what stands out over the last column costs less than the streaming variant's tiles of 64
 // rows, each of which reads its expert's weights again (us, streaming / tiled: E=40, k=5, H=1344, I=736
@@ -176,12 +181,15 @@ hipError_t validate(const FlashMoeLayerDesc* d) {
 // T=320 905 / 960, T=384 934 / 969, T=512 1054 / 976), and from about 14 rows on
 // the caller's row-major weights, which the streaming variant reads half a
 // cache line at a time (30B: T=192 309 / 318, T=256 318 / 318, T=320 346 / 320;
-// 235B: T=192 1030 / 1001, T=256 1055 / 1007, T=384 1142 / 1015).
+// 235B: T=192 1030 / 1001, T=256 1055 / 1007, T=384 1142 / 1015). float32 has a tiled kernel of its own,
+// from 10 rows an expert on: up to 9 the streaming variant's early tasks carry a tile each (us,
+// streaming / tiled, packed: 30B shape T=128 421 / 428, T=160 541 / 437, T=256 586 / 452; E=40, k=5,
+// H=1344, I=736 T=60 117 / 148, T=120 189 / 152; row-major: 30B T=128 548 / 487, T=256 595 / 510; E=16,
+// k=2, H=320, I=160 T=64 50 / 56, T=128 60 / 56).
 bool tiled_eligible(const FlashMoeLayerDesc& d, int tokens_num) {
-  return d.dtype == FLASH_MOE_BF16 && d.hidden >= 128 && d.intermediate >= 128 &&
-         tokens_num <= fmoe::tiled_max_tokens() &&
-         static_cast<long long>(tokens_num) * d.hidden * 2 < (1ll << 32) &&
-         static_cast<long long>(d.intermediate) * d.hidden * 4 < (1ll << 32);
+  const long long esz = d.dtype == FLASH_MOE_BF16 ? 2 : 4;
+  return d.hidden >= 128 && d.intermediate >= 128 && tokens_num <= fmoe::tiled_max_tokens() &&
+         tokens_num * esz * d.hidden < (1ll << 32) && 2 * esz * d.intermediate * d.hidden < (1ll << 32);
 }
 
 // What the choice of a kernel depends on beside the layer and the batch.
@@ -218,8 +226,13 @@ int split_row_blocks(const FlashMoeLayerDesc& d, int tokens_num, const Machine& 
 int sched_for(const FlashMoeLayerDesc& d, int tokens_num, const Machine& m) {
   if (d.sched == FLASH_MOE_SCHED_STREAM) return FLASH_MOE_SCHED_STREAM;
   if (!tiled_eligible(d, tokens_num)) return FLASH_MOE_SCHED_STREAM;
-  if (d.sched == FLASH_MOE_SCHED_TILED) return FLASH_MOE_SCHED_TILED;
   const long long rows = static_cast<long long>(tokens_num) * d.top_k;
+  if (d.dtype == FLASH_MOE_F32) {
+    if (m.traced) return FLASH_MOE_SCHED_STREAM;  // the float32 tiled kernel writes no task records
+    if (d.sched == FLASH_MOE_SCHED_TILED) return FLASH_MOE_SCHED_TILED;
+    return rows >= static_cast<long long>(kAutoTiledRowsF32) * d.experts ? FLASH_MOE_SCHED_TILED : FLASH_MOE_SCHED_STREAM;
+  }
+  if (d.sched == FLASH_MOE_SCHED_TILED) return FLASH_MOE_SCHED_TILED;
   const bool packed = (d.flags & (FLASH_MOE_FLAG_PACK_WEIGHTS | FLASH_MOE_FLAG_WEIGHTS_PREPACKED)) != 0;
   // Row-major weights of moderate size: the split-k kernel is faster as far as it goes (us, tiled /
   // split-k, 30B shape: T=224 309 / 277, T=256 313 / 292, with four hot experts 327 / 307; H=1024,
@@ -321,6 +334,12 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
     // a down task in four parts, two of them to a workgroup, unless that leaves CUs without one
     p.split_down = d.intermediate >= 256 && std::min<long long>(slots, d.experts) * (d.hidden / 128) < p.n_groups ? 8 : 4;
   }
+  const bool tiled = sched_for(d, T, m) == FLASH_MOE_SCHED_TILED;
+  if (tiled && d.dtype == FLASH_MOE_F32) {
+    p.n_groups = std::min(2 * m.n_groups, kMaxGroups);  // two workgroups of four waves a CU
+    p.n_workers = p.n_groups * 4;
+    p.early = 1;  // (the last selection raises FLAG_ROUTED)
+  }
   p.max_mtiles = L.max_mtiles;
   p.spin_limit = l->spin_limit;
   p.tokens = (d.flags & FLASH_MOE_FLAG_RMSNORM) ? static_cast<const void*>(l->ws + L.xn) : tokens;
@@ -337,7 +356,7 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   // T=8192 6770 / 10930: the streaming variant's row tiles of one expert each fetch its
   // weights again, and the row-major rows stream at the higher rate then); bf16 batches are
   // faster on the packed copy at every size.
-  const bool use_packed = pack && !(d.dtype == FLASH_MOE_F32 &&
+  const bool use_packed = pack && !(d.dtype == FLASH_MOE_F32 && !tiled &&
                                     static_cast<long long>(T) * d.top_k >= 16ll * d.experts);
   p.ffn1_packed = use_packed ? l->ws + L.pack1 : prepacked ? d.ffn1_weights : nullptr;
   p.ffn2_packed = use_packed ? l->ws + L.pack2 : prepacked ? d.ffn2_weights : nullptr;
@@ -366,6 +385,14 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   p.trace = l->trace;
   p.trace_cap = l->trace_cap;
   return p;
+}
+
+hipError_t launch_layer(const fmoe::Params& p, int dtype, int sched, hipStream_t stream) {
+  if (sched == FLASH_MOE_SCHED_TILED)
+    return dtype == FLASH_MOE_BF16 ? fmoe::launch_tiled_kernel(p, p.n_groups, stream)
+                                   : fmoe::launch_tiled_f32_kernel(p, p.n_groups, stream);
+  return p.split ? fmoe::launch_split_kernel(p, p.n_groups, stream)
+                 : fmoe::launch_stream_kernel(p, dtype, p.n_groups, stream);
 }
 
 }  // namespace
@@ -488,6 +515,7 @@ int flashMoeCreate(FlashMoeLauncher** out, const FlashMoeLayerDesc* desc, void* 
   if ((e = fmoe::prepare_stream_kernel()) != hipSuccess) return fail(e);
   if ((e = fmoe::prepare_split_kernel()) != hipSuccess) return fail(e);
   if ((e = fmoe::prepare_tiled_kernel()) != hipSuccess) return fail(e);
+  if ((e = fmoe::prepare_tiled_f32_kernel()) != hipSuccess) return fail(e);
   // Waits happen inside the kernels, so every workgroup of a launch must be resident at
   // once: one per CU, which the kernels' resources allow only if nothing else is asked of them.
   int per_cu = 0;
@@ -497,6 +525,8 @@ int flashMoeCreate(FlashMoeLauncher** out, const FlashMoeLayerDesc* desc, void* 
   if (per_cu < 1) return fail(hipErrorLaunchOutOfResources);
   if ((e = fmoe::tiled_kernel_occupancy(&per_cu)) != hipSuccess) return fail(e);
   if (per_cu < 1) return fail(hipErrorLaunchOutOfResources);
+  if ((e = fmoe::tiled_f32_kernel_occupancy(&per_cu)) != hipSuccess) return fail(e);
+  if (per_cu < 2) return fail(hipErrorLaunchOutOfResources);
   if ((e = hipMalloc(reinterpret_cast<void**>(&l->ws), l->layout.total)) != hipSuccess)
     return fail(e);
   if ((e = hipHostMalloc(reinterpret_cast<void**>(&l->host_error), 64, hipHostMallocDefault)) !=
@@ -567,13 +597,7 @@ int flashMoeLaunch(FlashMoeLauncher* l, const void* tokens, void* output, int to
   if (l->desc.flags & FLASH_MOE_FLAG_RMSNORM)
     FMOE_HIP_CHECK(fmoe::launch_rmsnorm(tokens, l->desc.norm_weight, l->ws + l->layout.xn, l->desc.dtype,
                                         tokens_num, l->desc.hidden, l->desc.norm_eps, stream));
-  if (flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED) {
-    FMOE_HIP_CHECK(fmoe::launch_tiled_kernel(p, p.n_groups, stream));
-  } else if (p.split) {
-    FMOE_HIP_CHECK(fmoe::launch_split_kernel(p, p.n_groups, stream));
-  } else {
-    FMOE_HIP_CHECK(fmoe::launch_stream_kernel(p, l->desc.dtype, p.n_groups, stream));
-  }
+  FMOE_HIP_CHECK(launch_layer(p, l->desc.dtype, flashMoeSchedFor(l, tokens_num), stream));
   return hipSuccess;
 }
 
@@ -622,6 +646,7 @@ hipError_t static_device(int device, const StaticDevice** out) {
     FMOE_HIP_CHECK(fmoe::prepare_stream_kernel());
     FMOE_HIP_CHECK(fmoe::prepare_split_kernel());
     FMOE_HIP_CHECK(fmoe::prepare_tiled_kernel());
+    FMOE_HIP_CHECK(fmoe::prepare_tiled_f32_kernel());
     // as in flashMoeCreate: every workgroup of a launch must be resident at once
     int per_cu = 0;
     FMOE_HIP_CHECK(fmoe::stream_kernel_occupancy(FLASH_MOE_BF16, &per_cu));
@@ -632,6 +657,8 @@ hipError_t static_device(int device, const StaticDevice** out) {
     if (per_cu < 1) FMOE_FAIL(hipErrorLaunchOutOfResources, "the split-k kernel does not fit a CU");
     FMOE_HIP_CHECK(fmoe::tiled_kernel_occupancy(&per_cu));
     if (per_cu < 1) FMOE_FAIL(hipErrorLaunchOutOfResources, "the tiled kernel does not fit a CU");
+    FMOE_HIP_CHECK(fmoe::tiled_f32_kernel_occupancy(&per_cu));
+    if (per_cu < 2) FMOE_FAIL(hipErrorLaunchOutOfResources, "the float32 tiled kernel does not fit a CU twice");
     // the error word starts at zero (the array is zero-initialised with the code object,
     // but a process may have failed launches behind it)
     FMOE_HIP_CHECK(hipMemset(static_cast<unsigned char*>(ptr) + kScratchErrorOffset, 0, 256));
@@ -725,13 +752,7 @@ int flashMoeLaunchNoAlloc(const FlashMoeLayerDesc* desc, const void* tokens, voi
   if (desc->flags & FLASH_MOE_FLAG_RMSNORM)
     FMOE_HIP_CHECK(fmoe::launch_rmsnorm(tokens, desc->norm_weight, l.ws + l.layout.xn, desc->dtype, tokens_num,
                                         desc->hidden, desc->norm_eps, stream));
-  if (sched == FLASH_MOE_SCHED_TILED) {
-    FMOE_HIP_CHECK(fmoe::launch_tiled_kernel(p, p.n_groups, stream));
-  } else if (p.split) {
-    FMOE_HIP_CHECK(fmoe::launch_split_kernel(p, p.n_groups, stream));
-  } else {
-    FMOE_HIP_CHECK(fmoe::launch_stream_kernel(p, desc->dtype, p.n_groups, stream));
-  }
+  FMOE_HIP_CHECK(launch_layer(p, desc->dtype, sched, stream));
   return hipSuccess;
 }
 
@@ -798,7 +819,7 @@ int flashMoeReadIntermediate(FlashMoeLauncher* l, int tokens_num, void* h, void*
   const size_t esz = l->desc.dtype == FLASH_MOE_BF16 ? 2 : 4;
   const size_t rows = static_cast<size_t>(tokens_num) * l->desc.top_k;
   const size_t row_bytes = esz * l->desc.intermediate;
-  const bool tiled = flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED;
+  const bool tiled = l->desc.dtype == FLASH_MOE_BF16 && flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED;
   const size_t pitch = tiled ? esz * fmoe::tiled_h_pitch(l->desc.intermediate) : row_bytes;
   if (rows != 0)
     FMOE_HIP_CHECK(hipMemcpy2D(h, row_bytes, l->ws + l->layout.h, pitch, row_bytes, rows, hipMemcpyDeviceToHost));
@@ -813,7 +834,7 @@ int flashMoeReadDownRows(FlashMoeLauncher* l, int tokens_num, void* y, int* elem
   if (tokens_num < 0 || tokens_num > l->desc.max_tokens)
     FMOE_FAIL(hipErrorInvalidValue, "tokens_num = %i", tokens_num);
   FMOE_HIP_CHECK(hipStreamSynchronize(stream));
-  const bool tiled = flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED;
+  const bool tiled = l->desc.dtype == FLASH_MOE_BF16 && flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED;
   const size_t rows = static_cast<size_t>(tokens_num) * l->desc.top_k;
   const size_t bytes = rows * l->desc.hidden * (tiled ? 2 : 4);
   const size_t kept = (l->layout.xn - l->layout.y);  // the region's size up to the next one

@@ -56,13 +56,6 @@ constexpr int split_lds_bytes(int rb) {
 }
 static_assert(split_lds_bytes(2) + 64 <= 160 * 1024, "LDS of a workgroup");
 
-// LDS operations of this wave are done, then the workgroup barrier (loads from memory stay in flight)
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // A tile as the tables hold it: at most 16 * RB rows of one expert.
 struct SplitTile {
   int expert, row0, rows;

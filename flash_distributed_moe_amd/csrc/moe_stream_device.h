@@ -1,7 +1,9 @@
 // What the streaming and the split-k kernel share: the routing tasks of bf16 layers, the wait for
 // a phase flag, the register transpose of row-major weights and the combine tasks.
 #pragma once
+#ifndef FMOE_PARAMS_IN_KERNARG
 #define FMOE_PARAMS_IN_KERNARG 1
+#endif
 #include "moe_device.h"
 
 namespace fmoe {
@@ -11,6 +13,147 @@ constexpr int ROUTER_LD = ROUTER_KC + 4;  // LDS row stride in floats (bank spre
 constexpr int ROUTER_LDS_FLOATS = 2 * ROUTER_EXP * ROUTER_LD;  // per wave
 
 extern __shared__ __align__(16) float lds_dyn[];  // ROUTER_LDS_FLOATS per wave
+
+// The logits are computed by "dot" tasks: one wave takes 8 tokens x 8 experts,
+// one (token, expert) chain per lane. Token rows and expert rows arrive with
+// fully coalesced 16-byte loads, are converted to float once and staged in the
+// wave's private LDS slice in k-chunks, and feed one sequential chain per lane
+// (k ascending). Each chain ends as a 64-bit candidate key in HBM. A "select"
+// task per token waits for all of the token's expert groups and picks the
+// winners. (bf16 layers of suitable shape run the chains on the matrix core: router_dot16_task.)
+template <typename DT>
+__device__ __noinline__ void router_dot_task(ParamsRef pv, int tg, int eg) {
+  ParamsRef p = uniform_params(pv);
+  typedef typename DT::elem elem;
+  constexpr int EPV = DT::EPV;
+  constexpr int CH_ROW = ROUTER_KC / EPV;               // 16-byte chunks per staged row
+  constexpr int NLD = ROUTER_EXP * CH_ROW / 64;         // loads per lane per tile and chunk
+  // Params is reached through a generic reference; keep what the loops need in
+  // registers so that LDS stores do not force reloads.
+  const int H = p.H, E = p.E, T = p.T;
+  const int lane = lane_id();
+  const int ti = lane >> 3, ei = lane & 7;
+  const int t = tg * ROUTER_TOK + ti;
+  const int e = eg * ROUTER_EXP + ei;
+  float* ws = lds_dyn + (threadIdx.x >> 6) * ROUTER_LDS_FLOATS;  // [ROUTER_EXP][ROUTER_LD]
+  float* xs = ws + ROUTER_EXP * ROUTER_LD;                       // [ROUTER_TOK][ROUTER_LD]
+  const elem* gate = reinterpret_cast<const elem*>(p.gate);
+  const elem* tokens = reinterpret_cast<const elem*>(p.tokens);
+
+  // PF k-chunks of global loads are in flight ahead of the chunk being consumed
+  constexpr int PF = 1;  // deeper prefetch measured slower (registers)
+  uint4 wr[PF][NLD], xr[PF][NLD];
+  auto issue = [&](uint4(&wq)[NLD], uint4(&xq)[NLD], int c0) {  // global -> registers
+    if (c0 >= H) return;
+    const int ch_row = min(ROUTER_KC, H - c0) / EPV;
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      // no branches around the loads: rows past the tile (short last chunk)
+      // re-read the last row and are dropped when staging
+      const int c = i * 64 + lane;
+      const int row = min(c / ch_row, ROUTER_EXP - 1), col = c % ch_row;
+      const int er = min(eg * ROUTER_EXP + row, E - 1);
+      const int tr = min(tg * ROUTER_TOK + row, T - 1);
+      wq[i] = ld16(gate + static_cast<size_t>(er) * H + c0 + col * EPV);
+      xq[i] = ld16(tokens + static_cast<size_t>(tr) * H + c0 + col * EPV);
+    }
+  };
+  auto stage = [&](const uint4(&wq)[NLD], const uint4(&xq)[NLD], int n) {  // -> float rows in LDS
+    const int ch_row = n / EPV;
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const int c = i * 64 + lane;
+      const int row = c / ch_row, col = c % ch_row;
+      if (row < ROUTER_EXP) {
+        float wf[EPV], xf[EPV];
+        unpack<DT>(wq[i], wf);
+        unpack<DT>(xq[i], xf);
+#pragma unroll
+        for (int q = 0; q < EPV; q += 4) {
+          *reinterpret_cast<float4*>(ws + row * ROUTER_LD + col * EPV + q) =
+              make_float4(wf[q], wf[q + 1], wf[q + 2], wf[q + 3]);
+          *reinterpret_cast<float4*>(xs + row * ROUTER_LD + col * EPV + q) =
+              make_float4(xf[q], xf[q + 1], xf[q + 2], xf[q + 3]);
+        }
+      }
+    }
+  };
+
+  float acc = 0.0f;
+  const float* wrow = ws + ei * ROUTER_LD;
+  const float* xrow = xs + ti * ROUTER_LD;
+  auto consume = [&](int n) {
+    // 32 k per block; the next block's LDS reads are in flight while this
+    // block's chain runs (n is a multiple of 64)
+    float4 wa[8], xa[8], wb[8], xb[8];
+    auto lds_load = [&](float4(&w)[8], float4(&x)[8], int k) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        w[q] = *reinterpret_cast<const float4*>(wrow + k + 4 * q);
+        x[q] = *reinterpret_cast<const float4*>(xrow + k + 4 * q);
+      }
+    };
+    auto chain = [&](const float4(&w)[8], const float4(&x)[8]) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        if constexpr (EPV == 8) {
+          acc = __builtin_fmaf(x[q].x, w[q].x, acc);
+          acc = __builtin_fmaf(x[q].y, w[q].y, acc);
+          acc = __builtin_fmaf(x[q].z, w[q].z, acc);
+          acc = __builtin_fmaf(x[q].w, w[q].w, acc);
+        } else {
+          acc = __fadd_rn(acc, __fmul_rn(x[q].x, w[q].x));
+          acc = __fadd_rn(acc, __fmul_rn(x[q].y, w[q].y));
+          acc = __fadd_rn(acc, __fmul_rn(x[q].z, w[q].z));
+          acc = __fadd_rn(acc, __fmul_rn(x[q].w, w[q].w));
+        }
+      }
+    };
+    if (n == ROUTER_KC) {
+      // full chunk: straight-line code, so the two register sets simply
+      // alternate and no copies are needed between blocks
+      lds_load(wa, xa, 0);
+#pragma unroll
+      for (int k = 0; k < ROUTER_KC; k += 64) {
+        lds_load(wb, xb, k + 32);
+        chain(wa, xa);
+        if (k + 64 < ROUTER_KC) lds_load(wa, xa, k + 64);
+        chain(wb, xb);
+      }
+    } else {
+      for (int k = 0; k < n; k += 32) {
+        lds_load(wa, xa, k);
+        chain(wa, xa);
+      }
+    }
+  };
+
+#pragma unroll
+  for (int j = 0; j < PF; ++j) issue(wr[j], xr[j], j * ROUTER_KC);
+  for (int c0 = 0; c0 < H; c0 += PF * ROUTER_KC) {
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      const int cj = c0 + j * ROUTER_KC;
+      if (cj < H) {
+        const int n = min(ROUTER_KC, H - cj);
+        stage(wr[j], xr[j], n);
+        lds_wave_sync();
+        issue(wr[j], xr[j], cj + PF * ROUTER_KC);
+        consume(n);
+        lds_wave_sync();
+      }
+    }
+  }
+
+  const bool valid = (t < T) && (e < E);
+  if (valid) {
+    float v = acc;
+    if (p.bias != nullptr) v = __fadd_rn(v, as_global(p.bias)[e]);
+    stc(&p.cand[static_cast<size_t>(t) * E + e], make_key(v, e, true));
+  }
+  fence_release();
+  if (ei == 0 && t < T) add_relaxed(&p.tok_arrive[t], 1u);
+}
 
 // The same chains on the matrix core, for bf16 layers: V_MFMA_F32_16X16X4_F32 adds
 // its four products to the accumulator one after the other in k order, one
@@ -161,6 +304,13 @@ __device__ __noinline__ void router_select_task(ParamsRef pv, int t) {
                     reinterpret_cast<double*>(lds_dyn + (threadIdx.x >> 6) * ROUTER_LDS_FLOATS));
   const unsigned old = wave_arrive(&p.ctl->router_done.v);
   if (p.early && old == static_cast<unsigned>(p.T) - 1u) broadcast_flag(p, FLAG_ROUTED);
+}
+
+// LDS operations of this wave are done, then the workgroup barrier (loads from memory stay in flight)
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
 // ----------------------------------------------------------------------- waits

@@ -1,0 +1,460 @@
+// Persistent MoE kernel, tiled variant of float32 layers for gfx950: batches where an expert sees
+// more rows than a streaming tile shares its weights with.
+//
+// Two workgroups of 4 waves per CU draw task tickets. Stages as in the bf16 tiled kernel:
+//   router   8 tokens x 8 experts a wave (the streaming kernel's chains), then a selection a token
+//   scan, scatter
+//   gate/up  (row tile, 128 h columns), down (row tile, 256 output columns): up to 96 token rows x
+//            256 weight rows, k stepped by 32; a wave owns 64 weight rows x all token rows
+//   combine  (token, 256 columns), as in the streaming kernel
+//
+// The products run on the bf16 matrix cores, sixteen times as fast as the float32 ones here. Both
+// operands are split into three bf16 parts, x = hi + mid + lo: each part is the rest rounded to
+// nearest, 8 significant bits each, so the three hold all 24 bits of a float exactly (down to values
+// of 2^-109, whose lowest part is subnormal). Of the nine products of parts the six largest are
+// accumulated in float32: hi*hi, hi*mid, mid*hi, mid*mid, hi*lo, lo*hi; what is left out is below
+// 2^-25 of a product, less than the one rounding of a float32 multiplication. A sum of K products is
+// rounded 6*K/32 times instead of K times. The layer's error against float64, relative 2-norm, float32
+// matrix instructions (streaming kernel) / this: 30B shape T=256 1.85e-6 / 1.72e-6, T=512 1.84e-6 /
+// 1.71e-6; E=40, k=5, H=1344, I=736 T=900 1.29e-6 / 1.16e-6; E=10, k=3, H=320, I=2016 T=2000 9.4e-7 / 8.2e-7.
+//
+// Bound by HBM up to some 40 rows an expert, above by splitting and products together. us, streaming /
+// this, 30B shape: T=256 586 / 444, T=512 800 / 466, T=1024 1077 / 585 (2.43 GB and 77 GFLOP: 132
+// TFLOP/s of float32); row-major weights T=1024 1076 / 627; E=32 T=4096 2400 / 1450.
+//
+// A value that is no finite number, or rounds to none in bf16, has no such parts: its products come
+// out as infinities or NaN. A wave whose sums hold one multiplies its block again with the float32
+// matrix instructions, so such inputs give what they give in the streaming kernel.
+//
+// Weights go straight to registers (no other wave of the workgroup reads them), 16 bytes per lane and
+// load, one 32-k step ahead, and are split there; token rows are split once per workgroup, on
+// their way to LDS. The k of a fragment is permuted the way the loads bring it: lane group g of a
+// matrix operand holds k = 4g..4g+3 and 16+4g..16+4g+3 of a step, in both operands.
+//
+// Replaces, for this regime, the reference's moeKernel (src/hip/kernel/moeKernel.h:37-107).
+#include <type_traits>
+
+#include "moe_stream_device.h"
+#include "moe_tiled_device.h"
+
+namespace fmoe {
+
+constexpr int F_JB = 6;              // 16-row token blocks of the tallest row tile
+constexpr int F_TM = 16 * F_JB;      // 96 token rows
+constexpr int F_TN = 256;            // weight rows of a task
+constexpr int F_WAVES = T_THREADS / 64;
+
+// LDS of a workgroup: two steps of token rows, [row block][part][lane] of 16 bytes, then
+// the tile's rows; the routing tasks use it from its first byte on before that.
+constexpr int f_stage_bytes(int jb) { return (jb + (jb & 1)) * 3 * 1024; }
+constexpr int F_SIDE_OFF = 2 * f_stage_bytes(F_JB);
+constexpr int F_LDS_BYTES = F_SIDE_OFF + F_TM * 8 > F_WAVES * ROUTER_LDS_FLOATS * 4 ? F_SIDE_OFF + F_TM * 8 : F_WAVES * ROUTER_LDS_FLOATS * 4;
+static_assert(2 * (F_LDS_BYTES + 256) <= 160 * 1024, "two workgroups a CU");
+
+// four floats -> two words of each part
+__device__ __forceinline__ void split4(const uint4& v, u32x4 (&p)[3], int at) {
+  const unsigned in[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    float a = __uint_as_float(in[2 * q]), b = __uint_as_float(in[2 * q + 1]);
+    const unsigned hi = pack_bf16(a, b);
+    a -= bf16_lo(hi);
+    b -= bf16_hi(hi);
+    const unsigned mid = pack_bf16(a, b);
+    a -= bf16_lo(mid);
+    b -= bf16_hi(mid);
+    p[0][at + q] = hi;
+    p[1][at + q] = mid;
+    p[2][at + q] = pack_bf16(a, b);
+  }
+}
+__device__ __forceinline__ f32x4 mma_bf16(const u32x4& a, const u32x4& b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// 16 bytes at a lane's offset plus a uniform one; AUX 2: non-temporal
+template <int AUX>
+__device__ __forceinline__ uint4 ld16_buffer(const CoherentBuffer& b, unsigned off, unsigned uniform_off) {
+  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(b.rsrc, static_cast<int>(off), static_cast<int>(uniform_off), AUX);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// What a task multiplies. Weight block i (16 of the wave's 64 rows): this lane's 16 bytes of the
+// k-step of 16 number q are at wbase + woff + wblock[i] + q * wstep.
+struct FloatOperands {
+  const unsigned char* wbase;  // uniform
+  unsigned woff;               // this lane's 16 bytes of block 0, k-step 0
+  unsigned wblock[4];          // uniform: bytes from block 0 to block i
+  unsigned wstep;              // uniform
+  const unsigned char* tbase;  // uniform: tokens or h
+  unsigned toff[F_JB];         // this thread's 16 bytes of token load q at step 0
+  int ksteps;                  // k / 32
+};
+
+// acc[i][j] = weight block i x token block j over ksteps * 32 k. Step k, from the loads of the steps
+// before it: its weights are split, the token rows of step k+1 are split and go to the other LDS
+// buffer, the loads of the token rows of k+2 and of the weights of k+1 go out, then the products.
+// The splitting (44 vector instructions a weight block and step) is what the step pays for beside the
+// products; the other wave of the SIMD multiplies meanwhile. A second step of weights in flight gained
+// nothing (30B shape, us, T=512 490 against 466, T=768 536 / 522, T=1024 585 / 585), nor did splitting
+// the next step's weights between the products of this one (two sets of parts do not fit the
+// registers: T=768 641, T=1024 753).
+template <int JB, bool ONCE>
+__device__ __forceinline__ void float_gemm(const FloatOperands& op, f32x4 (&acc)[4][JB]) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int r16 = lane & 15, g = lane >> 4;
+  unsigned char* lds = reinterpret_cast<unsigned char*>(lds_dyn);
+  // The 16-byte slot of (lane group g, row r) in a fragment: 16 g + (r ^ 4 g), so that the rows and
+  // groups a wave writes together fall into different banks.
+  const int rd = (16 * g + (r16 ^ (4 * g))) * 16;
+  // Token load q brings 16 bytes (four k) of row 32 q + tid / 8: chunk tid % 8 of the row's 128 bytes.
+  const int c = tid & 7, trow = tid >> 3;
+  const int wr = (trow >> 4) * 3072 + ((c & 3) * 16 + ((trow & 15) ^ (4 * (c & 3)))) * 16 + (c >> 2) * 8;
+  constexpr int NT = (JB + 1) / 2;
+  const bool odd_half = (JB & 1) && tid >= 128;  // uniform in a wave: rows of the last load that do not exist
+
+  // (through buffer descriptors: a lane offset and a uniform one, no 64-bit address per lane)
+  const CoherentBuffer wbuf = coherent_buffer(op.wbase, 0xFFFFFFFFu), tbuf = coherent_buffer(op.tbase, 0xFFFFFFFFu);
+  uint4 tr[NT], aw[4][2];
+  auto load_t = [&](int k) {
+#pragma unroll
+    for (int q = 0; q < NT; ++q) tr[q] = ld16_buffer<0>(tbuf, op.toff[q], static_cast<unsigned>(k) * 128u);
+  };
+  auto store_t = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      u32x4 p[3];
+      split4(tr[q], p, 0);
+      if (q + 1 < NT || !odd_half) {
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+          *reinterpret_cast<uint2*>(lds + buf * f_stage_bytes(JB) + q * 6144 + m * 1024 + wr) = make_uint2(p[m][0], p[m][1]);
+      }
+    }
+  };
+  auto load_w = [&](int k) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        aw[i][h] = ld16_buffer<ONCE ? 2 : 0>(wbuf, op.woff, static_cast<unsigned>(2 * k + h) * op.wstep + op.wblock[i]);
+      }
+  };
+  const int last = op.ksteps - 1;
+  load_t(0);
+  load_w(0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < JB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  store_t(0);
+  load_t(min(1, last));
+  lds_barrier();
+  auto step = [&](int k, auto b_tag) {
+    constexpr int B = decltype(b_tag)::value;
+    u32x4 a[4][3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      split4(aw[i][0], a[i], 0);
+      split4(aw[i][1], a[i], 2);
+    }
+    store_t(B ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    load_t(min(k + 2, last));
+    load_w(min(k + 1, last));
+    __builtin_amdgcn_sched_barrier(0);
+    // a token block's fragments are read under the products of the one before it, and not earlier
+    const unsigned char* st = lds + B * f_stage_bytes(JB) + rd;
+    u32x4 b[2][3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) b[0][m] = *reinterpret_cast<const u32x4*>(st + m * 1024);
+#pragma unroll
+    for (int j = 0; j < JB; ++j) {
+      if (j + 1 < JB) {
+#pragma unroll
+        for (int m = 0; m < 3; ++m) b[(j + 1) & 1][m] = *reinterpret_cast<const u32x4*>(st + (j + 1) * 3072 + m * 1024);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int pr = 0; pr < 6; ++pr) {
+        constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i][j] = mma_bf16(a[i][pa[pr]], b[j & 1][pb[pr]], acc[i][j]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    lds_barrier();
+  };
+  // The first two steps stand in front of the loop: the compiler counts the loads a wait may leave in
+  // flight from the orders of all ways that lead there.
+  auto pair = [&](int k) {
+    step(k, std::integral_constant<int, 0>{});
+    step(k + 1, std::integral_constant<int, 1>{});
+  };
+  pair(0);  // (k >= 128)
+  int k = 2;
+  asm volatile("; end of the first pair" ::: "memory");
+  for (; k + 1 < op.ksteps; k += 2) pair(k);
+  if (k < op.ksteps) step(k, std::integral_constant<int, 0>{});
+}
+
+// The same block again with the float32 matrix instructions, for sums that are no finite numbers:
+// operands straight from memory, one wave on its own.
+template <int JB>
+__device__ __forceinline__ void float_gemm_exact(const FloatOperands& op, const unsigned (&trow)[JB], f32x4 (&acc)[4][JB]) {
+#pragma unroll
+  for (int j = 0; j < JB; ++j) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int q = 0; q < 2 * op.ksteps; ++q) {
+      const uint4 b = ld16(op.tbase + trow[j] + static_cast<size_t>(q) * 64);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        acc[i][j] = mma16<F32>(ld16(op.wbase + op.wblock[i] + static_cast<size_t>(q) * op.wstep + op.woff), b, acc[i][j]);
+    }
+  }
+}
+
+// One tile task. gate/up: h[row, n0 .. n0+128) (refExpertFFN1.h:51-65); wave w holds gate rows
+// n0+32w.. and the matching up rows, so SiLU(gate)*up happens in registers. down:
+// y[t*K+slot, n0 .. n0+256) = w * (h[row] . W2[e]^T) (refFullMoe.h:58-65, src/hip/kernel/tasks/ffn2Task.h:37-40),
+// float rows with the gate weight applied, as the streaming kernel leaves them. Both are written
+// through, 64 bytes of a row at a time, from the accumulators.
+template <int JB, bool down>
+__device__ __noinline__ void float_task(ParamsRef pv, int expert_in, int row0_in, int rows_in, int shared_in, int nblk_in) {
+  ParamsRef p = uniform_params(pv);
+  const int expert = uni(expert_in), row0 = uni(row0_in), rows = uni(rows_in);
+  const bool packed = uni((down ? p.ffn2_packed : p.ffn1_packed) != nullptr ? 1 : 0) != 0;
+  // weights that no other tile reads pass through the caches without staying; row-major ones come half a
+  // line at a time and have to stay
+  const bool shared = uni(shared_in) != 0 || !packed;
+  const int H = uni(p.H), I = uni(p.I), K = uni(p.K);
+  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int nblk = uni(nblk_in);
+  const int cols = down ? 64 : 32;                        // of a wave
+  const int nw = (down ? H : I) / cols, w0 = nblk * F_WAVES + wave;
+  const int wblk = min(w0, nw - 1);
+  const int* perm = uni(p.perm) + row0;
+  uint2* side = reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(lds_dyn) + F_SIDE_OFF);  // row -> (token, slot), weight
+  FloatOperands op;
+  const int kk = down ? I : H;
+  op.ksteps = kk >> 5;
+  if (packed) {
+    op.wbase = uni(reinterpret_cast<const unsigned char*>(down ? p.ffn2_packed : p.ffn1_packed)) + (static_cast<size_t>(expert) * nw + wblk) * (static_cast<size_t>(kk / 16) * 4096);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) op.wblock[i] = static_cast<unsigned>(i * 1024);
+    op.woff = static_cast<unsigned>(lane * 16);
+    op.wstep = 4096u;
+  } else if (down) {
+    op.wbase = uni(reinterpret_cast<const unsigned char*>(p.ffn2)) + (static_cast<size_t>(expert) * H + 64 * wblk) * I * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) op.wblock[i] = static_cast<unsigned>(16 * i) * static_cast<unsigned>(I * 4);
+    op.woff = static_cast<unsigned>(r16) * static_cast<unsigned>(I * 4) + g * 16;
+    op.wstep = 64u;
+  } else {
+    op.wbase = uni(reinterpret_cast<const unsigned char*>(p.ffn1)) + (static_cast<size_t>(expert) * 2 * I + 32 * wblk) * H * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) op.wblock[i] = static_cast<unsigned>((i & 1) * 16 + (i >> 1) * I) * static_cast<unsigned>(H * 4);
+    op.woff = static_cast<unsigned>(r16) * static_cast<unsigned>(H * 4) + g * 16;
+    op.wstep = 64u;
+  }
+  op.tbase = down ? uni(reinterpret_cast<const unsigned char*>(p.h)) + static_cast<size_t>(row0) * I * 4
+                  : uni(reinterpret_cast<const unsigned char*>(p.tokens));
+  auto row_offset = [&](int row) {
+    const int r = min(row, rows - 1);
+    return down ? static_cast<unsigned>(r) * static_cast<unsigned>(I * 4)
+                : static_cast<unsigned>(ldc(&perm[r]) / K) * static_cast<unsigned>(H * 4);
+  };
+#pragma unroll
+  for (int q = 0; q < (JB + 1) / 2; ++q) op.toff[q] = row_offset(32 * q + (tid >> 3)) + (tid & 7) * 16;
+  if (down && tid < rows)
+    side[tid] = make_uint2(static_cast<unsigned>(ldc(&perm[tid])), __float_as_uint(ldc(&uni(p.row_w)[row0 + tid])));
+
+  f32x4 acc[4][JB];
+  if (shared) {
+    float_gemm<JB, false>(op, acc);
+  } else {
+    float_gemm<JB, true>(op, acc);
+  }
+  if (w0 >= nw) return;  // this wave's columns do not exist: it has multiplied the last ones that do
+  float t = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < JB; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) t = __builtin_fmaf(acc[i][j][v], 0.0f, t);
+  if (__any(t != 0.0f)) {
+    unsigned trow[JB];
+#pragma unroll
+    for (int j = 0; j < JB; ++j) trow[j] = row_offset(16 * j + r16) + g * 16;
+    float_gemm_exact<JB>(op, trow, acc);
+  }
+
+  if (!down) {
+    float* h = uni(reinterpret_cast<float*>(p.h)) + static_cast<size_t>(row0) * I + 32 * w0 + 4 * g;
+#pragma unroll
+    for (int j = 0; j < JB; ++j) {
+      const int row = 16 * j + r16;
+      if (row < rows) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          unsigned hv[4];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) hv[v] = __float_as_uint(silu_mul(acc[i][j][v], acc[2 + i][j][v]));
+          st16_through(h + static_cast<size_t>(row) * I + 16 * i, make_uint4(hv[0], hv[1], hv[2], hv[3]));
+        }
+      }
+    }
+  } else {
+    float* y = uni(p.y) + 64 * w0 + 4 * g;
+#pragma unroll
+    for (int j = 0; j < JB; ++j) {
+      const int row = 16 * j + r16;
+      if (row < rows) {
+        const uint2 d = side[row];
+        const float w = __uint_as_float(d.y);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          st16_through(y + static_cast<size_t>(d.x) * H + 16 * i,
+                       make_uint4(__float_as_uint(acc[i][j][0] * w), __float_as_uint(acc[i][j][1] * w),
+                                  __float_as_uint(acc[i][j][2] * w), __float_as_uint(acc[i][j][3] * w)));
+      }
+    }
+  }
+}
+
+template <bool down>
+__device__ __forceinline__ void float_tile(ParamsRef p, const TileDesc& t, int nblk) {
+  switch (uni((t.rows + 15) >> 4)) {
+    case 1: float_task<1, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
+    case 2: float_task<2, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
+    case 3: float_task<3, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
+    case 4: float_task<4, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
+    case 5: float_task<5, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
+    default: float_task<6, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
+  }
+}
+
+// ---------------------------------------------------------------- worker loop
+// Routing, scan and scatter tasks are handed out statically: every workgroup of the launch is
+// resident (two a CU; the launcher asks). The GEMM tasks come from one queue per XCD, as in the bf16
+// tiled kernel; the other workgroup of the CU covers what a task waits for at its ends.
+__global__ __launch_bounds__(T_THREADS, 2) __attribute__((disable_tail_calls)) void moe_tiled_f32_kernel(
+    const Params params) {
+  ParamsRef p = kernel_params();
+  __shared__ WgShared sh;
+  if (threadIdx.x == 0) {
+    sh.ticket = 0u;
+    sh.ok = 1u;
+    sh.flag[0] = sh.flag[1] = sh.flag[2] = sh.flag[3] = 0u;
+  }
+  __syncthreads();
+  Control* ctl = p.ctl;
+  const int T = p.T, E = p.E;
+  const int G = static_cast<int>(gridDim.x), b = static_cast<int>(blockIdx.x);
+  const int wave = uni(static_cast<int>(threadIdx.x >> 6));
+  const int me = wave * G + b, waves = G * F_WAVES;
+
+  const int n_eg = (E + ROUTER_EXP - 1) / ROUTER_EXP;
+  const int n_dot = (T + ROUTER_TOK - 1) / ROUTER_TOK * n_eg;
+  for (int i = me; i < n_dot; i += waves) router_dot_task<F32>(p, i / n_eg, i % n_eg);
+  for (int t = me; t < T; t += waves) {
+    if (!wave_wait_ge(&p.tok_arrive[t], static_cast<unsigned>(n_eg), ctl, p.spin_limit)) break;
+    router_select_task(p, t);
+  }
+  bool ok = wg_wait_flag(p, FLAG_ROUTED, &sh);
+  const int n_es = (E + SCAN_EXPERTS - 1) / SCAN_EXPERTS;
+  if (ok && b < n_es) {
+    tiled_expert_scan_task(p, b);
+    if (wg_arrive<false>(&ctl->scan_done.v, &sh) == static_cast<unsigned>(n_es) - 1u) tiled_scan_task<F_TM, 16>(p);
+  }
+  if (ok) ok = wg_wait_flag(p, FLAG_SCAN, &sh);
+  const int n_sc = (T + RT_TOK - 1) / RT_TOK;
+  for (int i = b; ok && i < n_sc; i += G) {
+    tiled_scatter_task(p, i);
+    if (wg_arrive<false>(&ctl->perm_done.v, &sh) == static_cast<unsigned>(n_sc) - 1u) wg_broadcast_flag(p, FLAG_PERM);
+  }
+  if (ok) ok = wg_wait_flag(p, FLAG_PERM, &sh);
+
+  const unsigned nm = ok ? ldc(&ctl->n_mtiles.v) : 0u;
+  const unsigned nt1 = static_cast<unsigned>((p.I + 127) / 128), nt2 = static_cast<unsigned>((p.H + 255) / 256);
+  const unsigned n2_total = nm * nt2;
+  const int home = xcc_id();
+  for (int hop = 0; ok && hop < 8; ++hop) {
+    const unsigned q = static_cast<unsigned>((home + hop) & 7);
+    const unsigned lo = nm * q / 8u, hi = nm * (q + 1u) / 8u;
+    const unsigned q1 = (hi - lo) * nt1, q2 = (hi - lo) * nt2;
+    while (ok) {
+      if (threadIdx.x == 0) sh.ticket = add_relaxed(&ctl->xq[q].v, 1u);
+      __syncthreads();
+      const unsigned j = uni(static_cast<int>(sh.ticket));
+      __syncthreads();
+      if (j >= q1 + q2) break;
+      if (j < q1) {
+        const unsigned m = lo + j / nt1;
+        const TileDesc tile = ld_tile(&p.mtiles[m]);
+        float_tile<false>(p, tile, static_cast<int>(j % nt1));
+        wg_arrive<false>(&p.g1_done[m].v, &sh);
+      } else {
+        const unsigned jj = j - q1, m = lo + jj / nt2;
+        const TileDesc tile = ld_tile(&p.mtiles[m]);
+        ok = wg_wait_ge(p, &p.g1_done[m].v, nt1, &sh);
+        if (ok) {
+          float_tile<true>(p, tile, static_cast<int>(jj % nt2));
+          if (wg_arrive<false>(&ctl->g2_done.v, &sh) == n2_total - 1u) wg_broadcast_flag(p, FLAG_G2);
+        }
+      }
+    }
+  }
+  if (ok && n2_total != 0u) ok = wg_wait_flag(p, FLAG_G2, &sh);
+  if (ok) {
+    const unsigned ncomb = static_cast<unsigned>((p.H + COMBINE_COLS - 1) / COMBINE_COLS);
+    combine_items<F32>(p, static_cast<unsigned>(me), static_cast<unsigned>(T) * ncomb, ncomb, static_cast<unsigned>(me), 0u, 0);
+  }
+
+  // The last workgroup out returns every counter to zero for the next launch.
+  fence_release();
+  __syncthreads();
+  if (threadIdx.x == 0) sh.ok = (add_relaxed(&ctl->exit_count.v, 1u) == static_cast<unsigned>(G) - 1u) ? 1u : 0u;
+  __syncthreads();
+  if (sh.ok) {
+    const unsigned err = ldc(&ctl->error.v);
+    if (err != 0u) {
+      recover_after_error(p, err, static_cast<int>(threadIdx.x), T_THREADS);
+      __syncthreads();
+    }
+    const unsigned nmr = min(ldc(&ctl->n_mtiles.v), static_cast<unsigned>(p.max_mtiles));
+    for (unsigned i = threadIdx.x; i < nmr; i += T_THREADS) stc(&p.g1_done[i].v, 0u);
+    for (int i = threadIdx.x; i < G; i += T_THREADS)
+      for (int f = 0; f < 4; ++f) stc(&p.wgflags[i].f[f], 0u);
+    if (threadIdx.x < 8) stc(&ctl->xq[threadIdx.x].v, 0u);
+    if (threadIdx.x == 0) {
+      stc(&ctl->launches.v, ldc(&ctl->launches.v) + 1u);
+      stc(&ctl->router_done.v, 0u);
+      stc(&ctl->scan_done.v, 0u);
+      stc(&ctl->perm_done.v, 0u);
+      stc(&ctl->g2_done.v, 0u);
+      stc(&ctl->n_mtiles.v, 0u);
+      stc(&ctl->exit_count.v, 0u);
+    }
+  }
+}
+
+hipError_t launch_tiled_f32_kernel(const Params& p, int grid, hipStream_t stream) {
+  hipLaunchKernelGGL(moe_tiled_f32_kernel, dim3(grid), dim3(T_THREADS), F_LDS_BYTES, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t prepare_tiled_f32_kernel() {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(moe_tiled_f32_kernel),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, F_LDS_BYTES);
+}
+
+hipError_t tiled_f32_kernel_occupancy(int* per_cu) {
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, moe_tiled_f32_kernel, T_THREADS, F_LDS_BYTES);
+}
+
+}  // namespace fmoe

@@ -30,8 +30,7 @@
 #include <type_traits>
 #include <utility>
 
-#define FMOE_PARAMS_IN_KERNARG 1
-#include "moe_device.h"
+#include "moe_tiled_device.h"
 
 namespace fmoe {
 
@@ -43,117 +42,12 @@ constexpr int TM_MAX = 32 * JT_MAX;  // 320 token rows
 constexpr int TN = 256;            // weight rows per tile
 constexpr int KS = 64;             // k per LDS stage
 constexpr int ROWB = KS * 2;       // bytes of a row per stage: one 128-byte line
-constexpr int T_THREADS = 256;
 constexpr int WAVES = T_THREADS / 64;  // one per SIMD
 constexpr int NLD = 8;             // 8-row loads per wave, operand and stage
 constexpr int G1_COLS = TN / 2;    // h columns per gate/up task
-constexpr int RT_TOK = 32;         // tokens per scatter task
 constexpr int CMB_TOK = 8;         // tokens per combine task at most
 
 extern __shared__ __align__(16) unsigned char lds_raw[];
-
-// ---------------------------------------------------------- workgroup helpers
-// Values that are the same in every lane but that the compiler cannot prove so
-// (they come through a struct reference): pin them to scalar registers, so
-// loops and branches on them stay scalar.
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-template <typename T>
-__device__ __forceinline__ T* uni(T* ptr) {
-  const unsigned long long v = reinterpret_cast<unsigned long long>(ptr);
-  const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(v));
-  const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(v >> 32));
-  return reinterpret_cast<T*>((static_cast<unsigned long long>(hi) << 32) | lo);
-}
-
-struct WgShared {  // small static LDS block
-  unsigned ticket;
-  unsigned next;
-  unsigned ok;
-  unsigned flag[4];
-};
-
-// Thread 0 waits (bounded) for *p >= target; every thread learns the outcome.
-__device__ __forceinline__ bool wg_wait_ge(ParamsRef p, const unsigned* ptr, unsigned target,
-                                           WgShared* sh) {
-  if (threadIdx.x == 0) {
-    unsigned ok = 1u;
-    if (ld_relaxed(ptr) < target) {
-      const long long t0 = wall_clock64();
-      unsigned spins = 0;
-      while (ld_relaxed(ptr) < target) {
-        if ((++spins & 31u) == 0u && ld_relaxed(&p.ctl->error.v) != 0u) {
-          ok = 0u;
-          break;
-        }
-        if (wall_clock64() - t0 > p.spin_limit) {
-          or_relaxed(&p.ctl->error.v, ERR_TIMEOUT);
-          ok = 0u;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(16);
-      }
-    }
-    sh->ok = ok;
-  }
-  __syncthreads();
-  const bool ok = sh->ok != 0u;
-  __syncthreads();
-  fence_acquire();
-  return ok;
-}
-
-__device__ __forceinline__ bool wg_wait_flag(ParamsRef p, int which, WgShared* sh) {
-  if (sh->flag[which] != 0u) return true;  // seen before by this workgroup
-  const bool ok = wg_wait_ge(p, &p.wgflags[blockIdx.x].f[which], 1u, sh);
-  if (ok && threadIdx.x == 0) sh->flag[which] = 1u;
-  __syncthreads();
-  return ok;
-}
-
-// All threads' stores have completed, then one thread bumps the counter. Tile
-// data (h, y) is written through to device-coherent memory, so completion is
-// all a reader on another XCD needs (WRITEBACK adds an agent-scope release for
-// data written with ordinary cached stores; no task does that at present).
-// Readers of h and y use ordinary loads: every cache line of them has a single
-// writer and is not read before it is final, so no reader can hold a stale copy.
-template <bool WRITEBACK>
-__device__ __forceinline__ unsigned wg_arrive(unsigned* counter, WgShared* sh) {
-  fence_release();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    if (WRITEBACK) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    sh->ticket = add_relaxed(counter, 1u);
-  }
-  __syncthreads();
-  const unsigned old = sh->ticket;
-  __syncthreads();
-  return old;
-}
-
-// The same, and the workgroup's next ticket from `queue` in the same trip to
-// memory: thread 0 sends both atomics before it looks at either result.
-__device__ __forceinline__ unsigned wg_arrive_and_draw(unsigned* counter, unsigned* queue,
-                                                       unsigned& next, WgShared* sh) {
-  fence_release();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned old = add_relaxed(counter, 1u);
-    const unsigned nxt = add_relaxed(queue, 1u);
-    sh->ticket = old;
-    sh->next = nxt;
-  }
-  __syncthreads();
-  const unsigned old = sh->ticket;
-  next = sh->next;
-  __syncthreads();
-  return old;
-}
-
-__device__ __forceinline__ void wg_broadcast_flag(ParamsRef p, int which) {
-  const int n = p.n_groups;
-  WgFlags* flags = p.wgflags;
-  for (int g = threadIdx.x; g < n; g += blockDim.x) st_relaxed(&flags[g].f[which], 1u);
-}
 
 // ------------------------------------------------- direct-to-LDS load helpers
 #define FMOE_G1 __attribute__((address_space(1)))
@@ -371,91 +265,6 @@ __device__ __noinline__ void tiled_router_task(ParamsRef pv, int blk) {
   }
 }
 
-
-// ----------------------------------------------------------------------- scan
-// Same tables as the streaming variant's scan, in two steps. Expert scan: one
-// wave per expert walks the expert's mask words 64 at a time and writes the
-// running count in front of every word (word_prefix) and the expert's total.
-// Final scan: one wave turns the totals into row offsets and the row-tile table
-// (an expert's rows in as few tiles of at most TM_MAX rows as possible, of equal size).
-constexpr int SCAN_EXPERTS = T_THREADS / 64;  // experts per expert-scan task
-
-__device__ __noinline__ void tiled_expert_scan_task(ParamsRef pv, int blk) {
-  ParamsRef p = uniform_params(pv);
-  const int E = uni(p.E), W = uni(p.W), T = uni(p.T);
-  const unsigned long long* masks = uni(p.masks);
-  int* word_prefix = uni(p.word_prefix);
-  int* expert_count = uni(p.expert_count);
-  const int lane = threadIdx.x & 63;
-  const int e = uni(blk) * SCAN_EXPERTS + uni(threadIdx.x >> 6);
-  if (e >= E) return;
-  const int wact = (T + 63) >> 6;
-  int base = 0;
-  for (int w0 = 0; w0 < wact; w0 += 64) {
-    const int w = w0 + lane;
-    const int c = w < wact ? __popcll(ldc(&masks[static_cast<size_t>(e) * W + w])) : 0;
-    const int incl = wave_inclusive_scan(c);
-    if (w < wact) stc(&word_prefix[static_cast<size_t>(e) * W + w], base + incl - c);
-    base += __shfl(incl, 63, 64);
-  }
-  if (lane == 0) stc(&expert_count[e], base);
-}
-
-__device__ __noinline__ void tiled_scan_task(ParamsRef pv) {
-  ParamsRef p = uniform_params(pv);
-  const RouteTables r = route_tables(p);
-  const int tid = threadIdx.x;
-  if (tid < 64) {
-    const int lane = tid;
-    const int epl = (r.E + 63) >> 6;
-    int base = 0, tile_base = 0;
-    for (int j = 0; j < epl; ++j) {
-      const int e = lane + 64 * j;
-      const int c = e < r.E ? ldc(&r.expert_count[e]) : 0;
-      const int incl = wave_inclusive_scan(c);
-      const int off = base + incl - c;
-      // balanced tiles of at most TM_MAX rows, whole 32-row blocks
-      const int nt = (c + TM_MAX - 1) / TM_MAX;
-      const int per = nt > 0 ? ((c + nt - 1) / nt + 31) / 32 * 32 : 0;
-      const int tincl = wave_inclusive_scan(nt);
-      const int toff = tile_base + tincl - nt;
-      if (e < r.E) {
-        stc(&r.expert_offset[e], off);
-        int done = 0;
-        for (int i = 0; i < nt; ++i) {
-          const int left = c - done;
-          const int tr = min(per, left);
-          if (toff + i < r.max_mtiles) {
-            stc16(&r.mtiles[toff + i],
-                  make_uint4(static_cast<unsigned>(e), static_cast<unsigned>(off + done),
-                             static_cast<unsigned>(tr), 0u));
-          }
-          done += tr;
-        }
-      }
-      base += __shfl(incl, 63, 64);
-      tile_base += __shfl(tincl, 63, 64);
-    }
-    if (lane == 0) {
-      stc(&r.expert_offset[r.E], base);
-      if (tile_base > r.max_mtiles) {
-        or_relaxed(&p.ctl->error.v, ERR_CAPACITY);
-        tile_base = 0;
-      }
-      stc(&p.ctl->n_mtiles.v, static_cast<unsigned>(tile_base));
-    }
-  }
-  fence_release();
-  __syncthreads();
-  wg_broadcast_flag(p, FLAG_SCAN);
-}
-
-__device__ void tiled_scatter_task(ParamsRef p, int blk) {
-  const RouteTables r = route_tables(p);
-  const int i0 = blk * RT_TOK * r.K;
-  const int n = min(RT_TOK * r.K, r.T * r.K - i0);
-  for (int i = threadIdx.x; i < n; i += T_THREADS) scatter_entry(r, i0 + i);
-}
 
 // -------------------------------------------------------------- the GEMM tile
 // Operands go HBM/L2 -> LDS directly (global_load_lds_dwordx4: lane l's 16 bytes
@@ -1447,11 +1256,6 @@ __device__ __noinline__ void tiled_combine_task(ParamsRef pv, int blk, int tok_i
 // steals from the next queue. Dependencies stay inside one queue and point to
 // smaller tickets, so whoever holds them is already running. Combine tasks
 // come from a last global counter once every queue is empty.
-__device__ __forceinline__ int xcc_id() {
-  // HW_REG_XCC_ID (20), bits 0..3
-  return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 7;
-}
-
 // The launch parameters are read in place and the task calls keep the local
 // calling convention, as in the streaming variant (see its worker loop).
 // ODD: I is an odd number of 32-k steps (a kernel of its own: as a branch of this one it cost every
@@ -1536,7 +1340,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
       ok = wg_wait_ge(p, &ctl->scan_done.v, n_es, &sh);
       if (ok) {
         if (p.trace) t_ready = wall_clock64();
-        tiled_scan_task(p);
+        tiled_scan_task<TM_MAX, 32>(p);
         trace(tk, 1, 0, t_fetch, t_ready);
       }
     } else {

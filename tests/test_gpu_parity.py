@@ -255,6 +255,62 @@ def check_tile_heights(rows, H, I):
         case.close()
 
 
+@pytest.mark.parametrize("rows,H,I", [
+    (1, 128, 128), (15, 128, 128), (16, 192, 160), (17, 320, 224), (33, 128, 288), (49, 448, 128), (64, 256, 352),
+    (65, 576, 672), (81, 64 * 9, 32 * 9), (96, 256, 256), (97, 320, 160), (193, 192, 224), (400, 512, 416),
+])
+def test_tiled_float32(rows, H, I):
+    """The float32 tiled kernel at the edges of its tiles (16 to 96 rows), column blocks (128 of I, 256 of
+    H) and k (even and odd numbers of 32-k steps): row-major weights against the oracle, and the packed
+    copy must give the same bits."""
+    cfg = synth.MoeConfig("tiled_f32", rows, H, 2, 2, I, "f32")
+    print("tiled float32", rows, H, I, flush=True)
+    case = GpuCase(cfg, seed=rows + I, sched=_lib.SCHED_TILED)
+    try:
+        assert case.launcher.sched_for(rows) == _lib.SCHED_TILED
+        out = case.run()
+        case.check_routing(case.inp["tokens"], case.launcher.routing(rows))
+        case.check_outputs(case.inp["tokens"], out, nthreads=4)
+        assert torch.equal(case.run(), out)
+        packed = GpuCase(cfg, seed=rows + I, sched=_lib.SCHED_TILED, inputs=case.inp, pack_weights=True)
+        try:
+            assert torch.equal(packed.run(), out)
+        finally:
+            packed.close()
+    finally:
+        case.close()
+
+
+def test_tiled_float32_values_without_bf16_parts():
+    """Infinities, NaN, values that round to infinity in bf16 and tiny ones among the expert weights: the
+    float32 tiled kernel gives what the streaming kernel's float32 instructions give, element by element:
+    the same infinities and NaN, and finite values within the tolerance of float32 layers."""
+    cfg = synth.MoeConfig("tiled_f32", 150, 256, 4, 2, 160, "f32")
+    dev = torch.device("cuda:0")
+    inp = synth.make_inputs_torch(cfg, 5, dev)
+    f1, f2 = inp["ffn1"], inp["ffn2"]
+    f1[0, 3, 7] = float("inf")
+    f1[0, cfg.I + 70, 250] = -float("inf")
+    f1[1, 5, 9] = float("nan")
+    f1[2, 11, 0] = 3.4e38
+    f1[2, cfg.I + 11, 1] = 1e-38
+    f2[2, 17, 3] = float("inf")
+    f2[3, 20:40] *= 1e-30
+    ref = GpuCase(cfg, seed=5, sched=_lib.SCHED_STREAM, inputs=inp)
+    case = GpuCase(cfg, seed=5, sched=_lib.SCHED_TILED, inputs=inp)
+    try:
+        want, got = ref.run(), case.run()
+        assert torch.isnan(want).any() and torch.isinf(want).any() and torch.isfinite(want).any()
+        assert torch.equal(torch.isnan(want), torch.isnan(got))
+        assert torch.equal(torch.isposinf(want), torch.isposinf(got)) and torch.equal(torch.isneginf(want), torch.isneginf(got))
+        fin = torch.isfinite(want)
+        rms = float(want[fin].double().pow(2).clamp(max=1e30).mean().sqrt())
+        assert float(((want - got).abs()[fin] - 2e-5 * want.abs()[fin]).max()) <= 2e-5 * rms
+    finally:
+        case.close()
+        ref.close()
+
+
 @pytest.mark.parametrize("E,k,last", [(128, 4, 256), (96, 4, 336), (64, 2, 512)])
 def test_auto_row_major_leaves_the_streaming_variant_with_the_split_k_kernel(E, k, last):
     """AUTO sends row-major bf16 batches of 14 to 24 rows an expert to the streaming variant for its
