@@ -335,6 +335,18 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
     p.split_down = d.intermediate >= 256 && std::min<long long>(slots, d.experts) * (d.hidden / 128) < p.n_groups ? 8 : 4;
   }
   const bool tiled = sched_for(d, T, m) == FLASH_MOE_SCHED_TILED;
+  // How the bf16 tiled kernel starts. 1: logit chains of 16 tokens x 32 experts a workgroup, in two rounds
+  // at most, and selections spread over all waves, while a wave has two of them at most (30B shape, us,
+  // without / with: T=450 300 / 282, T=600 302 / 285, T=900 312 / 299, T=1500 330 / 325, T=2048 353 / 356;
+  // E=256, H=1024, I=512, T=1024 242 / 231; E=16, k=2, H=320, I=160, T=4000 74 / 78). 2: router tasks of 16
+  // or 32 tokens x all experts. Both without a scan phase, while the mask words fit LDS (as 2 against 0:
+  // T=2048 345 / 340, row-major 359 / 355; E=16 T=4000 74 / 70). 0: tickets for all of it; so with a trace.
+  if (tiled && d.dtype == FLASH_MOE_BF16) {
+    p.dot16 = d.experts * ((T + 63) / 64) > fmoe::SHORT_MASK_WORDS || T > 65535 || m.traced ? 0
+              : T <= 6 * m.n_groups && ((T + 15) / 16) * ((d.experts + 31) / 32) <= 2 * m.n_groups ? 1
+                                                                                                  : 2;
+    p.early = p.dot16;  // (the last selection raises FLAG_ROUTED)
+  }
   if (tiled && d.dtype == FLASH_MOE_F32) {
     p.n_groups = std::min(2 * m.n_groups, kMaxGroups);  // two workgroups of four waves a CU
     p.n_workers = p.n_groups * 4;

@@ -26,6 +26,7 @@ constexpr int ROUTER_TOK = 8;    // streaming variant: tokens per router dot tas
 constexpr int ROUTER_EXP = 8;    // streaming variant: experts per router dot task
 constexpr int DOT16_KC = 256;    // streaming variant, matrix-core router: k per LDS stage
 constexpr int SCAN_LDS_WORDS = 1024;  // mask words (experts x 64-token words) the small-batch scan keeps in LDS
+constexpr int SHORT_MASK_WORDS = 8192;  // the same for the tiled kernel's short prologue
 constexpr int SPLIT_MAX_SLOTS = 2048;  // split-k kernel: (token, slot) entries its tables hold
 constexpr int EARLY_MAX_TOKENS = 384;  // batches up to this size may take their gate/up weights before the routing is known
 // Elements from one row of h to the next in the bf16 tiled variant: whole 128-byte lines.
@@ -127,7 +128,8 @@ struct Params {
   int split_spec;                  //    1: its workgroups ask for gate/up weights before the routing is known
   int split_down;                  //    waves that share a down task: 4 or 8
   int dot16;                       // 1 (streaming variant, bf16): the logit chains run on the matrix core, 16 tokens x
-                                   //    16 experts per workgroup, on the first workgroups before they take tickets
+                                   //    16 experts per workgroup, on the first workgroups before they take tickets;
+                                   //    bf16 tiled variant: how it starts (see the launcher)
   // What the last worker out needs when a launch has raised an error bit: it fills `out`
   // with NaN, returns the workspace's leading zero_words 32-bit words (counters, flags,
   // masks; `ctl` is the workspace's first byte) to zero, and adds the bits to *host_error

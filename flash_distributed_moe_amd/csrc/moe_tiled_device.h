@@ -124,6 +124,41 @@ __device__ __noinline__ void tiled_expert_scan_task(ParamsRef pv, int blk) {
   if (lane == 0) stc(&expert_count[e], base);
 }
 
+// Expert e's c rows, from permuted row `off` on, as balanced tiles of at most TM rows, whole blocks of
+// BLK rows. Called by a whole wave, lanes in expert order; returns the number of tiles so far.
+template <int TM, int BLK>
+__device__ __forceinline__ int scan_tiles(const RouteTables& r, int e, int c, int off, int tile_base) {
+  const int nt = (c + TM - 1) / TM;
+  const int per = nt > 0 ? ((c + nt - 1) / nt + BLK - 1) / BLK * BLK : 0;
+  const int tincl = wave_inclusive_scan(nt);
+  const int toff = tile_base + tincl - nt;
+  if (e < r.E) {
+    stc(&r.expert_offset[e], off);
+    int done = 0;
+    for (int i = 0; i < nt; ++i) {
+      const int tr = min(per, c - done);
+      if (toff + i < r.max_mtiles) {
+        stc16(&r.mtiles[toff + i],
+              make_uint4(static_cast<unsigned>(e), static_cast<unsigned>(off + done), static_cast<unsigned>(tr),
+                         nt > 1 ? 1u : 0u));
+      }
+      done += tr;
+    }
+  }
+  return tile_base + __shfl(tincl, 63, 64);
+}
+// the totals behind it: rows of all experts and tiles
+__device__ __forceinline__ void scan_totals(ParamsRef p, const RouteTables& r, int lane, int rows, int tiles) {
+  if (lane == 0) {
+    stc(&r.expert_offset[r.E], rows);
+    if (tiles > r.max_mtiles) {
+      or_relaxed(&p.ctl->error.v, ERR_CAPACITY);
+      tiles = 0;
+    }
+    stc(&p.ctl->n_mtiles.v, static_cast<unsigned>(tiles));
+  }
+}
+
 template <int TM, int BLK>
 __device__ __noinline__ void tiled_scan_task(ParamsRef pv) {
   ParamsRef p = uniform_params(pv);
@@ -137,37 +172,10 @@ __device__ __noinline__ void tiled_scan_task(ParamsRef pv) {
       const int e = lane + 64 * j;
       const int c = e < r.E ? ldc(&r.expert_count[e]) : 0;
       const int incl = wave_inclusive_scan(c);
-      const int off = base + incl - c;
-      // balanced tiles of at most TM rows, whole blocks of BLK rows
-      const int nt = (c + TM - 1) / TM;
-      const int per = nt > 0 ? ((c + nt - 1) / nt + BLK - 1) / BLK * BLK : 0;
-      const int tincl = wave_inclusive_scan(nt);
-      const int toff = tile_base + tincl - nt;
-      if (e < r.E) {
-        stc(&r.expert_offset[e], off);
-        int done = 0;
-        for (int i = 0; i < nt; ++i) {
-          const int left = c - done;
-          const int tr = min(per, left);
-          if (toff + i < r.max_mtiles) {
-            stc16(&r.mtiles[toff + i],
-                  make_uint4(static_cast<unsigned>(e), static_cast<unsigned>(off + done),
-                             static_cast<unsigned>(tr), nt > 1 ? 1u : 0u));
-          }
-          done += tr;
-        }
-      }
+      tile_base = scan_tiles<TM, BLK>(r, e, c, base + incl - c, tile_base);
       base += __shfl(incl, 63, 64);
-      tile_base += __shfl(tincl, 63, 64);
     }
-    if (lane == 0) {
-      stc(&r.expert_offset[r.E], base);
-      if (tile_base > r.max_mtiles) {
-        or_relaxed(&p.ctl->error.v, ERR_CAPACITY);
-        tile_base = 0;
-      }
-      stc(&p.ctl->n_mtiles.v, static_cast<unsigned>(tile_base));
-    }
+    scan_totals(p, r, lane, base, tile_base);
   }
   fence_release();
   __syncthreads();

@@ -30,6 +30,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "moe_stream_device.h"
 #include "moe_tiled_device.h"
 
 namespace fmoe {
@@ -71,6 +72,14 @@ __device__ __forceinline__ void load_to_lds(unsigned off, const unsigned char* b
                : "memory");
 }
 
+
+typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
+// 16 bytes of LDS at a byte address. The k-loops address LDS by number: the dynamic block's
+// base is looked up in memory wherever its name is used inside a function that is not inlined,
+// and a scalar load in the loop makes every LDS read in flight be waited for.
+__device__ __forceinline__ v4u_t lds_read16(unsigned addr) {
+  return *(const FMOE_L3 v4u_t*)addr;
+}
 
 // --------------------------------------------------------------------- router
 // Logits as in test/singleGPU/cpp/moe/reference/refGemm.h:21-24: one chain per
@@ -266,6 +275,254 @@ __device__ __noinline__ void tiled_router_task(ParamsRef pv, int blk) {
 }
 
 
+// ------------------------------------------------------------ the short router
+// The same chains where a batch has too few 16-token tasks for the CUs: 16 tokens x 32 experts a
+// workgroup, as the streaming kernel's router_dot16_task does it for 16 experts. Waves 0 and 1 only
+// multiply, one 16x16 chain each; waves 2 and 3 load 32 bytes of a row, widen them to float and leave
+// them in LDS in the order the instruction wants them (see router_dot16_task), two stages of 256 k, the
+// loads of four stages in flight. k past H counts as zero: a sum is never -0, so adding +0 leaves it.
+// Bound by the chains (512 dependent instructions of 32 cycles at H=2048). The logits go to memory
+// as candidate keys and any wave picks a token's winners once all its keys are in.
+constexpr int DOT32_AHEAD = 4;
+constexpr int DOT32_STAGE_BYTES = 3 * DOT16_OP_BYTES;  // experts 0..15, 16..31, tokens
+constexpr int DOT32_LDS_BYTES = 2 * DOT32_STAGE_BYTES;
+
+__device__ __noinline__ void router_dot32_task(ParamsRef pv, int tg_in, int eg_in) {
+  ParamsRef p = uniform_params(pv);
+  const int H = uni(p.H), E = uni(p.E), T = uni(p.T), tg = uni(tg_in), eg = uni(eg_in);
+  const int lane = lane_id();
+  const int wave = uni(static_cast<int>(threadIdx.x >> 6));
+  const int nc = (H + DOT16_KC - 1) / DOT16_KC;
+  const unsigned lds0 = uni(static_cast<unsigned>(reinterpret_cast<size_t>((FMOE_L3 unsigned char*)lds_raw)));
+  if (wave < 2) {
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    const unsigned wmine = lds0 + wave * DOT16_OP_BYTES + lane * 16, xmine = lds0 + 2 * DOT16_OP_BYTES + lane * 16;
+    v4u_t wc, xc, wn, xn;
+    lds_barrier();  // stage 0 is written
+    wc = lds_read16(wmine);
+    xc = lds_read16(xmine);
+    for (int c = 0; c < nc; ++c) {
+      const unsigned st = (c & 1) * DOT32_STAGE_BYTES, st_next = ((c + 1) & 1) * DOT32_STAGE_BYTES;
+#pragma unroll
+      for (int g = 0; g < DOT16_GROUPS; ++g) {
+        if (g + 1 < DOT16_GROUPS) {
+          wn = lds_read16(wmine + st + (g + 1) * 1024);
+          xn = lds_read16(xmine + st + (g + 1) * 1024);
+        } else {
+          // every read of this stage has returned: it may be refilled, and the next one is
+          // complete once the others have arrived too
+          lds_barrier();
+          if (c + 1 < nc) {
+            wn = lds_read16(wmine + st_next);
+            xn = lds_read16(xmine + st_next);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(wc[i]), __uint_as_float(xc[i]), acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        wc = wn;
+        xc = xn;
+      }
+    }
+    // acc[v] of lane l: expert 32*eg + 16*wave + 4*(l/16) + v, token 16*tg + l%16
+    const int t = tg * 16 + (lane & 15);
+    const int e0 = eg * 32 + wave * 16 + 4 * (lane >> 4);
+    if (eg * 32 + wave * 16 < E) {
+      if (t < T) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int e = e0 + v;
+          if (e < E) {
+            float x = acc[v];
+            if (p.bias != nullptr) x = __fadd_rn(x, as_global(p.bias)[e]);
+            stc(&p.cand[static_cast<size_t>(t) * E + e], make_key(x, e, true));
+          }
+        }
+      }
+      fence_release();
+      if (lane < 16 && t < T) add_relaxed(&p.tok_arrive[t], 1u);
+    }
+  } else {
+    // unit n of this lane: operand n / 2, (row, 16-k group) as in router_dot16_task: four lanes
+    // cover 128 contiguous bytes of a row
+    const int hl = (wave - 2) * 64 + lane;
+    const unsigned short* src[6];
+    unsigned dst[6];
+    int gk[2];
+#pragma unroll
+    for (int n = 0; n < 6; ++n) {
+      const int idx = hl + 128 * (n & 1);
+      const int row = (idx & 63) >> 2, g = (idx >> 6) * 4 + (idx & 3);
+      gk[n & 1] = g * 16;
+      const unsigned short* base =
+          n < 4 ? reinterpret_cast<const unsigned short*>(p.gate) + static_cast<size_t>(min(eg * 32 + 16 * (n >> 1) + row, E - 1)) * H
+                : reinterpret_cast<const unsigned short*>(p.tokens) + static_cast<size_t>(min(tg * 16 + row, T - 1)) * H;
+      src[n] = base;
+      dst[n] = lds0 + (n >> 1) * DOT16_OP_BYTES + g * 1024 + row * 16;
+    }
+    struct Regs {
+      uint4 a[6], b[6];
+    };
+    auto load = [&](Regs& r, int c) {  // past the last k: the row's first ones again, counted as zero
+#pragma unroll
+      for (int n = 0; n < 6; ++n) {
+        const int k = c * DOT16_KC + gk[n & 1];
+        const unsigned short* at = src[n] + (k < H ? k : 0);
+        r.a[n] = ld16(at);
+        r.b[n] = ld16(at + 8);
+      }
+    };
+    auto widen = [&](const Regs& r, int c) {
+#pragma unroll
+      for (int n = 0; n < 6; ++n) {
+        const unsigned keep = c * DOT16_KC + gk[n & 1] < H ? 0xFFFFFFFFu : 0u;
+        const unsigned hi = keep & 0xFFFF0000u;
+        const uint4 a = make_uint4(r.a[n].x & keep, r.a[n].y & keep, r.a[n].z & keep, r.a[n].w & keep);
+        const uint4 b = make_uint4(r.b[n].x & keep, r.b[n].y & keep, r.b[n].z & keep, r.b[n].w & keep);
+        const unsigned d = dst[n] + (c & 1) * DOT32_STAGE_BYTES;
+        auto put = [&](unsigned off, unsigned v0, unsigned v1, unsigned v2, unsigned v3) {
+          *(FMOE_L3 v4u_t*)(d + off) = v4u_t{v0, v1, v2, v3};
+        };
+        put(0, a.x << 16, a.z << 16, b.x << 16, b.z << 16);
+        put(256, a.x & hi, a.z & hi, b.x & hi, b.z & hi);
+        put(512, a.y << 16, a.w << 16, b.y << 16, b.w << 16);
+        put(768, a.y & hi, a.w & hi, b.y & hi, b.w & hi);
+      }
+    };
+    Regs r[DOT32_AHEAD];
+#pragma unroll
+    for (int i = 0; i < DOT32_AHEAD; ++i) load(r[i], i);
+    for (int c0 = 0; c0 < nc; c0 += DOT32_AHEAD) {
+#pragma unroll
+      for (int i = 0; i < DOT32_AHEAD; ++i) {
+        if (c0 + i < nc) {
+          widen(r[i], c0 + i);
+          load(r[i], c0 + i + DOT32_AHEAD);
+          lds_barrier();  // the stage is written; the multiplying waves are done with the one before
+        }
+      }
+    }
+    lds_barrier();  // the multiplying waves have read everything: the LDS is free again
+  }
+}
+
+// Winners of the tokens t, t + stride, ... of one wave, up to four at a time: their keys are asked
+// for together, and what was written is waited for once (one token after the other each costs
+// four trips to memory). Returns false if a wait failed.
+constexpr int SELECT_BATCH = 4;
+__device__ __noinline__ bool select_tokens_task(ParamsRef pv, int t_in, int stride_in) {
+  ParamsRef p = uniform_params(pv);
+  constexpr int MAXEPL = MAX_EXPERTS / 64;
+  const int T = uni(p.T), E = uni(p.E), stride = uni(stride_in), lane = lane_id();
+  const unsigned arrivals = static_cast<unsigned>((E + 15) >> 4);
+  double* lex = reinterpret_cast<double*>(lds_raw) + uni(static_cast<int>(threadIdx.x >> 6)) * MAX_TOPK;
+  unsigned done = 0;
+  for (int t0 = uni(t_in); t0 < T; t0 += SELECT_BATCH * stride) {
+    unsigned val[SELECT_BATCH][MAXEPL];
+#pragma unroll
+    for (int b = 0; b < SELECT_BATCH; ++b) {
+      const int t = t0 + b * stride;
+      if (t < T && !wave_wait_ge(&p.tok_arrive[t], arrivals, p.ctl, p.spin_limit)) return false;
+    }
+#pragma unroll
+    for (int b = 0; b < SELECT_BATCH; ++b) {
+      const int t = min(t0 + b * stride, T - 1);
+#pragma unroll
+      for (int j = 0; j < MAXEPL; ++j) {
+        const int e = lane + 64 * j;
+        // the ordered logit bits are the upper half of a candidate key
+        val[b][j] = e < E ? static_cast<unsigned>(ldc(&p.cand[static_cast<size_t>(t) * E + e]) >> 32) : 0u;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < SELECT_BATCH; ++b) {
+      const int t = t0 + b * stride;
+      if (t < T) {
+        if (lane == 0) stc(&p.tok_arrive[t], 0u);
+        router_select_max(p, t, val[b], lex);
+        ++done;
+      }
+    }
+  }
+  if (done != 0u) {
+    fence_release();
+    unsigned old = 0;
+    if (lane == 0) old = add_relaxed(&p.ctl->router_done.v, done);
+    if (uni(static_cast<int>(old)) + static_cast<int>(done) == T) broadcast_flag(p, FLAG_ROUTED);
+  }
+  return true;
+}
+
+// ------------------------------------------------------- the short scan and scatter
+// Where the mask words of the batch fit LDS, the workgroups that write a share of the permutation
+// (256 entries each) build the tables they need for it themselves; the first of them also writes
+// the row-tile table and what the host may read back.
+constexpr int SHORT_PRE_OFF = (SHORT_MASK_WORDS + MAX_EXPERTS) * 8;  // (rows of the mask table have an odd pitch)
+constexpr int SHORT_CNT_OFF = SHORT_PRE_OFF + (SHORT_MASK_WORDS + MAX_EXPERTS) * 2;
+constexpr int SHORT_OFF_OFF = SHORT_CNT_OFF + MAX_EXPERTS * 4;
+constexpr int SHORT_LDS_BYTES = SHORT_OFF_OFF + MAX_EXPERTS * 4;
+
+__device__ __noinline__ void short_scatter_task(ParamsRef pv, int blk_in) {
+  ParamsRef p = uniform_params(pv);
+  const RouteTables r = route_tables(p);
+  const int blk = uni(blk_in), tid = threadIdx.x, lane = tid & 63;
+  const int wact = (r.T + 63) >> 6, nw = r.E * wact, pitch = wact | 1;
+  unsigned long long* lmask = reinterpret_cast<unsigned long long*>(lds_raw);
+  unsigned short* lpre = reinterpret_cast<unsigned short*>(lds_raw + SHORT_PRE_OFF);  // rows of the expert before the word
+  int* lcnt = reinterpret_cast<int*>(lds_raw + SHORT_CNT_OFF);
+  int* loff = reinterpret_cast<int*>(lds_raw + SHORT_OFF_OFF);
+  const int i = blk * T_THREADS + tid;
+  const int e = i < r.T * r.K ? ldc(&r.topk_idx[i]) : -1;
+  for (int w0 = tid; w0 < nw; w0 += 4 * T_THREADS) {
+    unsigned long long m[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int w = min(w0 + q * T_THREADS, nw - 1);
+      m[q] = ldc(&r.masks[static_cast<size_t>(w / wact) * r.W + w % wact]);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (w0 + q * T_THREADS < nw) {
+        const int w = w0 + q * T_THREADS;
+        lmask[w / wact * pitch + w % wact] = m[q];
+      }
+  }
+  __syncthreads();
+  if (tid < r.E) {
+    int c = 0;
+#pragma unroll 4
+    for (int w = 0; w < wact; ++w) {
+      lpre[tid * pitch + w] = static_cast<unsigned short>(c);
+      c += __popcll(lmask[tid * pitch + w]);
+    }
+    lcnt[tid] = c;
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const int epl = (r.E + 63) >> 6;
+    int base = 0, tile_base = 0;
+    for (int j = 0; j < epl; ++j) {
+      const int x = lane + 64 * j;
+      const int c = x < r.E ? lcnt[x] : 0;
+      const int incl = wave_inclusive_scan(c);
+      const int off = base + incl - c;
+      if (x < r.E) loff[x] = off;
+      if (blk == 0) tile_base = scan_tiles<TM_MAX, 32>(r, x, c, off, tile_base);
+      base += __shfl(incl, 63, 64);
+    }
+    if (blk == 0) scan_totals(p, r, lane, base, tile_base);
+  }
+  __syncthreads();
+  if (blk == 0 && tid < r.E) stc(&r.expert_count[tid], lcnt[tid]);
+  if (e >= 0) {
+    const int t = i / r.K, wd = t >> 6;
+    const int w = e * pitch + wd;
+    stc(&r.perm[loff[e] + lpre[w] + __popcll(lmask[w] & ((1ull << (t & 63)) - 1ull))], i);
+  }
+}
+
 // -------------------------------------------------------------- the GEMM tile
 // Operands go HBM/L2 -> LDS directly (global_load_lds_dwordx4: lane l's 16 bytes
 // land at LDS base + 16*l, from any global address), in stages of 64 k: one
@@ -300,16 +557,8 @@ __device__ __noinline__ void tiled_router_task(ParamsRef pv, int blk) {
 // chose the vector-register form of the instruction, which cannot reach a[...]).
 // The first instruction of every accumulator takes the constant 0 as its
 // addend, so nothing zeroes them.
-typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
 constexpr int JB_MAX = 2 * JT_MAX;  // 16-row token blocks of the tallest tile
 constexpr int JB_ACC = 16;          // of these, the ones whose accumulators are in a[...]
-
-// 16 bytes of LDS at a byte address. The k-loops address LDS by number: the dynamic block's
-// base is looked up in memory wherever its name is used inside a function that is not inlined,
-// and a scalar load in the loop makes every LDS read in flight be waited for.
-__device__ __forceinline__ v4u_t lds_read16(unsigned addr) {
-  return *(const FMOE_L3 v4u_t*)addr;
-}
 
 template <bool INIT, bool IN_V>
 __device__ __forceinline__ void mma(const v4u_t& a, const v4u_t& b, f32x4& c) {
@@ -1088,7 +1337,7 @@ __device__ __noinline__ void tiled_odd_down_task(ParamsRef pv, const TileDesc& t
 }
 
 constexpr int TILED_LDS_BYTES = NOTE_OFF + NOTE_BYTES;
-static_assert(TILED_LDS_BYTES >= ROUTER_LDS_BYTES && TILED_LDS_BYTES + 256 <= 160 * 1024, "LDS of a workgroup");
+static_assert(TILED_LDS_BYTES >= DOT32_LDS_BYTES && TILED_LDS_BYTES >= SHORT_LDS_BYTES && TILED_LDS_BYTES >= ROUTER_LDS_BYTES && TILED_LDS_BYTES + 256 <= 160 * 1024, "LDS of a workgroup");
 
 // combine: out[t] = sum over slots, in slot order, of w[t,slot] * y[t*K+slot]
 // (refFullMoe.h:35,62-65): y holds each slot's down-projection row rounded to bf16; weight
@@ -1309,8 +1558,34 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
     }
   };
 
-  // ---- prologue: router, scan, scatter from the global counter
-  while (ok) {
+  // ---- prologue, few tokens: handed out statically (every workgroup of the launch is resident)
+  if (p.dot16) {
+    const int G = static_cast<int>(n_groups), b = static_cast<int>(blockIdx.x), wave = uni(static_cast<int>(threadIdx.x >> 6));
+    const int Ti = static_cast<int>(T), n_eg = (p.E + 31) >> 5, n_dot = ((Ti + 15) >> 4) * n_eg;
+    if (p.dot16 == 1) {
+      for (int i = b; i < n_dot; i += G) router_dot32_task(p, i / n_eg, i % n_eg);
+      const int sel_groups = min(n_dot, G);
+      // (a wait that fails has raised an error bit, which every later wait sees)
+      if (b < sel_groups) (void)select_tokens_task(p, b + sel_groups * wave, WAVES * sel_groups);
+    } else {
+      for (int i = b; i < static_cast<int>(n_rt); i += G) {
+        if (rt2) {
+          tiled_router_task<2>(p, i);
+        } else {
+          tiled_router_task<1>(p, i);
+        }
+        if (wg_arrive<false>(&ctl->router_done.v, &sh) == n_rt - 1u) wg_broadcast_flag(p, FLAG_ROUTED);
+      }
+    }
+    const int n_perm = (Ti * p.K + T_THREADS - 1) / T_THREADS;
+    if (b < n_perm) ok = wg_wait_flag(p, FLAG_ROUTED, &sh);
+    for (int i = b; ok && i < n_perm; i += G) {
+      short_scatter_task(p, i);
+      if (wg_arrive<false>(&ctl->perm_done.v, &sh) == static_cast<unsigned>(n_perm) - 1u) wg_broadcast_flag(p, FLAG_PERM);
+    }
+  }
+  // ---- prologue otherwise: router, scan, scatter from the global counter
+  while (ok && !p.dot16) {
     const long long t_fetch = p.trace ? wall_clock64() : 0;
     if (threadIdx.x == 0) sh.ticket = first ? blockIdx.x : n_groups + add_relaxed(&ctl->ticket.v, 1u);
     first = false;
@@ -1356,11 +1631,11 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
 
   // ---- GEMM tasks from the per-XCD queues
   unsigned nm = 0, n2_total = 0;
-  if (ok) ok = wg_wait_flag(p, FLAG_SCAN, &sh);
+  if (ok && !p.dot16) ok = wg_wait_flag(p, FLAG_SCAN, &sh);
+  if (ok) ok = wg_wait_flag(p, FLAG_PERM, &sh);
   if (ok) {
     nm = ldc(&ctl->n_mtiles.v);
     n2_total = nm * nt2;
-    ok = wg_wait_flag(p, FLAG_PERM, &sh);
   }
   for (int hop = 0; ok && hop < 8; ++hop) {
     const unsigned q = static_cast<unsigned>((home + hop) & 7);
@@ -1441,6 +1716,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
   }
 
   // The last workgroup out returns every counter to zero for the next launch.
+  fence_release();  // flags this wave has raised for others have landed before anybody clears them
   __syncthreads();
   if (threadIdx.x == 0) sh.ok = (add_relaxed(&ctl->exit_count.v, 1u) == n_groups - 1u) ? 1u : 0u;
   __syncthreads();
@@ -1456,6 +1732,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
       stc(&p.wgflags[g].f[FLAG_SCAN], 0u);
       stc(&p.wgflags[g].f[FLAG_PERM], 0u);
       stc(&p.wgflags[g].f[FLAG_G2], 0u);
+      stc(&p.wgflags[g].f[FLAG_ROUTED], 0u);
     }
     if (threadIdx.x < 8) stc(&ctl->xq[threadIdx.x].v, 0u);
     if (threadIdx.x == 0) {

@@ -83,3 +83,42 @@ def test_a_task_is_signalled_behind_a_full_wait_for_its_stores(gemm_task):
                 partial = ins
         else:
             raise AssertionError("no wait in front of instruction %d" % at)
+
+
+def _registers(text):
+    found = set()
+    for bank, lo, hi, bank1, one in re.findall(r"\b([va])\[(\d+):(\d+)\]|\b([va])(\d+)\b", text):
+        found |= {(bank, r) for r in range(int(lo), int(hi) + 1)} if bank else {(bank1, int(one))}
+    return found
+
+
+def test_accumulators_are_left_alone_until_they_are_written(functions):
+    """The tiled kernel's matrix instructions stand in assembly, so the compiler does not know that their
+    results take a while: wherever it copies an accumulator between registers (it may where two ways
+    through the code meet) it would read the old value. So nothing but matrix instructions may touch a
+    result for 16 wait states (a 16x16x32 product takes four passes of four cycles, and the wait the
+    hardware does not make by itself is less), along the straight line behind it."""
+    checked = 0
+    for name, code in functions.items():
+        if not re.search("tiled_gemm_task|tiled_odd_down_task", name):
+            continue
+        ins = [i for _, i, _ in code]
+        for at, op in enumerate(ins):
+            if not op.startswith("v_mfma"):
+                continue
+            checked += 1
+            result, waited = _registers(op.split(None, 1)[1].split(", ")[0]), 0
+            for later in ins[at + 1:at + 40]:
+                if waited >= 16 or later.startswith(("s_branch", "s_cbranch", "s_setpc")):
+                    break
+                if later.startswith("s_nop"):
+                    waited += int(later.split()[1]) + 1
+                elif later.startswith("v_mfma"):
+                    a, b = later.split(None, 1)[1].split(", ")[1:3]
+                    assert not result & (_registers(a) | _registers(b)), "%s: %s | %s" % (name, op, later)
+                    waited += 4
+                else:
+                    if later.startswith(("v_", "ds_", "global_", "buffer_", "scratch_")) and " " in later:
+                        assert not result & _registers(later.split(None, 1)[1]), "%s: %s | %s" % (name, op, later)
+                    waited += 1
+    assert checked > 10000

@@ -238,6 +238,31 @@ def test_tiled_ragged_columns(rows, H, I):
     check_tile_heights(rows, H, I)
 
 
+@pytest.mark.parametrize("T,H,E,k", [
+    (40, 128, 17, 3),       # a second group of experts with one expert; one token a wave at most
+    (1000, 192, 33, 2),     # a last 256-k stage that is partly empty
+    (1536, 320, 70, 8),     # the last size of the spread-out chains; two tokens a wave
+    (1537, 320, 70, 8),     # router tasks of all experts, no scan phase
+    (1000, 512, 256, 6),    # two rounds of 16-token x 32-expert tasks
+    (2048, 128, 256, 2),    # the last size whose mask words fit LDS
+    (2049, 128, 256, 2),    # the first whose do not
+])
+def test_tiled_starts(T, H, E, k):
+    """The ways the tiled kernel gets from tokens to row tiles, at the edges of their ranges: routing
+    tables bit for bit, outputs against the oracle, and the same from a second launch."""
+    cfg = synth.MoeConfig("starts", T, H, E, k, 128, "bf16", hot=3)
+    print("tiled starts", T, H, E, k, flush=True)
+    case = GpuCase(cfg, seed=T + E, sched=_lib.SCHED_TILED)
+    try:
+        assert case.launcher.sched_for(T) == _lib.SCHED_TILED
+        out = case.run()
+        case.check_routing(case.inp["tokens"], case.launcher.routing(T))
+        case.check_outputs(case.inp["tokens"], out, nthreads=4)
+        assert torch.equal(case.run(), out)
+    finally:
+        case.close()
+
+
 def check_tile_heights(rows, H, I):
     cfg = synth.MoeConfig("heights", rows, H, 2, 2, I, "bf16")
     print("tile heights", rows, H, I, flush=True)
