@@ -24,7 +24,7 @@
 namespace fmoe {
 hipError_t launch_stream_kernel(const Params& p, int dtype, int grid, hipStream_t stream);
 hipError_t prepare_stream_kernel();
-hipError_t launch_split_kernel(const Params& p, int grid, hipStream_t stream);
+hipError_t launch_split_kernel(const Params& p, int dtype, int grid, hipStream_t stream);
 hipError_t prepare_split_kernel();
 hipError_t split_kernel_occupancy(int* per_cu);
 hipError_t pack_weights(const void* src, void* dst, int dtype, int E, int H, int I, int which,
@@ -203,22 +203,34 @@ int dot16_tasks_of(const FlashMoeLayerDesc& d, int tokens_num) {
   return ((tokens_num + 15) / 16) * ((d.experts + 15) / 16);
 }
 
+// The others take 8 tokens x 8 experts per wave.
+int dot_tasks_of(const FlashMoeLayerDesc& d, int tokens_num) {
+  return ((tokens_num + fmoe::ROUTER_TOK - 1) / fmoe::ROUTER_TOK) * ((d.experts + fmoe::ROUTER_EXP - 1) / fmoe::ROUTER_EXP);
+}
+
 // Whether the streaming variant runs this batch on its split-k kernel, and on how many 16-row
-// blocks a tile: 0 (no), 1 or 2. bf16; the shapes of the matrix-core router, with at most half of the
+// blocks a tile: 0 (no), 1 or 2. For bf16 the shapes of the matrix-core router, with at most half of the
 // workgroups on it (the others have asked for weights by then); k of at least a step a wave in
 // either projection; tables that fit the kernel's LDS; 4 KiB of router weights (where the
-// loads go that nobody needs); h rows that 31 bits address; no trace. One block up to 9 rows an expert on
+// loads go that nobody needs); h rows that 31 bits address; no trace. float32: any H from 128 on (its logit
+// chains take 8 tokens x 8 experts a wave: four waves of half of the workgroups at most), one block, up to
+// where the tiled variant takes over (figures in the kernel's file). bf16: one block up to 9 rows an expert on
 // average, two up to 24 (us, streaming kernel / one / two blocks, 30B shape: T=96 235 / 221 / 222,
 // T=144 260 / 230 / 229, T=160 252 / 228 / 225, T=200 266 / 253 / 234, T=256 275 / 301 / 241; 235B
 // shape: T=128 808 / 791 / 791, T=160 816 / 805 / 799, T=200 855 / 904 / 812, T=256 876 / 1124 / 836;
 // four hot experts, 30B: T=160 345 / 253 / 243, T=256 458 / 279 / 270).
 int split_row_blocks(const FlashMoeLayerDesc& d, int tokens_num, const Machine& m) {
   const long long slots = static_cast<long long>(tokens_num) * d.top_k;
-  if (d.dtype != FLASH_MOE_BF16 || d.hidden % fmoe::DOT16_KC != 0 || d.intermediate < 128 ||
-      slots > fmoe::SPLIT_MAX_SLOTS || slots > 24ll * d.experts ||
+  if (d.intermediate < 128 || slots > fmoe::SPLIT_MAX_SLOTS ||
       d.experts * ((tokens_num + 63) / 64) > fmoe::SCAN_LDS_WORDS ||
-      static_cast<long long>(d.experts) * d.hidden < 2048 || slots * d.intermediate * 2 >= (1ll << 31) ||
-      dot16_tasks_of(d, tokens_num) > m.n_groups / 2 || m.traced)
+      static_cast<long long>(d.experts) * d.hidden < 2048 || slots * d.intermediate * 4 >= (1ll << 31) || m.traced)
+    return 0;
+  if (d.dtype == FLASH_MOE_F32)
+    return d.hidden >= 128 && slots < static_cast<long long>(kAutoTiledRowsF32) * d.experts &&
+                   dot_tasks_of(d, tokens_num) <= 4 * (m.n_groups / 2)
+               ? 1
+               : 0;
+  if (d.hidden % fmoe::DOT16_KC != 0 || slots > 24ll * d.experts || dot16_tasks_of(d, tokens_num) > m.n_groups / 2)
     return 0;
   return slots <= 9ll * d.experts ? 1 : 2;
 }
@@ -296,8 +308,7 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   // task must be among the tickets the workers start with: they go to the first
   // workgroups, four dot tasks and four select/scan tasks each (half of the
   // workgroups at most, to leave workers for the weights).
-  const int dot_tasks = ((T + fmoe::ROUTER_TOK - 1) / fmoe::ROUTER_TOK) *
-                        ((d.experts + fmoe::ROUTER_EXP - 1) / fmoe::ROUTER_EXP);
+  const int dot_tasks = dot_tasks_of(d, T);
   // bf16 layers run the logit chains on the matrix core, 16 tokens x 16 experts
   // per workgroup, while every such task finds a workgroup of its own
   const int dot16_tasks = dot16_tasks_of(d, T);
@@ -331,8 +342,13 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   if (p.split) {
     p.early = 1;
     p.split_spec = reaches_experts ? 1 : 0;
-    // a down task in four parts, two of them to a workgroup, unless that leaves CUs without one
-    p.split_down = d.intermediate >= 256 && std::min<long long>(slots, d.experts) * (d.hidden / 128) < p.n_groups ? 8 : 4;
+    // a down task in four parts, two of them to a workgroup, unless that leaves CUs without one or (float32) the
+    // number of 64-column tasks is odd
+    const bool eight_steps = d.intermediate >= (d.dtype == FLASH_MOE_BF16 ? 256 : 128);
+    p.split_down = d.hidden % 128 != 0 ||
+                           (eight_steps && std::min<long long>(slots, d.experts) * (d.hidden / 128) < p.n_groups)
+                       ? 8
+                       : 4;
   }
   const bool tiled = sched_for(d, T, m) == FLASH_MOE_SCHED_TILED;
   // How the bf16 tiled kernel starts. 1: logit chains of 16 tokens x 32 experts a workgroup, in two rounds
@@ -403,7 +419,7 @@ hipError_t launch_layer(const fmoe::Params& p, int dtype, int sched, hipStream_t
   if (sched == FLASH_MOE_SCHED_TILED)
     return dtype == FLASH_MOE_BF16 ? fmoe::launch_tiled_kernel(p, p.n_groups, stream)
                                    : fmoe::launch_tiled_f32_kernel(p, p.n_groups, stream);
-  return p.split ? fmoe::launch_split_kernel(p, p.n_groups, stream)
+  return p.split ? fmoe::launch_split_kernel(p, dtype, p.n_groups, stream)
                  : fmoe::launch_stream_kernel(p, dtype, p.n_groups, stream);
 }
 

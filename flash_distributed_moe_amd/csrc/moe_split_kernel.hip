@@ -1,5 +1,5 @@
 // Persistent MoE kernel, split-k variant for gfx950: batches of up to 24 rows an expert (bf16,
-// tiles of one or two 16-row blocks). A wave of the streaming
+// tiles of one or two 16-row blocks) or fewer than 10 (float32, one block). A wave of the streaming
 // variant carries a task of 64 weight rows over the whole of k alone: with few experts in use
 // most waves have no task at all and the others need 256 KiB each through one wave's window of
 // loads (one token on the 30B shape: 192 tasks on 2048 waves), and with many the launch ends in
@@ -21,6 +21,9 @@
 // T=200 266 -> 234, T=256 275 -> 241; row-major T=32 249 -> 226, T=128 290 -> 261; 235B T=1 102 -> 87,
 // T=64 759 -> 762, T=256 876 -> 836. Four hot experts: T=16 146 -> 120, T=128 317 -> 240 (a tile of more
 // rows than an early task carries starts over there; here it is several tiles).
+// float32, weights packed in place, streaming kernel -> here: E=8, H=256, I=128, k=2 T=16 44.8 -> 26.4; 30B
+// shape T=1 105.9 -> 67.3, T=4 133.8 -> 127.6, T=16 304 -> 289, T=64 397 -> 399, T=128 420 -> 412 (with four hot
+// experts 829 -> 454), T=159 543 -> 433; E=40, k=5, H=1344, I=736 T=1 91.6 -> 49.6, T=79 135 -> 113.
 //
 // Where the batch reaches most experts, the first workgroups (as many as whole experts fill; those
 // with a routing task behind it) ask for the first window of (expert b / nt1, columns b % nt1)
@@ -72,7 +75,7 @@ __device__ __forceinline__ SplitTile split_tile(const uint2* tiles, int i) {
 
 // The window: U k-steps of four 16-row weight blocks and RB blocks of token rows. PACKED weights
 // are one run of 4 KiB a step; row-major ones four row-order loads (see fragment_from_row_order).
-template <bool PACKED, bool DOWN, int RB>
+template <typename DT, bool PACKED, bool DOWN, int RB>
 struct SplitStream {
   static constexpr int NP = PACKED ? 1 : 4;
   static constexpr int U = split_u(RB);
@@ -123,7 +126,7 @@ struct SplitStream {
     for (int i = 0; i < 4; ++i) {
       const uint4 w = PACKED ? a[u][i] : fragment_from_row_order(a[u][i], pull_from);
 #pragma unroll
-      for (int r = 0; r < RB; ++r) acc[i][r] = mma16<BF16>(w, b[u][r], acc[i][r]);
+      for (int r = 0; r < RB; ++r) acc[i][r] = mma16<DT>(w, b[u][r], acc[i][r]);
     }
   }
   // this wave's partial sums of a task go to LDS, and the accumulators back to zero
@@ -138,7 +141,7 @@ struct SplitStream {
   }
 };
 
-template <bool PACKED, int RB>
+template <typename DT, bool PACKED, int RB>
 __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_split_kernel(const Params params) {
   ParamsRef p = kernel_params();
   __shared__ unsigned lds_flag[4];
@@ -156,6 +159,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   const int T = p.T, E = p.E, H = p.H, K = p.K, I = p.I, W = p.W;
   unsigned char* lds = reinterpret_cast<unsigned char*>(lds_dyn);
   constexpr int U = split_u(RB), TILE_ROWS = 16 * RB;
+  constexpr int ESZ = 16 / DT::EPV;
   unsigned short* lperm = reinterpret_cast<unsigned short*>(lds + SPLIT_PERM_OFF);  // permuted row -> token*K + slot
   unsigned short* ltok = reinterpret_cast<unsigned short*>(lds + SPLIT_TOK_OFF);    // permuted row -> token
   float* lw = reinterpret_cast<float*>(lds + SPLIT_W_OFF);      // permuted row -> gate weight
@@ -165,16 +169,23 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   int* spec_tile = reinterpret_cast<int*>(lds + SPLIT_SPEC_OFF);  // expert -> its early tile, or -1
   int* note = reinterpret_cast<int*>(lds + SPLIT_NOTE_OFF);
 
-  const int n_eg = (E + 15) >> 4;
-  const int n_dot = ((T + 15) >> 4) * n_eg;
+  // logit chains: bf16 16 tokens x 16 experts a workgroup, float32 8 x 8 a wave
+  constexpr int DOT = DT::EPV == 8 ? 16 : ROUTER_EXP;
+  const int n_eg = (E + DOT - 1) / DOT;
+  const int n_dot = ((T + DOT - 1) / DOT) * n_eg;
+  const int n_rt = DT::EPV == 8 ? n_dot : min(n_dot, G >> 1);  // workgroups with routing tasks
   const int nt1 = I / (16 * G1_NB), nt2 = H / (16 * G2_NB);
-  const int ks1 = H >> 5, ks2 = I >> 5;
+  const int ks1 = H / (4 * DT::EPV), ks2 = I / (4 * DT::EPV);  // steps of 64 bytes a row
   const int pull_from = (((lane & 15) << 2) | (lane >> 4)) << 2;
 
   // ---- routing: logit chains on the first workgroups, then one select a wave there
-  if (b < n_dot) {
-    router_dot16_task(p, b / n_eg, b % n_eg);
-    for (int t = b + n_dot * wave; t < T; t += 8 * n_dot) {
+  if (b < n_rt) {
+    if constexpr (DT::EPV == 8) {
+      router_dot16_task(p, b / n_eg, b % n_eg);
+    } else {
+      for (int q = b + n_rt * wave; q < n_dot; q += 8 * n_rt) router_dot_task<DT>(p, q / n_eg, q % n_eg);
+    }
+    for (int t = b + n_rt * wave; t < T; t += 8 * n_rt) {
       if (!wave_wait_ge(&p.tok_arrive[t], static_cast<unsigned>(n_eg), ctl, p.spin_limit)) break;
       router_select_task(p, t);
     }
@@ -193,7 +204,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   int ntiles = 0;
   int cnt = 0;  // tasks this workgroup has finished: its parity names the set of partial sums
   {
-    SplitStream<PACKED, false, RB> st;
+    SplitStream<DT, PACKED, false, RB> st;
     st.cb = coherent_buffer(p.h, 0u);
     auto weights = [&](int expert, int nblk) {
       if constexpr (PACKED) {
@@ -202,12 +213,12 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
         st.astep = 4096;
       } else {
         const unsigned char* w13 = reinterpret_cast<const unsigned char*>(p.ffn1) +
-                                   static_cast<size_t>(expert) * 2 * I * H * 2 + k0 * 64 + row_order_chunk() * 16;
+                                   static_cast<size_t>(expert) * 2 * I * H * ESZ + k0 * 64 + row_order_chunk() * 16;
         const int n0 = nblk * (16 * G1_NB) + row_order_row();
 #pragma unroll
         for (int q = 0; q < G1_NB; ++q) {
-          st.ap[q] = w13 + static_cast<size_t>(n0 + 16 * q) * H * 2;
-          st.ap[G1_NB + q] = w13 + static_cast<size_t>(I + n0 + 16 * q) * H * 2;
+          st.ap[q] = w13 + static_cast<size_t>(n0 + 16 * q) * H * ESZ;
+          st.ap[G1_NB + q] = w13 + static_cast<size_t>(I + n0 + 16 * q) * H * ESZ;
         }
         st.astep = 64;
       }
@@ -325,7 +336,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
 #pragma unroll
       for (int r = 0; r < RB; ++r)
         st.bp[r] = reinterpret_cast<const unsigned char*>(p.tokens) +
-                   (static_cast<size_t>(ltok[t.row0 + min(16 * r + r16, t.rows - 1)]) * H + k0 * 32 + g * 8) * 2;
+                   static_cast<size_t>(ltok[t.row0 + min(16 * r + r16, t.rows - 1)]) * H * ESZ + k0 * 64 + g * 16;
       st.bstep = 64;
     };
     auto next_task = [&]() {
@@ -362,13 +373,18 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
           unsigned hv[4];
 #pragma unroll
           for (int k = 0; k < 4; ++k) {  // (one after the other, for the same reason)
-            hv[k] = f2bf(silu_mul(s[k], v[k]));
+            const float x = silu_mul(s[k], v[k]);
+            hv[k] = DT::EPV == 8 ? f2bf(x) : __float_as_uint(x);
             __builtin_amdgcn_sched_barrier(0);
           }
-          const unsigned lo = hv[0] | (hv[1] << 16), hi = hv[2] | (hv[3] << 16);
-          stc(reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned short*>(p.h) +
-                                                    static_cast<size_t>(t.row0 + row) * I + n0 + 16 * i + 4 * g),
-              static_cast<unsigned long long>(lo) | (static_cast<unsigned long long>(hi) << 32));
+          const size_t at = static_cast<size_t>(t.row0 + row) * I + n0 + 16 * i + 4 * g;
+          if constexpr (DT::EPV == 8) {
+            const unsigned lo = hv[0] | (hv[1] << 16), hi = hv[2] | (hv[3] << 16);
+            stc(reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned short*>(p.h) + at),
+                static_cast<unsigned long long>(lo) | (static_cast<unsigned long long>(hi) << 32));
+          } else {
+            st16_through(reinterpret_cast<float*>(p.h) + at, make_uint4(hv[0], hv[1], hv[2], hv[3]));
+          }
         }
       }
     };
@@ -442,8 +458,8 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     const int n_tasks = ntiles * per_tile;
     int ntask = b < n_tasks ? (n_tasks - b + G - 1) / G : 0;
     if (ntask > 0) {
-      SplitStream<PACKED, true, RB> st;
-      st.cb = coherent_buffer(p.h, static_cast<unsigned>(T * K * I * 2));
+      SplitStream<DT, PACKED, true, RB> st;
+      st.cb = coherent_buffer(p.h, static_cast<unsigned>(T * K * I * ESZ));
       int lq = b, cq = b;
       auto next_task = [&]() {
         if (lq < n_tasks) {
@@ -455,15 +471,15 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
             st.astep = 4096;
           } else {
             const unsigned char* w2 = reinterpret_cast<const unsigned char*>(p.ffn2) +
-                                      static_cast<size_t>(t.expert) * H * I * 2 + d0 * 64 + row_order_chunk() * 16;
+                                      static_cast<size_t>(t.expert) * H * I * ESZ + d0 * 64 + row_order_chunk() * 16;
             const int n0 = nblk * (16 * G2_NB) + row_order_row();
 #pragma unroll
-            for (int q = 0; q < st.NP; ++q) st.ap[q] = w2 + static_cast<size_t>(n0 + 16 * q) * I * 2;
+            for (int q = 0; q < st.NP; ++q) st.ap[q] = w2 + static_cast<size_t>(n0 + 16 * q) * I * ESZ;
             st.astep = 64;
           }
 #pragma unroll
           for (int r = 0; r < RB; ++r)
-            st.boff[r] = static_cast<unsigned>(((t.row0 + min(16 * r + r16, t.rows - 1)) * I + d0 * 32 + g * 8) * 2);
+            st.boff[r] = static_cast<unsigned>((t.row0 + min(16 * r + r16, t.rows - 1)) * I * ESZ + d0 * 64 + g * 16);
           st.bstep = 64;
           st.left = steps2;
           lq += G;
@@ -567,7 +583,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     const unsigned nc = static_cast<unsigned>(T) * ncomb;
     const unsigned slot = static_cast<unsigned>(wave * G + b);
     if (slot < nc && wait_flag(p, FLAG_G2, lds_flag, lds_poller))
-      combine_items<BF16>(p, slot, nc, ncomb, static_cast<unsigned>(b * 8 + wave), 0u, 0);
+      combine_items<DT>(p, slot, nc, ncomb, static_cast<unsigned>(b * 8 + wave), 0u, 0);
   }
 
   // ---- the last workgroup out returns every counter to zero for the next launch
@@ -596,20 +612,24 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
 }
 
 namespace {
-// The four kernels, and the dynamic LDS each is launched with.
+// The kernels, and the dynamic LDS each is launched with.
 struct SplitUse {
   const void* kernel;
   int lds;
 };
-const SplitUse kSplitUses[] = {{reinterpret_cast<const void*>(moe_split_kernel<true, 1>), split_lds_bytes(1)},
-                               {reinterpret_cast<const void*>(moe_split_kernel<false, 1>), split_lds_bytes(1)},
-                               {reinterpret_cast<const void*>(moe_split_kernel<true, 2>), split_lds_bytes(2)},
-                               {reinterpret_cast<const void*>(moe_split_kernel<false, 2>), split_lds_bytes(2)}};
+const SplitUse kSplitUses[] = {{reinterpret_cast<const void*>(moe_split_kernel<BF16, true, 1>), split_lds_bytes(1)},
+                               {reinterpret_cast<const void*>(moe_split_kernel<BF16, false, 1>), split_lds_bytes(1)},
+                               {reinterpret_cast<const void*>(moe_split_kernel<BF16, true, 2>), split_lds_bytes(2)},
+                               {reinterpret_cast<const void*>(moe_split_kernel<BF16, false, 2>), split_lds_bytes(2)},
+                               {reinterpret_cast<const void*>(moe_split_kernel<F32, true, 1>), split_lds_bytes(1)},
+                               {reinterpret_cast<const void*>(moe_split_kernel<F32, false, 1>), split_lds_bytes(1)}};
 }  // namespace
 
-hipError_t launch_split_kernel(const Params& p, int grid, hipStream_t stream) {
-  auto* kernel = p.split == 1 ? (p.ffn1_packed != nullptr ? moe_split_kernel<true, 1> : moe_split_kernel<false, 1>)
-                              : (p.ffn1_packed != nullptr ? moe_split_kernel<true, 2> : moe_split_kernel<false, 2>);
+hipError_t launch_split_kernel(const Params& p, int dtype, int grid, hipStream_t stream) {
+  const bool packed = p.ffn1_packed != nullptr;
+  auto* kernel = dtype == DT_F32 ? (packed ? moe_split_kernel<F32, true, 1> : moe_split_kernel<F32, false, 1>)
+                 : p.split == 1  ? (packed ? moe_split_kernel<BF16, true, 1> : moe_split_kernel<BF16, false, 1>)
+                                 : (packed ? moe_split_kernel<BF16, true, 2> : moe_split_kernel<BF16, false, 2>);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), split_lds_bytes(p.split), stream, p);
   return hipGetLastError();
 }

@@ -50,8 +50,8 @@ enum { FLASH_MOE_SCHED_AUTO = 0, FLASH_MOE_SCHED_STREAM = 1, FLASH_MOE_SCHED_TIL
  *      row-major expert weights into a packed second copy in its workspace
  *      (+3*E*H*I elements of device memory). The caller's tensors stay the external
  *      format and must stay valid: a launch reads whichever form is faster for its
- *      batch (bf16: always the copy; float32: the caller's tensors from 16 rows an
- *      expert on). After changing them call flashMoeRefreshWeights.
+ *      batch (the copy, but for float32 batches of 16 rows an expert and more that run
+ *      the streaming variant). After changing them call flashMoeRefreshWeights.
  *  FLASH_MOE_FLAG_WEIGHTS_PREPACKED ffn1_weights / ffn2_weights already hold the
  *      packed layout (made by flashMoePackWeights into buffers of the caller's, or
  *      by flashMoePackWeightsInPlace): no second copy anywhere; the row-major form

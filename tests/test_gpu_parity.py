@@ -454,13 +454,33 @@ def test_prepacked_weights_equal_unpacked(name, T, sched):
     (0, (98, 256, 8, 2, 256)),           # 24.5 rows an expert
 ])
 def test_split_k_small_batches(blocks, shape):
-    """Small bf16 batches (at most 24 rows an expert): the split-k kernel at the edges of its k
+    _check_split_k(blocks, shape, "bf16")
+
+
+@pytest.mark.parametrize("blocks,shape", [
+    (1, (1, 128, 16, 2, 128)),           # one k-step a wave in either projection; 64-column tasks in pairs, one pair
+    (1, (3, 192, 16, 2, 160)),           # an odd number of 64-column tasks: eight parts of a down task; odd k-steps
+    (1, (16, 256, 8, 2, 128)),           # tiny: most workgroups without a task
+    (1, (1, 2048, 16, 8, 768)),          # one token, full windows
+    (1, (33, 1344, 40, 5, 736)),         # 21 column blocks of 64; 84 and 46 k-steps over the eight waves
+    (1, (77, 320, 16, 2, 160)),          # 9.6 rows an expert, ragged last chunk of the chains
+    (1, (64, 2048, 64, 8, 416, 4)),      # four experts with 64 rows: several tiles each
+    (1, (127, 256, 256, 9, 128, 3)),     # 512 chain tasks: four waves of each routing workgroup; two mask words
+    (0, (129, 256, 256, 9, 128)),        # 544 of them: the streaming kernel
+    (0, (36, 256, 4, 1, 128)),           # too few router weights for the loads nobody needs
+])
+def test_split_k_small_batches_float32(blocks, shape):
+    _check_split_k(blocks, shape, "f32")
+
+
+def _check_split_k(blocks, shape, dtype):
+    """Small batches (bf16: at most 24 rows an expert, float32: fewer than 10): the split-k kernel at the edges of its k
     parts, tiles and tables, on row-major weights against the oracle; the packed copy gives the same
     bits, and so does a second launch (every counter is back at zero). `blocks`: the 16-row blocks
     of its tiles, 0 just outside its range (another kernel runs, the packed copy's may differ)."""
     T, H, E, k, I = shape[:5]
-    cfg = synth.MoeConfig("split", T, H, E, k, I, "bf16", hot=shape[5] if len(shape) > 5 else 0)
-    print("split-k", shape, flush=True)
+    cfg = synth.MoeConfig("split", T, H, E, k, I, dtype, hot=shape[5] if len(shape) > 5 else 0)
+    print("split-k", dtype, shape, flush=True)
     case = GpuCase(cfg, seed=T + E)
     try:
         assert case.launcher.split_blocks_for(T) == blocks
