@@ -22,8 +22,8 @@
 // T=64 759 -> 762, T=256 876 -> 836. Four hot experts: T=16 146 -> 120, T=128 317 -> 240 (a tile of more
 // rows than an early task carries starts over there; here it is several tiles).
 // float32, weights packed in place, streaming kernel -> here: E=8, H=256, I=128, k=2 T=16 44.8 -> 26.4; 30B
-// shape T=1 105.9 -> 67.3, T=4 133.8 -> 127.6, T=16 304 -> 289, T=64 397 -> 399, T=128 420 -> 412 (with four hot
-// experts 829 -> 454), T=159 543 -> 433; E=40, k=5, H=1344, I=736 T=1 91.6 -> 49.6, T=79 135 -> 113.
+// shape T=1 105.9 -> 67.8, T=4 133.8 -> 127.7, T=16 302 -> 286, T=64 397 -> 397, T=128 420 -> 408 (with four hot
+// experts 837 -> 449), T=159 543 -> 433; E=40, k=5, H=1344, I=736 T=1 91.6 -> 49.9, T=79 135 -> 113.
 //
 // Where the batch reaches most experts, the first workgroups (as many as whole experts fill; those
 // with a routing task behind it) ask for the first window of (expert b / nt1, columns b % nt1)
@@ -59,6 +59,51 @@ constexpr int split_lds_bytes(int rb) {
 }
 static_assert(split_lds_bytes(2) + 64 <= 160 * 1024, "LDS of a workgroup");
 
+// Which steps of a task's k a wave takes. `runs` false (batches that leave most experts unused: a CU has
+// a task at most): one of `parts` equal stretches. Otherwise every parts-th run of four steps (256 bytes of a
+// row; of two or one where the steps do not divide into such runs), from one of up to four places
+// that moves with the task's column block and once around: the eight waves then read a stretch of
+// 32 KiB (packed) or 2 KiB of each row, and the CUs do not all read at the same offset of their rows, which for
+// pitches of 4 KiB and more are the same channels. us, equal stretches / as here, packed: bf16 30B shape T=64
+// 209.9 / 207.0, 235B T=64 742 / 733, T=200 797 / 788, float32 30B T=128 412 / 408; row-major: bf16 30B
+// T=64 241.6 / 238.4, T=200 273.6 / 268.5, 235B T=64 888 / 860, T=200 1009 / 970, float32 30B T=64 499 / 474,
+// T=128 521 / 498; E=60, k=4, H=2304, I=1408 T=100 (no two steps divide) packed 210 / 211.5, row-major
+// 262 / 252. Without the moving start, bf16 row-major 235B T=64 933, float32 30B T=128 576; runs of two with
+// it 900 and 537, of eight 880 and 501; starts next to each other instead of far apart, float32 row-major
+// H=4096, I=512 T=100 389 instead of 373.
+struct SplitSteps {
+  int first, count;       // first step, number of steps
+  int jump;               // from the last step of a run to the wave's next
+  int shift, mask;        // steps of a run: 1 << shift, less one
+  int starts, apart;      // places where it may start, less one: 0, 1 or 3; runs from one to the next
+  __device__ __forceinline__ int start(int column) const { return ((column & starts) * apart) << shift; }
+  __device__ __forceinline__ int at(int start) const { return first + (start >> shift) * (jump + mask); }
+  __device__ __forceinline__ int span() const { return (count >> shift) * (jump + mask); }
+};
+__device__ __forceinline__ SplitSteps split_steps(int steps, int part, int log_parts, bool runs) {
+  SplitSteps s;
+  const int parts = 1 << log_parts;
+  s.shift = 0;
+  if (runs) {
+    s.shift = max(0, min(2, __builtin_ctz(steps) - log_parts));
+    const int n = steps >> (s.shift + log_parts);  // runs that every wave has
+    s.starts = n >= 4 ? 3 : n >= 2 ? 1 : 0;
+    s.apart = n >= 4 ? n >> 2 : 1;
+    s.first = part << s.shift;
+    s.count = (((steps >> s.shift) - part + parts - 1) >> log_parts) << s.shift;
+    s.jump = ((parts - 1) << s.shift) + 1;
+    s.mask = (1 << s.shift) - 1;
+  } else {
+    s.first = (steps * part) >> log_parts;
+    s.count = ((steps * (part + 1)) >> log_parts) - s.first;
+    s.jump = 1;
+    s.apart = 1;
+    s.mask = 0;
+    s.starts = 0;
+  }
+  return s;
+}
+
 // A tile as the tables hold it: at most 16 * RB rows of one expert.
 struct SplitTile {
   int expert, row0, rows;
@@ -83,7 +128,11 @@ struct SplitStream {
   const unsigned char* ap[NP];   // where the next step's weights are
   const unsigned char* bp[RB];   // ... and its token rows (gate/up)
   unsigned boff[RB];             // ... or h rows, as offsets (down)
-  int astep, bstep, left;        // bytes to the next step (0 behind the last task); steps left of the task
+  int astep, bstep;              // bytes to the next step (0 behind the last task) ...
+  int ajump, bjump, mask;        // ... from the last step of a run on; steps of a run - 1
+  int aspan, bspan;              // from the task's first step to behind its last
+  int left;                      // steps left of the task
+  int turn;                      // ... when the pointers go back to its first step (0: they do not any more)
   CoherentBuffer cb;
 
   // Packed weights pass through the caches without staying, also where an expert has several tiles
@@ -94,17 +143,18 @@ struct SplitStream {
 #pragma unroll
     for (int i = 0; i < 4; ++i) a[u][i] = PACKED ? ld16_once(ap[0] + i * 1024) : ld16(ap[i]);
 #pragma unroll
-    for (int q = 0; q < NP; ++q) ap[q] += astep;
+    for (int q = 0; q < NP; ++q) ap[q] += ((left - 1) & mask) == 0 ? ajump : astep;
   }
   __device__ __forceinline__ void load_b(int u) {
+    const int step = ((left - 1) & mask) == 0 ? bjump : bstep;
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       if (DOWN) {
         b[u][r] = ld16_agent(cb, boff[r]);
-        boff[r] += static_cast<unsigned>(bstep);
+        boff[r] += static_cast<unsigned>(step);
       } else {
         b[u][r] = ld16(bp[r]);
-        bp[r] += bstep;
+        bp[r] += step;
       }
     }
   }
@@ -118,8 +168,27 @@ struct SplitStream {
       bp[r] = reinterpret_cast<const unsigned char*>(somewhere);
       boff[r] = 0u;
     }
-    astep = bstep = 0;
+    astep = bstep = ajump = bjump = mask = 0;
     left = 0x7FFFFFFF;
+    turn = 0;
+  }
+  // A step's loads (of A: weights, of B: token rows) are out: on to the next one, or to the next task.
+  template <bool A, bool B, typename NextTask>
+  __device__ __forceinline__ void advance(NextTask next_task) {
+    if (--left != turn) return;
+    if (left == 0) {
+      next_task();
+      return;
+    }
+    turn = 0;
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+      if (A) ap[q] -= aspan;
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      if (B && DOWN) boff[r] -= static_cast<unsigned>(bspan);
+      if (B && !DOWN) bp[r] -= bspan;
+    }
   }
   __device__ __forceinline__ void mma(int u, int pull_from, f32x4 (&acc)[4][RB]) {
 #pragma unroll
@@ -194,7 +263,8 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   // ---- gate/up weights before the routing is known
   const int n_spec_experts = p.split_spec ? min(G / nt1, E) : 0;
   const int n_spec = n_spec_experts * nt1;  // workgroups b < n_spec
-  const int k0 = ks1 * wave / 8, steps1 = ks1 * (wave + 1) / 8 - k0;
+  const SplitSteps sk1 = split_steps(ks1, wave, 3, p.split_spec != 0);
+  const int steps1 = sk1.count;
   f32x4 acc[4][RB];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -207,10 +277,13 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     SplitStream<DT, PACKED, false, RB> st;
     st.cb = coherent_buffer(p.h, 0u);
     auto weights = [&](int expert, int nblk) {
+      const int start = sk1.start(nblk), k0 = sk1.at(start);
       if constexpr (PACKED) {
         const size_t task = static_cast<size_t>(expert) * nt1 + nblk;
         st.ap[0] = reinterpret_cast<const unsigned char*>(p.ffn1_packed) + (task * ks1 + k0) * 4096 + lane * 16;
         st.astep = 4096;
+        st.ajump = 4096 * sk1.jump;
+        st.aspan = 4096 * sk1.span();
       } else {
         const unsigned char* w13 = reinterpret_cast<const unsigned char*>(p.ffn1) +
                                    static_cast<size_t>(expert) * 2 * I * H * ESZ + k0 * 64 + row_order_chunk() * 16;
@@ -221,8 +294,12 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
           st.ap[G1_NB + q] = w13 + static_cast<size_t>(I + n0 + 16 * q) * H * ESZ;
         }
         st.astep = 64;
+        st.ajump = 64 * sk1.jump;
+        st.aspan = 64 * sk1.span();
       }
       st.left = steps1;
+      st.turn = start;
+      st.mask = sk1.mask;
     };
     if (b < n_spec) {
       weights(b / nt1, b % nt1);
@@ -233,7 +310,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     for (int u = 0; u < U; ++u) {
       st.load_a(u);
       // (a task shorter than the window: the slots behind it are filled again below)
-      if (u + 1 == steps1) st.park(p.gate);
+      st.template advance<true, false>([&] { st.park(p.gate); });
       __builtin_amdgcn_sched_barrier(0);
     }
 
@@ -332,18 +409,21 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     int lq = rank;  // next task of the rest to load, and (cq) to finish
     int cq = rank;
     bool cspec = my_spec >= 0;
-    auto rows_of = [&](const SplitTile& t) {
+    auto rows_of = [&](const SplitTile& t, int nblk) {
+      const int k0 = sk1.at(sk1.start(nblk));
 #pragma unroll
       for (int r = 0; r < RB; ++r)
         st.bp[r] = reinterpret_cast<const unsigned char*>(p.tokens) +
                    static_cast<size_t>(ltok[t.row0 + min(16 * r + r16, t.rows - 1)]) * H * ESZ + k0 * 64 + g * 16;
       st.bstep = 64;
+      st.bjump = 64 * sk1.jump;
+      st.bspan = 64 * sk1.span();
     };
     auto next_task = [&]() {
       if (lq < n_tasks) {
         const SplitTile t = split_tile(tiles, lq / nt1);
         weights(t.expert, lq % nt1);
-        rows_of(t);
+        rows_of(t, lq % nt1);
         lq += G;
       } else {
         st.park(p.gate);
@@ -391,19 +471,19 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     if (ntask > 0) {
       if (my_spec >= 0 && steps1 >= U) {
         // the window is this task's: its token rows join it
-        rows_of(split_tile(tiles, my_spec));
-        if (steps1 == U) {
-          st.left = 0;
-        } else {
-          st.left = steps1 - U;
-        }
+        rows_of(split_tile(tiles, my_spec), b % nt1);
+        st.left = steps1;
+        st.turn = sk1.start(b % nt1);
+        st.mask = sk1.mask;
 #pragma unroll
-        for (int u = 0; u < U; ++u) st.load_b(u);
-        if (st.left == 0) next_task();
+        for (int u = 0; u < U; ++u) {
+          st.load_b(u);
+          st.template advance<false, true>(next_task);
+        }
       } else {
         if (my_spec >= 0) {
           weights(b / nt1, b % nt1);
-          rows_of(split_tile(tiles, my_spec));
+          rows_of(split_tile(tiles, my_spec), b % nt1);
         } else {
           next_task();
         }
@@ -411,7 +491,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
         for (int u = 0; u < U; ++u) {
           st.load_a(u);
           st.load_b(u);
-          if (--st.left == 0) next_task();
+          st.template advance<true, true>(next_task);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -424,7 +504,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
           st.load_a(u);
           st.load_b(u);
           __builtin_amdgcn_sched_barrier(0);
-          if (--st.left == 0) next_task();
+          st.template advance<true, true>(next_task);
           if (--cleft == 0) {
             finish();
             if (--ntask == 0) return true;
@@ -454,7 +534,8 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
       old = __builtin_amdgcn_readfirstlane(old);
       if (old == static_cast<unsigned>(G) - 1u) broadcast_flag(p, FLAG_PERM);
     }
-    const int d0 = ks2 * sub / parts, steps2 = ks2 * (sub + 1) / parts - d0;
+    const SplitSteps sk2 = split_steps(ks2, sub, parts == 8 ? 3 : 2, p.split_spec != 0);
+    const int steps2 = sk2.count;
     const int n_tasks = ntiles * per_tile;
     int ntask = b < n_tasks ? (n_tasks - b + G - 1) / G : 0;
     if (ntask > 0) {
@@ -465,10 +546,13 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
         if (lq < n_tasks) {
           const SplitTile t = split_tile(tiles, lq / per_tile);
           const int nblk = parts == 8 ? lq % per_tile : (lq % per_tile) * 2 + grp;
+          const int start = sk2.start(nblk), d0 = sk2.at(start);
           if constexpr (PACKED) {
             const size_t task = static_cast<size_t>(t.expert) * nt2 + nblk;
             st.ap[0] = reinterpret_cast<const unsigned char*>(p.ffn2_packed) + (task * ks2 + d0) * 4096 + lane * 16;
             st.astep = 4096;
+            st.ajump = 4096 * sk2.jump;
+            st.aspan = 4096 * sk2.span();
           } else {
             const unsigned char* w2 = reinterpret_cast<const unsigned char*>(p.ffn2) +
                                       static_cast<size_t>(t.expert) * H * I * ESZ + d0 * 64 + row_order_chunk() * 16;
@@ -476,12 +560,18 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
 #pragma unroll
             for (int q = 0; q < st.NP; ++q) st.ap[q] = w2 + static_cast<size_t>(n0 + 16 * q) * I * ESZ;
             st.astep = 64;
+            st.ajump = 64 * sk2.jump;
+            st.aspan = 64 * sk2.span();
           }
 #pragma unroll
           for (int r = 0; r < RB; ++r)
             st.boff[r] = static_cast<unsigned>((t.row0 + min(16 * r + r16, t.rows - 1)) * I * ESZ + d0 * 64 + g * 16);
           st.bstep = 64;
+          st.bjump = 64 * sk2.jump;
+          st.bspan = 64 * sk2.span();
           st.left = steps2;
+          st.turn = start;
+          st.mask = sk2.mask;
           lq += G;
         } else {
           st.park(p.gate);
@@ -490,14 +580,14 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
       // The weights of the first window go out before the wait, the h rows behind it: both walk
       // through the same steps.
       next_task();
-      const int lq0 = lq;
+      const int lq0 = lq, turn0 = st.turn;
       unsigned boff0[RB];
 #pragma unroll
       for (int r = 0; r < RB; ++r) boff0[r] = st.boff[r];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         st.load_a(u);
-        if (--st.left == 0) next_task();
+        st.template advance<true, false>(next_task);
         __builtin_amdgcn_sched_barrier(0);
       }
       ok = wait_flag(p, FLAG_PERM, lds_flag, lds_poller);
@@ -505,19 +595,26 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
         const unsigned char* keep[st.NP];
 #pragma unroll
         for (int q = 0; q < st.NP; ++q) keep[q] = st.ap[q];
+        const int keep_step = st.astep, keep_jump = st.ajump;
         lq = lq0;
 #pragma unroll
         for (int r = 0; r < RB; ++r) st.boff[r] = boff0[r];
         st.bstep = 64;
+        st.bjump = 64 * sk2.jump;
+        st.bspan = 64 * sk2.span();
         st.left = steps2;
+        st.turn = turn0;
+        st.mask = sk2.mask;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           st.load_b(u);
-          if (--st.left == 0) next_task();
+          st.template advance<false, true>(next_task);
           __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int q = 0; q < st.NP; ++q) st.ap[q] = keep[q];
+        st.astep = keep_step;
+        st.ajump = keep_jump;
         auto finish = [&]() {
           const SplitTile t = split_tile(tiles, cq / per_tile);
           const int n0 = (parts == 8 ? cq % per_tile : (cq % per_tile) * 2 + grp) * (16 * G2_NB);
@@ -551,7 +648,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
             st.load_a(u);
             st.load_b(u);
             __builtin_amdgcn_sched_barrier(0);
-            if (--st.left == 0) next_task();
+            st.template advance<true, true>(next_task);
             if (--cleft == 0) {
               finish();
               if (--ntask == 0) return true;
