@@ -87,8 +87,8 @@ def measured_traffic(workload, weights):
 
 
 def kernel_of(tiled, dtype):
-    """The kernel a workload of this file runs (its bf16 decode batches have at most 24 rows an expert)."""
-    return "moe_tiled_kernel" if tiled else "moe_split_kernel" if dtype == "bf16" else "moe_stream_kernel"
+    """The kernel a workload of this file runs (its small batches have at most 24 rows an expert, float32 4)."""
+    return "moe_tiled_kernel" if tiled else "moe_split_kernel"
 
 
 def record_traffic(workload, weights, fetch_kib, write_kib, kernel):
