@@ -1,4 +1,4 @@
-// What the streaming and the split-k kernel share: the routing tasks of bf16 layers, the wait for
+// What the streaming and the split-k kernel share: the routing tasks, the wait for
 // a phase flag, the register transpose of row-major weights and the combine tasks.
 #pragma once
 #ifndef FMOE_PARAMS_IN_KERNARG

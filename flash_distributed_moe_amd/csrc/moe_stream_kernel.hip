@@ -17,7 +17,7 @@
 // The down projection reads h rows that other workers wrote, so its B operand
 // uses coherent loads.
 //
-// bf16 batches of up to 24 rows an expert run the split-k variant instead (moe_split_kernel.hip),
+// bf16 batches of up to 24 rows an expert, float32 ones below 10, run the split-k variant instead (moe_split_kernel.hip),
 // with the same routing and combine, whose workgroups share a task's k. It has a file of its own
 // because the float32 kernel's time depends on where its loops lie (see build.py).
 //
