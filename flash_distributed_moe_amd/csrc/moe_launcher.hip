@@ -86,6 +86,10 @@ constexpr int kAutoTiledRowsPacked = 26;
 constexpr int kAutoTiledRowsRowMajor = 14;
 constexpr int kAutoTiledRowsF32 = 10;
 
+bool keeps_bf16_rows(const FlashMoeLayerDesc& d) {  // the tiled variant's y (see moe_params.h)
+  return d.dtype == FLASH_MOE_BF16 && !fmoe::tiled_ragged(d.hidden, d.intermediate);
+}
+
 // need_tiled: the tiled variant may run on this workspace.
 Layout make_layout(const FlashMoeLayerDesc& d, bool need_tiled) {
   Layout L{};
@@ -120,15 +124,16 @@ Layout make_layout(const FlashMoeLayerDesc& d, bool need_tiled) {
   // caches, so its rows are whole 128-byte lines: no line then holds rows of two tiles.
   L.h = take(esz * rows * (need_tiled ? fmoe::tiled_h_pitch(d.intermediate) : d.intermediate));
   // y: the streaming variant keeps every (token, slot) row in float, the tiled variant in
-  // bf16. When every batch that asks for the tiled variant gets it (tiled_all) and AUTO hands
-  // it the large batches, the streaming one only ever sees batches below the switch-over.
-  const bool tiled_all = need_tiled && static_cast<long long>(d.max_tokens) * d.hidden * 2 < (1ll << 32);
+  // bf16 (ragged shapes: in float). When every batch that asks for the tiled variant gets it (tiled_all) and AUTO
+  // hands it the large batches, the streaming one only ever sees batches below the switch-over.
+  const bool bf16_rows = need_tiled && keeps_bf16_rows(d);
+  const bool tiled_all = bf16_rows && static_cast<long long>(d.max_tokens) * d.hidden * 2 < (1ll << 32);
   const size_t stream_rows =
       tiled_all && d.sched == FLASH_MOE_SCHED_TILED ? 0
       : tiled_all && d.sched == FLASH_MOE_SCHED_AUTO ? std::min<size_t>(rows, kAutoTiledRowsPacked * static_cast<size_t>(d.experts))
                                                      : rows;
   L.y = take(std::max(sizeof(float) * stream_rows * d.hidden,
-                      need_tiled ? fmoe::tiled_y_bytes(rows, d.hidden) : 0));
+                      bf16_rows ? fmoe::tiled_y_bytes(rows, d.hidden) : 0));
   L.xn = take((d.flags & FLASH_MOE_FLAG_RMSNORM) ? esz * static_cast<size_t>(d.max_tokens) * d.hidden : 0);
   const bool pack = (d.flags & FLASH_MOE_FLAG_PACK_WEIGHTS) != 0;
   L.pack1 = take(pack ? esz * d.experts * 2 * d.intermediate * d.hidden : 0);
@@ -174,8 +179,8 @@ hipError_t validate(const FlashMoeLayerDesc* d) {
 // weights that it can address with 32-bit byte offsets. H need be no multiple of its 256 columns nor I
 // one of 128: what stands out over the last column costs less than the streaming variant's tiles of 64
 // rows, each of which reads its expert's weights again (us, streaming / tiled: E=40, k=5, H=1344, I=736
-// T=200 107 / 107, T=400 150 / 105, T=8000 1112 / 391; E=16, k=2, H=320, I=160 T=300 58 / 48, T=4000
-// 201 / 74; E=100, k=6, H=3904, I=1952 T=600 1044 / 956, T=4000 3746 / 1386). AUTO takes it once an expert sees about 26
+// T=208 111 / 99, T=600 173 / 115, T=8000 1118 / 453; E=16, k=2, H=320, I=160 T=208 55 / 44, T=4000
+// 202 / 79; E=100, k=6, H=3904, I=1952 T=434 941 / 925, T=4000 3746 / 1497). AUTO takes it once an expert sees about 26
 // rows on average when the weights are packed (30B shape, us, streaming / tiled:
 // T=320 284 / 301, T=384 293 / 301, T=448 314 / 299, T=512 339 / 304; 235B shape:
 // T=320 905 / 960, T=384 934 / 969, T=512 1054 / 976), and from about 14 rows on
@@ -366,6 +371,7 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
               : T <= 6 * m.n_groups && ((T + 15) / 16) * ((d.experts + 31) / 32) <= 2 * m.n_groups ? 1
                                                                                                   : 2;
     p.early = p.dot16;  // (the last selection raises FLAG_ROUTED)
+    p.n_workers = p.n_groups * 4;
   }
   if (tiled && d.dtype == FLASH_MOE_F32) {
     p.n_groups = std::min(2 * m.n_groups, kMaxGroups);  // two workgroups of four waves a CU
@@ -736,9 +742,10 @@ int flashMoeLaunchNoAlloc(const FlashMoeLayerDesc* desc, const void* tokens, voi
   l.num_cus = kMaxGroups;
   int sched = sched_for(l.desc, tokens_num, machine(l));
   l.layout = make_layout(l.desc, sched == FLASH_MOE_SCHED_TILED);
-  if (sched == FLASH_MOE_SCHED_TILED && desc->sched == FLASH_MOE_SCHED_AUTO &&
+  if (sched == FLASH_MOE_SCHED_TILED && (desc->sched == FLASH_MOE_SCHED_AUTO || !keeps_bf16_rows(l.desc)) &&
       l.layout.total > static_cast<size_t>(FLASH_MOE_NOALLOC_SCRATCH_BYTES)) {
-    // AUTO: the streaming variant's workspace is smaller, and it serves any batch
+    // The streaming variant's workspace is smaller and it serves any batch: so for AUTO, and for layers whose
+    // tiled variant only adds the padding of h's rows to it.
     sched = FLASH_MOE_SCHED_STREAM;
     l.desc.sched = FLASH_MOE_SCHED_STREAM;
     l.layout = make_layout(l.desc, false);
@@ -866,7 +873,7 @@ int flashMoeReadDownRows(FlashMoeLauncher* l, int tokens_num, void* y, int* elem
   if (tokens_num < 0 || tokens_num > l->desc.max_tokens)
     FMOE_FAIL(hipErrorInvalidValue, "tokens_num = %i", tokens_num);
   FMOE_HIP_CHECK(hipStreamSynchronize(stream));
-  const bool tiled = l->desc.dtype == FLASH_MOE_BF16 && flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED;
+  const bool tiled = keeps_bf16_rows(l->desc) && flashMoeSchedFor(l, tokens_num) == FLASH_MOE_SCHED_TILED;
   const size_t rows = static_cast<size_t>(tokens_num) * l->desc.top_k;
   const size_t bytes = rows * l->desc.hidden * (tiled ? 2 : 4);
   const size_t kept = (l->layout.xn - l->layout.y);  // the region's size up to the next one

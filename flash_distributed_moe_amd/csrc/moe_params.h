@@ -29,6 +29,11 @@ constexpr int SCAN_LDS_WORDS = 1024;  // mask words (experts x 64-token words) t
 constexpr int SHORT_MASK_WORDS = 8192;  // the same for the tiled kernel's short prologue
 constexpr int SPLIT_MAX_SLOTS = 2048;  // split-k kernel: (token, slot) entries its tables hold
 constexpr int EARLY_MAX_TOKENS = 384;  // batches up to this size may take their gate/up weights before the routing is known
+// Shapes whose columns do not divide into the bf16 tiled variant's tasks (256 of H, 128 of I): kernels of
+// their own, which keep y as the streaming variant does (see tile_task).
+constexpr __host__ __device__ bool tiled_ragged(int hidden, int intermediate) {
+  return hidden % 256 != 0 || intermediate % 128 != 0;
+}
 // Elements from one row of h to the next in the bf16 tiled variant: whole 128-byte lines.
 constexpr __host__ __device__ int tiled_h_pitch(int intermediate) { return (intermediate + 63) & ~63; }
 constexpr int MAX_EXPERTS = 256;  // experts are spread 64 per wave register slot
@@ -87,7 +92,7 @@ struct TraceRec {
 struct Params {
   int T, E, H, K, I;
   int W;          // 64-bit mask words per expert (row stride of `masks`)
-  int n_workers;  // waves (skinny kernel) taking tickets
+  int n_workers;  // waves that take tickets (streaming variant) or items of the combine step
   int max_mtiles;
   long long spin_limit;  // bound on one dependency wait, 100 MHz ticks
 
@@ -114,7 +119,8 @@ struct Params {
   float* row_w;               // [T*K] gate weight of the permuted row
   TileDesc* mtiles;           // [max_mtiles]
   void* h;                    // [T*K, I] SwiGLU output, layer dtype; bf16 tiled variant: rows of tiled_h_pitch(I) elements
-  float* y;                   // [T*K, H] weighted down-projection rows, by t*K+slot
+  float* y;                   // [T*K, H] weighted down-projection rows, by t*K+slot; bf16 tiled variant, shapes that are
+                              // not ragged: bf16 rows without the weight
   Control* ctl;
   WgFlags* wgflags;                // [n_groups]
   ControlLine* g1_done;            // [max_mtiles] gate/up tasks finished per row tile

@@ -13,7 +13,7 @@
 //   scatter  32 tokens: permuted row of every (token, slot)
 //   gate/up  (row tile, 128 h columns): 256 token rows x 256 weight rows, gate
 //            and up rows side by side so that SiLU(gate)*up happens in registers
-//   down     (row tile, 256 output columns): same tile, weighted bf16 rows to y
+//   down     (row tile, 256 output columns): same tile, bf16 rows to y (ragged shapes: weighted float rows)
 //   combine  1 to 8 tokens: out = sum over slots of y
 // GEMM tile: up to 320 token rows x 256 weight rows, K stepped by 64; each wave
 // owns 64 weight rows x all token rows of it as 4 x (2*JT) MFMA 16x16x32 blocks
@@ -464,6 +464,7 @@ constexpr int SHORT_CNT_OFF = SHORT_PRE_OFF + (SHORT_MASK_WORDS + MAX_EXPERTS) *
 constexpr int SHORT_OFF_OFF = SHORT_CNT_OFF + MAX_EXPERTS * 4;
 constexpr int SHORT_LDS_BYTES = SHORT_OFF_OFF + MAX_EXPERTS * 4;
 
+template <bool RAGGED>
 __device__ __noinline__ void short_scatter_task(ParamsRef pv, int blk_in) {
   ParamsRef p = uniform_params(pv);
   const RouteTables r = route_tables(p);
@@ -475,6 +476,8 @@ __device__ __noinline__ void short_scatter_task(ParamsRef pv, int blk_in) {
   int* loff = reinterpret_cast<int*>(lds_raw + SHORT_OFF_OFF);
   const int i = blk * T_THREADS + tid;
   const int e = i < r.T * r.K ? ldc(&r.topk_idx[i]) : -1;
+  float weight = 0.0f;
+  if (RAGGED && i < r.T * r.K) weight = ldc(&r.topk_w[i]);
   for (int w0 = tid; w0 < nw; w0 += 4 * T_THREADS) {
     unsigned long long m[4];
 #pragma unroll
@@ -519,7 +522,9 @@ __device__ __noinline__ void short_scatter_task(ParamsRef pv, int blk_in) {
   if (e >= 0) {
     const int t = i / r.K, wd = t >> 6;
     const int w = e * pitch + wd;
-    stc(&r.perm[loff[e] + lpre[w] + __popcll(lmask[w] & ((1ull << (t & 63)) - 1ull))], i);
+    const int pos = loff[e] + lpre[w] + __popcll(lmask[w] & ((1ull << (t & 63)) - 1ull));
+    stc(&r.perm[pos], i);
+    if (RAGGED) stc(&r.row_w[pos], weight);
   }
 }
 
@@ -583,9 +588,9 @@ constexpr int stage_bytes_of(int jt) { return (TN + 32 * jt) * ROWB; }
 constexpr int nst_of(int jt) { return jt <= 5 ? 3 : 2; }
 constexpr int TILE_LDS_BYTES = 3 * stage_bytes_of(5);               // 159744
 static_assert(TILE_LDS_BYTES >= 2 * stage_bytes_of(JT_MAX), "stages");
-// behind the stages: the tile's destination rows for the down epilogue
+// behind the stages: the tile's destination rows for the down epilogue, and (ragged shapes) their gate weights
 constexpr int SIDE_OFF = TILE_LDS_BYTES;
-constexpr int SIDE_BYTES = TM_MAX * 4;
+constexpr int SIDE_BYTES = TM_MAX * 8;
 // and behind those one 16-byte line of words a GEMM task leaves for the worker loop: the ticket it
 // drew for the workgroup's next task. They live in
 // the dynamic block because a file-scope LDS variable written from a function that is not
@@ -1098,22 +1103,31 @@ __device__ __forceinline__ unsigned packed_run_offset(int q) {
 // by the combine task, which has instruction slots to spare; here every instruction of the
 // epilogue is one the matrix cores wait for.
 //
+// RAGGED: H is no multiple of 256 or I none of 128. The last task of a row tile may stand out over the
+// last column: a wave whose columns do not exist repeats the last ones that do, and its results are not
+// stored. These layers keep what the streaming variant computes for them, bit for bit: the division in
+// SwiGLU is a division, and y holds float rows that carry their gate weight, stored from the accumulators
+// (16 bytes a lane, 64 of a row). With bf16 rows as below they would be faster, but held in fewer bits than
+// their small batches: relative error against float64 2.87e-3 instead of 2.35e-3 (us, streaming variant / float
+// rows / bf16 rows, E=40, k=5, H=1344, I=736: T=260 127 / 101 / 98, T=2000 361 / 166 / 150, T=8000 1118 / 453 /
+// 375; E=100, k=6, H=3904, I=1952: T=1200 1622 / 1028 / 997, T=4000 3746 / 1497 / 1384).
+//
 // HALF (down): I is an odd number of 32-k steps (see tile_gemm).
-template <int JT, bool down, bool HALF = false>
+template <int JT, bool down, bool RAGGED = false, bool HALF = false>
 __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int rows, int nblk, unsigned* pend,
                                           unsigned* queue) {
   const int H = uni(p.H), I = uni(p.I), K = uni(p.K);
   const int wave = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
   // packed weights and enough stages: the deeper pipeline
-  const int hp = tiled_h_pitch(I);
+  const int hp = RAGGED ? tiled_h_pitch(I) : I;
   const int depth = HALF ? 0 : uni((down ? p.ffn2_packed : p.ffn1_packed) != nullptr ? direct_depth(JT, (down ? I : H) / KS) : 0);
   const int* perm = uni(p.perm) + row0;
   const int n0 = uni(nblk) * (down ? TN : G1_COLS);
-  // The last task of a row tile may stand out over the last column: a wave whose columns do not exist
-  // repeats the last ones that do, and its results are not stored.
-  const int wblk = down ? min(n0 / 64 + wave, H / 64 - 1) : min(n0 / 32 + wave, I / 32 - 1);
+  const int wcol = down ? n0 / 64 + wave : n0 / 32 + wave;  // the wave's column block, and the last that exists
+  const int wblk = RAGGED ? min(wcol, (down ? H / 64 : I / 32) - 1) : wcol;
   TileOperands op;
   int side_dst[2] = {-1, -1};
+  float side_w[2] = {0.0f, 0.0f};
   int nstages;
   if (down) {
     nstages = (I + KS - 1) / KS;
@@ -1182,6 +1196,7 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
       for (int k = 0; k < 2; ++k) {
         const int r = static_cast<int>(threadIdx.x) + k * T_THREADS;
         side_dst[k] = r < rows ? ldc(&perm[r]) : -1;
+        if (RAGGED && r < rows) side_w[k] = ldc(&uni(p.row_w)[row0 + r]);
       }
     }
   };
@@ -1208,7 +1223,8 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
       for (int i = 0; i < 2; ++i) {  // gate blocks 0, 1 with their up blocks 2, 3
         float hv[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) hv[v] = silu_mul_fast(acc[i][j][v], acc[2 + i][j][v]);
+        for (int v = 0; v < 4; ++v)
+          hv[v] = RAGGED ? silu_mul(acc[i][j][v], acc[2 + i][j][v]) : silu_mul_fast(acc[i][j][v], acc[2 + i][j][v]);
         uint2 pk;
         pk.x = pack_bf16(hv[0], hv[1]);
         pk.y = pack_bf16(hv[2], hv[3]);
@@ -1217,7 +1233,7 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
     __syncthreads();
     // 16 lanes store one row's 256 bytes; a wave stores 4 rows per instruction
     unsigned char* h = uni(reinterpret_cast<unsigned char*>(p.h)) + (static_cast<size_t>(row0) * hp + n0) * 2;
-    const bool live = n0 + (lane & 15) * 8 < I;  // the lane's columns exist
+    const bool live = !RAGGED || n0 + (lane & 15) * 8 < I;  // the lane's columns exist
     // (the reads of a batch first, then its stores: a store's assembly orders memory
     // operations around it, and one LDS round trip per store would add up to microseconds)
     constexpr int NIT = 8 * JT / WAVES, BATCH = 8;
@@ -1232,7 +1248,7 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
         const int row = ((it0 + u) * WAVES + wave) * 4 + (lane >> 4);
-        if (it0 + u < NIT && ((row < rows) & live))
+        if (it0 + u < NIT && (RAGGED ? (row < rows) & live : row < rows))
           st16_through(h + static_cast<size_t>(row) * hp * 2 + (lane & 15) * 16, v[u]);
       }
     }
@@ -1243,10 +1259,27 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
     for (int k = 0; k < 2; ++k) {
       const int r = static_cast<int>(threadIdx.x) + k * T_THREADS;
       if (r < TM_MAX) sdst[r] = side_dst[k];
+      if (RAGGED && r < TM_MAX) reinterpret_cast<float*>(sdst + TM_MAX)[r] = side_w[k];
     }
     __syncthreads();
+    if constexpr (RAGGED) {
+      if (wcol != wblk) return;
+      float* yf = uni(p.y) + 64 * wcol + 4 * kg;
+#pragma unroll
+      for (int j = 0; j < 2 * JT; ++j) {
+        const int dst = sdst[16 * j + r16];
+        const float w = reinterpret_cast<const float*>(sdst + TM_MAX)[16 * j + r16];
+        if (dst >= 0) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            st16_through(yf + static_cast<size_t>(dst) * H + 16 * i,
+                         make_uint4(__float_as_uint(acc[i][j][0] * w), __float_as_uint(acc[i][j][1] * w),
+                                    __float_as_uint(acc[i][j][2] * w), __float_as_uint(acc[i][j][3] * w)));
+        }
+      }
+      return;
+    }
     unsigned char* y = uni(reinterpret_cast<unsigned char*>(p.y)) + n0 * 2;
-    const bool live = n0 + (lane & 31) * 8 < H;  // the lane's columns exist
 #pragma unroll
     for (int part = 0; part < (JT + 3) / 4; ++part) {
 #pragma unroll
@@ -1278,7 +1311,7 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
         }
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
-          if ((dst[u] >= 0) & live) st16_through(y + static_cast<size_t>(dst[u]) * H * 2 + (lane & 31) * 16, v[u]);
+          if (dst[u] >= 0) st16_through(y + static_cast<size_t>(dst[u]) * H * 2 + (lane & 31) * 16, v[u]);
       }
       __syncthreads();
     }
@@ -1315,25 +1348,38 @@ __device__ __noinline__ void tiled_gemm_task(ParamsRef pv, const TileDesc& tile_
   }
 }
 
-// the down tasks of layers whose I is an odd number of 32-k steps
-__device__ __noinline__ void tiled_odd_down_task(ParamsRef pv, const TileDesc& tile_in, int nblk, unsigned* pend_in,
-                                                 unsigned* queue_in) {
+// the tasks of ragged layers, and their down tasks where I is an odd number of 32-k steps
+template <bool down, bool HALF>
+__device__ __forceinline__ void ragged_tile(ParamsRef pv, const TileDesc& tile_in, int nblk, unsigned* pend_in,
+                                            unsigned* queue_in) {
   ParamsRef p = uniform_params(pv);
   unsigned* pend = uni(pend_in);
   unsigned* queue = uni(queue_in);
   const int expert = uni(tile_in.expert), row0 = uni(tile_in.row0), rows = uni(tile_in.rows);
   switch ((rows + 31) >> 5) {
     case 1:
-    case 2: tile_task<2, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
-    case 3: tile_task<3, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
-    case 4: tile_task<4, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
-    case 5: tile_task<5, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
-    case 6: tile_task<6, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
-    case 7: tile_task<7, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
-    case 8: tile_task<8, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
-    case 9: tile_task<9, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
-    default: tile_task<10, true, true>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 2: tile_task<2, down, true, HALF>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 3: tile_task<3, down, true, HALF>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 4: tile_task<4, down, true, HALF>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 5: tile_task<5, down, true, HALF>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 6: tile_task<6, down, true, HALF>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 7: tile_task<7, down, true, HALF>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 8: tile_task<8, down, true, HALF>(p, expert, row0, rows, nblk, pend, queue); break;
+    case 9: tile_task<9, down, true, HALF>(p, expert, row0, rows, nblk, pend, queue); break;
+    default: tile_task<10, down, true, HALF>(p, expert, row0, rows, nblk, pend, queue); break;
   }
+}
+__device__ __noinline__ void tiled_ragged_gate_up_task(ParamsRef p, const TileDesc& tile, int nblk, unsigned* pend,
+                                                       unsigned* queue) {
+  ragged_tile<false, false>(p, tile, nblk, pend, queue);
+}
+__device__ __noinline__ void tiled_ragged_down_task(ParamsRef p, const TileDesc& tile, int nblk, unsigned* pend,
+                                                    unsigned* queue) {
+  ragged_tile<true, false>(p, tile, nblk, pend, queue);
+}
+__device__ __noinline__ void tiled_odd_down_task(ParamsRef p, const TileDesc& tile, int nblk, unsigned* pend,
+                                                 unsigned* queue) {
+  ragged_tile<true, true>(p, tile, nblk, pend, queue);
 }
 
 constexpr int TILED_LDS_BYTES = NOTE_OFF + NOTE_BYTES;
@@ -1507,9 +1553,9 @@ __device__ __noinline__ void tiled_combine_task(ParamsRef pv, int blk, int tok_i
 // come from a last global counter once every queue is empty.
 // The launch parameters are read in place and the task calls keep the local
 // calling convention, as in the streaming variant (see its worker loop).
-// ODD: I is an odd number of 32-k steps (a kernel of its own: as a branch of this one it cost every
-// task of the others half a microsecond).
-template <bool ODD>
+// RAGGED: see tile_task. ODD: I is an odd number of 32-k steps, which only ragged layers have (kernels of
+// their own: as a branch of this one the odd steps cost every task of the others half a microsecond).
+template <bool RAGGED, bool ODD>
 __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void moe_tiled_kernel(
     const Params params) {
   ParamsRef p = kernel_params();
@@ -1580,7 +1626,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
     const int n_perm = (Ti * p.K + T_THREADS - 1) / T_THREADS;
     if (b < n_perm) ok = wg_wait_flag(p, FLAG_ROUTED, &sh);
     for (int i = b; ok && i < n_perm; i += G) {
-      short_scatter_task(p, i);
+      short_scatter_task<RAGGED>(p, i);
       if (wg_arrive<false>(&ctl->perm_done.v, &sh) == static_cast<unsigned>(n_perm) - 1u) wg_broadcast_flag(p, FLAG_PERM);
     }
   }
@@ -1669,7 +1715,11 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
         const unsigned m = lo + j / nt1;
         if (p.trace) t_ready = wall_clock64();
         const TileDesc tile = ld_tile(&p.mtiles[m]);
-        tiled_gemm_task(p, tile, static_cast<int>(j % nt1), 0, pend, &ctl->xq[q].v);
+        if constexpr (RAGGED) {
+          tiled_ragged_gate_up_task(p, tile, static_cast<int>(j % nt1), pend, &ctl->xq[q].v);
+        } else {
+          tiled_gemm_task(p, tile, static_cast<int>(j % nt1), 0, pend, &ctl->xq[q].v);
+        }
         pend = &p.g1_done[m].v;
         trace(t_dyn0 + lo * nt1 + j, 3, m, t_fetch, t_ready);
         j = task_notes()[0];
@@ -1689,6 +1739,8 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
           if (p.trace) t_ready = wall_clock64();
           if constexpr (ODD) {
             tiled_odd_down_task(p, tile, static_cast<int>(jj % nt2), pend, &ctl->xq[q].v);
+          } else if constexpr (RAGGED) {
+            tiled_ragged_down_task(p, tile, static_cast<int>(jj % nt2), pend, &ctl->xq[q].v);
           } else {
             tiled_gemm_task(p, tile, static_cast<int>(jj % nt2), 1, pend, &ctl->xq[q].v);
           }
@@ -1701,9 +1753,16 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
     flush();
   }
 
-  // ---- combine tasks from the last global counter
+  // ---- combine tasks from the last global counter; float rows of y as the streaming variant sums them
   if (ok && n2_total != 0u) ok = wg_wait_ge(p, &ctl->g2_done.v, n2_total, &sh);
-  while (ok) {
+  if constexpr (RAGGED) {
+    if (ok) {
+      const unsigned ncomb = (static_cast<unsigned>(p.H) + COMBINE_COLS - 1u) / COMBINE_COLS;
+      const unsigned slot = static_cast<unsigned>(uni(static_cast<int>(threadIdx.x >> 6))) * n_groups + blockIdx.x;
+      combine_items<BF16>(p, slot, T * ncomb, ncomb, blockIdx.x, t_dyn0 + nm * (nt1 + nt2), p.trace ? wall_clock64() : 0);
+    }
+  }
+  while (!RAGGED && ok) {
     const long long t_fetch = p.trace ? wall_clock64() : 0;
     if (threadIdx.x == 0) sh.ticket = add_relaxed(&ctl->cticket.v, 1u);
     __syncthreads();
@@ -1751,17 +1810,19 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
 
 // Largest token count of the tiled variant: the launcher's capacity at top-1.
 int tiled_max_tokens() { return 1 << 21; }
-// y of the tiled variant: one bf16 row of H per (token, slot)
+// y of the tiled variant: one bf16 row of H per (token, slot); ragged shapes keep the streaming variant's float rows
 size_t tiled_y_bytes(size_t rows, size_t hidden) { return rows * hidden * 2; }
 
 hipError_t launch_tiled_kernel(const Params& p, int grid, hipStream_t stream) {
-  auto* kernel = p.I % KS == 0 ? moe_tiled_kernel<false> : moe_tiled_kernel<true>;
+  auto* kernel = !tiled_ragged(p.H, p.I) ? moe_tiled_kernel<false, false>
+                 : p.I % KS == 0         ? moe_tiled_kernel<true, false>
+                                         : moe_tiled_kernel<true, true>;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(T_THREADS), TILED_LDS_BYTES, stream, p);
   return hipGetLastError();
 }
 
 hipError_t prepare_tiled_kernel() {
-  for (auto* kernel : {moe_tiled_kernel<false>, moe_tiled_kernel<true>}) {
+  for (auto* kernel : {moe_tiled_kernel<false, false>, moe_tiled_kernel<true, false>, moe_tiled_kernel<true, true>}) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, TILED_LDS_BYTES);
     if (e != hipSuccess) return e;
@@ -1769,10 +1830,10 @@ hipError_t prepare_tiled_kernel() {
   return hipSuccess;
 }
 
-// the lesser of the two kernels' numbers of workgroups a CU holds
+// the least of the kernels' numbers of workgroups a CU holds
 hipError_t tiled_kernel_occupancy(int* per_cu) {
   *per_cu = 0x7FFFFFFF;
-  for (auto* kernel : {moe_tiled_kernel<false>, moe_tiled_kernel<true>}) {
+  for (auto* kernel : {moe_tiled_kernel<false, false>, moe_tiled_kernel<true, false>, moe_tiled_kernel<true, true>}) {
     int n = 0;
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, T_THREADS, TILED_LDS_BYTES);
     if (e != hipSuccess) return e;

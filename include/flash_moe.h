@@ -199,7 +199,9 @@ int flashMoeReadIntermediate(FlashMoeLauncher* l, int tokens_num, void* h, void*
  * y [tokens_num*top_k, H], row t*top_k+slot = h[row of (t, slot)] . W2[expert]^T.
  * The two variants keep them differently, which *elem_dtype and *weighted report:
  * the streaming variant float32, already multiplied by the slot's gate weight
- * (FLASH_MOE_F32, 1), the tiled variant bfloat16, unweighted (FLASH_MOE_BF16, 0).
+ * (FLASH_MOE_F32, 1), the tiled variant of bfloat16 layers with hidden a multiple of
+ * 256 and intermediate one of 128 bfloat16, unweighted (FLASH_MOE_BF16, 0); of other
+ * layers float32 and weighted too.
  * `y` must hold 4 bytes per element either way. Rows of slots without an expert
  * are undefined. hipErrorInvalidValue if the launcher's workspace keeps fewer rows
  * than asked for (the streaming variant of an AUTO launcher that hands larger

@@ -100,7 +100,7 @@ def test_accumulators_are_left_alone_until_they_are_written(functions):
     hardware does not make by itself is less), along the straight line behind it."""
     checked = 0
     for name, code in functions.items():
-        if not re.search("tiled_gemm_task|tiled_odd_down_task", name):
+        if not re.search("tiled_gemm_task|tiled_odd_down_task|tiled_ragged_(gate_up|down)_task", name):
             continue
         ins = [i for _, i, _ in code]
         for at, op in enumerate(ins):

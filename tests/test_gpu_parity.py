@@ -238,6 +238,41 @@ def test_tiled_ragged_columns(rows, H, I):
     check_tile_heights(rows, H, I)
 
 
+@pytest.mark.parametrize("T,H,E,k,I,hot,edges", [
+    (70, 192, 2, 2, 160, 0, False),       # one tile of three 32-row blocks; odd 32-k steps
+    (161, 320, 2, 2, 224, 0, True),       # k of 3.5 stages; norm and residual
+    (330, 448, 2, 2, 352, 0, False),      # two tiles an expert
+    (330, 576, 5, 3, 672, 2, False),
+    (400, 512, 4, 2, 160, 0, False),      # only I is ragged
+    (900, 320, 16, 2, 256, 3, True),      # only H is, in no whole stage of the logit chains
+    (70000, 128, 4, 1, 160, 0, False),    # beyond the short prologue
+])
+@pytest.mark.parametrize("packed", [False, True])
+def test_tiled_ragged_equals_the_streaming_variant(T, H, E, k, I, hot, edges, packed):
+    """Layers whose columns do not divide into the tiled variant's tasks are held in as many bits there as in
+    the streaming variant, which serves their small batches: the same sums in the same order, float rows that
+    carry their gate weight, one rounding. So the same bits."""
+    cfg = synth.MoeConfig("ragged", T, H, E, k, I, "bf16", hot=hot)
+    print("ragged", T, H, E, k, I, packed, flush=True)
+    dev = torch.device("cuda:0")
+    norm = synth.normal_torch(5, 9, (H,), 0.25, torch.float32, dev).add_(1.0).to(torch.bfloat16) if edges else None
+    make = lambda sched, inputs: GpuCase(cfg, seed=T + I, sched=sched, inputs=inputs, pack_weights=packed,
+                                         norm_weight=norm, residual=edges)
+    a = make(_lib.SCHED_STREAM, None)
+    try:
+        assert a.launcher.split_blocks_for(T) == 0
+        want = a.run()
+        b = make(_lib.SCHED_TILED, a.inp)
+        try:
+            assert b.launcher.sched_for(T) == _lib.SCHED_TILED
+            assert torch.equal(b.run(), want)
+            assert torch.equal(b.run(), want)
+        finally:
+            b.close()
+    finally:
+        a.close()
+
+
 @pytest.mark.parametrize("T,H,E,k", [
     (40, 128, 17, 3),       # a second group of experts with one expert; one token a wave at most
     (1000, 192, 33, 2),     # a last 256-k stage that is partly empty
