@@ -23,7 +23,7 @@
 // TFLOP/s of float32); row-major weights T=1024 1076 / 627; E=32 T=4096 2400 / 1450.
 //
 // A value that is no finite number, or rounds to none in bf16, has no such parts: its products come
-// out as infinities or NaN. A wave whose sums hold one multiplies its block again with the float32
+// out as infinities or NaN. A wave whose sums hold one multiplies that token row again with the float32
 // matrix instructions, so such inputs give what they give in the streaming kernel.
 //
 // Weights go straight to registers (no other wave of the workgroup reads them), 16 bytes per lane and
@@ -198,48 +198,13 @@ __device__ __forceinline__ void float_gemm(const FloatOperands& op, f32x4 (&acc)
   if (k < op.ksteps) step(k, std::integral_constant<int, 0>{});
 }
 
-// The same block again with the float32 matrix instructions, for sums that are no finite numbers:
-// operands straight from memory, one wave on its own.
-template <int JB>
-__device__ __forceinline__ void float_gemm_exact(const FloatOperands& op, const unsigned (&trow)[JB], f32x4 (&acc)[4][JB]) {
-#pragma unroll
-  for (int j = 0; j < JB; ++j) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int q = 0; q < 2 * op.ksteps; ++q) {
-      const uint4 b = ld16(op.tbase + trow[j] + static_cast<size_t>(q) * 64);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        acc[i][j] = mma16<F32>(ld16(op.wbase + op.wblock[i] + static_cast<size_t>(q) * op.wstep + op.woff), b, acc[i][j]);
-    }
-  }
-}
-
-// One tile task. gate/up: h[row, n0 .. n0+128) (refExpertFFN1.h:51-65); wave w holds gate rows
-// n0+32w.. and the matching up rows, so SiLU(gate)*up happens in registers. down:
-// y[t*K+slot, n0 .. n0+256) = w * (h[row] . W2[e]^T) (refFullMoe.h:58-65, src/hip/kernel/tasks/ffn2Task.h:37-40),
-// float rows with the gate weight applied, as the streaming kernel leaves them. Both are written
-// through, 64 bytes of a row at a time, from the accumulators.
-template <int JB, bool down>
-__device__ __noinline__ void float_task(ParamsRef pv, int expert_in, int row0_in, int rows_in, int shared_in, int nblk_in) {
-  ParamsRef p = uniform_params(pv);
-  const int expert = uni(expert_in), row0 = uni(row0_in), rows = uni(rows_in);
+// The weights of an operand: the 64 rows of a wave's column block `wblk`.
+template <bool down>
+__device__ __forceinline__ void float_weights(ParamsRef p, int expert, int wblk, FloatOperands& op) {
+  const int H = uni(p.H), I = uni(p.I), kk = down ? I : H;
+  const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
   const bool packed = uni((down ? p.ffn2_packed : p.ffn1_packed) != nullptr ? 1 : 0) != 0;
-  // weights that no other tile reads pass through the caches without staying; row-major ones come half a
-  // line at a time and have to stay
-  const bool shared = uni(shared_in) != 0 || !packed;
-  const int H = uni(p.H), I = uni(p.I), K = uni(p.K);
-  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
-  const int r16 = lane & 15, g = lane >> 4;
-  const int nblk = uni(nblk_in);
-  const int cols = down ? 64 : 32;                        // of a wave
-  const int nw = (down ? H : I) / cols, w0 = nblk * F_WAVES + wave;
-  const int wblk = min(w0, nw - 1);
-  const int* perm = uni(p.perm) + row0;
-  uint2* side = reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(lds_dyn) + F_SIDE_OFF);  // row -> (token, slot), weight
-  FloatOperands op;
-  const int kk = down ? I : H;
+  const int nw = down ? H / 64 : I / 32;
   op.ksteps = kk >> 5;
   if (packed) {
     op.wbase = uni(reinterpret_cast<const unsigned char*>(down ? p.ffn2_packed : p.ffn1_packed)) + (static_cast<size_t>(expert) * nw + wblk) * (static_cast<size_t>(kk / 16) * 4096);
@@ -260,6 +225,38 @@ __device__ __noinline__ void float_task(ParamsRef pv, int expert_in, int row0_in
     op.woff = static_cast<unsigned>(r16) * static_cast<unsigned>(H * 4) + g * 16;
     op.wstep = 64u;
   }
+}
+
+// One tile task. gate/up: h[row, n0 .. n0+128) (refExpertFFN1.h:51-65); wave w holds gate rows
+// n0+32w.. and the matching up rows, so SiLU(gate)*up happens in registers. down:
+// y[t*K+slot, n0 .. n0+256) = w * (h[row] . W2[e]^T) (refFullMoe.h:58-65, src/hip/kernel/tasks/ffn2Task.h:37-40),
+// float rows with the gate weight applied, as the streaming kernel leaves them. Both are written
+// through, 64 bytes of a row at a time, from the accumulators. Returns the token rows for which a sum of
+// the wave is no finite number: float_exact_rows writes those again.
+struct RowSet {
+  unsigned word[3];  // a bit a row
+  __device__ __forceinline__ unsigned any() const { return word[0] | word[1] | word[2]; }
+};
+static_assert(F_TM <= 96, "rows of a RowSet");
+template <int JB, bool down>
+__device__ __noinline__ RowSet float_task(ParamsRef pv, int expert_in, int row0_in, int rows_in, int shared_in, int nblk_in) {
+  ParamsRef p = uniform_params(pv);
+  const int expert = uni(expert_in), row0 = uni(row0_in), rows = uni(rows_in);
+  const bool packed = uni((down ? p.ffn2_packed : p.ffn1_packed) != nullptr ? 1 : 0) != 0;
+  // weights that no other tile reads pass through the caches without staying; row-major ones come half a
+  // line at a time and have to stay
+  const bool shared = uni(shared_in) != 0 || !packed;
+  const int H = uni(p.H), I = uni(p.I), K = uni(p.K);
+  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int nblk = uni(nblk_in);
+  const int cols = down ? 64 : 32;                        // of a wave
+  const int nw = (down ? H : I) / cols, w0 = nblk * F_WAVES + wave;
+  const int wblk = min(w0, nw - 1);
+  const int* perm = uni(p.perm) + row0;
+  uint2* side = reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(lds_dyn) + F_SIDE_OFF);  // row -> (token, slot), weight
+  FloatOperands op;
+  float_weights<down>(p, expert, wblk, op);
   op.tbase = down ? uni(reinterpret_cast<const unsigned char*>(p.h)) + static_cast<size_t>(row0) * I * 4
                   : uni(reinterpret_cast<const unsigned char*>(p.tokens));
   auto row_offset = [&](int row) {
@@ -278,19 +275,25 @@ __device__ __noinline__ void float_task(ParamsRef pv, int expert_in, int row0_in
   } else {
     float_gemm<JB, true>(op, acc);
   }
-  if (w0 >= nw) return;  // this wave's columns do not exist: it has multiplied the last ones that do
-  float t = 0.0f;
+  RowSet again = {{0u, 0u, 0u}};
+  if (w0 >= nw) return again;  // this wave's columns do not exist: it has multiplied the last ones that do
+  float t[JB], all = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int j = 0; j < JB; ++j) {
+    t[j] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < JB; ++j)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) t = __builtin_fmaf(acc[i][j][v], 0.0f, t);
-  if (__any(t != 0.0f)) {
-    unsigned trow[JB];
+      for (int v = 0; v < 4; ++v) t[j] = __builtin_fmaf(acc[i][j][v], 0.0f, t[j]);
+    all += t[j];
+  }
+  if (__any(all != 0.0f)) {
 #pragma unroll
-    for (int j = 0; j < JB; ++j) trow[j] = row_offset(16 * j + r16) + g * 16;
-    float_gemm_exact<JB>(op, trow, acc);
+    for (int j = 0; j < JB; ++j) {
+      const unsigned long long b = __ballot(t[j] != 0.0f && 16 * j + r16 < rows);  // a row's lanes stand 16 apart
+      const unsigned both = static_cast<unsigned>(b) | static_cast<unsigned>(b >> 32);
+      again.word[j >> 1] |= ((both | both >> 16) & 0xFFFFu) << (16 * (j & 1));
+    }
   }
 
   if (!down) {
@@ -324,18 +327,110 @@ __device__ __noinline__ void float_task(ParamsRef pv, int expert_in, int row0_in
       }
     }
   }
+  return again;
 }
 
+// The `again` rows of this wave's columns with the float32 matrix instructions, 16 at a time: operands straight
+// from memory, the wave on its own, EXACT_AHEAD steps of 16 k in flight. Every task of an infinite token's
+// experts does this (a NaN token has none), so the launch waits for it. us, 30B shape, packed, without / with
+// one / with eight infinite tokens: T=160 440 / 520 / 527, T=256 455 / 537 / 548, T=1024 598 / 650 / 657 (whole
+// blocks of the tile, no step in flight:
+// T=160 434 / 630 / 665, T=1024 600 / 1223 / 1257; streaming kernel T=160 546 / 545 / 552, T=1024 1664 / 1668 /
+// 1666). A function of its own: inlined in the tasks it cost every launch 1 %.
+constexpr int EXACT_AHEAD = 4;
+template <bool down>
+__device__ __noinline__ void float_exact_rows(ParamsRef pv, int expert_in, int row0_in, int nblk_in, RowSet again) {
+  ParamsRef p = uniform_params(pv);
+  const int expert = uni(expert_in), row0 = uni(row0_in);
+  const int H = uni(p.H), I = uni(p.I), K = uni(p.K);
+  const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+  const int w0 = uni(nblk_in) * F_WAVES + uni(static_cast<int>(threadIdx.x >> 6));
+  FloatOperands op;
+  float_weights<down>(p, expert, w0, op);
+  const int n = 2 * op.ksteps;  // (k >= 128: at least EXACT_AHEAD)
+  unsigned left[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) left[q] = uni(static_cast<int>(again.word[q]));
+  while ((left[0] | left[1] | left[2]) != 0u) {
+    int row = 0, found = 0;  // this lane's row: the r16-th of those left, or the last of them
+    while (found < 16 && (left[0] | left[1] | left[2]) != 0u) {
+      const int q = left[0] != 0u ? 0 : left[1] != 0u ? 1 : 2;
+      const unsigned word = q == 0 ? left[0] : q == 1 ? left[1] : left[2];
+      if (r16 >= found) row = 32 * q + __builtin_ctz(word);
+      ++found;
+      if (q == 0) left[0] &= left[0] - 1u;
+      if (q == 1) left[1] &= left[1] - 1u;
+      if (q == 2) left[2] &= left[2] - 1u;
+    }
+    const int entry = ldc(&uni(p.perm)[row0 + row]);
+    const unsigned char* b = down ? reinterpret_cast<const unsigned char*>(p.h) + static_cast<size_t>(row0 + row) * I * 4
+                                  : reinterpret_cast<const unsigned char*>(p.tokens) + static_cast<size_t>(entry / K) * H * 4;
+    b += g * 16;
+    uint4 aw[EXACT_AHEAD][4], bt[EXACT_AHEAD];
+    f32x4 sum[4];
+    auto load = [&](int u, int q) {
+      bt[u] = ld16(b + static_cast<size_t>(q) * 64);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) aw[u][i] = ld16(op.wbase + op.wblock[i] + static_cast<size_t>(q) * op.wstep + op.woff);
+    };
+    auto multiply = [&](int u) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[i] = mma16<F32>(aw[u][i], bt[u], sum[i]);
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < EXACT_AHEAD; ++u) load(u, u);
+    int q0 = 0;
+#pragma unroll 1
+    for (; q0 + EXACT_AHEAD <= n; q0 += EXACT_AHEAD) {
+#pragma unroll
+      for (int u = 0; u < EXACT_AHEAD; ++u) {
+        multiply(u);
+        load(u, min(q0 + u + EXACT_AHEAD, n - 1));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < EXACT_AHEAD - 1; ++u)
+      if (q0 + u < n) multiply(u);
+    fence_release();  // what the task has written here is overwritten
+    if (r16 < found) {
+      if (!down) {
+        float* h = reinterpret_cast<float*>(p.h) + static_cast<size_t>(row0 + row) * I + 32 * w0 + 4 * g;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          unsigned hv[4];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) hv[v] = __float_as_uint(silu_mul(sum[i][v], sum[2 + i][v]));
+          st16_through(h + 16 * i, make_uint4(hv[0], hv[1], hv[2], hv[3]));
+        }
+      } else {
+        const float w = ldc(&uni(p.row_w)[row0 + row]);
+        float* y = p.y + static_cast<size_t>(entry) * H + 64 * w0 + 4 * g;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          st16_through(y + 16 * i, make_uint4(__float_as_uint(sum[i][0] * w), __float_as_uint(sum[i][1] * w),
+                                              __float_as_uint(sum[i][2] * w), __float_as_uint(sum[i][3] * w)));
+      }
+    }
+  }
+}
+
+// Column block `nblk` of a row tile.
 template <bool down>
 __device__ __forceinline__ void float_tile(ParamsRef p, const TileDesc& t, int nblk) {
-  switch (uni((t.rows + 15) >> 4)) {
-    case 1: float_task<1, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
-    case 2: float_task<2, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
-    case 3: float_task<3, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
-    case 4: float_task<4, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
-    case 5: float_task<5, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
-    default: float_task<6, down>(p, t.expert, t.row0, t.rows, t.shared, nblk); break;
+  const int expert = uni(t.expert), row0 = uni(t.row0), rows = uni(t.rows), shared = uni(t.shared);
+  RowSet again;
+  switch ((rows + 15) >> 4) {
+    case 1: again = float_task<1, down>(p, expert, row0, rows, shared, nblk); break;
+    case 2: again = float_task<2, down>(p, expert, row0, rows, shared, nblk); break;
+    case 3: again = float_task<3, down>(p, expert, row0, rows, shared, nblk); break;
+    case 4: again = float_task<4, down>(p, expert, row0, rows, shared, nblk); break;
+    case 5: again = float_task<5, down>(p, expert, row0, rows, shared, nblk); break;
+    default: again = float_task<6, down>(p, expert, row0, rows, shared, nblk); break;
   }
+  if (uni(static_cast<int>(again.any())) != 0) float_exact_rows<down>(p, expert, row0, nblk, again);
 }
 
 // ---------------------------------------------------------------- worker loop

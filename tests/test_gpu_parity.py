@@ -341,6 +341,19 @@ def test_tiled_float32(rows, H, I):
         case.close()
 
 
+def same_values(want, got, scale=None):
+    """The same infinities and NaN, and finite values within the tolerance of float32 layers, each against
+    the root mean square of its own token row (or of `scale`, a part of its columns)."""
+    assert torch.equal(torch.isnan(want), torch.isnan(got))
+    assert torch.equal(torch.isposinf(want), torch.isposinf(got)) and torch.equal(torch.isneginf(want), torch.isneginf(got))
+    fin = torch.isfinite(want)
+    w, g = torch.where(fin, want, 0.0).double(), torch.where(fin, got, 0.0).double()
+    part = slice(None) if scale is None else scale
+    rms = (w[:, part].pow(2).sum(1, keepdim=True) / fin[:, part].sum(1, keepdim=True).clamp(min=1)).sqrt()
+    worst = ((w - g).abs() - 2e-5 * w.abs() - 2e-5 * rms)[:, part]
+    assert float(worst.max()) <= 0.0
+
+
 def test_tiled_float32_values_without_bf16_parts():
     """Infinities, NaN, values that round to infinity in bf16 and tiny ones among the expert weights: the
     float32 tiled kernel gives what the streaming kernel's float32 instructions give, element by element:
@@ -369,6 +382,63 @@ def test_tiled_float32_values_without_bf16_parts():
     finally:
         case.close()
         ref.close()
+
+
+@pytest.mark.parametrize("T,k,H,I,every", [(40, 1, 128, 128, 0), (97, 2, 192, 160, 0), (200, 2, 320, 224, 0),
+                                           (290, 1, 448, 288, 0), (97, 3, 192, 160, 5), (290, 3, 320, 224, 3), (96, 3, 128, 128, 1)])
+def test_tiled_float32_infinite_tokens(T, k, H, I, every):
+    """Tokens that hold infinities or values beyond bf16, in the first, a middle and the last row of tiles of
+    one to six row blocks, a few of a tile or (`every`) more than the 16 rows that are multiplied again
+    together: the gate/up rows and the outputs of the streaming kernel, those of the tokens beside them included."""
+    cfg = synth.MoeConfig("tiled_f32", T, H, 3, k, I, "f32")
+    print("tiled float32, infinite tokens", T, k, H, I, every, flush=True)
+    inp = synth.make_inputs_torch(cfg, T, torch.device("cuda:0"))
+    x = inp["tokens"]
+    x[0, 5], x[T // 2, H - 1], x[T - 1, 64] = float("inf"), -float("inf"), 3.4e38
+    if every:
+        x[::every, 9] = float("inf")
+    ref = GpuCase(cfg, seed=T, sched=_lib.SCHED_STREAM, inputs=inp)
+    case = GpuCase(cfg, seed=T, sched=_lib.SCHED_TILED, inputs=inp)
+    try:
+        want, got = ref.run(), case.run()
+        same_values(want, got)
+        rows = int(ref.launcher.routing(T)["counts"].sum())  # (no expert is chosen for a logit of minus infinity)
+        h = [torch.from_numpy(np.array(c.launcher.intermediate(T)))[:rows] for c in (ref, case)]
+        assert not torch.isfinite(h[0]).all()
+        same_values(*h)
+    finally:
+        case.close()
+        ref.close()
+
+
+def test_tiled_float32_infinite_tokens_hold_up_no_one_else():
+    """One infinite token sends a row block of each of its experts through the float32 instructions again, a
+    wave on its own. The launch may take 1.5 times as long for that."""
+    cfg = synth.MoeConfig("tiled_f32", 320, 2048, 16, 2, 768, "f32")
+    case = GpuCase(cfg, seed=3, sched=_lib.SCHED_TILED)
+    try:
+        x, out = case.inp["tokens"], torch.empty_like(case.inp["tokens"])
+
+        def us():
+            times = []
+            for _ in range(25):
+                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                a.record()
+                case.launcher.launch(x, out)
+                b.record()
+                b.synchronize()
+                times.append(a.elapsed_time(b) * 1e3)
+            return sorted(times)[12]
+
+        us()
+        plain = us()
+        x[100, 5] = float("inf")
+        poisoned = us()
+        print("  %.0f us, with an infinite token %.0f" % (plain, poisoned), flush=True)
+        assert not torch.isfinite(out[100]).any() and torch.isfinite(out[:100]).all()
+        assert poisoned <= 1.5 * plain
+    finally:
+        case.close()
 
 
 @pytest.mark.parametrize("E,k,last", [(128, 4, 256), (96, 4, 336), (64, 2, 512)])
