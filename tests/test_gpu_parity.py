@@ -358,7 +358,7 @@ def test_tiled_float32_values_without_bf16_parts():
     """Infinities, NaN, values that round to infinity in bf16 and tiny ones among the expert weights: the
     float32 tiled kernel gives what the streaming kernel's float32 instructions give, element by element:
     the same infinities and NaN, and finite values within the tolerance of float32 layers."""
-    cfg = synth.MoeConfig("tiled_f32", 150, 256, 4, 2, 160, "f32")
+    cfg = synth.MoeConfig("tiled_f32", 300, 256, 8, 2, 160, "f32")
     dev = torch.device("cuda:0")
     inp = synth.make_inputs_torch(cfg, 5, dev)
     f1, f2 = inp["ffn1"], inp["ffn2"]
@@ -368,17 +368,36 @@ def test_tiled_float32_values_without_bf16_parts():
     f1[2, 11, 0] = 3.4e38
     f1[2, cfg.I + 11, 1] = 1e-38
     f2[2, 17, 3] = float("inf")
-    f2[3, 20:40] *= 1e-30
     ref = GpuCase(cfg, seed=5, sched=_lib.SCHED_STREAM, inputs=inp)
     case = GpuCase(cfg, seed=5, sched=_lib.SCHED_TILED, inputs=inp)
     try:
         want, got = ref.run(), case.run()
         assert torch.isnan(want).any() and torch.isinf(want).any() and torch.isfinite(want).any()
-        assert torch.equal(torch.isnan(want), torch.isnan(got))
-        assert torch.equal(torch.isposinf(want), torch.isposinf(got)) and torch.equal(torch.isneginf(want), torch.isneginf(got))
-        fin = torch.isfinite(want)
-        rms = float(want[fin].double().pow(2).clamp(max=1e30).mean().sqrt())
-        assert float(((want - got).abs()[fin] - 2e-5 * want.abs()[fin]).max()) <= 2e-5 * rms
+        same_values(want, got)
+        # rows that no such weight reaches: a wrong ordinary value shows
+        assert int((torch.isfinite(want).all(1) & (want.abs().amax(1) < 1e3)).sum()) >= 5
+        broken = got + 1e-3 * (got.abs() < 1e3)
+        with pytest.raises(AssertionError):
+            same_values(want, broken)
+    finally:
+        case.close()
+        ref.close()
+
+
+def test_tiled_float32_tiny_weights():
+    """Down rows of 1e-28 and 1e-30 of the usual size, one expert a token, so that nothing larger is added:
+    the low parts of such values are still there (they end at 2^-109)."""
+    cfg = synth.MoeConfig("tiled_f32", 90, 256, 3, 1, 160, "f32")
+    inp = synth.make_inputs_torch(cfg, 6, torch.device("cuda:0"))
+    inp["ffn2"][:, 20:40] *= 1e-28
+    inp["ffn2"][:, 40:120] *= 1e-30
+    ref = GpuCase(cfg, seed=6, sched=_lib.SCHED_STREAM, inputs=inp)
+    case = GpuCase(cfg, seed=6, sched=_lib.SCHED_TILED, inputs=inp)
+    try:
+        want, got = ref.run(), case.run()
+        assert 0.0 < float(want[:, 40:120].abs().max()) < 1e-29
+        for part in (slice(0, 20), slice(20, 40), slice(40, 120), slice(120, 256)):
+            same_values(want, got, part)
     finally:
         case.close()
         ref.close()
