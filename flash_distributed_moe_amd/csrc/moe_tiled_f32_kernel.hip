@@ -10,11 +10,13 @@
 //
 // The products run on the bf16 matrix cores, sixteen times as fast as the float32 ones here. Both
 // operands are split into three bf16 parts, x = hi + mid + lo: each part is the rest rounded to
-// nearest, 8 significant bits each, so the three hold all 24 bits of a float exactly (down to values
-// of 2^-109, whose lowest part is subnormal). Of the nine products of parts the six largest are
-// accumulated in float32: hi*hi, hi*mid, mid*hi, mid*mid, hi*lo, lo*hi; what is left out is below
-// 2^-25 of a product, less than the one rounding of a float32 multiplication. A sum of K products is
-// rounded 6*K/32 times instead of K times. The layer's error against float64, relative 2-norm, float32
+// nearest, 8 significant bits each, so the three hold all 24 bits of a float exactly. Of the nine products
+// of parts the six largest are accumulated in float32: hi*hi, hi*mid, mid*hi, mid*mid, hi*lo, lo*hi. What
+// is left out, mid*lo and lo*mid above all, is below 2^-24 of a product (0.991 * 2^-24 for
+// 1.0038986 squared), about as much as one rounding of a float32 multiplication may be off: a sum that has one
+// product only can be off by 7.5e-8 where a float32 multiplication is by 5.9e-8. A sum of K products is
+// rounded 6*K/32 times instead of K times, which outweighs that from a few products on (K=128: 2.5 times
+// nearer). The layer's error against float64, relative 2-norm, float32
 // matrix instructions (streaming kernel) / this: 30B shape T=256 1.85e-6 / 1.72e-6, T=512 1.84e-6 /
 // 1.71e-6; E=40, k=5, H=1344, I=736 T=900 1.29e-6 / 1.16e-6; E=10, k=3, H=320, I=2016 T=2000 9.4e-7 / 8.2e-7.
 //
@@ -23,8 +25,12 @@
 // TFLOP/s of float32); row-major weights T=1024 1076 / 627; E=32 T=4096 2400 / 1450.
 //
 // A value that is no finite number, or rounds to none in bf16, has no such parts: its products come
-// out as infinities or NaN. A wave whose sums hold one multiplies that token row again with the float32
-// matrix instructions, so such inputs give what they give in the streaming kernel.
+// out as infinities or NaN. One below 2^-102 has parts below the smallest normal bf16 number, which lose
+// bits or vanish (an error below 2^-126): that shows where a whole sum is small. A wave whose sums hold an infinity, a NaN
+// or a value below 2^-64 that is not zero multiplies that token row again with the float32
+// matrix instructions, so such inputs give what they give in the streaming kernel. (Sums of ordinary values do
+// not come that near to zero. In a sum of 2^-64 and more, 2^-126 of a weight is less than a float's last bit
+// as long as a thousand of the token's values are below 2^28.)
 //
 // Weights go straight to registers (no other wave of the workgroup reads them), 16 bytes per lane and
 // load, one 32-k step ahead, and are split there; token rows are split once per workgroup, on
@@ -232,12 +238,14 @@ __device__ __forceinline__ void float_weights(ParamsRef p, int expert, int wblk,
 // y[t*K+slot, n0 .. n0+256) = w * (h[row] . W2[e]^T) (refFullMoe.h:58-65, src/hip/kernel/tasks/ffn2Task.h:37-40),
 // float rows with the gate weight applied, as the streaming kernel leaves them. Both are written
 // through, 64 bytes of a row at a time, from the accumulators. Returns the token rows for which a sum of
-// the wave is no finite number: float_exact_rows writes those again.
+// the wave is no finite number or a small one: float_exact_rows writes those again.
 struct RowSet {
   unsigned word[3];  // a bit a row
   __device__ __forceinline__ unsigned any() const { return word[0] | word[1] | word[2]; }
 };
 static_assert(F_TM <= 96, "rows of a RowSet");
+// twice the bits of 2^-64 and of infinity
+constexpr unsigned SUM_SMALL = ((127u - 64u) << 24) - 1u, SUM_INF = 0xFF000000u;
 template <int JB, bool down>
 __device__ __noinline__ RowSet float_task(ParamsRef pv, int expert_in, int row0_in, int rows_in, int shared_in, int nblk_in) {
   ParamsRef p = uniform_params(pv);
@@ -277,20 +285,28 @@ __device__ __noinline__ RowSet float_task(ParamsRef pv, int expert_in, int row0_
   }
   RowSet again = {{0u, 0u, 0u}};
   if (w0 >= nw) return again;  // this wave's columns do not exist: it has multiplied the last ones that do
-  float t[JB], all = 0.0f;
+  // twice a sum's bits have no sign; less one, zero is the largest of them
+  unsigned least[JB], most[JB], all_least = 0xFFFFFFFFu, all_most = 0u;
 #pragma unroll
   for (int j = 0; j < JB; ++j) {
-    t[j] = 0.0f;
+    least[j] = 0xFFFFFFFFu;
+    most[j] = 0u;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) t[j] = __builtin_fmaf(acc[i][j][v], 0.0f, t[j]);
-    all += t[j];
+      for (int v = 0; v < 4; ++v) {
+        const unsigned twice = __float_as_uint(acc[i][j][v]) << 1;
+        least[j] = min(least[j], twice - 1u);
+        most[j] = max(most[j], twice);
+      }
+    all_least = min(all_least, least[j]);
+    all_most = max(all_most, most[j]);
   }
-  if (__any(all != 0.0f)) {
+  if (__any(all_least < SUM_SMALL || all_most >= SUM_INF)) {
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
-      const unsigned long long b = __ballot(t[j] != 0.0f && 16 * j + r16 < rows);  // a row's lanes stand 16 apart
+      const unsigned long long b =
+          __ballot((least[j] < SUM_SMALL || most[j] >= SUM_INF) && 16 * j + r16 < rows);  // a row's lanes stand 16 apart
       const unsigned both = static_cast<unsigned>(b) | static_cast<unsigned>(b >> 32);
       again.word[j >> 1] |= ((both | both >> 16) & 0xFFFFu) << (16 * (j & 1));
     }

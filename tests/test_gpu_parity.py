@@ -385,19 +385,31 @@ def test_tiled_float32_values_without_bf16_parts():
 
 
 def test_tiled_float32_tiny_weights():
-    """Down rows of 1e-28 and 1e-30 of the usual size, one expert a token, so that nothing larger is added:
-    the low parts of such values are still there (they end at 2^-109)."""
+    """Down rows of 1e-28 to 1e-36 of the usual size, one expert a token, so that nothing larger is added: the
+    streaming kernel's values, also where the low parts of such weights are beyond bf16. The same for up rows,
+    and zeros among them stay zeros."""
     cfg = synth.MoeConfig("tiled_f32", 90, 256, 3, 1, 160, "f32")
     inp = synth.make_inputs_torch(cfg, 6, torch.device("cuda:0"))
     inp["ffn2"][:, 20:40] *= 1e-28
     inp["ffn2"][:, 40:120] *= 1e-30
+    inp["ffn2"][:, 128:160] *= 1e-33
+    inp["ffn2"][:, 160:200] *= 1e-35
+    inp["ffn2"][:, 200:210] = 0.0
+    inp["ffn2"][:, 210:220] *= 1e-36
+    inp["ffn1"][:, cfg.I + 40:cfg.I + 60] *= 1e-35
     ref = GpuCase(cfg, seed=6, sched=_lib.SCHED_STREAM, inputs=inp)
     case = GpuCase(cfg, seed=6, sched=_lib.SCHED_TILED, inputs=inp)
     try:
         want, got = ref.run(), case.run()
-        assert 0.0 < float(want[:, 40:120].abs().max()) < 1e-29
-        for part in (slice(0, 20), slice(20, 40), slice(40, 120), slice(120, 256)):
-            same_values(want, got, part)
+        assert 0.0 < float(want[:, 40:120].abs().max()) < 1e-29 and 0.0 < float(want[:, 210:220].abs().max()) < 1e-35
+        assert not got[:, 200:210].any()
+        for part in ((0, 20), (20, 40), (40, 120), (120, 128), (128, 160), (160, 200), (210, 220), (220, 256)):
+            print("  columns", part, flush=True)
+            same_values(want, got, slice(*part))
+        rows = int(ref.launcher.routing(cfg.T)["counts"].sum())
+        h = [torch.from_numpy(np.array(c.launcher.intermediate(cfg.T)))[:rows] for c in (ref, case)]
+        same_values(*h, slice(0, 40))
+        same_values(*h, slice(40, 60))
     finally:
         case.close()
         ref.close()
