@@ -219,9 +219,12 @@ int dot_tasks_of(const FlashMoeLayerDesc& d, int tokens_num) {
 // either projection; tables that fit the kernel's LDS; 4 KiB of router weights (where the
 // loads go that nobody needs); h rows that 31 bits address; no trace. float32: any H from 128 on (its logit
 // chains take 8 tokens x 8 experts a wave: four waves of half of the workgroups at most), one block, up to
-// where the tiled variant takes over (figures in the kernel's file); but row-major rows of whole 16 KiB with
-// two rows an expert and more stay with the streaming kernel (us, streaming / split-k, H=4096: E=128, k=8,
-// I=768 T=32 774 / 820, T=128 985 / 994; E=64, k=4, I=512 T=16 294 / 262, T=32 326 / 334). bf16: one block up to 9 rows an expert on
+// where the tiled variant takes over (figures in the kernel's file); but row-major gate/up rows of whole 16 KiB
+// stay with the streaming kernel from two rows an expert on, and from one where a workgroup has ten gate/up tasks
+// and more (us, streaming / split-k, H=4096: E=128, k=8, I=768 T=8 411 / 404, T=16 607 / 621, T=24 784 / 801, T=32
+// 796 / 834, T=128 959 / 969; E=64, k=4, I=512 T=16 302 / 247, T=24 302 / 302, T=32 312 / 321, T=64 368 / 356; E=16, k=2,
+// I=4096 T=8 552 / 494, T=16 626 / 653, T=64 689 / 680). The pitch of the down rows does not decide (H=2048,
+// I=4096, E=32, k=4 T=16 676 / 560, T=64 777 / 629; H=1024, I=8192, E=16, k=2 T=16 467 / 270). bf16: one block up to 9 rows an expert on
 // average, two up to 24 (us, streaming kernel / one / two blocks, 30B shape: T=96 235 / 221 / 222,
 // T=144 260 / 230 / 229, T=160 252 / 228 / 225, T=200 266 / 253 / 234, T=256 275 / 301 / 241; 235B
 // shape: T=128 808 / 791 / 791, T=160 816 / 805 / 799, T=200 855 / 904 / 812, T=256 876 / 1124 / 836;
@@ -236,7 +239,8 @@ int split_row_blocks(const FlashMoeLayerDesc& d, int tokens_num, const Machine& 
     return d.hidden >= 128 && slots < static_cast<long long>(kAutoTiledRowsF32) * d.experts &&
                    dot_tasks_of(d, tokens_num) <= 4 * (m.n_groups / 2) &&
                    ((d.flags & (FLASH_MOE_FLAG_PACK_WEIGHTS | FLASH_MOE_FLAG_WEIGHTS_PREPACKED)) != 0 ||
-                    d.hidden % 4096 != 0 || slots < 2ll * d.experts)
+                    d.hidden % 4096 != 0 || slots < d.experts ||
+                    (slots < 2ll * d.experts && d.experts * (d.intermediate / 32) < 10ll * m.n_groups))
                ? 1
                : 0;
   if (d.hidden % fmoe::DOT16_KC != 0 || slots > 24ll * d.experts || dot16_tasks_of(d, tokens_num) > m.n_groups / 2)

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from flash_distributed_moe_amd import _lib, synth
+from flash_distributed_moe_amd.flashMoeLauncher import MoeKernelLauncher
 from tests.moe_case import GpuCase
 
 pytestmark = pytest.mark.gpu
@@ -470,6 +471,27 @@ def test_tiled_float32_infinite_tokens_hold_up_no_one_else():
         assert poisoned <= 1.5 * plain
     finally:
         case.close()
+
+
+@pytest.mark.parametrize("E,k,H,I,split,stream", [
+    (128, 8, 4096, 640, (1, 8, 15), (16, 24, 32, 128)),   # 2560 gate/up tasks for 256 CUs
+    (128, 8, 4096, 608, (1, 16, 31), (32, 64)),           # 2432
+    (16, 2, 4096, 4096, (1, 8, 15), (16, 64)),
+    (128, 8, 4032, 640, (1, 16, 32, 128), ()),            # rows of another pitch
+])
+def test_row_major_float32_rows_of_16_kib(E, k, H, I, split, stream):
+    """Row-major float32 layers whose gate/up rows are whole 16 KiB leave the split-k kernel to smaller batches:
+    from two rows an expert on, and from one where a workgroup has ten tasks. Packed ones do not."""
+    dev = torch.device("cuda:0")
+    w = [torch.empty(s, dtype=torch.float32, device=dev) for s in ((E, H), (E, 2 * I, H), (E, H, I))]  # never read
+    for packed in (False, True):
+        l = MoeKernelLauncher()
+        l.create(*w, 256, l.getDistributedUniqueId(True), 0, 1, top_k=k, pack_weights=False, prepacked=packed)
+        try:
+            assert [l.split_blocks_for(t) for t in split] == [1] * len(split)
+            assert [l.split_blocks_for(t) for t in stream] == [int(packed)] * len(stream)
+        finally:
+            l.destroy()
 
 
 @pytest.mark.parametrize("E,k,last", [(128, 4, 256), (96, 4, 336), (64, 2, 512)])
