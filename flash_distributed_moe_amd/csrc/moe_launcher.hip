@@ -253,7 +253,6 @@ int sched_for(const FlashMoeLayerDesc& d, int tokens_num, const Machine& m) {
   if (!tiled_eligible(d, tokens_num)) return FLASH_MOE_SCHED_STREAM;
   const long long rows = static_cast<long long>(tokens_num) * d.top_k;
   if (d.dtype == FLASH_MOE_F32) {
-    if (m.traced) return FLASH_MOE_SCHED_STREAM;  // the float32 tiled kernel writes no task records
     if (d.sched == FLASH_MOE_SCHED_TILED) return FLASH_MOE_SCHED_TILED;
     return rows >= static_cast<long long>(kAutoTiledRowsF32) * d.experts ? FLASH_MOE_SCHED_TILED : FLASH_MOE_SCHED_STREAM;
   }
@@ -369,9 +368,9 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   // without / with: T=450 300 / 282, T=600 302 / 285, T=900 312 / 299, T=1500 330 / 325, T=2048 353 / 356;
   // E=256, H=1024, I=512, T=1024 242 / 231; E=16, k=2, H=320, I=160, T=4000 74 / 78). 2: router tasks of 16
   // or 32 tokens x all experts. Both without a scan phase, while the mask words fit LDS (as 2 against 0:
-  // T=2048 345 / 340, row-major 359 / 355; E=16 T=4000 74 / 70). 0: tickets for all of it; so with a trace.
+  // T=2048 345 / 340, row-major 359 / 355; E=16 T=4000 74 / 70). 0: tickets for all of it.
   if (tiled && d.dtype == FLASH_MOE_BF16) {
-    p.dot16 = d.experts * ((T + 63) / 64) > fmoe::SHORT_MASK_WORDS || T > 65535 || m.traced ? 0
+    p.dot16 = d.experts * ((T + 63) / 64) > fmoe::SHORT_MASK_WORDS || T > 65535 ? 0
               : T <= 6 * m.n_groups && ((T + 15) / 16) * ((d.experts + 31) / 32) <= 2 * m.n_groups ? 1
                                                                                                   : 2;
     p.early = p.dot16;  // (the last selection raises FLAG_ROUTED)

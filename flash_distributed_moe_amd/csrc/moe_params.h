@@ -80,8 +80,8 @@ struct TileDesc {  // one row tile: `rows` consecutive permuted rows of one expe
 // One record per executed task when tracing is on (times: 100 MHz wall clock).
 struct TraceRec {
   unsigned ticket;
-  unsigned kind;    // 0 router dot, 1 scan, 2 scatter, 3 gate/up, 4 down, 5 combine, 6 select
-  unsigned worker;  // workgroup * waves_per_group + wave
+  unsigned kind;    // 0 router dot, 1 scan, 2 scatter, 3 gate/up, 4 down, 5 combine, 6 select or expert scan
+  unsigned worker;  // streaming variant: workgroup * waves_per_group + wave; tiled one: workgroup
   unsigned aux;     // task-specific (row tile, token ...)
   long long t_fetch;  // before the ticket was drawn
   long long t_ready;  // dependencies satisfied, work starts

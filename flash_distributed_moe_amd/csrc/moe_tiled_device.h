@@ -69,6 +69,22 @@ __device__ __forceinline__ bool wg_wait_flag(ParamsRef p, int which, WgShared* s
   return ok;
 }
 
+// A task's record, written by the lanes where `writes` holds: one, and only while tracing is on.
+__device__ __forceinline__ void trace_task(ParamsRef p, bool writes, unsigned id, unsigned kind, unsigned aux,
+                                           long long t_fetch, long long t_ready) {
+  if (writes && id < p.trace_cap) {
+    const long long t_end = wall_clock64();
+    TraceRec* r = p.trace + id;
+    st16(r, u32x4{id, kind, blockIdx.x, aux});
+    st16(reinterpret_cast<char*>(r) + 16,
+         u32x4{static_cast<unsigned>(t_fetch), static_cast<unsigned>(t_fetch >> 32),
+               static_cast<unsigned>(t_ready), static_cast<unsigned>(t_ready >> 32)});
+    st16(reinterpret_cast<char*>(r) + 32,
+         u32x4{static_cast<unsigned>(t_end), static_cast<unsigned>(t_end >> 32), 0u, 0u});
+  }
+}
+__device__ __forceinline__ long long trace_clock(bool traced) { return traced ? wall_clock64() : 0; }
+
 // All threads' stores have completed, then one thread bumps the counter. Tile
 // data (h, y) is written through to device-coherent memory, so completion is
 // all a reader on another XCD needs (WRITEBACK adds an agent-scope release for

@@ -453,6 +453,8 @@ __device__ __forceinline__ void float_tile(ParamsRef p, const TileDesc& t, int n
 // Routing, scan and scatter tasks are handed out statically: every workgroup of the launch is
 // resident (two a CU; the launcher asks). The GEMM tasks come from one queue per XCD, as in the bf16
 // tiled kernel; the other workgroup of the CU covers what a task waits for at its ends.
+// traced: with task records (asked at run time: T=1024 on the 30B shape 577.2 -> 580.2 us)
+template <bool traced>
 __global__ __launch_bounds__(T_THREADS, 2) __attribute__((disable_tail_calls)) void moe_tiled_f32_kernel(
     const Params params) {
   ParamsRef p = kernel_params();
@@ -471,34 +473,51 @@ __global__ __launch_bounds__(T_THREADS, 2) __attribute__((disable_tail_calls)) v
 
   const int n_eg = (E + ROUTER_EXP - 1) / ROUTER_EXP;
   const int n_dot = (T + ROUTER_TOK - 1) / ROUTER_TOK * n_eg;
-  for (int i = me; i < n_dot; i += waves) router_dot_task<F32>(p, i / n_eg, i % n_eg);
-  for (int t = me; t < T; t += waves) {
-    if (!wave_wait_ge(&p.tok_arrive[t], static_cast<unsigned>(n_eg), ctl, p.spin_limit)) break;
-    router_select_task(p, t);
+  const bool lane0 = traced && lane_id() == 0, thread0 = traced && threadIdx.x == 0;
+  for (int i = me; i < n_dot; i += waves) {
+    const long long t0 = trace_clock(traced);
+    router_dot_task<F32>(p, i / n_eg, i % n_eg);
+    trace_task(p, lane0, i, 0, i, t0, t0);
   }
+  for (int t = me; t < T; t += waves) {
+    const long long t0 = trace_clock(traced);
+    if (!wave_wait_ge(&p.tok_arrive[t], static_cast<unsigned>(n_eg), ctl, p.spin_limit)) break;
+    const long long t1 = trace_clock(traced);
+    router_select_task(p, t);
+    trace_task(p, lane0, n_dot + t, 6, t, t0, t1);
+  }
+  long long t_fetch = trace_clock(traced);
   bool ok = wg_wait_flag(p, FLAG_ROUTED, &sh);
   const int n_es = (E + SCAN_EXPERTS - 1) / SCAN_EXPERTS;
+  const unsigned t_scan0 = static_cast<unsigned>(n_dot + T), t_scatter0 = t_scan0 + n_es;
   if (ok && b < n_es) {
+    const long long t_ready = trace_clock(traced);
     tiled_expert_scan_task(p, b);
     if (wg_arrive<false>(&ctl->scan_done.v, &sh) == static_cast<unsigned>(n_es) - 1u) tiled_scan_task<F_TM, 16>(p);
+    trace_task(p, thread0, t_scan0 + b, 1, b, t_fetch, t_ready);
   }
+  t_fetch = trace_clock(traced);
   if (ok) ok = wg_wait_flag(p, FLAG_SCAN, &sh);
   const int n_sc = (T + RT_TOK - 1) / RT_TOK;
   for (int i = b; ok && i < n_sc; i += G) {
+    const long long t_ready = trace_clock(traced);
     tiled_scatter_task(p, i);
     if (wg_arrive<false>(&ctl->perm_done.v, &sh) == static_cast<unsigned>(n_sc) - 1u) wg_broadcast_flag(p, FLAG_PERM);
+    trace_task(p, thread0, t_scatter0 + i, 2, i, t_fetch, t_ready);
   }
   if (ok) ok = wg_wait_flag(p, FLAG_PERM, &sh);
 
   const unsigned nm = ok ? ldc(&ctl->n_mtiles.v) : 0u;
   const unsigned nt1 = static_cast<unsigned>((p.I + 127) / 128), nt2 = static_cast<unsigned>((p.H + 255) / 256);
   const unsigned n2_total = nm * nt2;
+  const unsigned t_dyn0 = t_scatter0 + n_sc;
   const int home = xcc_id();
   for (int hop = 0; ok && hop < 8; ++hop) {
     const unsigned q = static_cast<unsigned>((home + hop) & 7);
     const unsigned lo = nm * q / 8u, hi = nm * (q + 1u) / 8u;
     const unsigned q1 = (hi - lo) * nt1, q2 = (hi - lo) * nt2;
     while (ok) {
+      t_fetch = trace_clock(traced);
       if (threadIdx.x == 0) sh.ticket = add_relaxed(&ctl->xq[q].v, 1u);
       __syncthreads();
       const unsigned j = uni(static_cast<int>(sh.ticket));
@@ -506,24 +525,30 @@ __global__ __launch_bounds__(T_THREADS, 2) __attribute__((disable_tail_calls)) v
       if (j >= q1 + q2) break;
       if (j < q1) {
         const unsigned m = lo + j / nt1;
+        const long long t_ready = trace_clock(traced);
         const TileDesc tile = ld_tile(&p.mtiles[m]);
         float_tile<false>(p, tile, static_cast<int>(j % nt1));
         wg_arrive<false>(&p.g1_done[m].v, &sh);
+        trace_task(p, thread0, t_dyn0 + lo * nt1 + j, 3, m, t_fetch, t_ready);
       } else {
         const unsigned jj = j - q1, m = lo + jj / nt2;
         const TileDesc tile = ld_tile(&p.mtiles[m]);
         ok = wg_wait_ge(p, &p.g1_done[m].v, nt1, &sh);
         if (ok) {
+          const long long t_ready = trace_clock(traced);
           float_tile<true>(p, tile, static_cast<int>(jj % nt2));
           if (wg_arrive<false>(&ctl->g2_done.v, &sh) == n2_total - 1u) wg_broadcast_flag(p, FLAG_G2);
+          trace_task(p, thread0, t_dyn0 + nm * nt1 + lo * nt2 + jj, 4, m, t_fetch, t_ready);
         }
       }
     }
   }
+  t_fetch = trace_clock(traced);
   if (ok && n2_total != 0u) ok = wg_wait_flag(p, FLAG_G2, &sh);
   if (ok) {
     const unsigned ncomb = static_cast<unsigned>((p.H + COMBINE_COLS - 1) / COMBINE_COLS);
-    combine_items<F32>(p, static_cast<unsigned>(me), static_cast<unsigned>(T) * ncomb, ncomb, static_cast<unsigned>(me), 0u, 0);
+    combine_items<F32>(p, static_cast<unsigned>(me), static_cast<unsigned>(T) * ncomb, ncomb, blockIdx.x,
+                       t_dyn0 + nm * (nt1 + nt2), t_fetch);
   }
 
   // The last workgroup out returns every counter to zero for the next launch.
@@ -554,18 +579,34 @@ __global__ __launch_bounds__(T_THREADS, 2) __attribute__((disable_tail_calls)) v
   }
 }
 
+namespace {
+const auto kPlain = moe_tiled_f32_kernel<false>, kTraced = moe_tiled_f32_kernel<true>;
+}  // namespace
+
 hipError_t launch_tiled_f32_kernel(const Params& p, int grid, hipStream_t stream) {
-  hipLaunchKernelGGL(moe_tiled_f32_kernel, dim3(grid), dim3(T_THREADS), F_LDS_BYTES, stream, p);
+  hipLaunchKernelGGL(p.trace ? kTraced : kPlain, dim3(grid), dim3(T_THREADS), F_LDS_BYTES, stream, p);
   return hipGetLastError();
 }
 
 hipError_t prepare_tiled_f32_kernel() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(moe_tiled_f32_kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, F_LDS_BYTES);
+  for (auto kernel : {kPlain, kTraced}) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, F_LDS_BYTES);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
+// the lesser of the two kernels' numbers of workgroups a CU holds
 hipError_t tiled_f32_kernel_occupancy(int* per_cu) {
-  return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, moe_tiled_f32_kernel, T_THREADS, F_LDS_BYTES);
+  *per_cu = 0x7FFFFFFF;
+  for (auto kernel : {kPlain, kTraced}) {
+    int n = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, T_THREADS, F_LDS_BYTES);
+    if (e != hipSuccess) return e;
+    if (n < *per_cu) *per_cu = n;
+  }
+  return hipSuccess;
 }
 
 }  // namespace fmoe

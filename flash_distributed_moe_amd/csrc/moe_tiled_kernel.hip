@@ -1554,8 +1554,10 @@ __device__ __noinline__ void tiled_combine_task(ParamsRef pv, int blk, int tok_i
 // The launch parameters are read in place and the task calls keep the local
 // calling convention, as in the streaming variant (see its worker loop).
 // RAGGED: see tile_task. ODD: I is an odd number of 32-k steps, which only ragged layers have (kernels of
-// their own: as a branch of this one the odd steps cost every task of the others half a microsecond).
-template <bool RAGGED, bool ODD>
+// their own: as a branch of this one the odd steps cost every task of the others half a microsecond). TRACED:
+// with task records (kernels of their own: asking at run time costs the others, 30B shape, us, with / without
+// the question: T=600 283.5 / 278.8, T=2048 row-major 367.3 / 359.5, T=8192 766.9 / 762.5).
+template <bool RAGGED, bool ODD, bool TRACED>
 __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void moe_tiled_kernel(
     const Params params) {
   ParamsRef p = kernel_params();
@@ -1578,7 +1580,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
   const unsigned t_escan0 = n_rt;
   const unsigned t_scan = n_rt + n_es;
   const unsigned t_scatter0 = t_scan + 1u;
-  const unsigned t_dyn0 = t_scatter0 + n_sc;
+  unsigned t_dyn0 = t_scatter0 + n_sc;
   const unsigned nt1 = static_cast<unsigned>((p.I + G1_COLS - 1) / G1_COLS);
   const unsigned nt2 = static_cast<unsigned>((p.H + TN - 1) / TN);
   // as few tokens to a combine task as one round of tasks allows (8 tokens always, us, 30B shape: T=600
@@ -1591,48 +1593,57 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
   const int home = xcc_id();
   bool first = true, ok = true;
 
+  constexpr bool traced = TRACED;
   auto trace = [&](unsigned id, unsigned kind, unsigned aux, long long t_fetch, long long t_ready) {
-    if (p.trace && threadIdx.x == 0 && id < p.trace_cap) {
-      const long long t_end = wall_clock64();
-      TraceRec* r = p.trace + id;
-      st16(r, u32x4{id, kind, blockIdx.x, aux});
-      st16(reinterpret_cast<char*>(r) + 16,
-           u32x4{static_cast<unsigned>(t_fetch), static_cast<unsigned>(t_fetch >> 32),
-                 static_cast<unsigned>(t_ready), static_cast<unsigned>(t_ready >> 32)});
-      st16(reinterpret_cast<char*>(r) + 32,
-           u32x4{static_cast<unsigned>(t_end), static_cast<unsigned>(t_end >> 32), 0u, 0u});
-    }
+    trace_task(p, traced && threadIdx.x == 0, id, kind, aux, t_fetch, t_ready);
   };
 
   // ---- prologue, few tokens: handed out statically (every workgroup of the launch is resident)
   if (p.dot16) {
     const int G = static_cast<int>(n_groups), b = static_cast<int>(blockIdx.x), wave = uni(static_cast<int>(threadIdx.x >> 6));
     const int Ti = static_cast<int>(T), n_eg = (p.E + 31) >> 5, n_dot = ((Ti + 15) >> 4) * n_eg;
+    // (records: router tasks, one for the selections of each wave, scatter tasks)
+    unsigned t_perm0 = n_rt;
     if (p.dot16 == 1) {
-      for (int i = b; i < n_dot; i += G) router_dot32_task(p, i / n_eg, i % n_eg);
+      for (int i = b; i < n_dot; i += G) {
+        const long long t0 = trace_clock(traced);
+        router_dot32_task(p, i / n_eg, i % n_eg);
+        trace(i, 0, i, t0, t0);
+      }
       const int sel_groups = min(n_dot, G);
-      // (a wait that fails has raised an error bit, which every later wait sees)
-      if (b < sel_groups) (void)select_tokens_task(p, b + sel_groups * wave, WAVES * sel_groups);
+      const int t = b + sel_groups * wave;
+      if (b < sel_groups && t < Ti) {
+        const long long t0 = trace_clock(traced);
+        // (a wait that fails has raised an error bit, which every later wait sees)
+        if (select_tokens_task(p, t, WAVES * sel_groups)) trace_task(p, traced && lane_id() == 0, n_dot + t, 6, t, t0, t0);
+      }
+      t_perm0 = n_dot + WAVES * sel_groups;
     } else {
       for (int i = b; i < static_cast<int>(n_rt); i += G) {
+        const long long t0 = trace_clock(traced);
         if (rt2) {
           tiled_router_task<2>(p, i);
         } else {
           tiled_router_task<1>(p, i);
         }
         if (wg_arrive<false>(&ctl->router_done.v, &sh) == n_rt - 1u) wg_broadcast_flag(p, FLAG_ROUTED);
+        trace(i, 0, i, t0, t0);
       }
     }
     const int n_perm = (Ti * p.K + T_THREADS - 1) / T_THREADS;
+    t_dyn0 = t_perm0 + n_perm;
+    const long long t_fetch = trace_clock(traced);
     if (b < n_perm) ok = wg_wait_flag(p, FLAG_ROUTED, &sh);
     for (int i = b; ok && i < n_perm; i += G) {
+      const long long t_ready = trace_clock(traced);
       short_scatter_task<RAGGED>(p, i);
       if (wg_arrive<false>(&ctl->perm_done.v, &sh) == static_cast<unsigned>(n_perm) - 1u) wg_broadcast_flag(p, FLAG_PERM);
+      trace(t_perm0 + i, 2, i, i == b ? t_fetch : t_ready, t_ready);
     }
   }
   // ---- prologue otherwise: router, scan, scatter from the global counter
   while (ok && !p.dot16) {
-    const long long t_fetch = p.trace ? wall_clock64() : 0;
+    const long long t_fetch = trace_clock(traced);
     if (threadIdx.x == 0) sh.ticket = first ? blockIdx.x : n_groups + add_relaxed(&ctl->ticket.v, 1u);
     first = false;
     __syncthreads();
@@ -1641,7 +1652,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
     if (tk >= t_dyn0) break;
     long long t_ready = 0;
     if (tk < n_rt) {
-      if (p.trace) t_ready = wall_clock64();
+      if (traced) t_ready = wall_clock64();
       if (rt2) {
         tiled_router_task<2>(p, static_cast<int>(tk));
       } else {
@@ -1652,7 +1663,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
     } else if (tk < t_scan) {
       ok = wg_wait_ge(p, &ctl->router_done.v, n_rt, &sh);
       if (ok) {
-        if (p.trace) t_ready = wall_clock64();
+        if (traced) t_ready = wall_clock64();
         tiled_expert_scan_task(p, static_cast<int>(tk - t_escan0));
         wg_arrive<false>(&ctl->scan_done.v, &sh);
         trace(tk, 6, tk - t_escan0, t_fetch, t_ready);
@@ -1660,14 +1671,14 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
     } else if (tk == t_scan) {
       ok = wg_wait_ge(p, &ctl->scan_done.v, n_es, &sh);
       if (ok) {
-        if (p.trace) t_ready = wall_clock64();
+        if (traced) t_ready = wall_clock64();
         tiled_scan_task<TM_MAX, 32>(p);
         trace(tk, 1, 0, t_fetch, t_ready);
       }
     } else {
       ok = wg_wait_flag(p, FLAG_SCAN, &sh);
       if (ok) {
-        if (p.trace) t_ready = wall_clock64();
+        if (traced) t_ready = wall_clock64();
         tiled_scatter_task(p, static_cast<int>(tk - t_scatter0));
         if (wg_arrive<false>(&ctl->perm_done.v, &sh) == n_sc - 1u) wg_broadcast_flag(p, FLAG_PERM);
         trace(tk, 2, tk - t_scatter0, t_fetch, t_ready);
@@ -1708,12 +1719,12 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
       }
     };
     while (ok) {
-      const long long t_fetch = p.trace ? wall_clock64() : 0;
+      const long long t_fetch = trace_clock(traced);
       if (j >= q1 + q2) break;
       long long t_ready = 0;
       if (j < q1) {
         const unsigned m = lo + j / nt1;
-        if (p.trace) t_ready = wall_clock64();
+        if (traced) t_ready = wall_clock64();
         const TileDesc tile = ld_tile(&p.mtiles[m]);
         if constexpr (RAGGED) {
           tiled_ragged_gate_up_task(p, tile, static_cast<int>(j % nt1), pend, &ctl->xq[q].v);
@@ -1736,7 +1747,7 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
         }
         ok = wg_wait_ge(p, &p.g1_done[m].v, nt1, &sh);
         if (ok) {
-          if (p.trace) t_ready = wall_clock64();
+          if (traced) t_ready = wall_clock64();
           if constexpr (ODD) {
             tiled_odd_down_task(p, tile, static_cast<int>(jj % nt2), pend, &ctl->xq[q].v);
           } else if constexpr (RAGGED) {
@@ -1759,17 +1770,17 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
     if (ok) {
       const unsigned ncomb = (static_cast<unsigned>(p.H) + COMBINE_COLS - 1u) / COMBINE_COLS;
       const unsigned slot = static_cast<unsigned>(uni(static_cast<int>(threadIdx.x >> 6))) * n_groups + blockIdx.x;
-      combine_items<BF16>(p, slot, T * ncomb, ncomb, blockIdx.x, t_dyn0 + nm * (nt1 + nt2), p.trace ? wall_clock64() : 0);
+      combine_items<BF16>(p, slot, T * ncomb, ncomb, blockIdx.x, t_dyn0 + nm * (nt1 + nt2), trace_clock(traced));
     }
   }
   while (!RAGGED && ok) {
-    const long long t_fetch = p.trace ? wall_clock64() : 0;
+    const long long t_fetch = trace_clock(traced);
     if (threadIdx.x == 0) sh.ticket = add_relaxed(&ctl->cticket.v, 1u);
     __syncthreads();
     const unsigned c = sh.ticket;
     __syncthreads();
     if (c >= ncmb) break;
-    const long long t_ready = p.trace ? wall_clock64() : 0;
+    const long long t_ready = trace_clock(traced);
     tiled_combine_task(p, static_cast<int>(c), cmb_tok);
     trace(t_dyn0 + nm * (nt1 + nt2) + c, 5, c, t_fetch, t_ready);
   }
@@ -1813,32 +1824,40 @@ int tiled_max_tokens() { return 1 << 21; }
 // y of the tiled variant: one bf16 row of H per (token, slot); ragged shapes keep the streaming variant's float rows
 size_t tiled_y_bytes(size_t rows, size_t hidden) { return rows * hidden * 2; }
 
+namespace {
+using TiledKernel = void (*)(const Params);
+// [ragged, ragged with an odd I or neither][with task records]
+const TiledKernel kTiledKernels[3][2] = {{moe_tiled_kernel<false, false, false>, moe_tiled_kernel<false, false, true>},
+                                         {moe_tiled_kernel<true, false, false>, moe_tiled_kernel<true, false, true>},
+                                         {moe_tiled_kernel<true, true, false>, moe_tiled_kernel<true, true, true>}};
+}  // namespace
+
 hipError_t launch_tiled_kernel(const Params& p, int grid, hipStream_t stream) {
-  auto* kernel = !tiled_ragged(p.H, p.I) ? moe_tiled_kernel<false, false>
-                 : p.I % KS == 0         ? moe_tiled_kernel<true, false>
-                                         : moe_tiled_kernel<true, true>;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(T_THREADS), TILED_LDS_BYTES, stream, p);
+  const int shape = !tiled_ragged(p.H, p.I) ? 0 : p.I % KS == 0 ? 1 : 2;
+  hipLaunchKernelGGL(kTiledKernels[shape][p.trace != nullptr], dim3(grid), dim3(T_THREADS), TILED_LDS_BYTES, stream, p);
   return hipGetLastError();
 }
 
 hipError_t prepare_tiled_kernel() {
-  for (auto* kernel : {moe_tiled_kernel<false, false>, moe_tiled_kernel<true, false>, moe_tiled_kernel<true, true>}) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, TILED_LDS_BYTES);
-    if (e != hipSuccess) return e;
-  }
+  for (const auto& kernels : kTiledKernels)
+    for (TiledKernel kernel : kernels) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, TILED_LDS_BYTES);
+      if (e != hipSuccess) return e;
+    }
   return hipSuccess;
 }
 
 // the least of the kernels' numbers of workgroups a CU holds
 hipError_t tiled_kernel_occupancy(int* per_cu) {
   *per_cu = 0x7FFFFFFF;
-  for (auto* kernel : {moe_tiled_kernel<false, false>, moe_tiled_kernel<true, false>, moe_tiled_kernel<true, true>}) {
-    int n = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, T_THREADS, TILED_LDS_BYTES);
-    if (e != hipSuccess) return e;
-    if (n < *per_cu) *per_cu = n;
-  }
+  for (const auto& kernels : kTiledKernels)
+    for (TiledKernel kernel : kernels) {
+      int n = 0;
+      const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, T_THREADS, TILED_LDS_BYTES);
+      if (e != hipSuccess) return e;
+      if (n < *per_cu) *per_cu = n;
+    }
   return hipSuccess;
 }
 

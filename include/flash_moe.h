@@ -238,7 +238,8 @@ int flashMoeSetWaitLimitMs(FlashMoeLauncher* l, double ms);
  * (a batch that would run the split-k kernel runs the streaming or the tiled one while tracing is
  * on, see flashMoeSchedFor: read a launch's stage outputs before tracing is switched);
  * kind: 0 router dot, 1 scan, 2 scatter, 3 gate/up, 4 down, 5 combine, 6 router
- * select; times in
+ * select (a wave's tokens) or an expert's scan; launches whose scatter tasks build the tables
+ * themselves have no kind 1; times in
  * ticks of the 100 MHz device wall clock. Read waits for `stream`, copies up to
  * max_records records to the host and marks all records unused (all bits set). */
 int flashMoeTraceEnable(FlashMoeLauncher* l, unsigned capacity);

@@ -235,3 +235,39 @@ def test_down_stage_alone(shape):
               flush=True)
     finally:
         case.close()
+
+
+@pytest.mark.parametrize("T,H,E,k,I,dt,start", [
+    (300, 256, 8, 2, 128, "bf16", "chains"),       # logit chains of 16 tokens x 32 experts, selections by wave
+    (1700, 256, 8, 2, 128, "bf16", "tokens"),      # router tasks of 16 tokens, no scan
+    (300, 320, 40, 3, 160, "bf16", "chains"),      # ragged columns
+    (2100, 128, 256, 2, 128, "bf16", "tickets"),   # mask words beyond LDS
+    (300, 256, 8, 2, 160, "f32", "float32"),
+])
+def test_a_trace_shows_the_launch_as_it_runs_without_one(T, H, E, k, I, dt, start):
+    """Tracing changes neither the variant nor the tasks: as many records of each kind as the untraced
+    launch has tasks, each once and in order of its times, and the same output bits."""
+    cfg = synth.MoeConfig("trace", T, H, E, k, I, dt)
+    case = GpuCase(cfg, seed=T, sched=2)
+    try:
+        want = case.run()
+        case.launcher.trace_enable(1 << 17)
+        assert case.launcher.sched_for(T) == 2
+        assert torch.equal(case.run(), want)
+        rec = case.launcher.trace_read()
+        counts = case.launcher.routing(T)["counts"]
+        case.launcher.trace_enable(0)
+        assert len(np.unique(rec["ticket"])) == len(rec)
+        assert (rec["t_fetch"] <= rec["t_ready"]).all() and (rec["t_ready"] <= rec["t_end"]).all()
+        got = np.bincount(rec["kind"], minlength=7)
+        up = lambda a, b: -(-a // b)
+        tiles = sum(up(int(c), 96 if dt == "f32" else 320) for c in counts)
+        expect = {0: {"chains": up(T, 16) * up(E, 32), "float32": up(T, 8) * up(E, 8)}.get(start, up(T, 16)),
+                  1: {"tickets": 1, "float32": up(E, 4)}.get(start, 0),
+                  2: up(T, 32) if start in ("tickets", "float32") else up(T * k, 256),
+                  3: tiles * up(I, 128), 4: tiles * up(H, 256)}
+        print("  records by kind", got, flush=True)
+        assert {q: int(got[q]) for q in expect} == expect
+        assert got[5] > 0 and (got[6] > 0) == (start != "tokens")
+    finally:
+        case.close()
