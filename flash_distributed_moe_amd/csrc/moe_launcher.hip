@@ -79,9 +79,9 @@ struct Layout {
 
 constexpr int kMaxGroups = 1024;  // workgroups a launch may use (one per CU)
 
-// AUTO hands a batch to the tiled variant from this many rows an expert on (on average):
-// packed weights / the caller's row-major weights / float32. Below it the streaming variant runs,
-// which is what its share of `y` is sized for (bf16).
+// AUTO hands a batch to the tiled variant from this many rows an expert on (on average; see auto_tiled_rows):
+// bf16, packed weights, which is what the streaming variant's share of `y` is sized for / the caller's row-major
+// weights / float32 at the least.
 constexpr int kAutoTiledRowsPacked = 26;
 constexpr int kAutoTiledRowsRowMajor = 14;
 constexpr int kAutoTiledRowsF32 = 10;
@@ -186,15 +186,36 @@ hipError_t validate(const FlashMoeLayerDesc* d) {
 // T=320 905 / 960, T=384 934 / 969, T=512 1054 / 976), and from about 14 rows on
 // the caller's row-major weights, which the streaming variant reads half a
 // cache line at a time (30B: T=192 309 / 318, T=256 318 / 318, T=320 346 / 320;
-// 235B: T=192 1030 / 1001, T=256 1055 / 1007, T=384 1142 / 1015). float32 has a tiled kernel of its own,
-// from 10 rows an expert on: up to 9 the streaming variant's early tasks carry a tile each (us,
-// streaming / tiled, packed: 30B shape T=128 421 / 428, T=160 541 / 437, T=256 586 / 452; E=40, k=5,
-// H=1344, I=736 T=60 117 / 148, T=120 189 / 152; row-major: 30B T=128 548 / 487, T=256 595 / 510; E=16,
-// k=2, H=320, I=160 T=64 50 / 56, T=128 60 / 56).
+// 235B: T=192 1030 / 1001, T=256 1055 / 1007, T=384 1142 / 1015). float32 has a tiled kernel of its own. For both
+// dtypes the line of layers with fewer tasks is in auto_tiled_rows.
 bool tiled_eligible(const FlashMoeLayerDesc& d, int tokens_num) {
   const long long esz = d.dtype == FLASH_MOE_BF16 ? 2 : 4;
   return d.hidden >= 128 && d.intermediate >= 128 && tokens_num <= fmoe::tiled_max_tokens() &&
          tokens_num * esz * d.hidden < (1ll << 32) && 2 * esz * d.intermediate * d.hidden < (1ll << 32);
+}
+
+// Rows an expert from which AUTO takes the tiled variant. Where few experts give it few tasks, a task of one
+// short row tile is the longer one, and the streaming variant stays ahead until its own tasks carry a
+// second row block (us, streaming / tiled):
+//   float32, packed: 30B shape T=160 561 / 463, T=256 570 / 474; E=64, k=4, H=1024, I=1408 T=160 266 / 266; E=16, k=2, H=2048,
+//     I=2048 T=80 250 / 242, T=96 287 / 251; but E=32, k=4, H=2048, I=768 T=80 175 / 192, T=96 190 / 195, T=128 230 / 199;
+//     E=40, k=5, H=1344, I=736 T=80 132 / 150, T=112 0.91 of the time, T=128 187 / 158; E=8, k=2, H=1024, I=1024 T=40 100 / 110, T=64 145 / 116
+//   float32, row-major: 30B T=160 560 / 523; E=64, k=4, H=2048, I=512 T=160 274 / 243; but I=1408, H=1024 T=160 295 / 328, T=256
+//     325 / 326, T=384 388 / 331; E=32, I=768 T=80 214 / 242, T=160 233 / 237, T=192 294 / 242; E=16, I=2048 T=80 286 / 329, T=128
+//     326 / 325, T=192 397 / 325; E=40 T=80 157 / 183, T=128 187 / 184, T=192 245 / 185
+//   bf16, row-major, ragged shapes (float rows of y): E=40, k=5, H=1344, I=736 T=112 98 / 98, T=128 101 / 97; E=100, k=6, H=3904,
+//     I=1952 T=233 0.90 of the streaming variant's time; but E=24, k=3, H=640, I=2016 T=144 85 / 101, T=160 107 / 101; E=16, k=2,
+//     H=320, I=160 T=144 41 / 44, T=192 46 / 44, T=208 54 / 44; E=8, k=2, H=2240, I=1056 T=96 89.5 / 90.6, T=104 92 / 91
+int auto_tiled_rows(const FlashMoeLayerDesc& d) {
+  const bool packed = (d.flags & (FLASH_MOE_FLAG_PACK_WEIGHTS | FLASH_MOE_FLAG_WEIGHTS_PREPACKED)) != 0;
+  const bool many_columns = static_cast<long long>(d.experts) * d.intermediate >= 1 << 15;
+  if (d.dtype == FLASH_MOE_F32) {
+    if (packed) return d.experts >= 64 || many_columns ? kAutoTiledRowsF32 : d.experts >= 40 ? 14 : 16;
+    return d.experts >= 96 || (d.experts >= 64 && d.intermediate <= 1024) ? kAutoTiledRowsF32 : d.experts >= 40 ? 16 : 22;
+  }
+  if (packed) return kAutoTiledRowsPacked;
+  if (fmoe::tiled_ragged(d.hidden, d.intermediate) && d.experts < 32) return many_columns ? 20 : kAutoTiledRowsPacked;
+  return kAutoTiledRowsRowMajor;
 }
 
 // What the choice of a kernel depends on beside the layer and the batch.
@@ -252,13 +273,9 @@ int sched_for(const FlashMoeLayerDesc& d, int tokens_num, const Machine& m) {
   if (d.sched == FLASH_MOE_SCHED_STREAM) return FLASH_MOE_SCHED_STREAM;
   if (!tiled_eligible(d, tokens_num)) return FLASH_MOE_SCHED_STREAM;
   const long long rows = static_cast<long long>(tokens_num) * d.top_k;
-  if (d.dtype == FLASH_MOE_F32) {
-    if (d.sched == FLASH_MOE_SCHED_TILED) return FLASH_MOE_SCHED_TILED;
-    return rows >= static_cast<long long>(kAutoTiledRowsF32) * d.experts ? FLASH_MOE_SCHED_TILED : FLASH_MOE_SCHED_STREAM;
-  }
   if (d.sched == FLASH_MOE_SCHED_TILED) return FLASH_MOE_SCHED_TILED;
   const bool packed = (d.flags & (FLASH_MOE_FLAG_PACK_WEIGHTS | FLASH_MOE_FLAG_WEIGHTS_PREPACKED)) != 0;
-  // Row-major weights of moderate size: the split-k kernel is faster as far as it goes (us, tiled /
+  // Row-major bf16 weights of moderate size: the split-k kernel is faster as far as it goes (us, tiled /
   // split-k, 30B shape: T=224 309 / 277, T=256 313 / 292, with four hot experts 327 / 307; H=1024,
   // I=512, 22 rows an expert 88 / 64; but 235B: T=224 975 / 1022, T=256 998 / 1067). The line lies
   // between an expert's 1.6 M (30B) and 6.3 M (235B) weights a matrix. Where the split-k kernel
@@ -266,11 +283,9 @@ int sched_for(const FlashMoeLayerDesc& d, int tokens_num, const Machine& m) {
   // tiled / streaming, H=2048, I=768, even routing and four hot experts: E=128, k=4, T=480 307 / 334
   // and 305 / 347; E=128, k=6, T=320 308 / 330 and 329 / 354; E=64, k=2, T=700 202 / 219 and
   // 133 / 153; E=96, k=4, T=400 275 / 273 and 273 / 293).
-  if (!packed && static_cast<long long>(d.hidden) * d.intermediate <= 3ll << 20 && split_row_blocks(d, tokens_num, m) != 0)
+  if (d.dtype == FLASH_MOE_BF16 && !packed && static_cast<long long>(d.hidden) * d.intermediate <= 3ll << 20 && split_row_blocks(d, tokens_num, m) != 0)
     return FLASH_MOE_SCHED_STREAM;
-  return rows >= static_cast<long long>(packed ? kAutoTiledRowsPacked : kAutoTiledRowsRowMajor) * d.experts
-             ? FLASH_MOE_SCHED_TILED
-             : FLASH_MOE_SCHED_STREAM;
+  return rows >= static_cast<long long>(auto_tiled_rows(d)) * d.experts ? FLASH_MOE_SCHED_TILED : FLASH_MOE_SCHED_STREAM;
 }
 
 // Whether any batch size up to max_tokens may run the tiled variant.

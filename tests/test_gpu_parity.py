@@ -494,6 +494,27 @@ def test_row_major_float32_rows_of_16_kib(E, k, H, I, split, stream):
             l.destroy()
 
 
+@pytest.mark.parametrize("dtype,packed,E,k,H,I,rows", [
+    ("f32", True, 128, 8, 512, 256, 10), ("f32", True, 64, 4, 512, 256, 10), ("f32", True, 16, 2, 512, 2048, 10),
+    ("f32", True, 60, 4, 512, 512, 14), ("f32", True, 39, 4, 512, 512, 16), ("f32", True, 8, 2, 1024, 1024, 16),
+    ("f32", False, 96, 4, 512, 2048, 10), ("f32", False, 64, 4, 512, 1024, 10), ("f32", False, 64, 4, 512, 1408, 16),
+    ("f32", False, 40, 5, 1344, 736, 16), ("f32", False, 32, 4, 512, 768, 22), ("f32", False, 16, 2, 512, 2048, 22),
+    ("bf16", False, 40, 5, 1344, 736, 14), ("bf16", False, 24, 3, 640, 2016, 20), ("bf16", False, 16, 2, 320, 160, 26),
+    ("bf16", True, 16, 2, 320, 160, 26),
+])
+def test_auto_takes_the_tiled_variant_from_its_line_on(dtype, packed, E, k, H, I, rows):
+    """Layers with few tasks stay on the streaming variant for more rows an expert."""
+    dt, dev = torch.bfloat16 if dtype == "bf16" else torch.float32, torch.device("cuda:0")
+    w = [torch.empty(s, dtype=dt, device=dev) for s in ((E, H), (E, 2 * I, H), (E, H, I))]  # never read
+    l = MoeKernelLauncher()
+    line = -(-rows * E // k)
+    l.create(*w, line + 1, l.getDistributedUniqueId(True), 0, 1, top_k=k, pack_weights=False, prepacked=packed)
+    try:
+        assert [l.sched_for(t) for t in (line - 1, line, line + 1)] == [_lib.SCHED_STREAM] + [_lib.SCHED_TILED] * 2
+    finally:
+        l.destroy()
+
+
 @pytest.mark.parametrize("E,k,last", [(128, 4, 256), (96, 4, 336), (64, 2, 512)])
 def test_auto_row_major_leaves_the_streaming_variant_with_the_split_k_kernel(E, k, last):
     """AUTO sends row-major bf16 batches of 14 to 24 rows an expert to the streaming variant for its
