@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from flash_distributed_moe_amd import synth
+from flash_distributed_moe_amd import _lib, synth
 from tests.moe_case import GpuCase
 
 pytestmark = pytest.mark.gpu
@@ -31,13 +31,15 @@ HOST_THREADS = max(1, min(os.cpu_count() or 1, int(os.environ.get("OMP_NUM_THREA
 _first_output = {}   # (config, T) -> output of the first variant run: later variants must match it
 
 
-def run_full(name, T=None, pack_weights=False, same_bits_as_first=False, fresh_relaunch=False):
+def run_full(name, T=None, pack_weights=False, same_bits_as_first=False, fresh_relaunch=False,
+             sched=_lib.SCHED_AUTO, runs=None):
     cfg = synth.CONFIGS[name] if isinstance(name, str) else name
     if T is not None:
         cfg = cfg.replace(T=T)
     print("full config", cfg.name, "T", cfg.T, "packed" if pack_weights else "caller's layout", flush=True)
-    case = GpuCase(cfg, pack_weights=pack_weights)
+    case = GpuCase(cfg, pack_weights=pack_weights, sched=sched)
     try:
+        assert runs is None or case.launcher.sched_for(cfg.T) == runs
         x = case.inp["tokens"]
         out = case.run()
         r = case.launcher.routing(cfg.T)
@@ -56,13 +58,13 @@ def run_full(name, T=None, pack_weights=False, same_bits_as_first=False, fresh_r
         out2 = case.run(inplace=True)
         assert torch.equal(out, out2)                 # deterministic; aliasing-safe
         if fresh_relaunch:
-            relaunch_with_fresh_tokens(case)
+            relaunch_with_fresh_tokens(case, sched)
         return r
     finally:
         case.close()
 
 
-def relaunch_with_fresh_tokens(case):
+def relaunch_with_fresh_tokens(case, sched=_lib.SCHED_AUTO):
     """The launcher that has just run the checked batch runs two more batches of the same
     size with other token contents, one eagerly and one as a replay of a captured graph, and
     each must equal bit for bit what a launcher that has never run anything returns for those
@@ -75,7 +77,7 @@ def relaunch_with_fresh_tokens(case):
     dt = torch.bfloat16 if cfg.dtype == "bf16" else torch.float32
     fresh = [synth.normal_torch(s, synth.STREAM_TOKENS, (cfg.T, cfg.H), 1.0, dt, case.dev) for s in (4242, 777)]
     assert not torch.equal(fresh[0], case.inp["tokens"])
-    other = GpuCase(cfg, inputs=case.inp, pack_weights=case.pack_weights)
+    other = GpuCase(cfg, inputs=case.inp, pack_weights=case.pack_weights, sched=sched)
     try:
         want = [other.run(tokens=f).clone() for f in fresh]
     finally:
@@ -103,7 +105,7 @@ def relaunch_with_fresh_tokens(case):
 
 @pytest.mark.parametrize("pack_weights", [False, True])
 def test_qwen3_30b_prefill(pack_weights):
-    # the tiled variant reads the caller's layout either way
+    # the tiled variant on the caller's layout and on the launcher's packed copy: the same bits
     run_full("qwen3_30b_prefill", pack_weights=pack_weights, same_bits_as_first=True, fresh_relaunch=True)
 
 
@@ -128,8 +130,17 @@ def test_qwen3_30b_imbalance():
 @pytest.mark.parametrize("pack_weights", [False, True])
 def test_f32_30b_large_batch(pack_weights):
     """The reference's own dtype and shape (src/hip/common/metadata.h:7-13) at a batch its GPU
-    path cannot hold (capacity about 85 tokens, src/hip/moeKernelLauncher.hip:117-135): the
-    streaming variant with several row tiles an expert. With its own packed copy the
-    launcher reads the row-major tensors at this size (legacy CreateLauncher's case)."""
+    path cannot hold (capacity about 85 tokens, src/hip/moeKernelLauncher.hip:117-135): the tiled
+    float32 kernel, on the row-major tensors or on the launcher's packed copy."""
     cfg = synth.MoeConfig("f32_30b_t1024", 1024, 2048, 128, 8, 768, "f32")
-    run_full(cfg, pack_weights=pack_weights, same_bits_as_first=True, fresh_relaunch=not pack_weights)
+    run_full(cfg, pack_weights=pack_weights, same_bits_as_first=True, fresh_relaunch=not pack_weights, runs=_lib.SCHED_TILED)
+
+
+@pytest.mark.parametrize("pack_weights", [False, True])
+def test_f32_30b_large_batch_streaming(pack_weights):
+    """The same layer where the streaming variant is asked for: several row tiles an expert. With its
+    own packed copy the launcher reads the row-major tensors from 16 rows an expert on, so both runs are the
+    same bits."""
+    cfg = synth.MoeConfig("f32_30b_t1024_streaming", 1024, 2048, 128, 8, 768, "f32")
+    run_full(cfg, pack_weights=pack_weights, same_bits_as_first=True, fresh_relaunch=pack_weights,
+             sched=_lib.SCHED_STREAM, runs=_lib.SCHED_STREAM)

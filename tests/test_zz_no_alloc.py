@@ -96,14 +96,19 @@ def test_no_alloc_equals_launcher_two_calls_in_a_row():
     assert torch.equal(g, no_alloc(big, inp_big, inp_big["tokens"], _lib.SCHED_STREAM))
 
 
-def test_no_alloc_takes_the_kernel_of_the_launcher():
+@pytest.mark.parametrize("Tmax,H,E,k,I,dt,Ts", [
+    (480, 256, 128, 4, 128, "bf16", (256, 480)),
+    (480, 256, 128, 4, 160, "bf16", (256, 480)),   # the tiled variant's h rows are padded: another workspace
+    (600, 320, 8, 2, 224, "f32", (30, 60, 600)),   # split-k, streaming and tiled float32 kernels
+])
+def test_no_alloc_takes_the_kernel_of_the_launcher(Tmax, H, E, k, I, dt, Ts):
     """A row-major AUTO batch between the split-k kernel's last size and the packed weights'
     switch-over: the number of CUs decides, and both entry points decide alike (the variants
     round differently, so equal bits are the same variant's)."""
     dev = torch.device("cuda:0")
-    cfg = synth.MoeConfig("between", 480, 256, 128, 4, 128, "bf16")
+    cfg = synth.MoeConfig("between", Tmax, H, E, k, I, dt)
     inp = synth.make_inputs_torch(cfg, 7907, dev)
-    for T in (256, 480):
+    for T in Ts:
         x = inp["tokens"][:T].contiguous()
         want = with_launcher(cfg, inp, x, _lib.SCHED_AUTO, pack_weights=False)
         assert torch.equal(no_alloc(cfg, inp, x, _lib.SCHED_AUTO), want)
