@@ -67,8 +67,10 @@ static_assert(split_lds_bytes(2) + 64 <= 160 * 1024, "LDS of a workgroup");
 // pitches of 4 KiB and more are the same channels. us, equal stretches / as here, packed: bf16 30B shape T=64
 // 209.9 / 207.0, 235B T=64 742 / 733, T=200 797 / 788, float32 30B T=128 412 / 408; row-major: bf16 30B
 // T=64 241.6 / 238.4, T=200 273.6 / 268.5, 235B T=64 888 / 860, T=200 1009 / 970, float32 30B T=64 499 / 474,
-// T=128 521 / 498; E=60, k=4, H=2304, I=1408 T=100 (no two steps divide) packed 210 / 211.5, row-major
-// 262 / 252. Without the moving start, bf16 row-major 235B T=64 933, float32 30B T=128 576; runs of two with
+// T=128 521 / 498. Where the steps do not divide into runs of two, row-major weights gain too (bf16 E=60, k=4,
+// H=2304, I=1408 T=100 262 / 251, T=200 289 / 276, E=128, k=8, H=2048, I=800 T=100 262 / 258), packed ones do not (E=60 T=100
+// 210.1 / 210.4, T=200 222.8 / 223.7; float32 E=128, k=8, H=2880, I=1440 T=64 964 / 978, E=64, k=6, H=2240, I=1376 T=100
+// 402 / 408): they go along, because both forms of the weights give the same bits. Without the moving start, bf16 row-major 235B T=64 933, float32 30B T=128 576; runs of two with
 // it 900 and 537, of eight 880 and 501; starts next to each other instead of far apart, float32 row-major
 // H=4096, I=512 T=100 389 instead of 373.
 struct SplitSteps {

@@ -20,9 +20,10 @@
 // matrix instructions (streaming kernel) / this: 30B shape T=256 1.85e-6 / 1.72e-6, T=512 1.84e-6 /
 // 1.71e-6; E=40, k=5, H=1344, I=736 T=900 1.29e-6 / 1.16e-6; E=10, k=3, H=320, I=2016 T=2000 9.4e-7 / 8.2e-7.
 //
-// Bound by HBM up to some 40 rows an expert, above by splitting and products together. us, streaming /
-// this, 30B shape: T=256 586 / 444, T=512 800 / 466, T=1024 1077 / 585 (2.43 GB and 77 GFLOP: 132
-// TFLOP/s of float32); row-major weights T=1024 1076 / 627; E=32 T=4096 2400 / 1450.
+// Bound by HBM up to some 40 rows an expert, above by splitting and products together: at T=1024 on the 30B shape
+// the matrix cores are busy 44 % of the SIMD cycles, other vector instructions take 30 %, and 2.79 GB are moved
+// of the 2.43 GB needed. us, streaming / this, 30B shape: T=256 586 / 444, T=512 800 / 466, T=1024 1077 / 585
+// (77 GFLOP: 132 TFLOP/s of float32); row-major weights T=1024 1076 / 627; E=32 T=4096 2400 / 1450.
 //
 // A value that is no finite number, or rounds to none in bf16, has no such parts: its products come
 // out as infinities or NaN. One below 2^-102 has parts below the smallest normal bf16 number, which lose
@@ -233,19 +234,22 @@ __device__ __forceinline__ void float_weights(ParamsRef p, int expert, int wblk,
   }
 }
 
+// Token rows of a tile.
+struct RowSet {
+  unsigned word[3];  // a bit a row
+  __device__ __forceinline__ unsigned any() const { return word[0] | word[1] | word[2]; }
+};
+static_assert(F_TM <= 96, "rows of a RowSet");
+// A sum's place in the order infinity, NaN, zero, small to large; the ordinary ones begin with 2^-64.
+__device__ __forceinline__ unsigned sum_order(float x) { return (__float_as_uint(x) << 1) + 0x01000000u; }
+constexpr unsigned SUM_ORDINARY = 0x01000000u + ((127u - 64u) << 24);
+
 // One tile task. gate/up: h[row, n0 .. n0+128) (refExpertFFN1.h:51-65); wave w holds gate rows
 // n0+32w.. and the matching up rows, so SiLU(gate)*up happens in registers. down:
 // y[t*K+slot, n0 .. n0+256) = w * (h[row] . W2[e]^T) (refFullMoe.h:58-65, src/hip/kernel/tasks/ffn2Task.h:37-40),
 // float rows with the gate weight applied, as the streaming kernel leaves them. Both are written
 // through, 64 bytes of a row at a time, from the accumulators. Returns the token rows for which a sum of
 // the wave is no finite number or a small one: float_exact_rows writes those again.
-struct RowSet {
-  unsigned word[3];  // a bit a row
-  __device__ __forceinline__ unsigned any() const { return word[0] | word[1] | word[2]; }
-};
-static_assert(F_TM <= 96, "rows of a RowSet");
-// twice the bits of 2^-64 and of infinity
-constexpr unsigned SUM_SMALL = ((127u - 64u) << 24) - 1u, SUM_INF = 0xFF000000u;
 template <int JB, bool down>
 __device__ __noinline__ RowSet float_task(ParamsRef pv, int expert_in, int row0_in, int rows_in, int shared_in, int nblk_in) {
   ParamsRef p = uniform_params(pv);
@@ -285,28 +289,22 @@ __device__ __noinline__ RowSet float_task(ParamsRef pv, int expert_in, int row0_
   }
   RowSet again = {{0u, 0u, 0u}};
   if (w0 >= nw) return again;  // this wave's columns do not exist: it has multiplied the last ones that do
-  // twice a sum's bits have no sign; less one, zero is the largest of them
-  unsigned least[JB], most[JB], all_least = 0xFFFFFFFFu, all_most = 0u;
+  unsigned least = 0xFFFFFFFFu;
 #pragma unroll
-  for (int j = 0; j < JB; ++j) {
-    least[j] = 0xFFFFFFFFu;
-    most[j] = 0u;
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < JB; ++j)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const unsigned twice = __float_as_uint(acc[i][j][v]) << 1;
-        least[j] = min(least[j], twice - 1u);
-        most[j] = max(most[j], twice);
-      }
-    all_least = min(all_least, least[j]);
-    all_most = max(all_most, most[j]);
-  }
-  if (__any(all_least < SUM_SMALL || all_most >= SUM_INF)) {
+      for (int v = 0; v < 4; ++v) least = min(least, sum_order(acc[i][j][v]));
+  if (__any(least < SUM_ORDINARY)) {
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
-      const unsigned long long b =
-          __ballot((least[j] < SUM_SMALL || most[j] >= SUM_INF) && 16 * j + r16 < rows);  // a row's lanes stand 16 apart
+      bool odd = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) odd |= sum_order(acc[i][j][v]) < SUM_ORDINARY && acc[i][j][v] != 0.0f;
+      const unsigned long long b = __ballot(odd && 16 * j + r16 < rows);  // a row's lanes stand 16 apart
       const unsigned both = static_cast<unsigned>(b) | static_cast<unsigned>(b >> 32);
       again.word[j >> 1] |= ((both | both >> 16) & 0xFFFFu) << (16 * (j & 1));
     }
