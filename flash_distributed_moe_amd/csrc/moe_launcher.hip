@@ -379,7 +379,8 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   }
   const bool tiled = sched_for(d, T, m) == FLASH_MOE_SCHED_TILED;
   // How the bf16 tiled kernel starts. 1: logit chains of 16 tokens x 32 experts a workgroup, in two rounds
-  // at most, and selections spread over all waves, while a wave has two of them at most (30B shape, us,
+  // at most, and selections spread over all waves of the workgroups that had a chain, while that is two of them a wave
+  // at most if every workgroup had one (of 1536 tokens and 32 experts 96 have: four a wave) (30B shape, us,
   // without / with: T=450 300 / 282, T=600 302 / 285, T=900 312 / 299, T=1500 330 / 325, T=2048 353 / 356;
   // E=256, H=1024, I=512, T=1024 242 / 231; E=16, k=2, H=320, I=160, T=4000 74 / 78). 2: router tasks of 16
   // or 32 tokens x all experts. Both without a scan phase, while the mask words fit LDS (as 2 against 0:
