@@ -70,7 +70,10 @@ static_assert(split_lds_bytes(2) + 64 <= 160 * 1024, "LDS of a workgroup");
 // T=128 521 / 498. Where the steps do not divide into runs of two, row-major weights gain too (bf16 E=60, k=4,
 // H=2304, I=1408 T=100 262 / 251, T=200 289 / 276, E=128, k=8, H=2048, I=800 T=100 262 / 258), packed ones do not (E=60 T=100
 // 210.1 / 210.4, T=200 222.8 / 223.7; float32 E=128, k=8, H=2880, I=1440 T=64 964 / 978, E=64, k=6, H=2240, I=1376 T=100
-// 402 / 408): they go along, because both forms of the weights give the same bits. Without the moving start, bf16 row-major 235B T=64 933, float32 30B T=128 576; runs of two with
+// 402 / 408): they go along, because both forms of the weights give the same bits. Down projections with rows of
+// whole 8 KiB keep the stretches as well (row-major, runs / stretches there, bf16 E=16, k=4, H=1024, I=4096 T=24 106.6 /
+// 100.4, I=8192 T=24 187.1 / 167.1, E=32, k=4, H=2048, I=4096 T=24 298.6 / 293.1; float32 E=16, k=4, H=1024, I=4096 T=24 199.9 /
+// 174.5, but H=2048, E=32 T=48 621 / 633; packed level: bf16 H=1024, I=4096 86.4 / 86.4, I=8192 145.2 / 144.9). Without the moving start, bf16 row-major 235B T=64 933, float32 30B T=128 576; runs of two with
 // it 900 and 537, of eight 880 and 501; starts next to each other instead of far apart, float32 row-major
 // H=4096, I=512 T=100 389 instead of 373.
 struct SplitSteps {
@@ -536,7 +539,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
       old = __builtin_amdgcn_readfirstlane(old);
       if (old == static_cast<unsigned>(G) - 1u) broadcast_flag(p, FLAG_PERM);
     }
-    const SplitSteps sk2 = split_steps(ks2, sub, parts == 8 ? 3 : 2, p.split_spec != 0);
+    const SplitSteps sk2 = split_steps(ks2, sub, parts == 8 ? 3 : 2, p.split_spec != 0 && I * ESZ % 8192 != 0);
     const int steps2 = sk2.count;
     const int n_tasks = ntiles * per_tile;
     int ntask = b < n_tasks ? (n_tasks - b + G - 1) / G : 0;

@@ -473,6 +473,23 @@ def test_tiled_float32_infinite_tokens_hold_up_no_one_else():
         case.close()
 
 
+@pytest.mark.parametrize("dtype,E,k,H,I", [("bf16", 16, 2, 512, 4096), ("f32", 16, 2, 512, 2048), ("bf16", 12, 3, 256, 8192)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_split_k_down_rows_of_8_kib(dtype, E, k, H, I, packed):
+    """Down rows of whole 8 KiB are walked in equal stretches by batches that reach most experts, as by smaller
+    ones. (With one run of gate/up steps a wave, those are the same in both:) a token's sums are the same bits."""
+    cfg = synth.MoeConfig("stretches", 2 * E, H, E, k, I, dtype)
+    case = GpuCase(cfg, seed=I, pack_weights=packed)
+    try:
+        small = (E - 1) // k
+        assert case.launcher.split_blocks_for(small) == case.launcher.split_blocks_for(cfg.T) == 1
+        out = case.run()
+        case.check_outputs(case.inp["tokens"], out)
+        assert torch.equal(case.run(tokens=case.inp["tokens"][:small].contiguous()), out[:small])
+    finally:
+        case.close()
+
+
 @pytest.mark.parametrize("E,k,H,I,split,stream", [
     (128, 8, 4096, 640, (1, 8, 15), (16, 24, 32, 128)),   # 2560 gate/up tasks for 256 CUs
     (128, 8, 4096, 608, (1, 16, 31), (32, 64)),           # 2432
