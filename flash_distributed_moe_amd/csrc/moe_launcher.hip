@@ -202,7 +202,8 @@ bool tiled_eligible(const FlashMoeLayerDesc& d, int tokens_num) {
 //     E=40, k=5, H=1344, I=736 T=80 132 / 150, T=112 0.91 of the time, T=128 187 / 158; E=8, k=2, H=1024, I=1024 T=40 100 / 110, T=64 145 / 116
 //   float32, row-major: 30B T=160 560 / 523; E=64, k=4, H=2048, I=512 T=160 274 / 243; but I=1408, H=1024 T=160 295 / 328, T=256
 //     325 / 326, T=384 388 / 331; E=32, I=768 T=80 214 / 242, T=160 233 / 237, T=192 294 / 242; E=16, I=2048 T=80 286 / 329, T=128
-//     326 / 325, T=192 397 / 325; E=40 T=80 157 / 183, T=128 187 / 184, T=192 245 / 185
+//     326 / 325, T=192 397 / 325; E=40 T=80 157 / 183, T=128 187 / 184, T=192 245 / 185; E=8, k=2, I=3584 at 22, 25 and 30 rows an
+//     expert H=4096 1.14, 1.11 and 0.84 of the streaming variant's time, H=2048 1.13, 0.81 and 0.82
 //   bf16, row-major, ragged shapes (float rows of y): E=40, k=5, H=1344, I=736 T=112 98 / 98, T=128 101 / 97; E=100, k=6, H=3904,
 //     I=1952 T=233 0.90 of the streaming variant's time; but E=24, k=3, H=640, I=2016 T=144 85 / 101, T=160 107 / 101; E=16, k=2,
 //     H=320, I=160 T=144 41 / 44, T=192 46 / 44, T=208 54 / 44; E=8, k=2, H=2240, I=1056 T=96 89.5 / 90.6, T=104 92 / 91
@@ -211,7 +212,8 @@ int auto_tiled_rows(const FlashMoeLayerDesc& d) {
   const bool many_columns = static_cast<long long>(d.experts) * d.intermediate >= 1 << 15;
   if (d.dtype == FLASH_MOE_F32) {
     if (packed) return d.experts >= 64 || many_columns ? kAutoTiledRowsF32 : d.experts >= 40 ? 14 : 16;
-    return d.experts >= 96 || (d.experts >= 64 && d.intermediate <= 1024) ? kAutoTiledRowsF32 : d.experts >= 40 ? 16 : 22;
+    if (d.experts >= 40) return d.experts >= 96 || (d.experts >= 64 && d.intermediate <= 1024) ? kAutoTiledRowsF32 : 16;
+    return d.experts < 16 && d.intermediate >= 2048 ? 26 : 22;
   }
   if (packed) return kAutoTiledRowsPacked;
   if (fmoe::tiled_ragged(d.hidden, d.intermediate) && d.experts < 32) return many_columns ? 20 : kAutoTiledRowsPacked;

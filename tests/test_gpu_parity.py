@@ -516,6 +516,7 @@ def test_row_major_float32_rows_of_16_kib(E, k, H, I, split, stream):
     ("f32", True, 60, 4, 512, 512, 14), ("f32", True, 39, 4, 512, 512, 16), ("f32", True, 8, 2, 1024, 1024, 16),
     ("f32", False, 96, 4, 512, 2048, 10), ("f32", False, 64, 4, 512, 1024, 10), ("f32", False, 64, 4, 512, 1408, 16),
     ("f32", False, 40, 5, 1344, 736, 16), ("f32", False, 32, 4, 512, 768, 22), ("f32", False, 16, 2, 512, 2048, 22),
+    ("f32", False, 8, 2, 512, 2048, 26), ("f32", False, 8, 2, 512, 1792, 22),
     ("bf16", False, 40, 5, 1344, 736, 14), ("bf16", False, 24, 3, 640, 2016, 20), ("bf16", False, 16, 2, 320, 160, 26),
     ("bf16", True, 16, 2, 320, 160, 26),
 ])
