@@ -582,6 +582,20 @@ __device__ __forceinline__ void mma(const v4u_t& a, const v4u_t& b, f32x4& c) {
   }
 }
 
+// The compiler does not see matrix instructions in the assembly above: keep the wait states between the
+// last of them and the first read of an accumulator, and the reads behind them (it may place the reads of what an
+// assembly does not name anywhere).
+template <int JT>
+__device__ __forceinline__ void settle(f32x4 (&acc)[4][JB_MAX]) {
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * JT; ++j) {
+      if (j < JB_ACC) asm volatile("" : "+a"(acc[i][j])); else asm volatile("" : "+v"(acc[i][j]));
+    }
+}
+
 constexpr int stage_bytes_of(int jt) { return (TN + 32 * jt) * ROWB; }
 // Stages of the LDS-staged pipeline: three where they fit. The tiles of a batch of some 40 to
 // 160 rows an expert are bound by how much of the weights is in flight, taller ones are not.
@@ -598,8 +612,6 @@ constexpr int SIDE_BYTES = TM_MAX * 8;
 constexpr int NOTE_OFF = SIDE_OFF + SIDE_BYTES;
 constexpr int NOTE_BYTES = 16;
 __device__ __forceinline__ unsigned* task_notes() { return reinterpret_cast<unsigned*>(lds_raw + NOTE_OFF); }
-constexpr int EPI_LD = TN * 2 + 16;              // bytes per row of the down epilogue's staging slab
-static_assert(128 * EPI_LD <= TILE_LDS_BYTES, "epilogue slab exceeds the stage buffers");
 
 struct TileOperands {
   const unsigned char* wbase;  // uniform: the weight matrix (or this wave's packed slice) the offsets are relative to
@@ -824,10 +836,7 @@ __device__ __forceinline__ void tile_gemm(const TileOperands& op, int nstages, f
   } else {
     stage(s, No{}, std::integral_constant<int, 0>{});
   }
-  // the compiler does not see matrix instructions in the assembly above: keep the wait states
-  // between the last of them and the first read of an accumulator
-  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-  __syncthreads();  // the stages are free for the epilogue
+  settle<JT>(acc);
 }
 
 // The same product when the weights come from the packed layout, on a deeper pipeline that
@@ -1068,11 +1077,8 @@ __device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nst
     constexpr int k = decltype(i)::value, r = 2 * D - 2 - k;
     stage(std::integral_constant<int, (1 + k) % D>{}, std::integral_constant<int, r < D + 1 ? r : D + 1>{}, No{}, s + k);
   });
-  // the compiler does not see matrix instructions in the assembly above: keep the wait states
-  // between the last of them and the first read of an accumulator
-  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+  settle<JT>(acc);
   wait_vm<0>();
-  __syncthreads();  // the stages are free for the epilogue
 }
 
 // Weights in the packed layout (the streaming variant's: per wave task and 32-k step four
@@ -1087,6 +1093,32 @@ __device__ __forceinline__ void tile_gemm_direct(const TileOperands& op, int nst
 static_assert(G1_NB == 2 && G2_NB == 4, "the tiled variant reads the packed layout as 32+32-row and 64-row tasks");
 __device__ __forceinline__ unsigned packed_run_offset(int q) {
   return static_cast<unsigned>((q >> 2) * 4096 + (q & 3) * 1024 + (threadIdx.x & 63) * 16);
+}
+
+// ------------------------------------------------------------------ epilogues
+// A lane ends with four consecutive columns of each 16-column block of its token row: 8 bytes of bf16, and
+// the four lanes of a token 32 bytes a block. Two neighbouring blocks change places between lanes 16
+// apart (V_PERMLANE16_SWAP: odd rows of 16 lanes of the first register against even rows of the second), and
+// every lane has 8 consecutive columns of the 32, the four lanes of a token 64 contiguous bytes: a store
+// instruction writes half lines of 16 rows, straight from the accumulators. No LDS, so no barrier and no trip
+// through it stands between a task's last matrix instruction and its stores, and the waves of a
+// workgroup leave the task one by one.
+__device__ __forceinline__ void swap_rows16(unsigned& a, unsigned& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+// the 16 bytes of this lane out of its packed values of two blocks, and the column (of the 32) they start at
+__device__ __forceinline__ uint4 pair_columns(uint2 a, uint2 b) {
+  swap_rows16(a.x, b.x);
+  swap_rows16(a.y, b.y);
+  return make_uint4(a.x, a.y, b.x, b.y);
+}
+__device__ __forceinline__ unsigned pair_column(int kg) { return static_cast<unsigned>((kg & 1) * 16 + (kg >> 1) * 8); }
+// st16_through at a uniform base and a lane's offset
+__device__ __forceinline__ void st16_through_at(unsigned char* base, unsigned off, const uint4& v) {
+  const v4u_t d = {v.x, v.y, v.z, v.w};
+  asm volatile("global_store_dwordx4 %0, %1, %2 sc1\n\ts_nop 1" : : "v"(off), "v"(d), "s"(base) : "memory");
 }
 
 // One GEMM tile task, gate/up or down, for a row tile of up to 32*JT rows.
@@ -1211,109 +1243,72 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
   } else {
     tile_gemm<JT, HALF>(op, nstages, acc, pend, queue, next, load_side);
   }
-  if (threadIdx.x == 0) task_notes()[0] = next;  // the epilogue's barriers publish it
-
-  const int r16 = lane & 15, kg = lane >> 4;
-  unsigned char* slab = lds_raw;
-  if (!down) {
-    constexpr int LD = G1_COLS * 2 + 16;  // slab row pitch in bytes
-#pragma unroll
-    for (int j = 0; j < 2 * JT; ++j)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {  // gate blocks 0, 1 with their up blocks 2, 3
-        float hv[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          hv[v] = RAGGED ? silu_mul(acc[i][j][v], acc[2 + i][j][v]) : silu_mul_fast(acc[i][j][v], acc[2 + i][j][v]);
-        uint2 pk;
-        pk.x = pack_bf16(hv[0], hv[1]);
-        pk.y = pack_bf16(hv[2], hv[3]);
-        *reinterpret_cast<uint2*>(slab + (j * 16 + r16) * LD + (wave * 32 + i * 16 + kg * 4) * 2) = pk;
-      }
-    __syncthreads();
-    // 16 lanes store one row's 256 bytes; a wave stores 4 rows per instruction
-    unsigned char* h = uni(reinterpret_cast<unsigned char*>(p.h)) + (static_cast<size_t>(row0) * hp + n0) * 2;
-    const bool live = !RAGGED || n0 + (lane & 15) * 8 < I;  // the lane's columns exist
-    // (the reads of a batch first, then its stores: a store's assembly orders memory
-    // operations around it, and one LDS round trip per store would add up to microseconds)
-    constexpr int NIT = 8 * JT / WAVES, BATCH = 8;
-#pragma unroll
-    for (int it0 = 0; it0 < NIT; it0 += BATCH) {
-      uint4 v[BATCH];
-#pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        const int row = ((it0 + u) * WAVES + wave) * 4 + (lane >> 4);
-        if (it0 + u < NIT) v[u] = *reinterpret_cast<const uint4*>(slab + row * LD + (lane & 15) * 16);
-      }
-#pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        const int row = ((it0 + u) * WAVES + wave) * 4 + (lane >> 4);
-        if (it0 + u < NIT && (RAGGED ? (row < rows) & live : row < rows))
-          st16_through(h + static_cast<size_t>(row) * hp * 2 + (lane & 15) * 16, v[u]);
-      }
-    }
-    __syncthreads();  // the slab is stage memory again
-  } else {
-    int* sdst = reinterpret_cast<int*>(lds_raw + SIDE_OFF);
+  // What the workgroup shares from here on goes to LDS in front of the one barrier behind the k-loop: the
+  // next ticket, and (down) where the rows go. It also says that nobody reads the stages any more.
+  int* sdst = reinterpret_cast<int*>(lds_raw + SIDE_OFF);
+  if (threadIdx.x == 0) task_notes()[0] = next;
+  if (down) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int r = static_cast<int>(threadIdx.x) + k * T_THREADS;
       if (r < TM_MAX) sdst[r] = side_dst[k];
       if (RAGGED && r < TM_MAX) reinterpret_cast<float*>(sdst + TM_MAX)[r] = side_w[k];
     }
-    __syncthreads();
-    if constexpr (RAGGED) {
-      if (wcol != wblk) return;
-      float* yf = uni(p.y) + 64 * wcol + 4 * kg;
+  }
+  __syncthreads();
+  if (RAGGED && wcol != wblk) return;  // these columns do not exist
+
+  const int r16 = lane & 15, kg = lane >> 4;
+  // token blocks below this one have all of their rows (a tile has more than 32 * (JT - 1); JT = 2: or fewer)
+  constexpr int FULL = JT == 2 ? 0 : 2 * (JT - 1);
+  const unsigned colb = pair_column(kg) * 2u;
+  if (!down) {
+    unsigned char* h = uni(reinterpret_cast<unsigned char*>(p.h)) + (static_cast<size_t>(row0) * hp + 32 * wcol) * 2;
+    const unsigned off = static_cast<unsigned>(r16) * static_cast<unsigned>(hp * 2) + colb;
 #pragma unroll
-      for (int j = 0; j < 2 * JT; ++j) {
-        const int dst = sdst[16 * j + r16];
-        const float w = reinterpret_cast<const float*>(sdst + TM_MAX)[16 * j + r16];
-        if (dst >= 0) {
+    for (int j = 0; j < 2 * JT; ++j) {
+      uint2 pk[2];
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            st16_through(yf + static_cast<size_t>(dst) * H + 16 * i,
-                         make_uint4(__float_as_uint(acc[i][j][0] * w), __float_as_uint(acc[i][j][1] * w),
-                                    __float_as_uint(acc[i][j][2] * w), __float_as_uint(acc[i][j][3] * w)));
-        }
+      for (int i = 0; i < 2; ++i) {  // gate blocks 0, 1 with their up blocks 2, 3
+        float hv[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          hv[v] = RAGGED ? silu_mul(acc[i][j][v], acc[2 + i][j][v]) : silu_mul_fast(acc[i][j][v], acc[2 + i][j][v]);
+        pk[i] = make_uint2(pack_bf16(hv[0], hv[1]), pack_bf16(hv[2], hv[3]));
       }
-      return;
+      const uint4 v = pair_columns(pk[0], pk[1]);
+      if (j < FULL || 16 * j + r16 < rows) st16_through_at(h + static_cast<size_t>(j) * (32 * hp), off, v);
     }
-    unsigned char* y = uni(reinterpret_cast<unsigned char*>(p.y)) + n0 * 2;
+  } else if constexpr (RAGGED) {
+    float* yf = uni(p.y) + 64 * wcol + 4 * kg;
 #pragma unroll
-    for (int part = 0; part < (JT + 3) / 4; ++part) {
+    for (int j = 0; j < 2 * JT; ++j) {
+      const int dst = sdst[16 * j + r16];
+      const float w = reinterpret_cast<const float*>(sdst + TM_MAX)[16 * j + r16];
+      if (dst >= 0) {
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        const int j = part * 8 + jj;
-        if (j < 2 * JT) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            uint2 pk;
-            pk.x = pack_bf16(acc[i][j][0], acc[i][j][1]);
-            pk.y = pack_bf16(acc[i][j][2], acc[i][j][3]);
-            *reinterpret_cast<uint2*>(slab + (jj * 16 + r16) * EPI_LD + (wave * 64 + i * 16 + kg * 4) * 2) = pk;
-          }
-        }
+        for (int i = 0; i < 4; ++i)
+          st16_through(yf + static_cast<size_t>(dst) * H + 16 * i,
+                       make_uint4(__float_as_uint(acc[i][j][0] * w), __float_as_uint(acc[i][j][1] * w),
+                                  __float_as_uint(acc[i][j][2] * w), __float_as_uint(acc[i][j][3] * w)));
       }
-      __syncthreads();
-      // 32 lanes store one row's 512 bytes at the row's (token, slot); a wave stores 2 rows per instruction
-      constexpr int BATCH = 8;
+    }
+  } else {
+    unsigned char* y = uni(reinterpret_cast<unsigned char*>(p.y)) + 128 * wcol + colb;
+    int dst[2 * JT];
 #pragma unroll
-      for (int it0 = 0; it0 < 128 / (2 * WAVES); it0 += BATCH) {
-        uint4 v[BATCH];
-        int dst[BATCH];
+    for (int j = 0; j < 2 * JT; ++j) dst[j] = sdst[16 * j + r16];
 #pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-          const int lr = ((it0 + u) * WAVES + wave) * 2 + (lane >> 5);  // row inside this part
-          const int row = part * 128 + lr;
-          dst[u] = row < 32 * JT ? sdst[row] : -1;
-          v[u] = *reinterpret_cast<const uint4*>(slab + lr * EPI_LD + (lane & 31) * 16);
-        }
+    for (int j = 0; j < 2 * JT; ++j) {
+      uint2 pk[4];
 #pragma unroll
-        for (int u = 0; u < BATCH; ++u)
-          if (dst[u] >= 0) st16_through(y + static_cast<size_t>(dst[u]) * H * 2 + (lane & 31) * 16, v[u]);
+      for (int i = 0; i < 4; ++i) pk[i] = make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
+      const uint4 lo = pair_columns(pk[0], pk[1]), hi = pair_columns(pk[2], pk[3]);
+      if (j < FULL || dst[j] >= 0) {
+        unsigned char* row = y + static_cast<size_t>(dst[j]) * H * 2;
+        st16_through(row, lo);
+        st16_through(row + 64, hi);
       }
-      __syncthreads();
     }
   }
 }
