@@ -436,6 +436,71 @@ __device__ __forceinline__ void router_select_max(ParamsRef p, int t,
   lds_wave_sync();
 }
 
+// The same for four tokens at once, one to a row of 16 lanes: lane r of a row holds the experts EPL*r ..
+// EPL*r + EPL-1 of its token, so among equals the lowest lane, and in it the lowest element, wins. A round's
+// cross-lane steps stay inside the row and serve all four tokens, and nothing goes through scalar registers: on one
+// token to a wave a selection is a chain of K rounds of some 20 dependent cross-lane and scalar steps plus the
+// softmax in double, about 1.8 us whatever the wave could do beside it. t: the row's
+// token, -1: none. `scratch`:
+// SELECT_ROWS_BYTES of LDS private to the wave.
+constexpr int SELECT_ROWS_BYTES = 4 * MAX_TOPK * 16;
+__device__ __forceinline__ unsigned row_max_u32(unsigned v) {
+  auto step = [](unsigned x, unsigned moved) { return x > moved ? x : moved; };
+  v = step(v, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, true)));   // lane ^ 1
+  v = step(v, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, true)));   // lane ^ 2
+  v = step(v, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xF, 0xF, true)));  // mirror in 8
+  v = step(v, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xF, 0xF, true)));  // mirror in 16
+  return v;
+}
+template <int EPL>
+__device__ __forceinline__ void router_select_rows(ParamsRef p, int t, unsigned (&val)[EPL], unsigned char* scratch) {
+  const int lane = lane_id(), row = lane >> 4, r = lane & 15;
+  const int K = p.K;
+  double* ex = reinterpret_cast<double*>(scratch);                        // [4][MAX_TOPK]
+  uint2* won = reinterpret_cast<uint2*>(scratch + 4 * MAX_TOPK * 8);      // [4][MAX_TOPK]: expert (or -1), ordered bits
+  // lanes of this row in front of this one
+  const unsigned long long before = ((1ull << r) - 1ull) << (16 * row);
+  for (int s = 0; s < K; ++s) {
+    unsigned m = val[0];
+#pragma unroll
+    for (int j = 1; j < EPL; ++j) m = val[j] > m ? val[j] : m;
+    const unsigned best = row_max_u32(m);
+    const bool owner = m == best && (__ballot(m == best) & before) == 0ull;
+    int at = EPL;  // the lowest of this lane's elements that is the best
+#pragma unroll
+    for (int j = EPL - 1; j >= 0; --j) at = val[j] == best ? j : at;
+    // (no admissible expert left: lane 0 owns the zeros, and the slot stays empty)
+    if (owner) won[row * MAX_TOPK + s] = make_uint2(best != 0u ? static_cast<unsigned>(EPL * r + at) : 0xFFFFFFFFu, best);
+    const int drop = owner ? at : EPL;
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) val[j] = j == drop ? 0u : val[j];
+  }
+  lds_wave_sync();
+  // softmax over the K winners (descending, so the first is the maximum), a lane to a (token, slot)
+  auto logit = [](unsigned bits) { return bits != 0u ? from_ordered_bits(bits) : -FLT_MAX; };
+  for (int i = lane; i < 4 * K; i += 64) {
+    const int q = i & 3, s = i >> 2;
+    const float mine = logit(won[q * MAX_TOPK + s].y), first = logit(won[q * MAX_TOPK].y);
+    ex[q * MAX_TOPK + s] = exp(static_cast<double>(mine) - static_cast<double>(first));
+  }
+  lds_wave_sync();
+  for (int i0 = 0; i0 < 4 * K; i0 += 64) {
+    const int i = i0 + lane, q = i & 3, s = i >> 2;
+    const int tq = __shfl(t, 16 * q, 64);
+    if (i < 4 * K && tq >= 0) {
+      double sum = 0.0;
+      for (int u = 0; u < K; ++u) sum += ex[q * MAX_TOPK + u];
+      const float w = sum <= 0.0 ? static_cast<float>(1.0 / static_cast<double>(K))
+                                 : static_cast<float>(ex[q * MAX_TOPK + s] / sum);
+      const int e = static_cast<int>(won[q * MAX_TOPK + s].x);
+      stc(&p.topk_idx[static_cast<size_t>(tq) * K + s], e);
+      stc(&p.topk_w[static_cast<size_t>(tq) * K + s], w);
+      if (e >= 0) or_relaxed(&p.masks[static_cast<size_t>(e) * p.W + (tq >> 6)], 1ull << (tq & 63));
+    }
+  }
+  lds_wave_sync();
+}
+
 // ------------------------------------------------------------- scan / scatter
 // The tables the scan and scatter tasks work on, held in registers (Params is
 // reached through a generic reference, which every store would force the

@@ -35,9 +35,6 @@
 
 namespace fmoe {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-
 constexpr int JT_MAX = 10;         // 32-row token blocks of the tallest row tile
 constexpr int TM_MAX = 32 * JT_MAX;  // 320 token rows
 constexpr int TN = 256;            // weight rows per tile
@@ -84,192 +81,219 @@ __device__ __forceinline__ v4u_t lds_read16(unsigned addr) {
 // --------------------------------------------------------------------- router
 // Logits as in test/singleGPU/cpp/moe/reference/refGemm.h:21-24: one chain per
 // output, k ascending, one rounding per step. The chain runs on the matrix
-// core: V_MFMA_F32_16X16X4_F32 and V_MFMA_F32_32X32X2_F32 add their four / two
-// products to the accumulator one after the other in k order (checked bit for bit
-// against a CPU fmaf chain), and a product of two bf16 values is exact in float, so
-// every step is the oracle's acc = fmaf(x, w, acc).
-// A task is 16 or 32 tokens x a slab of 128 experts. With 16 tokens a wave carries two
-// 16x16 chains (experts 16w..16w+15 and 64+16w..64+16w+15); with 32 tokens one 32x32
-// chain (experts 32w..32w+31), which does the work of four 16x16 chains with half the
-// operand reads and permutes per multiply-add, and in less time: with every CU on the
-// float matrix core the chip holds ~56 cycles per 1024 multiply-adds in the 32x32 shape
-// against ~70 in the 16x16 shape (32 nominal for both).
-// All waves load: 64 k of the token rows and the 128 expert rows per stage,
-// four stages deep, with coalesced direct-to-LDS loads. Stage rows are 144 bytes
-// (128 of data, 16 of padding), so the 16-byte reads of 16 rows at one k fall
-// into different banks. 16x16: lane l multiplies row l % 16 of both operands at
-// k = 4*s + l/16: of the eight bf16 a 16-byte read brings, elements l/16 and
-// 4 + l/16. 32x32: row l % 32 at k = 2*s + l/32: elements l/32, 2 + l/32, 4 + l/32,
-// 6 + l/32. Each is moved into the upper half of a zero word by one byte permute.
+// core: V_MFMA_F32_16X16X4_F32 adds its four products to the accumulator one after
+// the other in k order (checked bit for bit against a CPU fmaf chain), and a product
+// of two bf16 values is exact in float, so every step is the oracle's acc = fmaf(x, w, acc).
+// A task is 16 or 32 tokens x a slab of 128 experts; a wave carries the 16x16 chains of
+// its 32 experts (16w..16w+15 and 64+16w..64+16w+15) and each block of 16 tokens.
+//
+// Bound by the float matrix instructions: 32 cycles each, and the SIMD's vector unit does nothing else
+// meanwhile (measured: four of them take 128 cycles, with one vector instruction between them 141, with four 159,
+// with eight 203). So the loop has none: lane l multiplies row l % 16 of both operands at k = 4*g + l/16, and
+// DS_READ_U16_D16_HI brings that bf16 into the upper half of a register whose lower half stays zero: the
+// float itself. 33.8 cycles an instruction, whatever the number of CUs at work. (A byte permute an operand
+// behind 16-byte reads: 50; 32x32x2 instructions on such operands: 96 for the 64 they take.) With the
+// selection of four tokens a wave, a task at H=2048 with all CUs: 32 tokens 63 -> 43 us, 16 tokens 38 -> 25.6 us.
+//
+// All waves load: 64 k of the token rows and the 128 expert rows per stage, four stages deep, with coalesced
+// direct-to-LDS loads. Stage rows are 144 bytes (128 of data, 16 of padding), so the reads of 16 rows at one k
+// fall into different banks. Token rows are padded to whole wave-wide loads, so a load has one base.
 // Then selection as in refTopk.h:36-58 / refMoeGate.h:27-30.
 constexpr int RT16_TOK = 16;  // tokens of the small router task; the large one has twice as many
 constexpr int RT_ROW_BYTES = 144;
 constexpr int RT_STAGES = 4;
 constexpr int RT_NL = 6;                                  // loads per wave and stage
 constexpr int RT_STAGE_BYTES = WAVES * RT_NL * 1024;      // 24 KiB
-constexpr int RT_NROWS = 2 * RT16_TOK + 128;
-static_assert(RT_NROWS * 9 <= WAVES * RT_NL * 64, "router stage too small");
-constexpr int ROUTER_LDS_BYTES = RT_STAGES * RT_STAGE_BYTES + 2 * RT16_TOK * MAX_EXPERTS * 4 + WAVES * MAX_TOPK * 8;
+constexpr int rt_token_loads(int nb) { return (nb * RT16_TOK * 9 + 63) / 64; }
+static_assert(rt_token_loads(2) + 128 * 9 / 64 <= WAVES * RT_NL, "router stage too small");
+constexpr int ROUTER_LDS_BYTES = RT_STAGES * RT_STAGE_BYTES + 2 * RT16_TOK * MAX_EXPERTS * 4;
+static_assert(WAVES * SELECT_ROWS_BYTES <= RT_STAGES * RT_STAGE_BYTES, "selection scratch exceeds the stages");
 
-__device__ __forceinline__ void load_to_lds_addr(const unsigned char* addr, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-               :
-               : "v"(addr), "s"(lds_addr)
-               : "memory");
+// Sixteen groups of 4 k to a stage. A group's operands (one register a block of token or expert rows) pass
+// through a ring of four: the group three ahead is asked for in front of a group's instructions. Whole runs of groups
+// are one assembly block each, which ends when all of its reads have returned: no register the compiler knows of is
+// ever in flight. FMOE_RD: the operands of ring place q, at byte `off` of the rows' stage; FMOE_MM: its instructions.
+#define FMOE_RD2(q, off)                                                                                       \
+  "ds_read_u16_d16_hi %[x" #q "0], %[xa] offset:" #off "\n\tds_read_u16_d16_hi %[w" #q "0], %[wa] offset:" #off \
+  "\n\tds_read_u16_d16_hi %[w" #q "1], %[wa] offset:9216+" #off "\n\tds_read_u16_d16_hi %[x" #q               \
+  "1], %[xa] offset:2304+" #off "\n\t"
+#define FMOE_RD1(q, off)                                                                                       \
+  "ds_read_u16_d16_hi %[x" #q "0], %[xa] offset:" #off "\n\tds_read_u16_d16_hi %[w" #q "0], %[wa] offset:" #off \
+  "\n\tds_read_u16_d16_hi %[w" #q "1], %[wa] offset:9216+" #off "\n\t"
+#define FMOE_MM1(q)                                                                                            \
+  "v_mfma_f32_16x16x4_f32 %[c00], %[x" #q "0], %[w" #q "0], %[c00]\n\tv_mfma_f32_16x16x4_f32 %[c01], %[x" #q   \
+  "0], %[w" #q "1], %[c01]\n\t"
+#define FMOE_MM2(q)                                                                                            \
+  FMOE_MM1(q)                                                                                                  \
+  "v_mfma_f32_16x16x4_f32 %[c10], %[x" #q "1], %[w" #q "0], %[c10]\n\tv_mfma_f32_16x16x4_f32 %[c11], %[x" #q   \
+  "1], %[w" #q "1], %[c11]\n\t"
+#define FMOE_WAIT(n) "s_waitcnt lgkmcnt(" #n ")\n\t"
+// ask for the group at `off` into ring place r, multiply the one in place q, wait for the next (all but the `n` reads
+// of the two groups behind it)
+#define FMOE_STEP2(q, r, off) FMOE_RD2(r, off) FMOE_MM2(q) FMOE_WAIT(8)
+#define FMOE_STEP1(q, r, off) FMOE_RD1(r, off) FMOE_MM1(q) FMOE_WAIT(6)
+#define FMOE_STEPS(S)                                                                                                 \
+  S(0, 3, 24) S(1, 0, 32) S(2, 1, 40) S(3, 2, 48) S(0, 3, 56) S(1, 0, 64) S(2, 1, 72) S(3, 2, 80) S(0, 3, 88) S(1, 0, 96) \
+      S(2, 1, 104) S(3, 2, 112) S(0, 3, 120)
+#define FMOE_X1 [x00] "+&v"(o.x[0][0]), [x10] "+&v"(o.x[1][0]), [x20] "+&v"(o.x[2][0]), [x30] "+&v"(o.x[3][0])
+#define FMOE_X2 FMOE_X1, [x01] "+&v"(o.x[0][1]), [x11] "+&v"(o.x[1][1]), [x21] "+&v"(o.x[2][1]), [x31] "+&v"(o.x[3][1])
+#define FMOE_W                                                                                              \
+  [w00] "+&v"(o.w[0][0]), [w10] "+&v"(o.w[1][0]), [w20] "+&v"(o.w[2][0]), [w30] "+&v"(o.w[3][0]), [w01] "+&v"(o.w[0][1]), \
+      [w11] "+&v"(o.w[1][1]), [w21] "+&v"(o.w[2][1]), [w31] "+&v"(o.w[3][1])
+#define FMOE_C1 [c00] "+&v"(acc[0][0]), [c01] "+&v"(acc[0][1])
+#define FMOE_C2 FMOE_C1, [c10] "+&v"(acc[1][0]), [c11] "+&v"(acc[1][1])
+#define FMOE_ADDR [xa] "v"(xa), [wa] "v"(wa)
+
+template <int NB>
+struct RouterRing {
+  unsigned x[4][NB], w[4][2];  // (lower halves zero, always)
+};
+// the first three groups of a stage into their places
+template <int NB>
+__device__ __forceinline__ void router_first(RouterRing<NB>& o, unsigned xa, unsigned wa) {
+  if constexpr (NB == 2)
+    asm volatile(FMOE_RD2(0, 0) FMOE_RD2(1, 8) FMOE_RD2(2, 16) FMOE_WAIT(0) : FMOE_X2, FMOE_W : FMOE_ADDR : "memory");
+  else
+    asm volatile(FMOE_RD1(0, 0) FMOE_RD1(1, 8) FMOE_RD1(2, 16) FMOE_WAIT(0) : FMOE_X1, FMOE_W : FMOE_ADDR : "memory");
+}
+// groups 0..12 of a stage, and the reads of its last three
+template <int NB>
+__device__ __forceinline__ void router_stage(RouterRing<NB>& o, f32x4 (&acc)[NB][2], unsigned xa, unsigned wa) {
+  if constexpr (NB == 2)
+    asm volatile(FMOE_STEPS(FMOE_STEP2) FMOE_WAIT(0) : FMOE_X2, FMOE_W, FMOE_C2 : FMOE_ADDR : "memory");
+  else
+    asm volatile(FMOE_STEPS(FMOE_STEP1) FMOE_WAIT(0) : FMOE_X1, FMOE_W, FMOE_C1 : FMOE_ADDR : "memory");
+}
+// groups 13..15, and the first three of the next stage
+template <int NB>
+__device__ __forceinline__ void router_stage_end(RouterRing<NB>& o, f32x4 (&acc)[NB][2], unsigned xa, unsigned wa) {
+  if constexpr (NB == 2)
+    asm volatile(FMOE_RD2(0, 0) FMOE_MM2(1) FMOE_RD2(1, 8) FMOE_MM2(2) FMOE_RD2(2, 16) FMOE_MM2(3) FMOE_WAIT(0)
+                 : FMOE_X2, FMOE_W, FMOE_C2
+                 : FMOE_ADDR
+                 : "memory");
+  else
+    asm volatile(FMOE_RD1(0, 0) FMOE_MM1(1) FMOE_RD1(1, 8) FMOE_MM1(2) FMOE_RD1(2, 16) FMOE_MM1(3) FMOE_WAIT(0)
+                 : FMOE_X1, FMOE_W, FMOE_C1
+                 : FMOE_ADDR
+                 : "memory");
+}
+// the wait states between the last matrix instruction, which the compiler does not see, and the first read of a sum
+template <int NB>
+__device__ __forceinline__ void router_settle(f32x4 (&acc)[NB][2]) {
+  if constexpr (NB == 2)
+    asm volatile("s_nop 15\n\ts_nop 15" : FMOE_C2);
+  else
+    asm volatile("s_nop 15\n\ts_nop 15" : FMOE_C1);
 }
 
-template <int NB>  // 1: 16 tokens, 16x16 chains; 2: 32 tokens, 32x32 chains
+template <int NB>  // blocks of 16 tokens
 __device__ __noinline__ void tiled_router_task(ParamsRef pv, int blk) {
   constexpr int NTOK = NB * RT16_TOK;
-  constexpr int NROWS = NTOK + 128;
-  constexpr int NW = NB == 2 ? 1 : 2;  // expert rows a lane reads
+  constexpr int W_OFF = rt_token_loads(NB) * 1024;  // expert rows in a stage
   ParamsRef p = uniform_params(pv);
   const int T = uni(p.T), E = uni(p.E), H = uni(p.H);
   const unsigned char* tokens = uni(reinterpret_cast<const unsigned char*>(p.tokens));
   const unsigned char* gate = uni(reinterpret_cast<const unsigned char*>(p.gate));
   const float* bias = uni(p.bias);
   unsigned* keys = reinterpret_cast<unsigned*>(lds_raw + RT_STAGES * RT_STAGE_BYTES);  // [NTOK][MAX_EXPERTS]
-  double* sel = reinterpret_cast<double*>(keys + NTOK * MAX_EXPERTS);              // WAVES x MAX_TOPK
   const unsigned lds_addr = uni(static_cast<unsigned>(
       reinterpret_cast<size_t>((FMOE_L3 unsigned char*)lds_raw)));
   const int tid = threadIdx.x;
   const int wave = uni(tid >> 6), lane = tid & 63;
   const int t0 = uni(blk) * NTOK;
   const int nsteps = H >> 6;
-  // slot g of a stage (16 bytes): position g % 9 of row g / 9 (position 8 is padding);
-  // rows 0..NTOK-1 are the tokens, the next 128 the experts of the slab; slots past the last row repeat it
-  const int r16 = lane & 15, kq = lane >> 4;    // 16x16: row and k quarter
-  const int r32 = lane & 31, kh = lane >> 5;    // 32x32: row and k half
-  const unsigned pick = NB == 2 ? (kh == 0 ? 0x01000C0Cu : 0x03020C0Cu)
-                                : (kq == 0   ? 0x01000C0Cu
-                                   : kq == 1 ? 0x03020C0Cu
-                                   : kq == 2 ? 0x05040C0Cu
-                                             : 0x07060C0Cu);
-  const int xoff = (NB == 2 ? r32 : r16) * RT_ROW_BYTES;
-  const int woff0 = (NB == 2 ? NTOK + 32 * wave + r32 : NTOK + 16 * wave + r16) * RT_ROW_BYTES;
-  const int woff1 = (NTOK + 64 + 16 * wave + r16) * RT_ROW_BYTES;  // 16x16 only
+  const int r16 = lane & 15, kq = lane >> 4;  // row and k of the group
+  const unsigned xoff = lds_addr + r16 * RT_ROW_BYTES + 2 * kq;
+  const unsigned woff = xoff + W_OFF + wave * 16 * RT_ROW_BYTES;
+  RouterRing<NB> o;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    o.w[q][0] = o.w[q][1] = 0u;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) o.x[q][n] = 0u;
+  }
   for (int e0 = 0; e0 < E; e0 += 128) {
-    const unsigned char* src[RT_NL];
+    // slot g of the token or the expert rows (16 bytes): position g % 9 of row g / 9 (position 8 is padding); slots
+    // past the last row repeat it
+    unsigned off[RT_NL];
+    const unsigned char* base[RT_NL];
 #pragma unroll
     for (int i = 0; i < RT_NL; ++i) {
-      const int g = (wave * RT_NL + i) * 64 + lane;
-      const int row = min(g / 9, NROWS - 1);
-      const int pos = min(g % 9, 7);
-      const unsigned char* base =
-          row < NTOK ? tokens + static_cast<size_t>(min(t0 + row, T - 1)) * H * 2
-                     : gate + static_cast<size_t>(min(e0 + row - NTOK, E - 1)) * H * 2;
-      src[i] = base + pos * 16;
+      const int ld = wave * RT_NL + i;
+      const bool tok = ld < rt_token_loads(NB);
+      const int g = (tok ? ld : ld - rt_token_loads(NB)) * 64 + lane;
+      const int row = tok ? min(min(g / 9, NTOK - 1), T - 1 - t0) : min(min(g / 9, 127), E - 1 - e0);
+      off[i] = static_cast<unsigned>(row) * static_cast<unsigned>(H * 2) + static_cast<unsigned>(min(g % 9, 7) * 16);
+      base[i] = uni(tok ? tokens + static_cast<size_t>(t0) * H * 2 : gate + static_cast<size_t>(e0) * H * 2);
     }
     auto issue = [&](int step) {  // past the last step: the last one again, into a stage nobody reads
       const size_t koff = static_cast<size_t>(min(step, nsteps - 1)) * 128;
       const unsigned st = lds_addr + (step & (RT_STAGES - 1)) * RT_STAGE_BYTES + wave * (RT_NL * 1024);
 #pragma unroll
-      for (int i = 0; i < RT_NL; ++i) load_to_lds_addr(src[i] + koff, st + i * 1024);
+      for (int i = 0; i < RT_NL; ++i) load_to_lds(off[i], base[i] + koff, st + i * 1024);
     };
-    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};  // 16x16
-    f32x16 big;                                                               // 32x32
+    f32x4 acc[NB][2];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) big[i] = 0.f;
-    // Operands of half a stage (32 k): four 16-byte chunks of the token row and of the
-    // expert rows. While the 16 matrix instructions of one half run, the next half is
-    // read, one chunk of each row after every four; the scheduling barriers keep the
-    // reads from being gathered in front of their first use.
-    struct Half {
-      uint4 a[4], w[NW][4];
-    };
-    auto read_chunk = [&](Half& h, const unsigned char* hb, int c4) {
-      h.a[c4] = *reinterpret_cast<const uint4*>(hb + xoff + 16 * c4);
-      h.w[0][c4] = *reinterpret_cast<const uint4*>(hb + woff0 + 16 * c4);
-      if constexpr (NB == 1) h.w[1][c4] = *reinterpret_cast<const uint4*>(hb + woff1 + 16 * c4);
-    };
-    auto sel1 = [&](unsigned v) { return __uint_as_float(__builtin_amdgcn_perm(v, v, pick)); };
-    auto chain_and_read = [&](const Half& h, Half& nx, const unsigned char* nb) {
-#pragma unroll
-      for (int c4 = 0; c4 < 4; ++c4) {
-        if constexpr (NB == 2) {
-          big = __builtin_amdgcn_mfma_f32_32x32x2f32(sel1(h.a[c4].x), sel1(h.w[0][c4].x), big, 0, 0, 0);
-          big = __builtin_amdgcn_mfma_f32_32x32x2f32(sel1(h.a[c4].y), sel1(h.w[0][c4].y), big, 0, 0, 0);
-          big = __builtin_amdgcn_mfma_f32_32x32x2f32(sel1(h.a[c4].z), sel1(h.w[0][c4].z), big, 0, 0, 0);
-          big = __builtin_amdgcn_mfma_f32_32x32x2f32(sel1(h.a[c4].w), sel1(h.w[0][c4].w), big, 0, 0, 0);
-        } else {
-          const float xl = __uint_as_float(__builtin_amdgcn_perm(h.a[c4].y, h.a[c4].x, pick));
-          const float xh = __uint_as_float(__builtin_amdgcn_perm(h.a[c4].w, h.a[c4].z, pick));
-#pragma unroll
-          for (int j = 0; j < NW; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                xl, __uint_as_float(__builtin_amdgcn_perm(h.w[j][c4].y, h.w[j][c4].x, pick)), acc[j], 0, 0, 0);
-#pragma unroll
-          for (int j = 0; j < NW; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                xh, __uint_as_float(__builtin_amdgcn_perm(h.w[j][c4].w, h.w[j][c4].z, pick)), acc[j], 0, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        read_chunk(nx, nb, c4);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    };
+    for (int n = 0; n < NB; ++n) acc[n][0] = acc[n][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int st = 0; st < RT_STAGES; ++st) issue(st);
     wait_vm<(RT_STAGES - 1) * RT_NL>();
     __builtin_amdgcn_s_barrier();  // stage 0 is in
     asm volatile("" ::: "memory");
-    Half h0, h1;
-#pragma unroll
-    for (int c4 = 0; c4 < 4; ++c4) read_chunk(h0, lds_raw, c4);
+    router_first<NB>(o, xoff, woff);
     for (int st = 0; st < nsteps; ++st) {
-      chain_and_read(h0, h1, lds_raw + (st & (RT_STAGES - 1)) * RT_STAGE_BYTES + 64);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave no longer reads stage st
-      wait_vm<(RT_STAGES - 2) * RT_NL>();                 // its loads of stage st+1 are in
+      const unsigned at = static_cast<unsigned>(st & (RT_STAGES - 1)) * RT_STAGE_BYTES;
+      const unsigned next = static_cast<unsigned>((st + 1) & (RT_STAGES - 1)) * RT_STAGE_BYTES;
+      router_stage<NB>(o, acc, xoff + at, woff + at);  // (this wave no longer reads stage st)
+      wait_vm<(RT_STAGES - 2) * RT_NL>();              // its loads of stage st+1 are in
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       issue(st + RT_STAGES);
       // after the last step this reads a stage that is being refilled; the values are never used
-      chain_and_read(h1, h0, lds_raw + ((st + 1) & (RT_STAGES - 1)) * RT_STAGE_BYTES);
+      router_stage_end<NB>(o, acc, xoff + next, woff + next);
     }
+    router_settle<NB>(acc);
     wait_vm<0>();                  // nothing may land in a stage after this slab
     __builtin_amdgcn_s_barrier();  // the stages may be refilled for the next slab
     asm volatile("" ::: "memory");
-    if constexpr (NB == 2) {
-      // big[i] of lane l: token 8*(i/4) + 4*(l/32) + i%4, expert e0 + 32*wave + l%32
-      const int e = e0 + 32 * wave + r32;
+    // acc[n][j][v] of lane l: token 16*n + 4*(l/16) + v, expert e0 + 64*j + 16*wave + l%16
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int e = e0 + 64 * j + 16 * wave + r16;
       const float bv = (bias != nullptr && e < E) ? as_global(bias)[e] : 0.0f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float x = bias != nullptr ? __fadd_rn(big[i], bv) : big[i];
-        const int tl = 8 * (i >> 2) + 4 * kh + (i & 3);
-        if (e < MAX_EXPERTS) keys[tl * MAX_EXPERTS + e] = ordered_bits(x, e < E);
-      }
-    } else {
-      // acc[j][v] of lane l: token 4*(l/16) + v, expert e0 + 64*j + 16*wave + l%16
-      const int ea = e0 + 16 * wave + r16, eb = ea + 64;
-      const float bva = (bias != nullptr && ea < E) ? as_global(bias)[ea] : 0.0f;
-      const float bvb = (bias != nullptr && eb < E) ? as_global(bias)[eb] : 0.0f;
+      for (int n = 0; n < NB; ++n)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        float xa = acc[0][v], xb = acc[1][v];
-        if (bias != nullptr) {
-          xa = __fadd_rn(xa, bva);
-          xb = __fadd_rn(xb, bvb);
+        for (int v = 0; v < 4; ++v) {
+          const float x = bias != nullptr ? __fadd_rn(acc[n][j][v], bv) : acc[n][j][v];
+          if (e < MAX_EXPERTS) keys[(16 * n + 4 * kq + v) * MAX_EXPERTS + e] = ordered_bits(x, e < E);
         }
-        if (ea < MAX_EXPERTS) keys[(4 * kq + v) * MAX_EXPERTS + ea] = ordered_bits(xa, ea < E);
-        if (eb < MAX_EXPERTS) keys[(4 * kq + v) * MAX_EXPERTS + eb] = ordered_bits(xb, eb < E);
-      }
     }
   }
   __syncthreads();
-  // selection: every wave takes its share of the tokens
-  double* lex = sel + wave * MAX_TOPK;
-  for (int i = 0; i < NTOK / WAVES; ++i) {
-    const int tl = wave * (NTOK / WAVES) + i;
-    const int t = t0 + tl;
-    if (t < T) {
-      unsigned val[MAX_EXPERTS / 64];
+  // selection: four tokens of every block of 16 to a wave, in the memory of the stages
+#pragma unroll 1
+  for (int n = 0; n < NB; ++n) {
+    const int tl = 16 * n + 4 * wave + kq;
+    const int t = t0 + tl < T ? t0 + tl : -1;
+    auto select = [&](auto epl) {
+      constexpr int EPL = decltype(epl)::value;
+      unsigned val[EPL];
 #pragma unroll
-      for (int j = 0; j < MAX_EXPERTS / 64; ++j) {
-        const int e = lane + 64 * j;
-        val[j] = e < E ? keys[tl * MAX_EXPERTS + e] : 0u;
+      for (int j = 0; j < EPL; j += 4) {
+        const uint4 v = *reinterpret_cast<const uint4*>(keys + tl * MAX_EXPERTS + EPL * r16 + j);
+        val[j] = v.x;
+        val[j + 1] = v.y;
+        val[j + 2] = v.z;
+        val[j + 3] = v.w;
       }
-      router_select_max(p, t, val, lex);
+      router_select_rows<EPL>(p, t, val, lds_raw + wave * SELECT_ROWS_BYTES);
+    };
+    if (E <= 128) {
+      select(std::integral_constant<int, 8>{});
+    } else {
+      select(std::integral_constant<int, 16>{});
     }
   }
 }

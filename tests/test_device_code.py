@@ -92,15 +92,10 @@ def _registers(text):
     return found
 
 
-def test_accumulators_are_left_alone_until_they_are_written(functions):
-    """The tiled kernel's matrix instructions stand in assembly, so the compiler does not know that their
-    results take a while: wherever it copies an accumulator between registers (it may where two ways
-    through the code meet) it would read the old value. So nothing but matrix instructions may touch a
-    result for 16 wait states (a 16x16x32 product takes four passes of four cycles, and the wait the
-    hardware does not make by itself is less), along the straight line behind it."""
+def _check_accumulators(functions, tasks):
     checked = 0
     for name, code in functions.items():
-        if not re.search("tiled_gemm_task|tiled_odd_down_task|tiled_ragged_(gate_up|down)_task", name):
+        if not re.search(tasks, name):
             continue
         ins = [i for _, i, _ in code]
         for at, op in enumerate(ins):
@@ -121,4 +116,20 @@ def test_accumulators_are_left_alone_until_they_are_written(functions):
                     if later.startswith(("v_", "ds_", "global_", "buffer_", "scratch_")) and " " in later:
                         assert not result & _registers(later.split(None, 1)[1]), "%s: %s | %s" % (name, op, later)
                     waited += 1
-    assert checked > 10000
+    return checked
+
+
+def test_accumulators_are_left_alone_until_they_are_written(functions):
+    """The tiled kernel's matrix instructions stand in assembly, so the compiler does not know that their
+    results take a while: wherever it copies an accumulator between registers (it may where two ways
+    through the code meet) it would read the old value. So nothing but matrix instructions may touch a
+    result for 16 wait states (a 16x16x32 product takes four passes of four cycles, and the wait the
+    hardware does not make by itself is less), along the straight line behind it."""
+    assert _check_accumulators(functions, "tiled_gemm_task|tiled_odd_down_task|tiled_ragged_(gate_up|down)_task") > 10000
+
+
+def test_router_chains_are_left_alone_until_they_are_written(functions):
+    """The same for the router's chains, which stand in assembly too: 16x16x4 float products of eight passes, ten wait
+    states."""
+    # 16 groups of 4 and of 2 instructions a stage
+    assert _check_accumulators(functions, "tiled_router_task") == 16 * 4 + 16 * 2

@@ -7,6 +7,7 @@ import torch
 
 from flash_distributed_moe_amd import _lib, synth
 from flash_distributed_moe_amd.flashMoeLauncher import MoeKernelLauncher
+from oracle import oracle
 from tests.moe_case import GpuCase
 
 pytestmark = pytest.mark.gpu
@@ -295,6 +296,35 @@ def test_tiled_starts(T, H, E, k):
         case.check_routing(case.inp["tokens"], case.launcher.routing(T))
         case.check_outputs(case.inp["tokens"], out, nthreads=4)
         assert torch.equal(case.run(), out)
+    finally:
+        case.close()
+
+
+@pytest.mark.parametrize("T,H,E,k,sched", [
+    (4099, 192, 128, 32, _lib.SCHED_TILED),  # 32-token router tasks, the last of 3 tokens; the most slots
+    (4100, 128, 200, 17, _lib.SCHED_TILED),  # two slabs of experts, the second partly empty; more slots than a row has lanes
+    (2100, 64, 40, 5, _lib.SCHED_TILED),     # 16-token tasks of one stage; the last of 4 tokens
+])
+@pytest.mark.parametrize("admitted", ["all", "three"])
+def test_router_winners(T, H, E, k, sched, admitted):
+    """Equal logits (every expert's row of the router weights twice, so the lower index wins) and experts that
+    are never admitted (a bias of -inf leaves three, fewer than k): winners and weights against the oracle."""
+    cfg = synth.MoeConfig("winners", T, H, E, k, 64, "bf16")
+    print("winners", T, H, E, k, sched, admitted, flush=True)
+    inp = synth.make_inputs_torch(cfg, T + k, torch.device("cuda:0"))
+    inp["gate"][E // 2:2 * (E // 2)] = inp["gate"][:E // 2].clone()
+    if admitted == "three":
+        inp["bias"] = torch.full((E,), -float("inf"), device="cuda:0")
+        inp["bias"][[1, E // 2 + 1, E - 1]] = 0.0
+    case = GpuCase(cfg, sched=sched, inputs=inp)
+    try:
+        case.run()
+        routing = case.launcher.routing(T)
+        hw = case.host_weights()
+        idx, w = oracle.gate(inp["tokens"].float().cpu().numpy(), hw["gate"], k, bias=hw["bias"])
+        assert (idx < 0).any() == (admitted == "three")
+        assert np.array_equal(routing["topk_idx"], idx)
+        np.testing.assert_allclose(routing["topk_w"], w, rtol=2e-6, atol=1e-7)  # as in GpuCase.check_routing
     finally:
         case.close()
 
