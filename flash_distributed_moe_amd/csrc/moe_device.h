@@ -314,15 +314,6 @@ __device__ __forceinline__ f32x4 mma16<F32>(const uint4& a, const uint4& b, f32x
   return c;
 }
 
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const unsigned long long o = __shfl_xor(v, off, 64);
-    v = o > v ? o : v;
-  }
-  return v;
-}
-
 __device__ __forceinline__ int wave_inclusive_scan(int v) {
   const int lane = lane_id();
 #pragma unroll
@@ -334,18 +325,6 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
 }
 
 // --------------------------------------------------------------------- router
-// (order-preserving value bits, inverted index): the maximum key is the largest
-// value and, among equals, the lowest index. Values the reference's strict '>'
-// against lowest() never admits (NaN, -inf, -FLT_MAX) get key 0.
-__device__ __forceinline__ unsigned long long make_key(float v, int e, bool in_range) {
-  const bool valid = in_range && (v > -FLT_MAX);
-  unsigned u = __float_as_uint(v);
-  u = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-  return valid ? ((static_cast<unsigned long long>(u) << 32) |
-                  static_cast<unsigned long long>(0xFFFFFFFFu - static_cast<unsigned>(e)))
-               : 0ull;
-}
-
 // Orders this wave's LDS writes before its later LDS reads (other lanes' data)
 // without waiting for global loads that are still in flight.
 __device__ __forceinline__ void lds_wave_sync() {
@@ -499,6 +478,60 @@ __device__ __forceinline__ void router_select_rows(ParamsRef p, int t, unsigned 
     }
   }
   lds_wave_sync();
+}
+
+// The waits and trips to memory around that, where other workgroups' chains have left their logits in p.cand: winners of
+// the tokens 4*i .. 4*i+3 by one wave. Returns how many tokens they are, once their entries are in memory; 0 if the
+// wait failed. A wave's tokens are asked for together, and its caller counts them with one atomic: a counter takes 90
+// of those a microsecond, so that counting every token by itself, as a selection a wave does, held up the last
+// of 600 tokens by 7 us. target: chain tasks a token has.
+constexpr int SELECT_TOK = 4;
+__device__ __noinline__ int router_select4_task(ParamsRef pv, int i_in, unsigned target_in, unsigned char* scratch) {
+  ParamsRef p = uniform_params(pv);
+  const int T = __builtin_amdgcn_readfirstlane(p.T), E = __builtin_amdgcn_readfirstlane(p.E);
+  const unsigned target = __builtin_amdgcn_readfirstlane(target_in);
+  const int t0 = __builtin_amdgcn_readfirstlane(i_in) * SELECT_TOK;
+  const int lane = lane_id(), row = lane >> 4, r = lane & 15;
+  const int n = min(SELECT_TOK, T - t0);
+  {
+    const unsigned* mine = &p.tok_arrive[t0 + min(lane, n - 1)];
+    const long long since = wall_clock64();
+    for (unsigned spins = 1; __ballot(ld_relaxed(mine) < target) != 0ull; ++spins) {
+      if ((spins & 31u) == 0u && __ballot(ld_relaxed(&p.ctl->error.v) != 0u) != 0ull) return 0;
+      if (wall_clock64() - since > p.spin_limit) {
+        if (lane == 0) or_relaxed(&p.ctl->error.v, ERR_TIMEOUT);
+        return 0;
+      }
+      __builtin_amdgcn_s_sleep(8);
+    }
+    fence_acquire();
+  }
+  if (lane < n) stc(&p.tok_arrive[t0 + lane], 0u);
+  // (past the last token the buffer reads zeros, past a token's last expert the next one's)
+  const CoherentBuffer keys = coherent_buffer(p.cand + static_cast<size_t>(t0) * E, static_cast<unsigned>(n * E) * 4u);
+  const int t = row < n ? t0 + row : -1;
+  auto select = [&](auto& val) {
+    constexpr int EPL = sizeof(val) / 4;
+    uint4 v[EPL / 4];
+#pragma unroll
+    for (int j = 0; j < EPL / 4; ++j) v[j] = ld16_agent(keys, static_cast<unsigned>(row * E + EPL * r + 4 * j) * 4u);
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+      const uint4& w = v[j >> 2];
+      const unsigned x = (j & 3) == 0 ? w.x : (j & 3) == 1 ? w.y : (j & 3) == 2 ? w.z : w.w;
+      val[j] = EPL * r + j < E ? x : 0u;
+    }
+    router_select_rows<EPL>(p, t, val, scratch);
+  };
+  if (E <= 128) {
+    unsigned val[8];
+    select(val);
+  } else {
+    unsigned val[16];
+    select(val);
+  }
+  fence_release();
+  return n;
 }
 
 // ------------------------------------------------------------- scan / scatter

@@ -111,7 +111,7 @@ Layout make_layout(const FlashMoeLayerDesc& d, bool need_tiled) {
   L.masks = take(sizeof(unsigned long long) * d.experts * L.W);
   L.tok_arrive = take(sizeof(unsigned) * d.max_tokens);
   L.zero_bytes = off;
-  L.cand = take(sizeof(unsigned long long) * d.max_tokens * d.experts);
+  L.cand = take(sizeof(unsigned) * d.max_tokens * d.experts);
   L.word_prefix = take(sizeof(int) * d.experts * L.W);
   L.topk_idx = take(sizeof(int) * rows);
   L.topk_w = take(sizeof(float) * rows);
@@ -426,7 +426,7 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   p.wgflags = reinterpret_cast<fmoe::WgFlags*>(w + L.wgflags);
   p.g1_done = reinterpret_cast<fmoe::ControlLine*>(w + L.g1_done);
   p.tok_arrive = reinterpret_cast<unsigned*>(w + L.tok_arrive);
-  p.cand = reinterpret_cast<unsigned long long*>(w + L.cand);
+  p.cand = reinterpret_cast<unsigned*>(w + L.cand);
   p.masks = reinterpret_cast<unsigned long long*>(w + L.masks);
   p.word_prefix = reinterpret_cast<int*>(w + L.word_prefix);
   p.topk_idx = reinterpret_cast<int*>(w + L.topk_idx);

@@ -124,7 +124,7 @@ struct Params {
   Control* ctl;
   WgFlags* wgflags;                // [n_groups]
   ControlLine* g1_done;            // [max_mtiles] gate/up tasks finished per row tile
-  unsigned long long* cand;        // [T,E] router candidate keys
+  unsigned* cand;                  // [T,E] ordered_bits of the logits, from the chains to the selections
   unsigned* tok_arrive;            // [T] expert groups of the token whose keys are in
   int n_groups;                    // workgroups in the grid
   int fuse_scatter;                // 1: the scan task also writes the permutation

@@ -252,16 +252,19 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   const int ks1 = H / (4 * DT::EPV), ks2 = I / (4 * DT::EPV);  // steps of 64 bytes a row
   const int pull_from = (((lane & 15) << 2) | (lane >> 4)) << 2;
 
-  // ---- routing: logit chains on the first workgroups, then one select a wave there
+  // ---- routing: logit chains on the first workgroups, then selections there, four tokens a wave
   if (b < n_rt) {
     if constexpr (DT::EPV == 8) {
       router_dot16_task(p, b / n_eg, b % n_eg);
     } else {
       for (int q = b + n_rt * wave; q < n_dot; q += 8 * n_rt) router_dot_task<DT>(p, q / n_eg, q % n_eg);
     }
-    for (int t = b + n_rt * wave; t < T; t += 8 * n_rt) {
-      if (!wave_wait_ge(&p.tok_arrive[t], static_cast<unsigned>(n_eg), ctl, p.spin_limit)) break;
-      router_select_task(p, t);
+    for (int i = b + n_rt * wave; i * SELECT_TOK < T; i += 8 * n_rt) {
+      const int n = router_select4_task(p, i, static_cast<unsigned>(n_eg), lds + wave * (ROUTER_LDS_FLOATS * 4));
+      if (n == 0) break;
+      unsigned old = 0;
+      if (lane == 0) old = add_relaxed(&ctl->router_done.v, static_cast<unsigned>(n));
+      if (__builtin_amdgcn_readfirstlane(static_cast<int>(old)) + n == T) broadcast_flag(p, FLAG_ROUTED);
     }
   }
 

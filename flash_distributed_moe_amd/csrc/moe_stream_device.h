@@ -18,7 +18,7 @@ extern __shared__ __align__(16) float lds_dyn[];  // ROUTER_LDS_FLOATS per wave
 // one (token, expert) chain per lane. Token rows and expert rows arrive with
 // fully coalesced 16-byte loads, are converted to float once and staged in the
 // wave's private LDS slice in k-chunks, and feed one sequential chain per lane
-// (k ascending). Each chain ends as a 64-bit candidate key in HBM. A "select"
+// (k ascending). Each chain ends as a candidate's ordered_bits in HBM. A "select"
 // task per token waits for all of the token's expert groups and picks the
 // winners. (bf16 layers of suitable shape run the chains on the matrix core: router_dot16_task.)
 template <typename DT>
@@ -149,7 +149,7 @@ __device__ __noinline__ void router_dot_task(ParamsRef pv, int tg, int eg) {
   if (valid) {
     float v = acc;
     if (p.bias != nullptr) v = __fadd_rn(v, as_global(p.bias)[e]);
-    stc(&p.cand[static_cast<size_t>(t) * E + e], make_key(v, e, true));
+    stc(&p.cand[static_cast<size_t>(t) * E + e], ordered_bits(v, true));
   }
   fence_release();
   if (ei == 0 && t < T) add_relaxed(&p.tok_arrive[t], 1u);
@@ -160,8 +160,9 @@ __device__ __noinline__ void router_dot_task(ParamsRef pv, int tg, int eg) {
 // rounding each, so a chain of them is the same sequential sum (and a dependent
 // chain issues back to back, 32 cycles an instruction: 512 of them for H = 2048
 // against 2048 dependent FMAs on the vector unit). A whole workgroup takes 16
-// tokens x 16 experts: wave 0 only multiplies, waves 1..4 prepare its operands so
-// that it has nothing else to do: they load 32 bytes of a row (16 k), widen them
+// tokens x 16 experts: wave 0 only multiplies, four waves on the other SIMDs (the float matrix
+// instructions and the vector unit of a SIMD take turns: with wave 4, which shares wave 0's, among them one
+// token takes 45.0 us instead of 44.3) prepare its operands so that it has nothing else to do: they load 32 bytes of a row (16 k), widen them
 // to float and leave them in LDS in the order the instruction wants them: the 16
 // k of a group as [k % 4][row][k / 4], so lane l of the multiplying wave (row
 // l % 16, k % 4 = l / 16) reads its operand of four consecutive instructions with
@@ -230,15 +231,15 @@ __device__ __noinline__ void router_dot16_task(ParamsRef pv, int tg, int eg) {
         if (e < E) {
           float x = acc[v];
           if (p.bias != nullptr) x = __fadd_rn(x, as_global(p.bias)[e]);
-          stc(&p.cand[static_cast<size_t>(t) * E + e], make_key(x, e, true));
+          stc(&p.cand[static_cast<size_t>(t) * E + e], ordered_bits(x, true));
         }
       }
     }
     fence_release();
     if (lane < 16 && t < T) add_relaxed(&p.tok_arrive[t], 1u);
-  } else if (wave <= 4) {
+  } else if (wave <= 3 || wave == 5) {  // (waves w and w + 4 share a SIMD)
     // lane -> (row, group): four lanes cover 128 contiguous bytes of a row
-    const int hl = (wave - 1) * 64 + lane;
+    const int hl = min(wave - 1, 3) * 64 + lane;
     const int row = (hl & 63) >> 2;
     const int g = (hl >> 6) * 4 + (hl & 3);
     const unsigned short* wsrc = reinterpret_cast<const unsigned short*>(p.gate) +
@@ -293,11 +294,11 @@ __device__ __noinline__ void router_select_task(ParamsRef pv, int t) {
   ParamsRef p = uniform_params(pv);
   constexpr int MAXEPL = MAX_EXPERTS / 64;
   const int lane = lane_id();
-  unsigned val[MAXEPL];  // the ordered logit bits are the upper half of a candidate key
+  unsigned val[MAXEPL];
 #pragma unroll
   for (int j = 0; j < MAXEPL; ++j) {
     const int e = lane + 64 * j;
-    val[j] = e < p.E ? static_cast<unsigned>(ldc(&p.cand[static_cast<size_t>(t) * p.E + e]) >> 32) : 0u;
+    val[j] = e < p.E ? ldc(&p.cand[static_cast<size_t>(t) * p.E + e]) : 0u;
   }
   if (lane == 0) stc(&p.tok_arrive[t], 0u);
   router_select_max(p, t, val,

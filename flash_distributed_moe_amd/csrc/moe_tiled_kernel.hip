@@ -306,7 +306,7 @@ __device__ __noinline__ void tiled_router_task(ParamsRef pv, int blk) {
 // them in LDS in the order the instruction wants them (see router_dot16_task), two stages of 256 k, the
 // loads of four stages in flight. k past H counts as zero: a sum is never -0, so adding +0 leaves it.
 // Bound by the chains (512 dependent instructions of 32 cycles at H=2048). The logits go to memory
-// as candidate keys and any wave picks a token's winners once all its keys are in.
+// and a wave picks the winners of four tokens once theirs are in.
 constexpr int DOT32_AHEAD = 4;
 constexpr int DOT32_STAGE_BYTES = 3 * DOT16_OP_BYTES;  // experts 0..15, 16..31, tokens
 constexpr int DOT32_LDS_BYTES = 2 * DOT32_STAGE_BYTES;
@@ -361,7 +361,7 @@ __device__ __noinline__ void router_dot32_task(ParamsRef pv, int tg_in, int eg_i
           if (e < E) {
             float x = acc[v];
             if (p.bias != nullptr) x = __fadd_rn(x, as_global(p.bias)[e]);
-            stc(&p.cand[static_cast<size_t>(t) * E + e], make_key(x, e, true));
+            stc(&p.cand[static_cast<size_t>(t) * E + e], ordered_bits(x, true));
           }
         }
       }
@@ -430,53 +430,6 @@ __device__ __noinline__ void router_dot32_task(ParamsRef pv, int tg_in, int eg_i
     }
     lds_barrier();  // the multiplying waves have read everything: the LDS is free again
   }
-}
-
-// Winners of the tokens t, t + stride, ... of one wave, up to four at a time: their keys are asked
-// for together, and what was written is waited for once (one token after the other each costs
-// four trips to memory). Returns false if a wait failed.
-constexpr int SELECT_BATCH = 4;
-__device__ __noinline__ bool select_tokens_task(ParamsRef pv, int t_in, int stride_in) {
-  ParamsRef p = uniform_params(pv);
-  constexpr int MAXEPL = MAX_EXPERTS / 64;
-  const int T = uni(p.T), E = uni(p.E), stride = uni(stride_in), lane = lane_id();
-  const unsigned arrivals = static_cast<unsigned>((E + 15) >> 4);
-  double* lex = reinterpret_cast<double*>(lds_raw) + uni(static_cast<int>(threadIdx.x >> 6)) * MAX_TOPK;
-  unsigned done = 0;
-  for (int t0 = uni(t_in); t0 < T; t0 += SELECT_BATCH * stride) {
-    unsigned val[SELECT_BATCH][MAXEPL];
-#pragma unroll
-    for (int b = 0; b < SELECT_BATCH; ++b) {
-      const int t = t0 + b * stride;
-      if (t < T && !wave_wait_ge(&p.tok_arrive[t], arrivals, p.ctl, p.spin_limit)) return false;
-    }
-#pragma unroll
-    for (int b = 0; b < SELECT_BATCH; ++b) {
-      const int t = min(t0 + b * stride, T - 1);
-#pragma unroll
-      for (int j = 0; j < MAXEPL; ++j) {
-        const int e = lane + 64 * j;
-        // the ordered logit bits are the upper half of a candidate key
-        val[b][j] = e < E ? static_cast<unsigned>(ldc(&p.cand[static_cast<size_t>(t) * E + e]) >> 32) : 0u;
-      }
-    }
-#pragma unroll
-    for (int b = 0; b < SELECT_BATCH; ++b) {
-      const int t = t0 + b * stride;
-      if (t < T) {
-        if (lane == 0) stc(&p.tok_arrive[t], 0u);
-        router_select_max(p, t, val[b], lex);
-        ++done;
-      }
-    }
-  }
-  if (done != 0u) {
-    fence_release();
-    unsigned old = 0;
-    if (lane == 0) old = add_relaxed(&p.ctl->router_done.v, done);
-    if (uni(static_cast<int>(old)) + static_cast<int>(done) == T) broadcast_flag(p, FLAG_ROUTED);
-  }
-  return true;
 }
 
 // ------------------------------------------------------- the short scan and scatter
@@ -1630,11 +1583,19 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
         trace(i, 0, i, t0, t0);
       }
       const int sel_groups = min(n_dot, G);
-      const int t = b + sel_groups * wave;
-      if (b < sel_groups && t < Ti) {
+      const int i0 = b + sel_groups * wave;
+      if (b < sel_groups && i0 * SELECT_TOK < Ti) {
         const long long t0 = trace_clock(traced);
-        // (a wait that fails has raised an error bit, which every later wait sees)
-        if (select_tokens_task(p, t, WAVES * sel_groups)) trace_task(p, traced && lane_id() == 0, n_dot + t, 6, t, t0, t0);
+        unsigned done = 0;
+        for (int i = i0; i * SELECT_TOK < Ti; i += WAVES * sel_groups) {
+          const int n = router_select4_task(p, i, static_cast<unsigned>((p.E + 15) >> 4), lds_raw + wave * SELECT_ROWS_BYTES);
+          if (n == 0) break;  // (a wait that fails has raised an error bit, which every later wait sees)
+          done += n;
+        }
+        unsigned old = 0;
+        if (lane_id() == 0) old = add_relaxed(&ctl->router_done.v, done);
+        if (uni(static_cast<int>(old + done)) == Ti) broadcast_flag(p, FLAG_ROUTED);
+        trace_task(p, traced && lane_id() == 0, n_dot + i0, 6, i0 * SELECT_TOK, t0, t0);
       }
       t_perm0 = n_dot + WAVES * sel_groups;
     } else {
