@@ -71,13 +71,13 @@ constexpr long long kMaxRows = 1ll << 21;  // max_tokens * top_k a launcher may 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 struct Layout {
-  size_t ctl, wgflags, g1_done, tok_arrive, cand, topk_idx, topk_w, masks, word_prefix,
+  size_t ctl, wgflags, posts, g1_done, tok_arrive, cand, topk_idx, topk_w, masks, word_prefix,
       expert_count, expert_offset, perm, row_w, mtiles, h, y, xn, pack1, pack2, total;
   size_t zero_bytes;  // leading region that must be zero before a launch
   int W, max_mtiles;
 };
 
-constexpr int kMaxGroups = 1024;  // workgroups a launch may use (one per CU)
+constexpr int kMaxGroups = 512;  // workgroups a launch may use: one per CU of 256, float32 tiled two
 
 // AUTO hands a batch to the tiled variant from this many rows an expert on (on average; see auto_tiled_rows):
 // bf16, packed weights, which is what the streaming variant's share of `y` is sized for / the caller's row-major
@@ -107,6 +107,7 @@ Layout make_layout(const FlashMoeLayerDesc& d, bool need_tiled) {
   // zero-initialised region first: control block, per-tile counters, masks
   L.ctl = take(sizeof(fmoe::Control));
   L.wgflags = take(sizeof(fmoe::WgFlags) * kMaxGroups);
+  L.posts = take(sizeof(unsigned) * fmoe::POST_PHASES * fmoe::POST_COPIES * kMaxGroups);
   L.g1_done = take(sizeof(fmoe::ControlLine) * L.max_mtiles);
   L.masks = take(sizeof(unsigned long long) * d.experts * L.W);
   L.tok_arrive = take(sizeof(unsigned) * d.max_tokens);
@@ -424,6 +425,7 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   char* w = l->ws;
   p.ctl = reinterpret_cast<fmoe::Control*>(w + L.ctl);
   p.wgflags = reinterpret_cast<fmoe::WgFlags*>(w + L.wgflags);
+  p.posts = reinterpret_cast<unsigned*>(w + L.posts);
   p.g1_done = reinterpret_cast<fmoe::ControlLine*>(w + L.g1_done);
   p.tok_arrive = reinterpret_cast<unsigned*>(w + L.tok_arrive);
   p.cand = reinterpret_cast<unsigned*>(w + L.cand);
@@ -760,8 +762,7 @@ int flashMoeLaunchNoAlloc(const FlashMoeLayerDesc* desc, const void* tokens, voi
   // (what does not fit is refused before any device is asked for; where the number of CUs
   // decides between the variants, below 26 rows an expert, the workspaces differ by the padding of
   // h's rows at most, and the streaming variant runs where only its own fits)
-  l.num_cus = kMaxGroups;
-  int sched = sched_for(l.desc, tokens_num, machine(l));
+  int sched = sched_for(l.desc, tokens_num, Machine{1024, false});
   l.layout = make_layout(l.desc, sched == FLASH_MOE_SCHED_TILED);
   if (sched == FLASH_MOE_SCHED_TILED && (desc->sched == FLASH_MOE_SCHED_AUTO || !keeps_bf16_rows(l.desc)) &&
       l.layout.total > static_cast<size_t>(FLASH_MOE_NOALLOC_SCRATCH_BYTES)) {

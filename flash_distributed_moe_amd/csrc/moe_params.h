@@ -70,6 +70,11 @@ struct alignas(128) WgFlags {
   unsigned f[32];
 };
 
+// Split-k kernel: a word a workgroup and hand-over, raised by the workgroup that has done its share, in every one of
+// POST_COPIES rows; a workgroup watches one of those. Raised means the number of the launch, so nobody lowers it.
+enum : int { POST_GATE_UP = 0, POST_DOWN = 1, POST_PHASES = 2 };
+constexpr int POST_COPIES = 8;
+
 struct TileDesc {  // one row tile: `rows` consecutive permuted rows of one expert
   int expert;
   int row0;
@@ -123,6 +128,7 @@ struct Params {
                               // not ragged: bf16 rows without the weight
   Control* ctl;
   WgFlags* wgflags;                // [n_groups]
+  unsigned* posts;                 // [POST_PHASES][POST_COPIES][n_groups]
   ControlLine* g1_done;            // [max_mtiles] gate/up tasks finished per row tile
   unsigned* cand;                  // [T,E] ordered_bits of the logits, from the chains to the selections
   unsigned* tok_arrive;            // [T] expert groups of the token whose keys are in

@@ -251,6 +251,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   const int nt1 = I / (16 * G1_NB), nt2 = H / (16 * G2_NB);
   const int ks1 = H / (4 * DT::EPV), ks2 = I / (4 * DT::EPV);  // steps of 64 bytes a row
   const int pull_from = (((lane & 15) << 2) | (lane >> 4)) << 2;
+  const unsigned raised = ldc(&ctl->launches.v) + 1u;  // (the last workgroup out moves it on)
 
   // ---- routing: logit chains on the first workgroups, then selections there, four tokens a wave
   if (b < n_rt) {
@@ -536,12 +537,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   if (ok) {
     fence_release();
     lds_barrier();
-    if (wave == 0) {
-      unsigned old = 0;
-      if (lane == 0) old = add_relaxed(&ctl->perm_done.v, 1u);
-      old = __builtin_amdgcn_readfirstlane(old);
-      if (old == static_cast<unsigned>(G) - 1u) broadcast_flag(p, FLAG_PERM);
-    }
+    if (tid < POST_COPIES) stc(&p.posts[(POST_GATE_UP * POST_COPIES + tid) * G + b], raised);
     const SplitSteps sk2 = split_steps(ks2, sub, parts == 8 ? 3 : 2, p.split_spec != 0 && I * ESZ % 8192 != 0);
     const int steps2 = sk2.count;
     const int n_tasks = ntiles * per_tile;
@@ -598,7 +594,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
         st.template advance<true, false>(next_task);
         __builtin_amdgcn_sched_barrier(0);
       }
-      ok = wait_flag(p, FLAG_PERM, lds_flag, lds_poller);
+      ok = wait_posts(p, p.posts + (POST_GATE_UP * POST_COPIES + b % POST_COPIES) * G, G, raised, &lds_flag[FLAG_PERM], &lds_poller[FLAG_PERM]);
       if (ok) {
         const unsigned char* keep[st.NP];
 #pragma unroll
@@ -678,16 +674,11 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   if (ok) {
     fence_release();
     lds_barrier();
-    if (wave == 0) {
-      unsigned old = 0;
-      if (lane == 0) old = add_relaxed(&ctl->g2_done.v, 1u);
-      old = __builtin_amdgcn_readfirstlane(old);
-      if (old == static_cast<unsigned>(G) - 1u) broadcast_flag(p, FLAG_G2);
-    }
+    if (tid < POST_COPIES) stc(&p.posts[(POST_DOWN * POST_COPIES + tid) * G + b], raised);
     const unsigned ncomb = static_cast<unsigned>((H + COMBINE_COLS - 1) / COMBINE_COLS);
     const unsigned nc = static_cast<unsigned>(T) * ncomb;
     const unsigned slot = static_cast<unsigned>(wave * G + b);
-    if (slot < nc && wait_flag(p, FLAG_G2, lds_flag, lds_poller))
+    if (slot < nc && wait_posts(p, p.posts + (POST_DOWN * POST_COPIES + b % POST_COPIES) * G, G, raised, &lds_flag[FLAG_G2], &lds_poller[FLAG_G2]))
       combine_items<DT>(p, slot, nc, ncomb, static_cast<unsigned>(b * 8 + wave), 0u, 0);
   }
 
@@ -700,16 +691,10 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     if (__builtin_amdgcn_readfirstlane(last) != 0u) {
       const unsigned err = ldc(&ctl->error.v);
       if (err != 0u) recover_after_error(p, err, lane, 64);
-      for (int q = lane; q < p.n_groups; q += 64) {
-        stc(&p.wgflags[q].f[FLAG_PERM], 0u);
-        stc(&p.wgflags[q].f[FLAG_G2], 0u);
-        stc(&p.wgflags[q].f[FLAG_ROUTED], 0u);
-      }
+      for (int q = lane; q < G; q += 64) stc(&p.wgflags[q].f[FLAG_ROUTED], 0u);
       if (lane == 0) {
         stc(&ctl->launches.v, ldc(&ctl->launches.v) + 1u);
         stc(&ctl->router_done.v, 0u);
-        stc(&ctl->perm_done.v, 0u);
-        stc(&ctl->g2_done.v, 0u);
         stc(&ctl->exit_count.v, 0u);
       }
     }

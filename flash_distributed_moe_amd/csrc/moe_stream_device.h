@@ -360,6 +360,55 @@ __device__ __forceinline__ bool wait_flag(ParamsRef p, int which, unsigned* lds_
   return ok != 0;
 }
 
+// The same wait for the first n of a row of posts: the polling wave reads all of them at once, so that nobody counts.
+// (A counter takes 90 atomics a microsecond: with 256 workgroups the last one waited up to 3 us for its turn, then
+// for the count to come back and for the flags it raised.)
+__device__ __forceinline__ bool wait_posts(ParamsRef p, const unsigned* posts, int n, unsigned raised, unsigned* lds_flag,
+                                           unsigned* lds_poller) {
+  const int lane = lane_id();
+  unsigned state = 0u;  // 1: all raised, 2: failed, 3: this wave polls
+  if (lane == 0) {
+    while (true) {
+      state = __hip_atomic_load(lds_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (state != 0u) break;
+      if (__hip_atomic_exchange(lds_poller, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u) {
+        state = 3u;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(8);
+    }
+  }
+  state = __builtin_amdgcn_readfirstlane(state);
+  if (state == 3u) {
+    const CoherentBuffer words = coherent_buffer(posts, static_cast<unsigned>(n) * 4u);
+    const long long t0 = wall_clock64();
+    unsigned spins = 0;
+    state = 1u;
+    int at = 4 * lane;  // this lane's next words that may be missing
+    while (true) {
+      if (at < n) {
+        const uint4 v = ld16_agent(words, static_cast<unsigned>(at) * 4u);
+        const bool missing = v.x != raised || (at + 1 < n && v.y != raised) || (at + 2 < n && v.z != raised) || (at + 3 < n && v.w != raised);
+        if (!missing) at += 256;
+      }
+      if (__ballot(at < n) == 0ull) break;
+      if ((++spins & 31u) == 0u && __builtin_amdgcn_readfirstlane(ld_relaxed(&p.ctl->error.v)) != 0u) {
+        state = 2u;
+        break;
+      }
+      if (wall_clock64() - t0 > p.spin_limit) {
+        if (lane == 0) or_relaxed(&p.ctl->error.v, ERR_TIMEOUT);
+        state = 2u;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(8);
+    }
+    if (lane == 0) __hip_atomic_store(lds_flag, state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  fence_acquire();
+  return state == 1u;
+}
+
 // ---------------------------------------------------------- row-major weights
 // Fragments of the caller's row-major weights: a fragment wants lane l to hold row l % 16,
 // 16-byte chunk l / 16 of a 64-byte row segment, which read that way makes every lane of a
