@@ -154,6 +154,14 @@ __device__ __forceinline__ void broadcast_flag(ParamsRef p, int which) {
   for (int g = lane_id(); g < n; g += 64) st_relaxed(&flags[g].f[which], 1u);
 }
 
+// A wave raises one post (see moe_params.h); what it stands for has to be in memory.
+__device__ __forceinline__ unsigned* post_row(ParamsRef p, int phase, int copy) {
+  return p.posts + (phase * POST_COPIES + copy) * POST_PITCH;
+}
+__device__ __forceinline__ void raise_post(ParamsRef p, int phase, int index, unsigned raised) {
+  if (lane_id() < POST_COPIES) stc(post_row(p, phase, lane_id()) + index, raised);
+}
+
 // A launch that raised an error bit (a bounded wait ran out, the tile table overflowed) has
 // left counters, masks and outputs in an arbitrary state. The last worker to leave makes
 // the failure visible and the launcher usable again without any help from the host, which
@@ -431,10 +439,10 @@ __device__ __forceinline__ unsigned row_max_u32(unsigned v) {
   v = step(v, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xF, 0xF, true)));  // mirror in 16
   return v;
 }
-template <int EPL>
-__device__ __forceinline__ void router_select_rows(ParamsRef p, int t, unsigned (&val)[EPL], unsigned char* scratch) {
+// emit(token, slot, expert or -1, weight) is called for each of the row's slots, by some lane.
+template <int EPL, typename Emit>
+__device__ __forceinline__ void router_select_rows(int K, int t, unsigned (&val)[EPL], unsigned char* scratch, Emit emit) {
   const int lane = lane_id(), row = lane >> 4, r = lane & 15;
-  const int K = p.K;
   double* ex = reinterpret_cast<double*>(scratch);                        // [4][MAX_TOPK]
   uint2* won = reinterpret_cast<uint2*>(scratch + 4 * MAX_TOPK * 8);      // [4][MAX_TOPK]: expert (or -1), ordered bits
   // lanes of this row in front of this one
@@ -471,13 +479,36 @@ __device__ __forceinline__ void router_select_rows(ParamsRef p, int t, unsigned 
       for (int u = 0; u < K; ++u) sum += ex[q * MAX_TOPK + u];
       const float w = sum <= 0.0 ? static_cast<float>(1.0 / static_cast<double>(K))
                                  : static_cast<float>(ex[q * MAX_TOPK + s] / sum);
-      const int e = static_cast<int>(won[q * MAX_TOPK + s].x);
-      stc(&p.topk_idx[static_cast<size_t>(tq) * K + s], e);
-      stc(&p.topk_w[static_cast<size_t>(tq) * K + s], w);
-      if (e >= 0) or_relaxed(&p.masks[static_cast<size_t>(e) * p.W + (tq >> 6)], 1ull << (tq & 63));
+      emit(tq, s, static_cast<int>(won[q * MAX_TOPK + s].x), w);
     }
   }
   lds_wave_sync();
+}
+// ... into the routing tables in memory
+template <int EPL>
+__device__ __forceinline__ void router_select_rows(ParamsRef p, int t, unsigned (&val)[EPL], unsigned char* scratch) {
+  router_select_rows<EPL>(p.K, t, val, scratch, [&](int tq, int s, int e, float w) {
+    stc(&p.topk_idx[static_cast<size_t>(tq) * p.K + s], e);
+    stc(&p.topk_w[static_cast<size_t>(tq) * p.K + s], w);
+    if (e >= 0) or_relaxed(&p.masks[static_cast<size_t>(e) * p.W + (tq >> 6)], 1ull << (tq & 63));
+  });
+}
+
+// The logits of the tokens t0 .. t0+n-1 (n <= 4) that chains elsewhere have left in memory, as router_select_rows wants
+// them. (Past the last token the buffer reads zeros, past a token's last expert the next one's.)
+template <int EPL>
+__device__ __forceinline__ void load_row_keys(ParamsRef p, int t0, int n, unsigned (&val)[EPL]) {
+  const int lane = lane_id(), row = lane >> 4, r = lane & 15, E = p.E;
+  const CoherentBuffer keys = coherent_buffer(p.cand + static_cast<size_t>(t0) * E, static_cast<unsigned>(n * E) * 4u);
+  uint4 v[EPL / 4];
+#pragma unroll
+  for (int j = 0; j < EPL / 4; ++j) v[j] = ld16_agent(keys, static_cast<unsigned>(row * E + EPL * r + 4 * j) * 4u);
+#pragma unroll
+  for (int j = 0; j < EPL; ++j) {
+    const uint4& w = v[j >> 2];
+    const unsigned x = (j & 3) == 0 ? w.x : (j & 3) == 1 ? w.y : (j & 3) == 2 ? w.z : w.w;
+    val[j] = EPL * r + j < E ? x : 0u;
+  }
 }
 
 // The waits and trips to memory around that, where other workgroups' chains have left their logits in p.cand: winners of
@@ -491,7 +522,7 @@ __device__ __noinline__ int router_select4_task(ParamsRef pv, int i_in, unsigned
   const int T = __builtin_amdgcn_readfirstlane(p.T), E = __builtin_amdgcn_readfirstlane(p.E);
   const unsigned target = __builtin_amdgcn_readfirstlane(target_in);
   const int t0 = __builtin_amdgcn_readfirstlane(i_in) * SELECT_TOK;
-  const int lane = lane_id(), row = lane >> 4, r = lane & 15;
+  const int lane = lane_id(), row = lane >> 4;
   const int n = min(SELECT_TOK, T - t0);
   {
     const unsigned* mine = &p.tok_arrive[t0 + min(lane, n - 1)];
@@ -507,28 +538,15 @@ __device__ __noinline__ int router_select4_task(ParamsRef pv, int i_in, unsigned
     fence_acquire();
   }
   if (lane < n) stc(&p.tok_arrive[t0 + lane], 0u);
-  // (past the last token the buffer reads zeros, past a token's last expert the next one's)
-  const CoherentBuffer keys = coherent_buffer(p.cand + static_cast<size_t>(t0) * E, static_cast<unsigned>(n * E) * 4u);
   const int t = row < n ? t0 + row : -1;
-  auto select = [&](auto& val) {
-    constexpr int EPL = sizeof(val) / 4;
-    uint4 v[EPL / 4];
-#pragma unroll
-    for (int j = 0; j < EPL / 4; ++j) v[j] = ld16_agent(keys, static_cast<unsigned>(row * E + EPL * r + 4 * j) * 4u);
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) {
-      const uint4& w = v[j >> 2];
-      const unsigned x = (j & 3) == 0 ? w.x : (j & 3) == 1 ? w.y : (j & 3) == 2 ? w.z : w.w;
-      val[j] = EPL * r + j < E ? x : 0u;
-    }
-    router_select_rows<EPL>(p, t, val, scratch);
-  };
   if (E <= 128) {
     unsigned val[8];
-    select(val);
+    load_row_keys<8>(p, t0, n, val);
+    router_select_rows<8>(p, t, val, scratch);
   } else {
     unsigned val[16];
-    select(val);
+    load_row_keys<16>(p, t0, n, val);
+    router_select_rows<16>(p, t, val, scratch);
   }
   fence_release();
   return n;

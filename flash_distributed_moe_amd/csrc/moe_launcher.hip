@@ -78,6 +78,7 @@ struct Layout {
 };
 
 constexpr int kMaxGroups = 512;  // workgroups a launch may use: one per CU of 256, float32 tiled two
+static_assert(kMaxGroups <= fmoe::POST_PITCH, "posts of a launch");
 
 // AUTO hands a batch to the tiled variant from this many rows an expert on (on average; see auto_tiled_rows):
 // bf16, packed weights, which is what the streaming variant's share of `y` is sized for / the caller's row-major
@@ -107,7 +108,7 @@ Layout make_layout(const FlashMoeLayerDesc& d, bool need_tiled) {
   // zero-initialised region first: control block, per-tile counters, masks
   L.ctl = take(sizeof(fmoe::Control));
   L.wgflags = take(sizeof(fmoe::WgFlags) * kMaxGroups);
-  L.posts = take(sizeof(unsigned) * fmoe::POST_PHASES * fmoe::POST_COPIES * kMaxGroups);
+  L.posts = take(sizeof(unsigned) * fmoe::POST_PHASES * fmoe::POST_COPIES * fmoe::POST_PITCH);
   L.g1_done = take(sizeof(fmoe::ControlLine) * L.max_mtiles);
   L.masks = take(sizeof(unsigned long long) * d.experts * L.W);
   L.tok_arrive = take(sizeof(unsigned) * d.max_tokens);
@@ -372,6 +373,7 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   if (p.split) {
     p.early = 1;
     p.split_spec = reaches_experts ? 1 : 0;
+    p.split_self = T <= fmoe::SPLIT_SELF_TOKENS;
     // a down task in four parts, two of them to a workgroup, unless that leaves CUs without one or (float32) the
     // number of 64-column tasks is odd
     const bool eight_steps = d.intermediate >= (d.dtype == FLASH_MOE_BF16 ? 256 : 128);

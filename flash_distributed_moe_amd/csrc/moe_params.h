@@ -28,6 +28,7 @@ constexpr int DOT16_KC = 256;    // streaming variant, matrix-core router: k per
 constexpr int SCAN_LDS_WORDS = 1024;  // mask words (experts x 64-token words) the small-batch scan keeps in LDS
 constexpr int SHORT_MASK_WORDS = 8192;  // the same for the tiled kernel's short prologue
 constexpr int SPLIT_MAX_SLOTS = 2048;  // split-k kernel: (token, slot) entries its tables hold
+constexpr int SPLIT_SELF_TOKENS = 32;  // ... tokens every workgroup may pick the winners of by itself
 constexpr int EARLY_MAX_TOKENS = 384;  // batches up to this size may take their gate/up weights before the routing is known
 // Shapes whose columns do not divide into the bf16 tiled variant's tasks (256 of H, 128 of I): kernels of
 // their own, which keep y as the streaming variant does (see tile_task).
@@ -72,8 +73,10 @@ struct alignas(128) WgFlags {
 
 // Split-k kernel: a word a workgroup and hand-over, raised by the workgroup that has done its share, in every one of
 // POST_COPIES rows; a workgroup watches one of those. Raised means the number of the launch, so nobody lowers it.
-enum : int { POST_GATE_UP = 0, POST_DOWN = 1, POST_PHASES = 2 };
+// (POST_ROUTE: a word a routing task.)
+enum : int { POST_ROUTE = 0, POST_GATE_UP = 1, POST_DOWN = 2, POST_PHASES = 3 };
 constexpr int POST_COPIES = 8;
+constexpr int POST_PITCH = 512;  // words of a row
 
 struct TileDesc {  // one row tile: `rows` consecutive permuted rows of one expert
   int expert;
@@ -128,7 +131,7 @@ struct Params {
                               // not ragged: bf16 rows without the weight
   Control* ctl;
   WgFlags* wgflags;                // [n_groups]
-  unsigned* posts;                 // [POST_PHASES][POST_COPIES][n_groups]
+  unsigned* posts;                 // [POST_PHASES][POST_COPIES][POST_PITCH]
   ControlLine* g1_done;            // [max_mtiles] gate/up tasks finished per row tile
   unsigned* cand;                  // [T,E] ordered_bits of the logits, from the chains to the selections
   unsigned* tok_arrive;            // [T] expert groups of the token whose keys are in
@@ -139,6 +142,7 @@ struct Params {
   int split;                       // 1, 2: the split-k kernel runs, on tiles of so many 16-row blocks
   int split_spec;                  //    1: its workgroups ask for gate/up weights before the routing is known
   int split_down;                  //    waves that share a down task: 4 or 8
+  int split_self;                  //    every workgroup picks all tokens' winners for itself
   int dot16;                       // 1 (streaming variant, bf16): the logit chains run on the matrix core, 16 tokens x
                                    //    16 experts per workgroup, on the first workgroups before they take tickets;
                                    //    bf16 tiled variant: how it starts (see the launcher)

@@ -12,12 +12,13 @@
 // (equal shares of equal tasks), the routing tables are built by every workgroup for itself in
 // LDS from the top-k entries, and there is one grid-wide dependency between gate/up and down,
 // under which the first window of down weights is on its way. T=64 on the 30B shape, us from the
-// launch's first workgroup: routed 21, tables 24, gate/up done 119 to 141, h everywhere 144, down
+// launch's first workgroup (before workgroups posted their arrivals): routed 21, tables 24, gate/up done 119 to 141, h everywhere 144, down
 // done 204, out 208.
 //
 // Bound by HBM from some 16 tokens on, below by the chain of waits (logit chains 14 us, selection,
 // gate/up, down, combine). Against the streaming kernel, us, 30B shape, weights packed in place:
-// T=1 59.5 -> 42 (routed 16, tables 19, gate/up 28, h everywhere 32, down 34), T=8 120 -> 103, T=16 164 -> 150, T=64 225 -> 217 (1.19 GB: 5.5 TB/s), T=128 243 -> 223,
+// T=1 59.5 -> 42 (routed 16, tables 19, gate/up 28, h everywhere 32, down 34; since every workgroup routes small
+// batches for itself and posts its arrivals, 44.4 -> 40.2 in a row of passes), T=8 120 -> 103, T=16 164 -> 150, T=64 225 -> 217 (1.19 GB: 5.5 TB/s), T=128 243 -> 223,
 // T=200 266 -> 234, T=256 275 -> 241; row-major T=32 249 -> 226, T=128 290 -> 261; 235B T=1 102 -> 87,
 // T=64 759 -> 762, T=256 876 -> 836. Four hot experts: T=16 146 -> 120, T=128 317 -> 240 (a tile of more
 // rows than an early task carries starts over there; here it is several tiles).
@@ -58,6 +59,10 @@ constexpr int split_lds_bytes(int rb) {
   return n > 8 * ROUTER_LDS_FLOATS * 4 ? n : 8 * ROUTER_LDS_FLOATS * 4;
 }
 static_assert(split_lds_bytes(2) + 64 <= 160 * 1024, "LDS of a workgroup");
+// small batches' winners, and what the waves need to find them, where the partial sums go later
+constexpr int SPLIT_SELF_OFF = SPLIT_PART_OFF;
+constexpr int SPLIT_SELECT_OFF = SPLIT_SELF_OFF + SPLIT_SELF_TOKENS * MAX_TOPK * 8;
+static_assert(SPLIT_SELECT_OFF + 8 * SELECT_ROWS_BYTES <= split_lds_bytes(1), "winners exceed the partial sums");
 
 // Which steps of a task's k a wave takes. `runs` false (batches that leave most experts unused: a CU has
 // a task at most): one of `parts` equal stretches. Otherwise every parts-th run of four steps (256 bytes of a
@@ -253,19 +258,21 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   const int pull_from = (((lane & 15) << 2) | (lane >> 4)) << 2;
   const unsigned raised = ldc(&ctl->launches.v) + 1u;  // (the last workgroup out moves it on)
 
-  // ---- routing: logit chains on the first workgroups, then selections there, four tokens a wave
+  // ---- routing: logit chains on the first workgroups, then (batches of more than SPLIT_SELF_TOKENS) selections there,
+  // four tokens a wave. Smaller batches have every workgroup pick all winners for itself, below: that saves the
+  // entries' way to memory and back and a wait in between (us, without / with: one token 41.8 / 40.2, T=11 123.2 /
+  // 120.9, E=8, H=256 float32 T=16 24.4 / 23.1; but T=40 199.1 / 200.3, T=64 205.7 / 207.6, H=512, E=64 float32 T=64 44.1 /
+  // 45.5).
+  const bool self = p.split_self != 0;
   if (b < n_rt) {
     if constexpr (DT::EPV == 8) {
-      router_dot16_task(p, b / n_eg, b % n_eg);
+      router_dot16_task(p, b / n_eg, b % n_eg, self ? b : -1, raised);
     } else {
-      for (int q = b + n_rt * wave; q < n_dot; q += 8 * n_rt) router_dot_task<DT>(p, q / n_eg, q % n_eg);
+      for (int q = b + n_rt * wave; q < n_dot; q += 8 * n_rt) router_dot_task<DT>(p, q / n_eg, q % n_eg, self ? q : -1, raised);
     }
-    for (int i = b + n_rt * wave; i * SELECT_TOK < T; i += 8 * n_rt) {
-      const int n = router_select4_task(p, i, static_cast<unsigned>(n_eg), lds + wave * (ROUTER_LDS_FLOATS * 4));
-      if (n == 0) break;
-      unsigned old = 0;
-      if (lane == 0) old = add_relaxed(&ctl->router_done.v, static_cast<unsigned>(n));
-      if (__builtin_amdgcn_readfirstlane(static_cast<int>(old)) + n == T) broadcast_flag(p, FLAG_ROUTED);
+    for (int i = b + n_rt * wave; !self && i * SELECT_TOK < T; i += 8 * n_rt) {
+      if (router_select4_task(p, i, static_cast<unsigned>(n_eg), lds + wave * (ROUTER_LDS_FLOATS * 4)) == 0) break;
+      raise_post(p, POST_ROUTE, i, raised);
     }
   }
 
@@ -324,20 +331,50 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     }
 
     // ---- tables, by every workgroup for itself
-    ok = wait_flag(p, FLAG_ROUTED, lds_flag, lds_poller);
+    ok = wait_posts(p, post_row(p, POST_ROUTE, b % POST_COPIES), self ? n_dot : (T + SELECT_TOK - 1) / SELECT_TOK, raised,
+                    &lds_flag[FLAG_ROUTED], &lds_poller[FLAG_ROUTED]);
     const int wact = (T + 63) >> 6;
     const int n = T * K;
     lds_barrier();  // the routing tasks' use of the LDS is over
+    int* self_idx = reinterpret_cast<int*>(lds + SPLIT_SELF_OFF);                        // [T][K]
+    float* self_w = reinterpret_cast<float*>(self_idx + SPLIT_SELF_TOKENS * MAX_TOPK);
+    if (self) {
+      for (int e = tid; e < E; e += 512) lmask[e] = 0ull;
+      lds_barrier();
+      for (int i = wave; ok && i * SELECT_TOK < T; i += 8) {
+        const int t0 = i * SELECT_TOK, nt = min(SELECT_TOK, T - t0), t = (lane >> 4) < nt ? t0 + (lane >> 4) : -1;
+        auto emit = [&](int tq, int s, int e, float w) {
+          self_idx[tq * K + s] = e;
+          self_w[tq * K + s] = w;
+          if (e >= 0) atomicOr(&lmask[e], 1ull << tq);
+          if (b == G - 1) {  // (what the host may read back)
+            stc(&p.topk_idx[tq * K + s], e);
+            stc(&p.topk_w[tq * K + s], w);
+          }
+        };
+        unsigned char* scratch = lds + SPLIT_SELECT_OFF + wave * SELECT_ROWS_BYTES;
+        if (E <= 128) {
+          unsigned val[8];
+          load_row_keys<8>(p, t0, nt, val);
+          router_select_rows<8>(K, t, val, scratch, emit);
+        } else {
+          unsigned val[16];
+          load_row_keys<16>(p, t0, nt, val);
+          router_select_rows<16>(K, t, val, scratch, emit);
+        }
+      }
+      lds_barrier();
+    }
     int ee[SPLIT_MAX_SLOTS / 512];
     float ww[SPLIT_MAX_SLOTS / 512];
     if (ok) {
 #pragma unroll
       for (int q = 0; q < SPLIT_MAX_SLOTS / 512; ++q) {
         const int i = tid + 512 * q;
-        ee[q] = i < n ? ldc(&p.topk_idx[i]) : -1;
-        ww[q] = i < n ? ldc(&p.topk_w[i]) : 0.0f;
+        ee[q] = i >= n ? -1 : self ? self_idx[i] : ldc(&p.topk_idx[i]);
+        ww[q] = i >= n ? 0.0f : self ? self_w[i] : ldc(&p.topk_w[i]);
       }
-      for (int i = tid; i < E * wact; i += 512) lmask[i] = ldc(&p.masks[static_cast<size_t>(i / wact) * W + i % wact]);
+      for (int i = tid; !self && i < E * wact; i += 512) lmask[i] = ldc(&p.masks[static_cast<size_t>(i / wact) * W + i % wact]);
     }
     lds_barrier();
     if (ok && wave == 0) {
@@ -537,7 +574,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   if (ok) {
     fence_release();
     lds_barrier();
-    if (tid < POST_COPIES) stc(&p.posts[(POST_GATE_UP * POST_COPIES + tid) * G + b], raised);
+    if (wave == 0) raise_post(p, POST_GATE_UP, b, raised);
     const SplitSteps sk2 = split_steps(ks2, sub, parts == 8 ? 3 : 2, p.split_spec != 0 && I * ESZ % 8192 != 0);
     const int steps2 = sk2.count;
     const int n_tasks = ntiles * per_tile;
@@ -594,7 +631,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
         st.template advance<true, false>(next_task);
         __builtin_amdgcn_sched_barrier(0);
       }
-      ok = wait_posts(p, p.posts + (POST_GATE_UP * POST_COPIES + b % POST_COPIES) * G, G, raised, &lds_flag[FLAG_PERM], &lds_poller[FLAG_PERM]);
+      ok = wait_posts(p, post_row(p, POST_GATE_UP, b % POST_COPIES), G, raised, &lds_flag[FLAG_PERM], &lds_poller[FLAG_PERM]);
       if (ok) {
         const unsigned char* keep[st.NP];
 #pragma unroll
@@ -674,11 +711,11 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   if (ok) {
     fence_release();
     lds_barrier();
-    if (tid < POST_COPIES) stc(&p.posts[(POST_DOWN * POST_COPIES + tid) * G + b], raised);
+    if (wave == 0) raise_post(p, POST_DOWN, b, raised);
     const unsigned ncomb = static_cast<unsigned>((H + COMBINE_COLS - 1) / COMBINE_COLS);
     const unsigned nc = static_cast<unsigned>(T) * ncomb;
     const unsigned slot = static_cast<unsigned>(wave * G + b);
-    if (slot < nc && wait_posts(p, p.posts + (POST_DOWN * POST_COPIES + b % POST_COPIES) * G, G, raised, &lds_flag[FLAG_G2], &lds_poller[FLAG_G2]))
+    if (slot < nc && wait_posts(p, post_row(p, POST_DOWN, b % POST_COPIES), G, raised, &lds_flag[FLAG_G2], &lds_poller[FLAG_G2]))
       combine_items<DT>(p, slot, nc, ncomb, static_cast<unsigned>(b * 8 + wave), 0u, 0);
   }
 
@@ -691,10 +728,8 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     if (__builtin_amdgcn_readfirstlane(last) != 0u) {
       const unsigned err = ldc(&ctl->error.v);
       if (err != 0u) recover_after_error(p, err, lane, 64);
-      for (int q = lane; q < G; q += 64) stc(&p.wgflags[q].f[FLAG_ROUTED], 0u);
       if (lane == 0) {
         stc(&ctl->launches.v, ldc(&ctl->launches.v) + 1u);
-        stc(&ctl->router_done.v, 0u);
         stc(&ctl->exit_count.v, 0u);
       }
     }

@@ -304,12 +304,16 @@ def test_tiled_starts(T, H, E, k):
     (4099, 192, 128, 32, _lib.SCHED_TILED),  # 32-token router tasks, the last of 3 tokens; the most slots
     (4100, 128, 200, 17, _lib.SCHED_TILED),  # two slabs of experts, the second partly empty; more slots than a row has lanes
     (2100, 64, 40, 5, _lib.SCHED_TILED),     # 16-token tasks of one stage; the last of 4 tokens
+    (601, 128, 200, 17, _lib.SCHED_TILED),   # selections spread over the workgroups, the last of one token
+    (32, 256, 200, 32, _lib.SCHED_AUTO),     # split-k kernel: every workgroup picks the winners, four tokens to each of its waves
+    (33, 256, 120, 17, _lib.SCHED_AUTO),     # the first size whose winners are picked once
+    (1, 256, 97, 32, _lib.SCHED_AUTO),
 ])
 @pytest.mark.parametrize("admitted", ["all", "three"])
 def test_router_winners(T, H, E, k, sched, admitted):
     """Equal logits (every expert's row of the router weights twice, so the lower index wins) and experts that
     are never admitted (a bias of -inf leaves three, fewer than k): winners and weights against the oracle."""
-    cfg = synth.MoeConfig("winners", T, H, E, k, 64, "bf16")
+    cfg = synth.MoeConfig("winners", T, H, E, k, 128, "bf16")
     print("winners", T, H, E, k, sched, admitted, flush=True)
     inp = synth.make_inputs_torch(cfg, T + k, torch.device("cuda:0"))
     inp["gate"][E // 2:2 * (E // 2)] = inp["gate"][:E // 2].clone()
