@@ -383,17 +383,20 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
                        : 4;
   }
   const bool tiled = sched_for(d, T, m) == FLASH_MOE_SCHED_TILED;
-  // How the bf16 tiled kernel starts. 1: logit chains of 16 tokens x 32 experts a workgroup, in two rounds
-  // at most, and selections spread over all waves of the workgroups that had a chain, while that is two of them a wave
-  // at most if every workgroup had one (of 1536 tokens and 32 experts 96 have: four a wave) (30B shape, us,
-  // without / with: T=450 300 / 282, T=600 302 / 285, T=900 312 / 299, T=1500 330 / 325, T=2048 353 / 356;
-  // E=256, H=1024, I=512, T=1024 242 / 231; E=16, k=2, H=320, I=160, T=4000 74 / 78). 2: router tasks of 16
-  // or 32 tokens x all experts. Both without a scan phase, while the mask words fit LDS (as 2 against 0:
+  // How the bf16 tiled kernel starts. 1: logit chains of 16 tokens x 32 experts a workgroup, and selections spread over
+  // the waves of the workgroups that had a chain. 2: router tasks of 16 or 32 tokens x all experts, which select for
+  // themselves: chains twice as long (15 us for 7 at H=2048) and some 4 us of trips to memory less. So 1 while one
+  // round of its tasks does and the chains are long enough (us, 1 / 2, 30B shape: T=450 266.0 / 273.6, T=600 270.9 /
+  // 277.6, T=900 277.9 / 283.6, two rounds T=1200 300.7 / 296.6, T=1500 309.4 / 304.1; 235B shape T=700 942 / 959;
+  // E=64, k=4, I=512: H=512 T=1000 65.0 / 64.0, H=1024 T=700 79.4 / 81.2, H=1536 T=700 104.6 / 109.1; E=32, H=768 T=800 55.3 /
+  // 56.5; E=16, H=320 T=1200 56.5 / 53.7) and a selecting wave has one or two tasks. Both without a scan phase, while the mask words fit LDS (as 2 against 0:
   // T=2048 345 / 340, row-major 359 / 355; E=16 T=4000 74 / 70). 0: tickets for all of it.
   if (tiled && d.dtype == FLASH_MOE_BF16) {
+    const int chain_k = d.hidden * ((d.experts + 127) / 128);  // of a router task of all experts
     p.dot16 = d.experts * ((T + 63) / 64) > fmoe::SHORT_MASK_WORDS || T > 65535 ? 0
-              : T <= 6 * m.n_groups && ((T + 15) / 16) * ((d.experts + 31) / 32) <= 2 * m.n_groups ? 1
-                                                                                                  : 2;
+              : T <= 6 * m.n_groups && chain_k >= 768 && ((T + 15) / 16) * ((d.experts + 31) / 32) <= m.n_groups
+                  ? 1
+                  : 2;
     p.early = p.dot16;  // (the last selection raises FLAG_ROUTED)
     p.n_workers = p.n_groups * 4;
   }

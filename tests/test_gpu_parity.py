@@ -283,6 +283,11 @@ def test_tiled_ragged_equals_the_streaming_variant(T, H, E, k, I, hot, edges, pa
     (1000, 512, 256, 6),    # two rounds of 16-token x 32-expert tasks
     (2048, 128, 256, 2),    # the last size whose mask words fit LDS
     (2049, 128, 256, 2),    # the first whose do not
+    (40, 768, 17, 3),       # spread-out chains: the least H; a group of experts with one expert
+    (1000, 832, 33, 2),     # a last 256-k stage that is partly empty
+    (1024, 768, 100, 4),    # 256 workgroups with a chain task each
+    (1025, 768, 100, 4),    # one task too many for that
+    (300, 384, 200, 6),     # two slabs of experts count twice
 ])
 def test_tiled_starts(T, H, E, k):
     """The ways the tiled kernel gets from tokens to row tiles, at the edges of their ranges: routing
