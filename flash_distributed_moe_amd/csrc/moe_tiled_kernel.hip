@@ -1092,6 +1092,26 @@ __device__ __forceinline__ uint4 pair_columns(uint2 a, uint2 b) {
   return make_uint4(a.x, a.y, b.x, b.y);
 }
 __device__ __forceinline__ unsigned pair_column(int kg) { return static_cast<unsigned>((kg & 1) * 16 + (kg >> 1) * 8); }
+// Tiles of more than 256 rows go through LDS instead, where rows become whole again: they come in numbers, from experts
+// that draw far more tokens than others, and there whole rows are ahead (30B shape, four hot experts, T=16384, us, half
+// lines / whole rows: 1387 / 1374; tiles of up to 256 rows, T=8192: 736 / 738). What they gain was only measured as time.
+constexpr int EPI_LD = TN * 2 + 16;  // bytes per row of the down slab
+static_assert(128 * EPI_LD <= TILE_LDS_BYTES && TM_MAX * (G1_COLS * 2 + 16) <= TILE_LDS_BYTES, "epilogue slab exceeds the stage buffers");
+// eight rows' reads first, then their stores: a store's assembly orders memory operations around it, and one LDS round
+// trip a store would add up to microseconds
+template <int N, typename Read, typename Store>
+__device__ __forceinline__ void for_rows(Read read, Store store) {
+#pragma unroll
+  for (int i0 = 0; i0 < N; i0 += 8) {
+    uint4 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i0 + u < N) v[u] = read(i0 + u);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i0 + u < N) store(i0 + u, v[u]);
+  }
+}
 // st16_through at a uniform base and a lane's offset
 __device__ __forceinline__ void st16_through_at(unsigned char* base, unsigned off, const uint4& v) {
   const v4u_t d = {v.x, v.y, v.z, v.w};
@@ -1239,7 +1259,56 @@ __device__ __forceinline__ void tile_task(ParamsRef p, int expert, int row0, int
   // token blocks below this one have all of their rows (a tile has more than 32 * (JT - 1); JT = 2: or fewer)
   constexpr int FULL = JT == 2 ? 0 : 2 * (JT - 1);
   const unsigned colb = pair_column(kg) * 2u;
-  if (!down) {
+  if constexpr (!RAGGED && JT > 8) {
+    unsigned char* slab = lds_raw;
+    if (!down) {
+      constexpr int LD = G1_COLS * 2 + 16;  // slab row pitch in bytes
+#pragma unroll
+      for (int j = 0; j < 2 * JT; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          float hv[4];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) hv[v] = silu_mul_fast(acc[i][j][v], acc[2 + i][j][v]);
+          *reinterpret_cast<uint2*>(slab + (j * 16 + r16) * LD + (wave * 32 + i * 16 + kg * 4) * 2) =
+              make_uint2(pack_bf16(hv[0], hv[1]), pack_bf16(hv[2], hv[3]));
+        }
+      __syncthreads();
+      // 16 lanes store one row's 256 bytes
+      unsigned char* h = uni(reinterpret_cast<unsigned char*>(p.h)) + (static_cast<size_t>(row0) * hp + 32 * (wcol - wave)) * 2;
+      for_rows<8 * JT / WAVES>([&](int it) { return *reinterpret_cast<const uint4*>(slab + ((it * WAVES + wave) * 4 + kg) * LD + r16 * 16); },
+                               [&](int it, const uint4& v) {
+                                 const int row = (it * WAVES + wave) * 4 + kg;
+                                 if (row < rows) st16_through(h + static_cast<size_t>(row) * hp * 2 + r16 * 16, v);
+                               });
+      __syncthreads();  // the slab is stage memory again
+    } else {
+      unsigned char* y = uni(reinterpret_cast<unsigned char*>(p.y)) + 128 * (wcol - wave);
+#pragma unroll
+      for (int part = 0; part < (JT + 3) / 4; ++part) {
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) {
+          const int j = part * 8 + jj;
+          if (j < 2 * JT) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              *reinterpret_cast<uint2*>(slab + (jj * 16 + r16) * EPI_LD + (wave * 64 + i * 16 + kg * 4) * 2) =
+                  make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
+          }
+        }
+        __syncthreads();
+        // 32 lanes store one row's 512 bytes at the row's (token, slot)
+        for_rows<128 / (2 * WAVES)>(
+            [&](int it) { return *reinterpret_cast<const uint4*>(slab + ((it * WAVES + wave) * 2 + (lane >> 5)) * EPI_LD + (lane & 31) * 16); },
+            [&](int it, const uint4& v) {
+              const int row = part * 128 + (it * WAVES + wave) * 2 + (lane >> 5);
+              const int dst = row < 32 * JT ? sdst[row] : -1;
+              if (dst >= 0) st16_through(y + static_cast<size_t>(dst) * H * 2 + (lane & 31) * 16, v);
+            });
+        __syncthreads();
+      }
+    }
+  } else if (!down) {
     unsigned char* h = uni(reinterpret_cast<unsigned char*>(p.h)) + (static_cast<size_t>(row0) * hp + 32 * wcol) * 2;
     const unsigned off = static_cast<unsigned>(r16) * static_cast<unsigned>(hp * 2) + colb;
 #pragma unroll
