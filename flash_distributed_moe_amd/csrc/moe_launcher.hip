@@ -386,15 +386,16 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   // How the bf16 tiled kernel starts. 1: logit chains of 16 tokens x 32 experts a workgroup, and selections spread over
   // the waves of the workgroups that had a chain. 2: router tasks of 16 or 32 tokens x all experts, which select for
   // themselves: chains twice as long (15 us for 7 at H=2048) and some 4 us of trips to memory less. So 1 while one
-  // round of its tasks does and the chains are long enough (us, 1 / 2, 30B shape: T=450 266.0 / 273.6, T=600 270.9 /
+  // round of its tasks does and the chains are long enough or the selections few (us, 1 / 2, 30B shape: T=450 266.0 / 273.6, T=600 270.9 /
   // 277.6, T=900 277.9 / 283.6, two rounds T=1200 300.7 / 296.6, T=1500 309.4 / 304.1; 235B shape T=700 942 / 959;
   // E=64, k=4, I=512: H=512 T=1000 65.0 / 64.0, H=1024 T=700 79.4 / 81.2, H=1536 T=700 104.6 / 109.1; E=32, H=768 T=800 55.3 /
-  // 56.5; E=16, H=320 T=1200 56.5 / 53.7) and a selecting wave has one or two tasks. Both without a scan phase, while the mask words fit LDS (as 2 against 0:
+  // 56.5; E=16, H=320 T=1200 56.5 / 53.7; k=2: E=8, H=256 T=300 37.8 / 37.8, E=16, H=512 T=400 41.6 / 42.6, E=32, H=512
+  // T=500 43.8 / 44.4, but k=4, E=64, H=256 T=512 43.0 / 42.0) and a selecting wave has one or two tasks. Both without a scan phase, while the mask words fit LDS (as 2 against 0:
   // T=2048 345 / 340, row-major 359 / 355; E=16 T=4000 74 / 70). 0: tickets for all of it.
   if (tiled && d.dtype == FLASH_MOE_BF16) {
     const int chain_k = d.hidden * ((d.experts + 127) / 128);  // of a router task of all experts
     p.dot16 = d.experts * ((T + 63) / 64) > fmoe::SHORT_MASK_WORDS || T > 65535 ? 0
-              : T <= 6 * m.n_groups && chain_k >= 768 && ((T + 15) / 16) * ((d.experts + 31) / 32) <= m.n_groups
+              : T <= 6 * m.n_groups && (T <= 512 || chain_k >= 768) && ((T + 15) / 16) * ((d.experts + 31) / 32) <= m.n_groups
                   ? 1
                   : 2;
     p.early = p.dot16;  // (the last selection raises FLAG_ROUTED)

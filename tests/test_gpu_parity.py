@@ -287,7 +287,8 @@ def test_tiled_ragged_equals_the_streaming_variant(T, H, E, k, I, hot, edges, pa
     (1000, 832, 33, 2),     # a last 256-k stage that is partly empty
     (1024, 768, 100, 4),    # 256 workgroups with a chain task each
     (1025, 768, 100, 4),    # one task too many for that
-    (300, 384, 200, 6),     # two slabs of experts count twice
+    (600, 384, 200, 6),     # two slabs of experts count twice
+    (513, 512, 64, 4),      # the first size whose chains are too short
 ])
 def test_tiled_starts(T, H, E, k):
     """The ways the tiled kernel gets from tokens to row tiles, at the edges of their ranges: routing
