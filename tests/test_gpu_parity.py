@@ -277,10 +277,12 @@ def test_tiled_ragged_equals_the_streaming_variant(T, H, E, k, I, hot, edges, pa
 
 @pytest.mark.parametrize("T,H,E,k", [
     (40, 128, 17, 3),       # a second group of experts with one expert; one token a wave at most
-    (1000, 192, 33, 2),     # a last 256-k stage that is partly empty
-    (1536, 320, 70, 8),     # the last size of the spread-out chains; two tokens a wave
-    (1537, 320, 70, 8),     # router tasks of all experts, no scan phase
-    (1000, 512, 256, 6),    # two rounds of 16-token x 32-expert tasks
+    (1000, 192, 33, 2),     # chains too short to be spread out: router tasks of all experts, no scan phase
+    (1536, 320, 70, 8),
+    (1537, 320, 70, 8),
+    (1000, 512, 256, 6),    # ... because spread-out chains would take two rounds
+    (1536, 768, 33, 2),     # the last size of spread-out chains; two selections a wave
+    (1537, 768, 33, 2),     # the first beyond it
     (2048, 128, 256, 2),    # the last size whose mask words fit LDS
     (2049, 128, 256, 2),    # the first whose do not
     (40, 768, 17, 3),       # spread-out chains: the least H; a group of experts with one expert
