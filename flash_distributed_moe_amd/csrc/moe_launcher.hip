@@ -383,21 +383,29 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
                        : 4;
   }
   const bool tiled = sched_for(d, T, m) == FLASH_MOE_SCHED_TILED;
-  // How the bf16 tiled kernel starts. 1: logit chains of 16 tokens x 32 experts a workgroup, and selections spread over
-  // the waves of the workgroups that had a chain. 2: router tasks of 16 or 32 tokens x all experts, which select for
-  // themselves: chains twice as long (15 us for 7 at H=2048) and some 4 us of trips to memory less. So 1 while one
-  // round of its tasks does and the chains are long enough or the selections few (us, 1 / 2, 30B shape: T=450 266.0 / 273.6, T=600 270.9 /
-  // 277.6, T=900 277.9 / 283.6, two rounds T=1200 300.7 / 296.6, T=1500 309.4 / 304.1; 235B shape T=700 942 / 959;
-  // E=64, k=4, I=512: H=512 T=1000 65.0 / 64.0, H=1024 T=700 79.4 / 81.2, H=1536 T=700 104.6 / 109.1; E=32, H=768 T=800 55.3 /
-  // 56.5; E=16, H=320 T=1200 56.5 / 53.7; k=2: E=8, H=256 T=300 37.8 / 37.8, E=16, H=512 T=400 41.6 / 42.6, E=32, H=512
-  // T=500 43.8 / 44.4, but k=4, E=64, H=256 T=512 43.0 / 42.0) and a selecting wave has one or two tasks. Both without a scan phase, while the mask words fit LDS (as 2 against 0:
-  // T=2048 345 / 340, row-major 359 / 355; E=16 T=4000 74 / 70). 0: tickets for all of it.
+  // How the bf16 tiled kernel starts. 1: logit chains of 16 tokens x 32 experts a workgroup, in as many rounds as that takes, and
+  // selections spread over the waves of the workgroups that had a chain. 2: router tasks of 16 or 32 tokens, which walk through the
+  // experts in slabs of 128 one after the other and select for themselves. Both without a scan phase, while the mask words fit
+  // LDS (as 2 against 0: T=2048 345 / 340, row-major 359 / 355; E=16 T=4000 74 / 70). 0: tickets for all of it.
+  // At H=2048 a slab takes 20 us and a round 11; against that stand the hand-over of the logits, a count by every four
+  // tokens and one by every chain. In these proportions (a quarter unit is 1.4 ns) the line below, fitted to 549 pairs of times:
+  // E=8 to 256, H=128 to 4096, T=110 to 4000. Beyond 512 tokens it takes the better start or one that is within 1 %. Up to there one
+  // round is taken from 256 k on, which is at most 1.7 us behind (E=16: H=512 T=300 45.4 / 46.5, but H=320 46.5 / 45.9, E=96, H=320
+  // 57.5 / 55.8) and 1.4 us ahead; left to router tasks: H=128 T=300 E=16 41.4 / 40.0; not E=144 T=450 54.0 / 55.3.
+  // us, 1 / 2: 30B shape T=600 285.6 / 292.5, T=1000 298.7 / 302.2, two rounds T=1040 311.8 / 308.0; H=512, I=256, k=4: E=32 T=600
+  // 50.4 / 50.8, T=1000 57.2 / 56.5; E=16, I=512, k=2, H=2048: T=2500 139.8 / 142.2, T=4000 147.0 / 145.4; two slabs (I=512, k=8):
+  //   E=160 one round H=2048 T=700 269.4 / 295.5; two: T=820 282.7 / 299.5, T=1500 306.4 / 317.5; H=4096 T=820 482.6 / 519.0,
+  //   T=1500 514.4 / 544.6; H=1024 T=820 158.2 / 164.1
+  //   E=200 two: H=512 T=800 82.9 / 84.0, T=1000 85.8 / 85.3; H=2048 T=1024 325.2 / 337.6; three: H=1024 T=1200 199.6 / 196.8; H=2048
+  //   T=1500 350.4 / 352.6; H=4096 T=1500 629.6 / 642.7
+  //   E=256 two: H=1024 T=520 207.4 / 213.5, T=1024 217.8 / 220.2; three: H=2048 T=1200 396.3 / 398.7, T=1500 404.2 / 404.5
+  // (More tokens than 16 a workgroup never pass, so that a wave has one selection at most.)
   if (tiled && d.dtype == FLASH_MOE_BF16) {
-    const int chain_k = d.hidden * ((d.experts + 127) / 128);  // of a router task of all experts
-    p.dot16 = d.experts * ((T + 63) / 64) > fmoe::SHORT_MASK_WORDS || T > 65535 ? 0
-              : T <= 6 * m.n_groups && (T <= 512 || chain_k >= 768) && ((T + 15) / 16) * ((d.experts + 31) / 32) <= m.n_groups
-                  ? 1
-                  : 2;
+    const int chains = ((T + 15) / 16) * ((d.experts + 31) / 32), rounds = (chains + m.n_groups - 1) / m.n_groups;
+    const int slabs = (d.experts + 127) / 128;
+    const bool spread = (T <= 512 && rounds == 1 && d.hidden * slabs >= 256) ||
+                        (T <= 16 * m.n_groups && 4ll * d.hidden * (7 * slabs - 4 * rounds) > 2000ll + 5ll * T + 12ll * chains);
+    p.dot16 = d.experts * ((T + 63) / 64) > fmoe::SHORT_MASK_WORDS || T > 65535 ? 0 : spread ? 1 : 2;
     p.early = p.dot16;  // (the last selection raises FLAG_ROUTED)
     p.n_workers = p.n_groups * 4;
   }

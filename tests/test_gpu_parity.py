@@ -275,28 +275,52 @@ def test_tiled_ragged_equals_the_streaming_variant(T, H, E, k, I, hot, edges, pa
         a.close()
 
 
-@pytest.mark.parametrize("T,H,E,k", [
-    (40, 128, 17, 3),       # a second group of experts with one expert; one token a wave at most
-    (1000, 192, 33, 2),     # chains too short to be spread out: router tasks of all experts, no scan phase
-    (1536, 320, 70, 8),
-    (1537, 320, 70, 8),
-    (1000, 512, 256, 6),    # ... because spread-out chains would take two rounds
-    (1536, 768, 33, 2),     # the last size of spread-out chains; two selections a wave
-    (1537, 768, 33, 2),     # the first beyond it
-    (2048, 128, 256, 2),    # the last size whose mask words fit LDS
-    (2049, 128, 256, 2),    # the first whose do not
-    (40, 768, 17, 3),       # spread-out chains: the least H; a group of experts with one expert
-    (1000, 832, 33, 2),     # a last 256-k stage that is partly empty
-    (1024, 768, 100, 4),    # 256 workgroups with a chain task each
-    (1025, 768, 100, 4),    # one task too many for that
-    (600, 384, 200, 6),     # two slabs of experts count twice
-    (513, 512, 64, 4),      # the first size whose chains are too short
+def tiled_start(case):
+    """How the tiled kernel gets from tokens to row tiles, and its records of kind 0 (logits) and 6 (selections), from a
+    traced launch, which starts as one without a trace does."""
+    case.launcher.trace_enable(1 << 17)
+    case.run()
+    kinds = np.bincount(case.launcher.trace_read()["kind"], minlength=7)
+    case.launcher.trace_enable(0)
+    return "tickets" if kinds[1] else "chains" if kinds[6] else "tokens", int(kinds[0]), int(kinds[6])
+
+
+# chains: logit chains of 16 tokens x 32 experts, on 256 workgroups; tokens: router tasks of all experts, in slabs of 128;
+# tickets: router, scan and scatter one after the other
+@pytest.mark.parametrize("T,H,E,k,start", [
+    (40, 128, 17, 3, "tokens"),
+    (1000, 192, 33, 2, "tokens"),
+    (1536, 320, 70, 8, "tokens"),
+    (1537, 320, 70, 8, "tokens"),
+    (1000, 512, 256, 6, "tokens"),
+    (1536, 768, 33, 2, "tokens"),
+    (1537, 768, 33, 2, "tokens"),
+    (2048, 128, 256, 2, "tokens"),    # the last size whose mask words fit LDS
+    (2049, 128, 256, 2, "tickets"),   # the first whose do not
+    (40, 768, 17, 3, "chains"),       # a group of experts with one expert
+    (1000, 832, 33, 2, "chains"),     # a last 256-k stage that is partly empty
+    (1024, 768, 100, 4, "tokens"),
+    (1025, 768, 100, 4, "tokens"),
+    (1024, 1024, 100, 4, "chains"),   # 256 workgroups with a chain task each
+    (1025, 1024, 100, 4, "tokens"),   # one slab does not pay for a second round
+    (513, 512, 64, 4, "chains"),
+    (512, 256, 64, 4, "chains"),      # the last size that needs no more than 256 k
+    (513, 256, 64, 4, "tokens"),
+    (512, 192, 64, 4, "tokens"),      # less than 256 k
+    (509, 128, 200, 17, "chains"),    # two slabs of 128 k; a last selection of one token
+    (557, 384, 200, 6, "chains"),     # two slabs against one round
+    (600, 384, 200, 6, "chains"),     # ... against two rounds, of which the second is short
+    (900, 1024, 160, 4, "chains"),
+    (1040, 1728, 256, 4, "chains"),   # ... against three
+    (1040, 1664, 256, 4, "tokens"),   # chains too short for that
+    (4096, 2176, 8, 1, "chains"),     # a selection for every wave of the launch
+    (4097, 2176, 8, 1, "tokens"),     # router tasks of 32 tokens, the last of one
 ])
-def test_tiled_starts(T, H, E, k):
+def test_tiled_starts(T, H, E, k, start):
     """The ways the tiled kernel gets from tokens to row tiles, at the edges of their ranges: routing
     tables bit for bit, outputs against the oracle, and the same from a second launch."""
     cfg = synth.MoeConfig("starts", T, H, E, k, 128, "bf16", hot=3)
-    print("tiled starts", T, H, E, k, flush=True)
+    print("tiled starts", T, H, E, k, start, flush=True)
     case = GpuCase(cfg, seed=T + E, sched=_lib.SCHED_TILED)
     try:
         assert case.launcher.sched_for(T) == _lib.SCHED_TILED
@@ -304,6 +328,11 @@ def test_tiled_starts(T, H, E, k):
         case.check_routing(case.inp["tokens"], case.launcher.routing(T))
         case.check_outputs(case.inp["tokens"], out, nthreads=4)
         assert torch.equal(case.run(), out)
+        up = lambda a, b: -(-a // b)
+        got = tiled_start(case)
+        assert got[0] == start
+        if start == "chains":
+            assert got[1:] == (up(T, 16) * up(E, 32), up(T, 4))
     finally:
         case.close()
 
