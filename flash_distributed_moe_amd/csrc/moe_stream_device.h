@@ -397,6 +397,8 @@ __device__ __forceinline__ bool wait_posts(ParamsRef p, const unsigned* posts, i
     state = 1u;
     int at = 4 * lane;  // this lane's next words that may be missing
     while (true) {
+      // (The load is no atomic one, which carries 8 bytes at most: without this the compiler may take words it has read.)
+      asm volatile("" ::: "memory");
       if (at < n) {
         const uint4 v = ld16_agent(words, static_cast<unsigned>(at) * 4u);
         const bool missing = v.x != raised || (at + 1 < n && v.y != raised) || (at + 2 < n && v.z != raised) || (at + 3 < n && v.w != raised);

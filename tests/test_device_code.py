@@ -133,3 +133,19 @@ def test_router_chains_are_left_alone_until_they_are_written(functions):
     states."""
     # 16 groups of 4 and of 2 instructions a stage
     assert _check_accumulators(functions, "tiled_router_task") == 16 * 4 + 16 * 2
+
+
+def test_every_look_at_the_posts_reads_them_again(functions):
+    """wait_posts polls with a load that is not atomic: it has to stand inside the loop around the wait's s_sleep 24."""
+    loops = 0
+    for name, code in functions.items():
+        if "moe_split_kernel" not in name:
+            continue
+        for at in [a for a, ins, _ in code if ins == "s_sleep 24"]:
+            back = [(a - target, target, a) for a, ins, target in code
+                    if ins.startswith(("s_cbranch", "s_branch")) and target is not None and target <= at < a]
+            assert back, "%s: no loop around 0x%x" % (name, at)
+            _, first, last = min(back)
+            assert any(first <= a < last and ins.startswith("buffer_load_dwordx4") and "sc1" in ins for a, ins, _ in code)
+            loops += 1
+    assert loops == 3 * 6  # routing, gate/up and down, in every instantiation
