@@ -166,7 +166,7 @@ __device__ __forceinline__ void raise_post(ParamsRef p, int phase, int index, un
 // left counters, masks and outputs in an arbitrary state. The last worker to leave makes
 // the failure visible and the launcher usable again without any help from the host, which
 // may be replaying a captured graph and never look: every element of `out` becomes NaN,
-// the workspace's zero region returns to zero (the count of completed launches apart), and
+// the workspace's zero region returns to zero (the count of completed launches apart; posts and their number together), and
 // the bits are added to the launcher's word in pinned host memory, where the next Launch
 // finds them. `tid` of `nthreads` threads of that worker call this; nobody else is running.
 __device__ __forceinline__ void recover_after_error(ParamsRef p, unsigned err, int tid, int nthreads) {

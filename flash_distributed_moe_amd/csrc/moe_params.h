@@ -48,6 +48,11 @@ struct alignas(128) ControlLine {
   unsigned v;
   unsigned pad[31];
 };
+struct alignas(128) LaunchLine {
+  unsigned v;       // completed launches (diagnostic)
+  unsigned posted;  // number the split-k kernel's last launch raised its posts to (see post_number)
+  unsigned pad[30];
+};
 struct Control {
   ControlLine ticket;       // next task number
   ControlLine router_done;  // tokens whose routing is final
@@ -56,7 +61,7 @@ struct Control {
   ControlLine exit_count;   // workers that have left the loop
   ControlLine n_mtiles;     // row tiles produced by the scan
   ControlLine error;        // sticky error bits
-  ControlLine launches;     // completed launches (diagnostic)
+  LaunchLine launches;
   ControlLine xq[8];        // tiled variant: per-XCD ticket counters of the GEMM tasks
   ControlLine cticket;      // tiled variant: combine tickets
   ControlLine scan_done;    // tiled variant: per-expert scan tasks finished
@@ -72,11 +77,16 @@ struct alignas(128) WgFlags {
 };
 
 // Split-k kernel: a word a workgroup and hand-over, raised by the workgroup that has done its share, in every one of
-// POST_COPIES rows; a workgroup watches one of those. Raised means the number of the launch, so nobody lowers it.
+// POST_COPIES rows; a workgroup watches one of those. Raised means the number of the launch, so nobody lowers it: launches
+// of this kernel count from 1 (0: never raised), and behind the last number all posts return to zero.
 // (POST_ROUTE: a word a routing task.)
 enum : int { POST_ROUTE = 0, POST_GATE_UP = 1, POST_DOWN = 2, POST_PHASES = 3 };
 constexpr int POST_COPIES = 8;
 constexpr int POST_PITCH = 512;  // words of a row
+constexpr __host__ __device__ unsigned post_number(unsigned posted) { return posted + 1u; }
+constexpr __host__ __device__ unsigned posted_by(unsigned number) { return number == 0xFFFFFFFFu ? 0u : number; }
+static_assert(post_number(posted_by(0xFFFFFFFFu)) == 1u && post_number(posted_by(0xFFFFFFFEu)) == 0xFFFFFFFFu,
+              "no launch may take a post that was never raised, or one from before the count came round, for its own");
 
 struct TileDesc {  // one row tile: `rows` consecutive permuted rows of one expert
   int expert;

@@ -256,7 +256,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   const int nt1 = I / (16 * G1_NB), nt2 = H / (16 * G2_NB);
   const int ks1 = H / (4 * DT::EPV), ks2 = I / (4 * DT::EPV);  // steps of 64 bytes a row
   const int pull_from = (((lane & 15) << 2) | (lane >> 4)) << 2;
-  const unsigned raised = ldc(&ctl->launches.v) + 1u;  // (the last workgroup out moves it on)
+  const unsigned raised = post_number(ldc(&ctl->launches.posted));  // (the last workgroup out moves it on)
 
   // ---- routing: logit chains on the first workgroups, then (batches of more than SPLIT_SELF_TOKENS) selections there,
   // four tokens a wave. Smaller batches have every workgroup pick all winners for itself, below: that saves the
@@ -719,7 +719,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
       combine_items<DT>(p, slot, nc, ncomb, static_cast<unsigned>(b * 8 + wave), 0u, 0);
   }
 
-  // ---- the last workgroup out returns every counter to zero for the next launch
+  // ---- the last workgroup out counts the launch
   __syncthreads();
   if (wave == 0) {
     fence_release();  // flags this wave has raised for others have landed before anybody clears them
@@ -728,8 +728,12 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     if (__builtin_amdgcn_readfirstlane(last) != 0u) {
       const unsigned err = ldc(&ctl->error.v);
       if (err != 0u) recover_after_error(p, err, lane, 64);
+      const unsigned posted = posted_by(raised);
+      if (posted == 0u)
+        for (int q = lane; q < POST_PHASES * POST_COPIES * POST_PITCH; q += 64) stc(&p.posts[q], 0u);
       if (lane == 0) {
         stc(&ctl->launches.v, ldc(&ctl->launches.v) + 1u);
+        stc(&ctl->launches.posted, posted);
         stc(&ctl->exit_count.v, 0u);
       }
     }
