@@ -1653,17 +1653,14 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
       }
       const int sel_groups = min(n_dot, G);
       const int i0 = b + sel_groups * wave;
+      // (the launcher takes this start while there are as many waves as selections, at least)
       if (b < sel_groups && i0 * SELECT_TOK < Ti) {
         const long long t0 = trace_clock(traced);
-        unsigned done = 0;
-        for (int i = i0; i * SELECT_TOK < Ti; i += WAVES * sel_groups) {
-          const int n = router_select4_task(p, i, static_cast<unsigned>((p.E + 15) >> 4), lds_raw + wave * SELECT_ROWS_BYTES);
-          if (n == 0) break;  // (a wait that fails has raised an error bit, which every later wait sees)
-          done += n;
-        }
+        const int n = router_select4_task(p, i0, static_cast<unsigned>((p.E + 15) >> 4), lds_raw + wave * SELECT_ROWS_BYTES);
         unsigned old = 0;
-        if (lane_id() == 0) old = add_relaxed(&ctl->router_done.v, done);
-        if (uni(static_cast<int>(old + done)) == Ti) broadcast_flag(p, FLAG_ROUTED);
+        if (lane_id() == 0) old = add_relaxed(&ctl->router_done.v, static_cast<unsigned>(n));
+        // (n = 0: a wait that failed has raised an error bit, which every later wait sees)
+        if (uni(static_cast<int>(old)) + n == Ti) broadcast_flag(p, FLAG_ROUTED);
         trace_task(p, traced && lane_id() == 0, n_dot + i0, 6, i0 * SELECT_TOK, t0, t0);
       }
       t_perm0 = n_dot + WAVES * sel_groups;
