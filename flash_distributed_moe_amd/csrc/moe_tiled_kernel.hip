@@ -1093,8 +1093,11 @@ __device__ __forceinline__ uint4 pair_columns(uint2 a, uint2 b) {
 }
 __device__ __forceinline__ unsigned pair_column(int kg) { return static_cast<unsigned>((kg & 1) * 16 + (kg >> 1) * 8); }
 // Tiles of more than 256 rows go through LDS instead, where rows become whole again: they come in numbers, from experts
-// that draw far more tokens than others, and there whole rows are ahead (30B shape, four hot experts, T=16384, us, half
-// lines / whole rows: 1387 / 1374; tiles of up to 256 rows, T=8192: 736 / 738). What they gain was only measured as time.
+// that draw far more tokens than others, and there whole rows are ahead. us, 30B shape, half lines at all heights / as here /
+// whole rows at all heights: four hot experts T=16384 1393 / 1382 / 1394, T=8192 725 / 723 / 768, T=2048 row-major 340 / 338 /
+// 358; 235B shape T=4096 1382 / 1389 / 1409. It is not for the bytes: FETCH_SIZE of T=8192 is 1.168, 1.231 and 1.206 M KiB, of T=16384
+// 1.816, 1.861 and 1.820 (WRITE_SIZE of half lines 1.7 % more): where an expert's tiles leave in two ways they drift apart
+// and share fewer weights in the L2.
 constexpr int EPI_LD = TN * 2 + 16;  // bytes per row of the down slab
 static_assert(128 * EPI_LD <= TILE_LDS_BYTES && TM_MAX * (G1_COLS * 2 + 16) <= TILE_LDS_BYTES, "epilogue slab exceeds the stage buffers");
 // eight rows' reads first, then their stores: a store's assembly orders memory operations around it, and one LDS round
@@ -1122,15 +1125,18 @@ __device__ __forceinline__ void st16_through_at(unsigned char* base, unsigned of
 //
 // gate/up: h[row, n0 .. n0+128) (test/singleGPU/cpp/moe/reference/refExpertFFN1.h:51-65).
 // h is [T*K, I] row-major, rows in permuted order. Wave w holds gate rows n0+32w.. and the
-// matching up rows, so SiLU(gate)*up happens in registers; the tile's 128 columns leave
-// through LDS as 256-byte row segments.
+// matching up rows, so SiLU(gate)*up happens in registers.
 //
 // down: y[t*K+slot, n0 .. n0+256) = h[row] . W2[e]^T (refFullMoe.h:58-65,
-// src/hip/kernel/tasks/ffn2Task.h:37-40), bf16, through LDS as 512-byte row segments, 128
-// rows at a time. The rows' destinations are fetched when the task starts and parked in LDS
-// behind the stages, so the epilogue waits for no memory. The slot's gate weight is applied
+// src/hip/kernel/tasks/ffn2Task.h:37-40), bf16. The rows' destinations are fetched when the task starts
+// and parked in LDS behind the stages, so the epilogue waits for no memory. The slot's gate weight is applied
 // by the combine task, which has instruction slots to spare; here every instruction of the
 // epilogue is one the matrix cores wait for.
+//
+// Tiles of up to 256 rows store 64-byte pieces of their rows straight from the accumulators, each wave its own columns; taller
+// ones go through LDS: gate/up as 256-byte row segments, down as 512-byte ones, 128 rows at a time. Only these end
+// with a barrier. Without one a wave may still read the destinations and the next ticket (sdst, task_notes) while others
+// are in the next task: both are written behind that task's k-loop, whose first barrier every wave reaches with its reads done.
 //
 // RAGGED: H is no multiple of 256 or I none of 128. The last task of a row tile may stand out over the
 // last column: a wave whose columns do not exist repeats the last ones that do, and its results are not

@@ -337,30 +337,38 @@ def test_tiled_starts(T, H, E, k, start):
         case.close()
 
 
-@pytest.mark.parametrize("T,H,E,k,sched", [
-    (4099, 192, 128, 32, _lib.SCHED_TILED),  # 32-token router tasks, the last of 3 tokens; the most slots
-    (4100, 128, 200, 17, _lib.SCHED_TILED),  # two slabs of experts, the second partly empty; more slots than a row has lanes
-    (2100, 64, 40, 5, _lib.SCHED_TILED),     # 16-token tasks of one stage; the last of 4 tokens
-    (601, 128, 200, 17, _lib.SCHED_TILED),   # selections spread over the workgroups, the last of one token
-    (32, 256, 200, 32, _lib.SCHED_AUTO),     # split-k kernel: every workgroup picks the winners, four tokens to each of its waves
-    (33, 256, 120, 17, _lib.SCHED_AUTO),     # the first size whose winners are picked once
-    (1, 256, 97, 32, _lib.SCHED_AUTO),
+@pytest.mark.parametrize("T,H,E,k,start", [
+    (4099, 192, 128, 32, "tickets"),  # 32-token router tasks, the last of 3 tokens; the most slots
+    (4100, 128, 200, 17, "tickets"),  # two slabs of experts, the second partly empty; more slots than a row has lanes
+    (2100, 64, 40, 5, "streaming"),   # too few k for the tiled variant: one token to a wave
+    (2100, 128, 40, 5, "tokens"),     # 16-token tasks, the last of 4 tokens
+    (601, 128, 200, 17, "tokens"),    # ... of two slabs; the last of 9 tokens
+    (509, 128, 200, 17, "chains"),    # selections spread over the workgroups, the last of one token
+    (511, 256, 120, 17, "chains"),    # ... of three tokens
+    (32, 256, 200, 32, "split-k"),    # every workgroup picks the winners, four tokens to each of its waves
+    (33, 256, 120, 17, "split-k"),    # the first size whose winners are picked once
+    (1, 256, 97, 32, "split-k"),
 ])
 @pytest.mark.parametrize("admitted", ["all", "three"])
-def test_router_winners(T, H, E, k, sched, admitted):
+def test_router_winners(T, H, E, k, start, admitted):
     """Equal logits (every expert's row of the router weights twice, so the lower index wins) and experts that
     are never admitted (a bias of -inf leaves three, fewer than k): winners and weights against the oracle."""
     cfg = synth.MoeConfig("winners", T, H, E, k, 128, "bf16")
-    print("winners", T, H, E, k, sched, admitted, flush=True)
+    print("winners", T, H, E, k, start, admitted, flush=True)
     inp = synth.make_inputs_torch(cfg, T + k, torch.device("cuda:0"))
     inp["gate"][E // 2:2 * (E // 2)] = inp["gate"][:E // 2].clone()
     if admitted == "three":
         inp["bias"] = torch.full((E,), -float("inf"), device="cuda:0")
         inp["bias"][[1, E // 2 + 1, E - 1]] = 0.0
-    case = GpuCase(cfg, sched=sched, inputs=inp)
+    case = GpuCase(cfg, sched=_lib.SCHED_AUTO if start == "split-k" else _lib.SCHED_TILED, inputs=inp)
+    tiled = start in ("chains", "tokens", "tickets")
     try:
+        assert (case.launcher.sched_for(T) == _lib.SCHED_TILED) == tiled
+        assert (case.launcher.split_blocks_for(T) != 0) == (start == "split-k")
         case.run()
         routing = case.launcher.routing(T)
+        if tiled:
+            assert tiled_start(case)[0] == start
         hw = case.host_weights()
         idx, w = oracle.gate(inp["tokens"].float().cpu().numpy(), hw["gate"], k, bias=hw["bias"])
         assert (idx < 0).any() == (admitted == "three")
