@@ -729,7 +729,11 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   __syncthreads();
   const int lane = lane_id();
   const int wave_in_group = threadIdx.x >> 6;
-  const int waves_per_group = blockDim.x >> 6;
+  constexpr int waves_per_group = 8;
+  // (Arguments lie in lines of 64 bytes that every launch fetches anew, and gridDim and blockDim behind Params in a line of their
+  // own, which this kernel need not wait for: us, with / without it, H=1600, I=768, E=5, k=4, T=6 58.3 / 57.3; row-major H=2880,
+  // I=1408, E=9, k=5, T=3 88.9 / 85.7. The float32 tiled kernel is compiled to a slower one that way, the others are level.)
+  const unsigned n_groups = static_cast<unsigned>(p.n_groups);
   Control* ctl = p.ctl;
   const unsigned T = static_cast<unsigned>(p.T);
   // dot tasks: 8 x 8 chains per wave, or (dot16) 16 x 16 per workgroup; those are
@@ -763,7 +767,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   const unsigned n_workers = static_cast<unsigned>(p.n_workers);
   bool first = true;
   const unsigned n_skip = dot16 ? n_dot : 0u;
-  unsigned first_tk = n_skip + static_cast<unsigned>(wave_in_group) * gridDim.x + blockIdx.x;
+  unsigned first_tk = n_skip + static_cast<unsigned>(wave_in_group) * n_groups + blockIdx.x;
   unsigned dyn_base = n_skip + n_workers;  // tickets below this are handed out statically
   unsigned late_lo = 0xFFFFFFFFu, late_skip = 0u;  // early mode: static tickets [late_lo, late_lo + late_skip)
   if (p.early) {
@@ -773,7 +777,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     // tasks on waves 0..3 (one per SIMD), select and scan tasks on waves 4..7.
     // Workers of those workgroups without a routing task take dynamic tickets.
     const unsigned nr = max(dot16 ? n_dot : (n_dot + 3u) / 4u, (T + 4u) / 4u);
-    const unsigned rest = gridDim.x - nr;
+    const unsigned rest = n_groups - nr;
     dyn_base = n_router + 1u + 8u * rest;
     if (n1 >= 8u * rest) {
       late_skip = 4u * rest;

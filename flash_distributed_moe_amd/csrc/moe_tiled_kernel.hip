@@ -1096,8 +1096,8 @@ __device__ __forceinline__ unsigned pair_column(int kg) { return static_cast<uns
 // that draw far more tokens than others, and there whole rows are ahead. us, 30B shape, half lines at all heights / as here /
 // whole rows at all heights: four hot experts T=16384 1393 / 1382 / 1394, T=8192 725 / 723 / 768, T=2048 row-major 340 / 338 /
 // 358; 235B shape T=4096 1382 / 1389 / 1409. It is not for the bytes: FETCH_SIZE of T=8192 is 1.168, 1.231 and 1.206 M KiB, of T=16384
-// 1.816, 1.861 and 1.820 (WRITE_SIZE of half lines 1.7 % more): where an expert's tiles leave in two ways they drift apart
-// and share fewer weights in the L2.
+// 1.816, 1.861 and 1.820 (WRITE_SIZE of half lines 1.7 % more): presumably an expert's tiles that leave in two ways drift
+// apart and share fewer weights in the L2.
 constexpr int EPI_LD = TN * 2 + 16;  // bytes per row of the down slab
 static_assert(128 * EPI_LD <= TILE_LDS_BYTES && TM_MAX * (G1_COLS * 2 + 16) <= TILE_LDS_BYTES, "epilogue slab exceeds the stage buffers");
 // eight rows' reads first, then their stores: a store's assembly orders memory operations around it, and one LDS round

@@ -149,3 +149,16 @@ def test_every_look_at_the_posts_reads_them_again(functions):
             assert any(first <= a < last and ins.startswith("buffer_load_dwordx4") and "sc1" in ins for a, ins, _ in code)
             loops += 1
     assert loops == 3 * 6  # routing, gate/up and down, in every instantiation
+
+
+def test_a_kernel_waits_for_no_more_lines_of_its_arguments_than_params_has(functions):
+    """Arguments are fetched anew for every launch, 64 bytes at a time. Params fills five such lines; gridDim and blockDim lie
+    behind it, and a kernel that asks for a sixth line starts later (1 to 3 us with small batches)."""
+    kernels = 0
+    for name, code in functions.items():
+        if re.search(r"moe_(split|stream|tiled|tiled_f32)_kernelI", name):
+            loads = [re.match(r"s_load_dword(x\d+)? \S+, s\[\d+:\d+\], 0x([0-9a-f]+)", ins) for _, ins, _ in code]
+            last = max(int(m.group(2), 16) + 4 * int((m.group(1) or "x1")[1:]) for m in loads if m)
+            assert 256 < last <= 320, "%s reads %d bytes of arguments" % (name, last)
+            kernels += 1
+    assert kernels == 6 + 2 + 2 + 6
