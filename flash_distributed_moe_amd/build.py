@@ -19,11 +19,13 @@ HIPCC_FLAGS = [
     "-Wno-return-type-c-linkage",
 ]
 
-# Flags of one source on top of those. The streaming kernel's time depends on where its loops lie
-# (functions are placed at 4-byte granularity, so any change in front of one moves it): float32, 30B
-# shape, T=700 905 or 918 us and T=1024 1071 or 1079 us for the same instructions; with the loops on
-# 64-byte boundaries 906 and 1073 wherever they are. The split-k kernel is 0.4 us slower with it.
-SOURCE_FLAGS = {"moe_stream_kernel.hip": ["-falign-loops=64"]}
+# Flags of one source on top of those. The streaming kernel's time depends on where its code lies: functions are placed at
+# 4-byte granularity, so any change in front of one moves it. With the loops on 64-byte boundaries float32 T=700 on the 30B
+# shape takes 906 us wherever it had taken 905 or 918 for the same instructions; with the functions on 4096-byte ones too
+# E=211, H=512, I=640, k=3, row-major, T=168 / 177 / 300 200.8 / 202.8 / 238.2 instead of 207.4 / 210.5 / 240.6, or
+# 204.4 / 206.8 / 239.3 as they happened to lie before; E=64, k=4 packed T=300 376.1 instead of 377.9 (375.8); bf16 level. The
+# split-k kernel is 0.4 us slower with aligned loops.
+SOURCE_FLAGS = {"moe_stream_kernel.hip": ["-falign-loops=64", "-falign-functions=4096"]}
 
 
 def sources():

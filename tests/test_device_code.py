@@ -41,6 +41,13 @@ def gemm_task(functions):
     return [ins for _, ins, _ in code]
 
 
+def test_streaming_tasks_lie_on_4096_byte_boundaries(functions):
+    """The streaming tasks' times depend on where they lie among each other by a percent or two (build.py)."""
+    tasks = [(name, code[0][0]) for name, code in functions.items() if re.search(r"fmoe\d+(gateup|gateup_early|down)_taskI", name)]
+    assert len(tasks) == 6 + 4 + 6
+    assert not [t for t in tasks if t[1] % 4096]
+
+
 def test_float32_sweeps_lie_on_64_byte_boundaries(functions):
     """The float32 streaming tasks lose about a percent to where their k-loops happen to lie
     (build.py), so those loops are aligned: every backward branch over the 256 matrix instructions of a round."""
