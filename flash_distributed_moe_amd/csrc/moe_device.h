@@ -463,20 +463,25 @@ __device__ __forceinline__ void router_select_rows(int K, int t, unsigned (&val)
     for (int j = 0; j < EPL; ++j) val[j] = j == drop ? 0u : val[j];
   }
   lds_wave_sync();
-  // softmax over the K winners (descending, so the first is the maximum), a lane to a (token, slot)
+  // softmax over the K winners (descending, so the first is the maximum), a lane to a (token, slot). The sum is taken in slot
+  // order, eight values on their way at a time: behind the last winner they are zeros.
   auto logit = [](unsigned bits) { return bits != 0u ? from_ordered_bits(bits) : -FLT_MAX; };
-  for (int i = lane; i < 4 * K; i += 64) {
-    const int q = i & 3, s = i >> 2;
-    const float mine = logit(won[q * MAX_TOPK + s].y), first = logit(won[q * MAX_TOPK].y);
-    ex[q * MAX_TOPK + s] = exp(static_cast<double>(mine) - static_cast<double>(first));
-  }
+  const int q = lane & 3, K8 = (K + 7) & ~7;
+  const float first = logit(won[q * MAX_TOPK].y);
+  for (int s = lane >> 2; s < K8; s += 16)
+    ex[q * MAX_TOPK + s] = s < K ? exp(static_cast<double>(logit(won[q * MAX_TOPK + s].y)) - static_cast<double>(first)) : 0.0;
   lds_wave_sync();
-  for (int i0 = 0; i0 < 4 * K; i0 += 64) {
-    const int i = i0 + lane, q = i & 3, s = i >> 2;
-    const int tq = __shfl(t, 16 * q, 64);
-    if (i < 4 * K && tq >= 0) {
-      double sum = 0.0;
-      for (int u = 0; u < K; ++u) sum += ex[q * MAX_TOPK + u];
+  double sum = 0.0;
+  for (int u = 0; u < K8; u += 8) {
+    double part[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) part[j] = ex[q * MAX_TOPK + u + j];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum += part[j];
+  }
+  const int tq = __shfl(t, 16 * q, 64);
+  if (tq >= 0) {
+    for (int s = lane >> 2; s < K; s += 16) {
       const float w = sum <= 0.0 ? static_cast<float>(1.0 / static_cast<double>(K))
                                  : static_cast<float>(ex[q * MAX_TOPK + s] / sum);
       emit(tq, s, static_cast<int>(won[q * MAX_TOPK + s].x), w);
