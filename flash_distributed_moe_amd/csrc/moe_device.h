@@ -423,9 +423,9 @@ __device__ __forceinline__ void router_select_max(ParamsRef p, int t,
   lds_wave_sync();
 }
 
-// The same for four tokens at once, one to a row of 16 lanes: lane r of a row holds the experts EPL*r ..
-// EPL*r + EPL-1 of its token, so among equals the lowest lane, and in it the lowest element, wins. A round's
-// cross-lane steps stay inside the row and serve all four tokens, and nothing goes through scalar registers: on one
+// The same for four tokens at once, one to a row of 16 lanes (or for two, one to two rows): lane r of a row holds the experts
+// EPL*r .. EPL*r + EPL-1 of its token, so among equals the lowest lane, and in it the lowest element, wins. A round's
+// cross-lane steps stay inside the row and serve all tokens, and nothing goes through scalar registers: on one
 // token to a wave a selection is a chain of K rounds of some 20 dependent cross-lane and scalar steps plus the
 // softmax in double, about 1.8 us whatever the wave could do beside it. t: the row's
 // token, -1: none. `scratch`:
@@ -439,19 +439,27 @@ __device__ __forceinline__ unsigned row_max_u32(unsigned v) {
   v = step(v, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xF, 0xF, true)));  // mirror in 16
   return v;
 }
-// emit(token, slot, expert or -1, weight) is called for each of the row's slots, by some lane.
-template <int EPL, typename Emit>
+// ... of two rows
+__device__ __forceinline__ unsigned row_pair_max_u32(unsigned v) {
+  v = row_max_u32(v);
+  const auto other = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return other[0] > other[1] ? other[0] : other[1];
+}
+// emit(token, slot, expert or -1, weight) is called for each of the token's slots, by some lane. LPT: lanes a token, 16 or
+// 32 (two tokens a wave).
+template <int EPL, int LPT, typename Emit>
 __device__ __forceinline__ void router_select_rows(int K, int t, unsigned (&val)[EPL], unsigned char* scratch, Emit emit) {
-  const int lane = lane_id(), row = lane >> 4, r = lane & 15;
+  constexpr int TOK = 64 / LPT;
+  const int lane = lane_id(), row = lane / LPT, r = lane % LPT;
   double* ex = reinterpret_cast<double*>(scratch);                        // [4][MAX_TOPK]
   uint2* won = reinterpret_cast<uint2*>(scratch + 4 * MAX_TOPK * 8);      // [4][MAX_TOPK]: expert (or -1), ordered bits
   // lanes of this row in front of this one
-  const unsigned long long before = ((1ull << r) - 1ull) << (16 * row);
+  const unsigned long long before = ((1ull << r) - 1ull) << (LPT * row);
   for (int s = 0; s < K; ++s) {
     unsigned m = val[0];
 #pragma unroll
     for (int j = 1; j < EPL; ++j) m = val[j] > m ? val[j] : m;
-    const unsigned best = row_max_u32(m);
+    const unsigned best = LPT == 16 ? row_max_u32(m) : row_pair_max_u32(m);
     const bool owner = m == best && (__ballot(m == best) & before) == 0ull;
     int at = EPL;  // the lowest of this lane's elements that is the best
 #pragma unroll
@@ -466,9 +474,9 @@ __device__ __forceinline__ void router_select_rows(int K, int t, unsigned (&val)
   // softmax over the K winners (descending, so the first is the maximum), a lane to a (token, slot). The sum is taken in slot
   // order, eight values on their way at a time: behind the last winner they are zeros.
   auto logit = [](unsigned bits) { return bits != 0u ? from_ordered_bits(bits) : -FLT_MAX; };
-  const int q = lane & 3, K8 = (K + 7) & ~7;
+  const int q = lane % TOK, K8 = (K + 7) & ~7;
   const float first = logit(won[q * MAX_TOPK].y);
-  for (int s = lane >> 2; s < K8; s += 16)
+  for (int s = lane / TOK; s < K8; s += LPT)
     ex[q * MAX_TOPK + s] = s < K ? exp(static_cast<double>(logit(won[q * MAX_TOPK + s].y)) - static_cast<double>(first)) : 0.0;
   lds_wave_sync();
   double sum = 0.0;
@@ -479,9 +487,9 @@ __device__ __forceinline__ void router_select_rows(int K, int t, unsigned (&val)
 #pragma unroll
     for (int j = 0; j < 8; ++j) sum += part[j];
   }
-  const int tq = __shfl(t, 16 * q, 64);
+  const int tq = __shfl(t, LPT * q, 64);
   if (tq >= 0) {
-    for (int s = lane >> 2; s < K; s += 16) {
+    for (int s = lane / TOK; s < K; s += LPT) {
       const float w = sum <= 0.0 ? static_cast<float>(1.0 / static_cast<double>(K))
                                  : static_cast<float>(ex[q * MAX_TOPK + s] / sum);
       emit(tq, s, static_cast<int>(won[q * MAX_TOPK + s].x), w);
@@ -490,9 +498,9 @@ __device__ __forceinline__ void router_select_rows(int K, int t, unsigned (&val)
   lds_wave_sync();
 }
 // ... into the routing tables in memory
-template <int EPL>
+template <int EPL, int LPT>
 __device__ __forceinline__ void router_select_rows(ParamsRef p, int t, unsigned (&val)[EPL], unsigned char* scratch) {
-  router_select_rows<EPL>(p.K, t, val, scratch, [&](int tq, int s, int e, float w) {
+  router_select_rows<EPL, LPT>(p.K, t, val, scratch, [&](int tq, int s, int e, float w) {
     stc(&p.topk_idx[static_cast<size_t>(tq) * p.K + s], e);
     stc(&p.topk_w[static_cast<size_t>(tq) * p.K + s], w);
     if (e >= 0) or_relaxed(&p.masks[static_cast<size_t>(e) * p.W + (tq >> 6)], 1ull << (tq & 63));
@@ -501,9 +509,9 @@ __device__ __forceinline__ void router_select_rows(ParamsRef p, int t, unsigned 
 
 // The logits of the tokens t0 .. t0+n-1 (n <= 4) that chains elsewhere have left in memory, as router_select_rows wants
 // them. (Past the last token the buffer reads zeros, past a token's last expert the next one's.)
-template <int EPL>
+template <int EPL, int LPT>
 __device__ __forceinline__ void load_row_keys(ParamsRef p, int t0, int n, unsigned (&val)[EPL]) {
-  const int lane = lane_id(), row = lane >> 4, r = lane & 15, E = p.E;
+  const int lane = lane_id(), row = lane / LPT, r = lane % LPT, E = p.E;
   const CoherentBuffer keys = coherent_buffer(p.cand + static_cast<size_t>(t0) * E, static_cast<unsigned>(n * E) * 4u);
   uint4 v[EPL / 4];
 #pragma unroll
@@ -517,18 +525,18 @@ __device__ __forceinline__ void load_row_keys(ParamsRef p, int t0, int n, unsign
 }
 
 // The waits and trips to memory around that, where other workgroups' chains have left their logits in p.cand: winners of
-// the tokens 4*i .. 4*i+3 by one wave. Returns how many tokens they are, once their entries are in memory; 0 if the
+// a wave's select_tokens tokens, the i-th such lot. Returns how many tokens they are, once their entries are in memory; 0 if the
 // wait failed. A wave's tokens are asked for together, and its caller counts them with one atomic: a counter takes 90
 // of those a microsecond, so that counting every token by itself, as a selection a wave does, held up the last
 // of 600 tokens by 7 us. target: chain tasks a token has.
-constexpr int SELECT_TOK = 4;
-__device__ __noinline__ int router_select4_task(ParamsRef pv, int i_in, unsigned target_in, unsigned char* scratch) {
+__device__ __noinline__ int router_select_tokens_task(ParamsRef pv, int i_in, unsigned target_in, unsigned char* scratch) {
   ParamsRef p = uniform_params(pv);
   const int T = __builtin_amdgcn_readfirstlane(p.T), E = __builtin_amdgcn_readfirstlane(p.E);
   const unsigned target = __builtin_amdgcn_readfirstlane(target_in);
-  const int t0 = __builtin_amdgcn_readfirstlane(i_in) * SELECT_TOK;
-  const int lane = lane_id(), row = lane >> 4;
-  const int n = min(SELECT_TOK, T - t0);
+  const int tok = select_tokens(E, __builtin_amdgcn_readfirstlane(p.K), T);
+  const int t0 = __builtin_amdgcn_readfirstlane(i_in) * tok;
+  const int lane = lane_id(), row = lane * tok >> 6;
+  const int n = min(tok, T - t0);
   {
     const unsigned* mine = &p.tok_arrive[t0 + min(lane, n - 1)];
     const long long since = wall_clock64();
@@ -546,12 +554,16 @@ __device__ __noinline__ int router_select4_task(ParamsRef pv, int i_in, unsigned
   const int t = row < n ? t0 + row : -1;
   if (E <= 128) {
     unsigned val[8];
-    load_row_keys<8>(p, t0, n, val);
-    router_select_rows<8>(p, t, val, scratch);
-  } else {
+    load_row_keys<8, 16>(p, t0, n, val);
+    router_select_rows<8, 16>(p, t, val, scratch);
+  } else if (tok == 4) {
     unsigned val[16];
-    load_row_keys<16>(p, t0, n, val);
-    router_select_rows<16>(p, t, val, scratch);
+    load_row_keys<16, 16>(p, t0, n, val);
+    router_select_rows<16, 16>(p, t, val, scratch);
+  } else {
+    unsigned val[8];
+    load_row_keys<8, 32>(p, t0, n, val);
+    router_select_rows<8, 32>(p, t, val, scratch);
   }
   fence_release();
   return n;

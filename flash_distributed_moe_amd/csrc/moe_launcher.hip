@@ -373,7 +373,6 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   if (p.split) {
     p.early = 1;
     p.split_spec = reaches_experts ? 1 : 0;
-    p.split_self = T <= fmoe::SPLIT_SELF_TOKENS;
     // a down task in four parts, two of them to a workgroup, unless that leaves CUs without one or (float32) the
     // number of 64-column tasks is odd
     const bool eight_steps = d.intermediate >= (d.dtype == FLASH_MOE_BF16 ? 256 : 128);
@@ -399,12 +398,12 @@ fmoe::Params make_params(const FlashMoeLauncher* l, const void* tokens, void* ou
   //   E=200 two: H=512 T=800 82.9 / 84.0, T=1000 85.8 / 85.3; H=2048 T=1024 325.2 / 337.6; three: H=1024 T=1200 199.6 / 196.8; H=2048
   //   T=1500 350.4 / 352.6; H=4096 T=1500 629.6 / 642.7
   //   E=256 two: H=1024 T=520 207.4 / 213.5, T=1024 217.8 / 220.2; three: H=2048 T=1200 396.3 / 398.7, T=1500 404.2 / 404.5
-  // (More tokens than 16 a workgroup never pass, so that a wave has one selection at most.)
+  // (Selections never outnumber the waves, so that each has one at most.)
   if (tiled && d.dtype == FLASH_MOE_BF16) {
     const int chains = ((T + 15) / 16) * ((d.experts + 31) / 32), rounds = (chains + m.n_groups - 1) / m.n_groups;
-    const int slabs = (d.experts + 127) / 128;
+    const int slabs = (d.experts + 127) / 128, tok = fmoe::select_tokens(d.experts, d.top_k, T);
     const bool spread = (T <= 512 && rounds == 1 && d.hidden * slabs >= 256) ||
-                        (T <= 16 * m.n_groups && 4ll * d.hidden * (7 * slabs - 4 * rounds) > 2000ll + 5ll * T + 12ll * chains);
+                        (T <= 4 * tok * m.n_groups && 4ll * d.hidden * (7 * slabs - 4 * rounds) > 2000ll + 5ll * T + 12ll * chains);
     p.dot16 = d.experts * ((T + 63) / 64) > fmoe::SHORT_MASK_WORDS || T > 65535 ? 0 : spread ? 1 : 2;
     p.early = p.dot16;  // (the last selection raises FLAG_ROUTED)
     p.n_workers = p.n_groups * 4;

@@ -29,6 +29,16 @@ constexpr int SCAN_LDS_WORDS = 1024;  // mask words (experts x 64-token words) t
 constexpr int SHORT_MASK_WORDS = 8192;  // the same for the tiled kernel's short prologue
 constexpr int SPLIT_MAX_SLOTS = 2048;  // split-k kernel: (token, slot) entries its tables hold
 constexpr int SPLIT_SELF_TOKENS = 32;  // ... tokens every workgroup may pick the winners of by itself
+// Tokens whose winners one wave picks side by side (router_select_rows), where other waves have left the logits in memory.
+// A winner costs a lane some 10 instructions and 5 for each expert it holds; of more than 128 experts those of four tokens
+// are 16 a lane, of two 8. Twice as many counts of selections against that: so two while there are few tokens to a winner.
+// us, one token / four / two, H=1024, I=256, E=256: k=32 T=1 43.9 / 44.6 / 40.7, T=31 97.0 / 101.1 / 96.8, k=16 T=8 56.4 /
+// 57.1 / 54.8, k=8 T=8 42.9 / 40.6 / 39.6; tiled, E=160, k=32: T=384 106.7 / 113.6 / 111.1, T=768 145.1 / 142.9 / 141.2, k=16 T=600 105.4 /
+// 103.7 / 104.0; float32 T=100 145.6 / 153.1 / 148.9.
+constexpr __host__ __device__ int select_tokens(int E, int K, int T) { return E > 128 && T <= 24 * K ? 2 : 4; }
+// Split-k kernel: every workgroup picks all winners for itself, while its eight waves do it in one go (E=256, k=8, T=24 so
+// with four tokens a wave 62.6 us, from the selections of other workgroups with two 61.6; k=32, T=31 101.1 / 96.8).
+constexpr __host__ __device__ bool split_self(int E, int K, int T) { return T <= 8 * select_tokens(E, K, T); }
 constexpr int EARLY_MAX_TOKENS = 384;  // batches up to this size may take their gate/up weights before the routing is known
 // Shapes whose columns do not divide into the bf16 tiled variant's tasks (256 of H, 128 of I): kernels of
 // their own, which keep y as the streaming variant does (see tile_task).
@@ -152,7 +162,6 @@ struct Params {
   int split;                       // 1, 2: the split-k kernel runs, on tiles of so many 16-row blocks
   int split_spec;                  //    1: its workgroups ask for gate/up weights before the routing is known
   int split_down;                  //    waves that share a down task: 4 or 8
-  int split_self;                  //    every workgroup picks all tokens' winners for itself
   int dot16;                       // 1 (streaming variant, bf16): the logit chains run on the matrix core, 16 tokens x
                                    //    16 experts per workgroup, on the first workgroups before they take tickets;
                                    //    bf16 tiled variant: how it starts (see the launcher)

@@ -258,20 +258,21 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
   const int pull_from = (((lane & 15) << 2) | (lane >> 4)) << 2;
   const unsigned raised = post_number(ldc(&ctl->launches.posted));  // (the last workgroup out moves it on)
 
-  // ---- routing: logit chains on the first workgroups, then (batches of more than SPLIT_SELF_TOKENS) selections there,
-  // four tokens a wave. Smaller batches have every workgroup pick all winners for itself, below: that saves the
+  // ---- routing: logit chains on the first workgroups, then (batches that split_self leaves out) selections there,
+  // four or two tokens a wave. Smaller batches have every workgroup pick all winners for itself, below: that saves the
   // entries' way to memory and back and a wait in between (us, without / with: one token 41.8 / 40.2, T=11 123.2 /
   // 120.9, E=8, H=256 float32 T=16 24.4 / 23.1; but T=40 199.1 / 200.3, T=64 205.7 / 207.6, H=512, E=64 float32 T=64 44.1 /
   // 45.5).
-  const bool self = p.split_self != 0;
+  const bool self = split_self(E, K, T);
+  const int tok = select_tokens(E, K, T);
   if (b < n_rt) {
     if constexpr (DT::EPV == 8) {
       router_dot16_task(p, b / n_eg, b % n_eg, self ? b : -1, raised);
     } else {
       for (int q = b + n_rt * wave; q < n_dot; q += 8 * n_rt) router_dot_task<DT>(p, q / n_eg, q % n_eg, self ? q : -1, raised);
     }
-    for (int i = b + n_rt * wave; !self && i * SELECT_TOK < T; i += 8 * n_rt) {
-      if (router_select4_task(p, i, static_cast<unsigned>(n_eg), lds + wave * (ROUTER_LDS_FLOATS * 4)) == 0) break;
+    for (int i = b + n_rt * wave; !self && i * tok < T; i += 8 * n_rt) {
+      if (router_select_tokens_task(p, i, static_cast<unsigned>(n_eg), lds + wave * (ROUTER_LDS_FLOATS * 4)) == 0) break;
       raise_post(p, POST_ROUTE, i, raised);
     }
   }
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     }
 
     // ---- tables, by every workgroup for itself
-    ok = wait_posts(p, post_row(p, POST_ROUTE, b % POST_COPIES), self ? n_dot : (T + SELECT_TOK - 1) / SELECT_TOK, raised,
+    ok = wait_posts(p, post_row(p, POST_ROUTE, b % POST_COPIES), self ? n_dot : (T + tok - 1) / tok, raised,
                     &lds_flag[FLAG_ROUTED], &lds_poller[FLAG_ROUTED]);
     const int wact = (T + 63) >> 6;
     const int n = T * K;
@@ -341,8 +342,8 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
     if (self) {
       for (int e = tid; e < E; e += 512) lmask[e] = 0ull;
       lds_barrier();
-      for (int i = wave; ok && i * SELECT_TOK < T; i += 8) {
-        const int t0 = i * SELECT_TOK, nt = min(SELECT_TOK, T - t0), t = (lane >> 4) < nt ? t0 + (lane >> 4) : -1;
+      for (int i = wave; ok && i * tok < T; i += 8) {
+        const int t0 = i * tok, nt = min(tok, T - t0), row = lane * tok >> 6, t = row < nt ? t0 + row : -1;
         auto emit = [&](int tq, int s, int e, float w) {
           self_idx[tq * K + s] = e;
           self_w[tq * K + s] = w;
@@ -355,12 +356,16 @@ __global__ __launch_bounds__(512) __attribute__((disable_tail_calls)) void moe_s
         unsigned char* scratch = lds + SPLIT_SELECT_OFF + wave * SELECT_ROWS_BYTES;
         if (E <= 128) {
           unsigned val[8];
-          load_row_keys<8>(p, t0, nt, val);
-          router_select_rows<8>(K, t, val, scratch, emit);
-        } else {
+          load_row_keys<8, 16>(p, t0, nt, val);
+          router_select_rows<8, 16>(K, t, val, scratch, emit);
+        } else if (tok == 4) {
           unsigned val[16];
-          load_row_keys<16>(p, t0, nt, val);
-          router_select_rows<16>(K, t, val, scratch, emit);
+          load_row_keys<16, 16>(p, t0, nt, val);
+          router_select_rows<16, 16>(K, t, val, scratch, emit);
+        } else {
+          unsigned val[8];
+          load_row_keys<8, 32>(p, t0, nt, val);
+          router_select_rows<8, 32>(K, t, val, scratch, emit);
         }
       }
       lds_barrier();

@@ -2,7 +2,7 @@
 // more rows than a streaming tile shares its weights with.
 //
 // Two workgroups of 4 waves per CU draw task tickets. Stages as in the bf16 tiled kernel:
-//   router   8 tokens x 8 experts a wave (the streaming kernel's chains), then selections of four tokens a wave
+//   router   8 tokens x 8 experts a wave (the streaming kernel's chains), then selections of four or two tokens a wave
 //   scan, scatter
 //   gate/up  (row tile, 128 h columns), down (row tile, 256 output columns): up to 96 token rows x
 //            256 weight rows, k stepped by 32; a wave owns 64 weight rows x all token rows
@@ -477,14 +477,15 @@ __global__ __launch_bounds__(T_THREADS, 2) __attribute__((disable_tail_calls)) v
     router_dot_task<F32>(p, i / n_eg, i % n_eg);
     trace_task(p, lane0, i, 0, i, t0, t0);
   }
-  for (int i = me; i * SELECT_TOK < T; i += waves) {
+  const int tok = select_tokens(E, p.K, T);
+  for (int i = me; i * tok < T; i += waves) {
     const long long t0 = trace_clock(traced);
-    const int n = router_select4_task(p, i, static_cast<unsigned>(n_eg), reinterpret_cast<unsigned char*>(lds_dyn + wave * ROUTER_LDS_FLOATS));
+    const int n = router_select_tokens_task(p, i, static_cast<unsigned>(n_eg), reinterpret_cast<unsigned char*>(lds_dyn + wave * ROUTER_LDS_FLOATS));
     if (n == 0) break;
     unsigned old = 0;
     if (lane_id() == 0) old = add_relaxed(&ctl->router_done.v, static_cast<unsigned>(n));
     if (uni(static_cast<int>(old)) + n == T) broadcast_flag(p, FLAG_ROUTED);
-    trace_task(p, lane0, n_dot + i, 6, i * SELECT_TOK, t0, t0);
+    trace_task(p, lane0, n_dot + i, 6, i * tok, t0, t0);
   }
   long long t_fetch = trace_clock(traced);
   bool ok = wg_wait_flag(p, FLAG_ROUTED, &sh);

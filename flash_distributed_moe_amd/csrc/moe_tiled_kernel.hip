@@ -288,7 +288,7 @@ __device__ __noinline__ void tiled_router_task(ParamsRef pv, int blk) {
         val[j + 2] = v.z;
         val[j + 3] = v.w;
       }
-      router_select_rows<EPL>(p, t, val, lds_raw + wave * SELECT_ROWS_BYTES);
+      router_select_rows<EPL, 16>(p, t, val, lds_raw + wave * SELECT_ROWS_BYTES);
     };
     if (E <= 128) {
       select(std::integral_constant<int, 8>{});
@@ -1658,16 +1658,16 @@ __global__ __launch_bounds__(T_THREADS) __attribute__((disable_tail_calls)) void
         trace(i, 0, i, t0, t0);
       }
       const int sel_groups = min(n_dot, G);
-      const int i0 = b + sel_groups * wave;
+      const int i0 = b + sel_groups * wave, tok = select_tokens(p.E, p.K, Ti);
       // (the launcher takes this start while there are as many waves as selections, at least)
-      if (b < sel_groups && i0 * SELECT_TOK < Ti) {
+      if (b < sel_groups && i0 * tok < Ti) {
         const long long t0 = trace_clock(traced);
-        const int n = router_select4_task(p, i0, static_cast<unsigned>((p.E + 15) >> 4), lds_raw + wave * SELECT_ROWS_BYTES);
+        const int n = router_select_tokens_task(p, i0, static_cast<unsigned>((p.E + 15) >> 4), lds_raw + wave * SELECT_ROWS_BYTES);
         unsigned old = 0;
         if (lane_id() == 0) old = add_relaxed(&ctl->router_done.v, static_cast<unsigned>(n));
         // (n = 0: a wait that failed has raised an error bit, which every later wait sees)
         if (uni(static_cast<int>(old)) + n == Ti) broadcast_flag(p, FLAG_ROUTED);
-        trace_task(p, traced && lane_id() == 0, n_dot + i0, 6, i0 * SELECT_TOK, t0, t0);
+        trace_task(p, traced && lane_id() == 0, n_dot + i0, 6, i0 * tok, t0, t0);
       }
       t_perm0 = n_dot + WAVES * sel_groups;
     } else {

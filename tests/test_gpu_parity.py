@@ -345,7 +345,14 @@ def test_tiled_starts(T, H, E, k, start):
     (601, 128, 200, 17, "tokens"),    # ... of two slabs; the last of 9 tokens
     (509, 128, 200, 17, "chains"),    # selections spread over the workgroups, the last of one token
     (511, 256, 120, 17, "chains"),    # ... of three tokens
-    (32, 256, 200, 32, "split-k"),    # every workgroup picks the winners, four tokens to each of its waves
+    (407, 128, 200, 17, "chains"),    # ... of two tokens a wave, the last of one
+    (409, 128, 200, 17, "chains"),    # the first size of so many winners with four; the last of one token
+    (32, 256, 120, 32, "split-k"),    # every workgroup picks the winners, four tokens to each of its waves
+    (32, 256, 200, 1, "split-k"),     # ... of which each lane holds 16 experts
+    (16, 256, 256, 9, "split-k"),     # ... two tokens
+    (15, 512, 129, 32, "split-k"),    # ... the last wave one
+    (17, 256, 256, 9, "split-k"),     # the first size of more than 128 experts whose winners are picked once
+    (32, 256, 200, 32, "split-k"),
     (33, 256, 120, 17, "split-k"),    # the first size whose winners are picked once
     (1, 256, 97, 32, "split-k"),
 ])
@@ -368,10 +375,13 @@ def test_router_winners(T, H, E, k, start, admitted):
         case.run()
         routing = case.launcher.routing(T)
         if tiled:
-            assert tiled_start(case)[0] == start
+            got = tiled_start(case)
+            assert got[0] == start
+            if start == "chains":
+                assert got[2] == -(-T // (2 if E > 128 and T <= 24 * k else 4))
         hw = case.host_weights()
         idx, w = oracle.gate(inp["tokens"].float().cpu().numpy(), hw["gate"], k, bias=hw["bias"])
-        assert (idx < 0).any() == (admitted == "three")
+        assert (idx < 0).any() == (admitted == "three" and k > 3)
         assert np.array_equal(routing["topk_idx"], idx)
         np.testing.assert_allclose(routing["topk_w"], w, rtol=2e-6, atol=1e-7)  # as in GpuCase.check_routing
     finally:
