@@ -513,7 +513,14 @@ __global__ __launch_bounds__(T_THREADS, 2) __attribute__((disable_tail_calls)) v
   const unsigned n2_total = nm * nt2;
   const unsigned t_dyn0 = t_scatter0 + n_sc;
   const int home = xcc_id();
-  for (int hop = 0; ok && hop < 8; ++hop) {
+  // While neither projection has more tasks than there are CUs, only the first workgroup of each (b and b + G/2 share
+  // one) takes tasks. Whoever came first did before, and where both of a CU's had one they took 73 us instead of 59 (down) or
+  // 134 instead of 113 (gate/up), for which the launch waited (E=3, k=3, H=2048, I=1024, T=300: some 8 of 96 tasks).
+  // us, everybody / so: that layer 243 / 226, T=600 293 / 252; E=13, k=8 T=64 200 / 183; E=16, k=2, T=300 200 / 182; E=32, k=4, T=200 (256
+  // tasks each) 234 / 196; I=512: H=1024, E=16, T=2000 172 / 152, E=3, T=64 level. With more tasks than CUs a second workgroup is needed.
+  const unsigned half = static_cast<unsigned>(G) / 2u;
+  const bool takes = static_cast<unsigned>(b) < half || nm * nt1 > half || n2_total > half;
+  for (int hop = 0; ok && takes && hop < 8; ++hop) {
     const unsigned q = static_cast<unsigned>((home + hop) & 7);
     const unsigned lo = nm * q / 8u, hi = nm * (q + 1u) / 8u;
     const unsigned q1 = (hi - lo) * nt1, q2 = (hi - lo) * nt2;

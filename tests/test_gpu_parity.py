@@ -431,6 +431,30 @@ def test_tiled_float32(rows, H, I):
         case.close()
 
 
+@pytest.mark.parametrize("H,I,one_a_cu", [(512, 256, True), (512, 288, False), (576, 256, False)])
+def test_tiled_float32_one_workgroup_a_cu(H, I, one_a_cu):
+    """128 row tiles: with two tasks each in both projections there are as many as CUs, and the first workgroup of
+    each takes them; with three in either everybody draws."""
+    cfg = synth.MoeConfig("one_a_cu", 640, H, 128, 2, I, "f32")
+    print("tiled float32, tasks", H, I, flush=True)
+    case = GpuCase(cfg, seed=H + I, sched=_lib.SCHED_TILED)
+    try:
+        out = case.run()
+        case.check_routing(case.inp["tokens"], case.launcher.routing(640))
+        case.check_outputs(case.inp["tokens"], out, nthreads=4)
+        case.launcher.trace_enable(1 << 14)
+        assert torch.equal(case.run(), out)
+        rec = case.launcher.trace_read()
+        case.launcher.trace_enable(0)
+        for kind, tasks in ((3, 128 * -(-I // 128)), (4, 128 * -(-H // 256))):
+            at = rec[rec["kind"] == kind]
+            assert len(at) == tasks
+            if one_a_cu:
+                assert at["worker"].max() < torch.cuda.get_device_properties(0).multi_processor_count
+    finally:
+        case.close()
+
+
 def same_values(want, got, scale=None):
     """The same infinities and NaN, and finite values within the tolerance of float32 layers, each against
     the root mean square of its own token row (or of `scale`, a part of its columns)."""
